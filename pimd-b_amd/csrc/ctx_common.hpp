@@ -10,6 +10,7 @@
 
 #include "pimdb_gpu.h"
 #include "exchange.hpp"
+#include "exchange_wide.hpp"
 #include "forces.hpp"
 #include "observables.hpp"
 
@@ -188,7 +189,8 @@ inline ForceArgs make_force_args(const pimdb_params& p, const Derived& d) {
     return fa;
 }
 
-// LDS of k_exchange_recursions (1024 threads per direction).
+// LDS that one workgroup running a whole recursion would need (1024 threads
+// per direction): the size of its device-memory workspace.
 inline size_t rec_lds_bytes(int N, int D) { return sizeof(double) * rec_shared_doubles(N, D, 1024 / WAVE); }
 
 inline size_t device_lds_limit() {
@@ -201,6 +203,33 @@ inline size_t device_lds_limit() {
         if (!lim) lim = 65536;
     }
     return lim;
+}
+
+// Whether a ring's recursions run with one workgroup per block of targets
+// (k_exchange_wide: the ring staged in every workgroup's LDS); larger rings
+// take k_exchange_recursions_gws.
+inline bool exchange_wide(int N, int D) { return xw_lds_bytes(N, D) <= device_lds_limit(); }
+
+// Both recursions of one ring.  pub: xw_pub_words(N) words holding XW_EMPTY
+// (exchange_wide rings); ws: 2 rec_lds_bytes(N, D) bytes (the others).
+inline void launch_exchange_recursions(int D, int N, double bt, double k, int pbc, double L, const double* x1,
+                                       const double* xP, double* V, double* Vb, double* Shi, double* Slo,
+                                       unsigned long long* pub, double* ws, int* status, hipStream_t s) {
+    if (exchange_wide(N, D)) {
+        const dim3 grid(xw_grid(N)), blk(XW_THREADS);
+        const size_t lds = xw_lds_bytes(N, D);
+        switch (D) {
+        case 1: hipLaunchKernelGGL(k_exchange_wide<1>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
+        case 2: hipLaunchKernelGGL(k_exchange_wide<2>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
+        default: hipLaunchKernelGGL(k_exchange_wide<3>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
+        }
+        return;
+    }
+    switch (D) {
+    case 1: hipLaunchKernelGGL(k_exchange_recursions_gws<1>, dim3(2), dim3(1024), 0, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status, ws); break;
+    case 2: hipLaunchKernelGGL(k_exchange_recursions_gws<2>, dim3(2), dim3(1024), 0, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status, ws); break;
+    default: hipLaunchKernelGGL(k_exchange_recursions_gws<3>, dim3(2), dim3(1024), 0, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status, ws); break;
+    }
 }
 
 inline void launch_cycle_energies(int D, int N, const double* x1, const double* xP, double k, int pbc, double L,

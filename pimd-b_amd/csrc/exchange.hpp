@@ -533,20 +533,8 @@ __device__ __forceinline__ void exchange_recursions_on(double* base, int N, doub
     else exchange_recursion<1, D>(N, bt, r, V, Vb, status, sh, threadIdx.x, blockDim.x);
 }
 
-// Both recursions with the workspace in LDS (rec_shared_doubles doubles of
-// dynamic shared memory).
-template <int D>
-static __global__ void __launch_bounds__(1024) k_exchange_recursions(int N, double bt, double k, int pbc, double L,
-                                                                     const double* __restrict__ x1,
-                                                                     const double* __restrict__ xP,
-                                                                     double* __restrict__ V, double* __restrict__ Vb,
-                                                                     double* __restrict__ Shi, double* __restrict__ Slo,
-                                                                     int* __restrict__ status) {
-    extern __shared__ double smem[];
-    exchange_recursions_on<D>(smem, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status);
-}
-
-// The same for rings whose workspace exceeds a workgroup's LDS: block b's
+// The recursions of rings that exceed a workgroup's LDS (smaller ones:
+// exchange_wide.hpp): block b's
 // workspace at ws + b rec_shared_doubles(N, D, waves), in device memory.  The
 // workspace is only touched between workgroup barriers or by the lane that
 // wrote it (the sequential passes read back their own stores), so the
@@ -651,7 +639,7 @@ __device__ __forceinline__ void exterior_force(int which, int l, int N, int lane
 
 // Adds the exterior spring forces into f for beads 1 and P:
 // f = F_exchange + f_phys (simulation.cpp:363-373: spring + physical).
-// Shi/Slo: the ring's prefix sums from k_exchange_recursions.
+// Shi/Slo: the ring's prefix sums from the recursions' kernel.
 template <int D>
 static __global__ void __launch_bounds__(256) k_exchange_forces(int N, int P, double bt, double k, int pbc, double L,
                                                          const double* __restrict__ Shi,

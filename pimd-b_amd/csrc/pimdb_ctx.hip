@@ -4,11 +4,11 @@
 // One MD step (Simulation::run body, src/simulation.cpp:246-259) is
 //   K1 k_momenta      O-step (+ deferred zeroMomentum of the previous step)
 //   K2 k_kick_drift   zeroMomentum, B, A          (or k_nm_propagate)
-//   K3 forces         s1: k_exchange_recursions (cycle energies on the fly)
+//   K3 forces         s1: k_exchange_wide (cycle energies on the fly)
 //                     s0: k_bead_forces (all beads, all pairs)
 //                     s0 after join: k_exchange_forces (beads 1 and P)
 //   K4 k_momenta      B, O-step, partial sums for zeroMomentum
-// The exchange chain (one long-latency workgroup) overlaps the pair forces
+// The exchange chain (few long-latency workgroups) overlaps the pair forces
 // on a second stream of default priority.
 #include <hip/hip_runtime.h>
 
@@ -39,6 +39,7 @@ struct pimdb_ctx {
     double *x = nullptr, *p = nullptr, *f = nullptr, *fext = nullptr;
     double *E = nullptr, *ET = nullptr, *V = nullptr, *Vb = nullptr, *prob = nullptr, *fex = nullptr;
     double *Shi = nullptr, *Slo = nullptr;   // link prefix sums of the ring (exterior forces)
+    unsigned long long* pub = nullptr;   // the recursions' published values (k_exchange_wide)
     double* xws = nullptr;   // the recursions' workspace in device memory, when it exceeds LDS
     double *C = nullptr, *CT = nullptr, *rot = nullptr, *com0 = nullptr, *com1 = nullptr;
     double *noise = nullptr, *obs = nullptr;
@@ -103,25 +104,11 @@ static void launch_bead_forces(pimdb_ctx* ctx, hipStream_t s) {
 }
 
 // Both recursions (cycle energies recomputed from the ring's prefix sums,
-// which block 0 also leaves in Shi/Slo for the exterior forces).
+// which are also left in Shi/Slo for the exterior forces).
 static void launch_exchange_forward(pimdb_ctx* ctx, hipStream_t s) {
-    const int N = ctx->N, P = ctx->P, D = ctx->D;
-    const double* x1 = ctx->x;
-    const double* xP = ctx->x + (size_t)(P - 1) * D * N;
-    if (ctx->xws) {   // a ring too large for the LDS of one workgroup
-        switch (D) {
-        case 1: hipLaunchKernelGGL(k_exchange_recursions_gws<1>, dim3(2), dim3(1024), 0, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status, ctx->xws); break;
-        case 2: hipLaunchKernelGGL(k_exchange_recursions_gws<2>, dim3(2), dim3(1024), 0, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status, ctx->xws); break;
-        default: hipLaunchKernelGGL(k_exchange_recursions_gws<3>, dim3(2), dim3(1024), 0, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status, ctx->xws); break;
-        }
-        return;
-    }
-    const size_t lds = rec_lds_bytes(N, D);
-    switch (D) {
-    case 1: hipLaunchKernelGGL(k_exchange_recursions<1>, dim3(2), dim3(1024), lds, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status); break;
-    case 2: hipLaunchKernelGGL(k_exchange_recursions<2>, dim3(2), dim3(1024), lds, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status); break;
-    default: hipLaunchKernelGGL(k_exchange_recursions<3>, dim3(2), dim3(1024), lds, s, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, x1, xP, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo, ctx->status); break;
-    }
+    launch_exchange_recursions(ctx->D, ctx->N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x,
+                               ctx->x + (size_t)(ctx->P - 1) * ctx->D * ctx->N, ctx->V, ctx->Vb, ctx->Shi, ctx->Slo,
+                               ctx->pub, ctx->xws, ctx->status, s);
 }
 
 // The stored triangle E (and its row-major copy), for the outputs and
@@ -374,10 +361,17 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     alloc(&ctx->Vb, sizeof(double) * (N + 1));
     alloc(&ctx->Shi, sizeof(double) * N);
     alloc(&ctx->Slo, sizeof(double) * N);
-    // both recursions' workspaces in device memory when one exceeds the LDS
-    // of a workgroup (the same kernel body; slower, no size limit of its own)
-    if (ctx->dv.bosonic && prm->exchange_algo != PIMDB_EXCHANGE_FACTORIAL && rec_lds_bytes(N, D) > device_lds_limit())
-        alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
+    if (ctx->dv.bosonic && prm->exchange_algo != PIMDB_EXCHANGE_FACTORIAL) {
+        // the recursions' published values, or both workspaces in device
+        // memory when the ring exceeds the LDS of a workgroup
+        if (exchange_wide(N, D)) {
+            alloc(&ctx->pub, 8 * xw_pub_words(N));
+            if (!rc && hipMemset(ctx->pub, 0xFF, 8 * xw_pub_words(N)) != hipSuccess)
+                rc = ctx->fail(PIMDB_E_HIP, "device initialisation failed");
+        } else {
+            alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
+        }
+    }
     alloc(&ctx->prob, sizeof(double) * (size_t)N * N);
     alloc(&ctx->fex, sizeof(double) * 2 * (size_t)D * N);
     alloc(&ctx->C, sizeof(double) * (size_t)P * P);
@@ -450,6 +444,7 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
                       ctx->nh.eta, ctx->nh.eta_dot, ctx->nh.eta_dot_dot, ctx->modes, ctx->xws};
     for (double* b : bufs)
         if (b) (void)hipFree(b);
+    if (ctx->pub) (void)hipFree(ctx->pub);
     if (ctx->status) (void)hipFree(ctx->status);
     if (ctx->ctr) (void)hipFree(ctx->ctr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);

@@ -20,10 +20,12 @@ using namespace pimdb;
 
 namespace {
 
-// Largest ring: V and Vb (N+1 each), Shi and Slo (N each), then the flag.
+// Largest ring: V and Vb (N+1 each), Shi and Slo (N each), then the flag and
+// the recursions' published values.
 constexpr int NOALLOC_MAX_N = 2048;
 constexpr size_t NOALLOC_FLAG = 4 * (size_t)(NOALLOC_MAX_N + 1);
-constexpr size_t NOALLOC_DOUBLES = NOALLOC_FLAG + 1;
+constexpr size_t NOALLOC_PUB = NOALLOC_FLAG + 1;
+constexpr size_t NOALLOC_DOUBLES = NOALLOC_PUB + 2 * (size_t)(NOALLOC_MAX_N + 1);
 
 __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 
@@ -31,10 +33,11 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex scratch_mu;
 double* scratch_ptr[NOALLOC_MAX_DEVICES] = {};
 
-// The flag starts every call at zero (a fill kernel, so that the call can be
-// recorded into a graph).
-__global__ void k_clear_flag(int* flag) {
+// The flag starts every call at zero and the published values empty (a fill
+// kernel, so that the call can be recorded into a graph).
+__global__ void k_clear_flag(int* flag, unsigned long long* pub, int words) {
     if (threadIdx.x == 0) *flag = 0;
+    for (int i = threadIdx.x; i < words; i += blockDim.x) pub[i] = XW_EMPTY;
 }
 
 // Device address of this device's scratch, looked up on its first use.
@@ -63,9 +66,8 @@ int scratch_base(double** out) {
 
 template <int D>
 void launch(int N, double bt, double k, int pbc, double L, const double* x1, const double* xP, double* V,
-            double* Vb, double* Shi, double* Slo, int* flag, double* grad, hipStream_t s) {
-    hipLaunchKernelGGL(k_exchange_recursions<D>, dim3(2), dim3(1024), rec_lds_bytes(N, D), s, N, bt, k, pbc, L, x1,
-                       xP, V, Vb, Shi, Slo, flag);
+            double* Vb, double* Shi, double* Slo, unsigned long long* pub, int* flag, double* grad, hipStream_t s) {
+    launch_exchange_recursions(D, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, nullptr, flag, s);
     if (grad)
         hipLaunchKernelGGL(k_exchange_vb_grad<D>, dim3((2 * N + 3) / 4), dim3(256), 0, s, N, bt, k, pbc, L, Shi,
                            Slo, V, Vb, x1, xP, grad);
@@ -99,12 +101,13 @@ extern "C" int pimdb_exchange_vb_grad_noalloc(int natoms, int ndim, double beta_
     double* Shi = Vb + (N + 1);
     double* Slo = Shi + N;
     int* flag = (int*)(base + NOALLOC_FLAG);
+    unsigned long long* pub = (unsigned long long*)(base + NOALLOC_PUB);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(64), 0, s, flag);
+    hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1024), 0, s, flag, pub, (int)xw_pub_words(N));
     switch (ndim) {
-    case 1: launch<1>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, flag, grad, s); break;
-    case 2: launch<2>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, flag, grad, s); break;
-    default: launch<3>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, flag, grad, s); break;
+    case 1: launch<1>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, pub, flag, grad, s); break;
+    case 2: launch<2>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, pub, flag, grad, s); break;
+    default: launch<3>(N, beta_t, spring_k, pbc, size, x1, xP, V, Vb, Shi, Slo, pub, flag, grad, s); break;
     }
     if (hipGetLastError() != hipSuccess) return PIMDB_E_HIP;
     if (VB && hipMemcpyAsync(VB, V + N, sizeof(double), hipMemcpyDeviceToDevice, s) != hipSuccess) return PIMDB_E_HIP;
