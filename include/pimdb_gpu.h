@@ -140,9 +140,11 @@ int pimdb_observables(pimdb_ctx* ctx, double* out);
  * PIMDB_E_STATE for a distinguishable system. */
 int pimdb_exchange_estimators(pimdb_ctx* ctx, double* prim, double* prob_distinct, double* prob_longest);
 
-/* Captures one MD step (device noise) in a hipGraph; later pimdb_step calls
- * with host_noise == NULL replay it.  No reference counterpart (the
- * reference has no graph capture). */
+/* Prepares the device-noise MD step for repeated use: a step that runs on two
+ * streams (rings beyond a workgroup's LDS) is captured in a hipGraph that
+ * later pimdb_step calls with host_noise == NULL replay; other steps are
+ * launched directly, which is faster, and need no preparation.  No reference
+ * counterpart (the reference has no graph capture). */
 int pimdb_graph_capture(pimdb_ctx* ctx);
 
 /* Average device time (ms) of `reps` launches of the physical-force kernel

@@ -360,6 +360,24 @@ __device__ __forceinline__ double wave_sum(double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
     return v;
 }
+// A double moved across lanes by DPP; lanes without a source get 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// Inclusive sums over the lanes of a wave by DPP (row_shr 1, 2, 4, 8, then the
+// last lane of rows 0 and 2 into the next row and of row 1 into rows 2 and 3).
+__device__ __forceinline__ double wave_scan(double v) {
+    v += dpp_or_zero<0x111, 0xF>(v);
+    v += dpp_or_zero<0x112, 0xF>(v);
+    v += dpp_or_zero<0x114, 0xF>(v);
+    v += dpp_or_zero<0x118, 0xF>(v);
+    v += dpp_or_zero<0x142, 0xA>(v);
+    v += dpp_or_zero<0x143, 0xC>(v);
+    return v;
+}
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, WAVE));
@@ -376,6 +394,10 @@ __device__ __forceinline__ double wave_bcast_uniform(double v, int src) {
     const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), src);
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
+
+// The wave's sum in every lane, without the LDS crossbar that wave_sum's
+// shuffles go through (a third of its latency).
+__device__ __forceinline__ double wave_total(double v) { return wave_bcast_uniform(wave_scan(v), WAVE - 1); }
 
 // ---- Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11) ----
 struct U4 { uint32_t x, y, z, w; };

@@ -620,14 +620,14 @@ __device__ __forceinline__ void exterior_force(int which, int l, int N, int lane
                                             : ring_ecyc<D>(r, d, r.Shi[j], r.Slo[j], shl, sll);
                 arg = V[col] + e + Vb[row + 1] - VN;
             }
-            const double ex = exp(-bt * arg);
+            const double ex = exp_minimax(-bt * arg);
             pr = link ? 1.0 - ex : 1.0 / (row + 1) * ex;
         }
 #pragma unroll
         for (int a = 0; a < D; ++a) S[a] += pr * d[a];
     }
 #pragma unroll
-    for (int a = 0; a < D; ++a) S[a] = wave_sum(S[a]);
+    for (int a = 0; a < D; ++a) S[a] = wave_total(S[a]);
     const double* link = which == 0 ? x2 : xPm1;
 #pragma unroll
     for (int a = 0; a < D; ++a) {

@@ -90,19 +90,11 @@ __device__ __forceinline__ XwShared xw_carve(double* p, int N, int D) {
     return s;
 }
 
-// A double moved across lanes by DPP; lanes without a source get 0.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_or_zero(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
 template <int CTRL, int ROWS>
 __device__ __forceinline__ DD dd_scan_step(DD v) {
     return dd_add(DD{dpp_or_zero<CTRL, ROWS>(v.hi), dpp_or_zero<CTRL, ROWS>(v.lo)}, v);
 }
-// Inclusive sums over the lanes of a wave (row_shr 1, 2, 4, 8, then the last
-// lane of row 0 / 2 into the next row and of row 1 into rows 2 and 3).
+// Inclusive sums over the lanes of a wave (wave_scan's steps).
 __device__ __forceinline__ DD dd_wave_scan(DD v) {
     v = dd_scan_step<0x111, 0xF>(v);
     v = dd_scan_step<0x112, 0xF>(v);
@@ -110,15 +102,6 @@ __device__ __forceinline__ DD dd_wave_scan(DD v) {
     v = dd_scan_step<0x118, 0xF>(v);
     v = dd_scan_step<0x142, 0xA>(v);
     v = dd_scan_step<0x143, 0xC>(v);
-    return v;
-}
-__device__ __forceinline__ double wave_scan(double v) {
-    v += dpp_or_zero<0x111, 0xF>(v);
-    v += dpp_or_zero<0x112, 0xF>(v);
-    v += dpp_or_zero<0x114, 0xF>(v);
-    v += dpp_or_zero<0x118, 0xF>(v);
-    v += dpp_or_zero<0x142, 0xA>(v);
-    v += dpp_or_zero<0x143, 0xC>(v);
     return v;
 }
 

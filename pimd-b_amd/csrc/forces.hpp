@@ -31,16 +31,19 @@ struct ForceArgs {
 constexpr int FORCE_TILE = 64;
 constexpr int FORCE_WAVES = 16;
 
+// The forces of particles tile*64 .. +63 of bead b by a workgroup of 1024
+// threads.  smem: the staged slice (GX: none) and the reduction.  Exchange
+// beads get the physical forces alone.  fpart (may be null): the tile's sums of
+// the external forces per axis at fpart[(b nt + tile) D + a], nt tiles per bead.
 // GX: the slice is read in place from device memory instead of being staged
 // in LDS (slices larger than a workgroup's LDS); the LDS then holds only the
 // reduction.
 template <int D, int KIND, bool GX = false>
-static __global__ void __launch_bounds__(FORCE_TILE * FORCE_WAVES)
-k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f, double* __restrict__ fext) {
-    extern __shared__ double smem[];
+__device__ __forceinline__ void bead_forces_tile(const ForceArgs& fa, int b, int tile, const double* __restrict__ x,
+                                                 double* __restrict__ f, double* __restrict__ fext,
+                                                 double* __restrict__ fpart, double* smem) {
     double* red = smem + (GX ? 0 : (size_t)D * fa.N);   // [FORCE_WAVES-1][D][FORCE_TILE]
     const int N = fa.N, P = fa.P;
-    const int b = blockIdx.y;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     const size_t bs = (size_t)D * N;
     const double* xb = x + bs * b;
@@ -48,12 +51,12 @@ k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f
     if constexpr (GX) {
         sx = xb;
     } else {
-        for (int e = tid; e < D * N; e += blockDim.x) smem[e] = xb[e];
+        for (int e = tid; e < D * N; e += FORCE_TILE * FORCE_WAVES) smem[e] = xb[e];
         __syncthreads();
         sx = smem;
     }
 
-    const int i = blockIdx.x * FORCE_TILE + lane;
+    const int i = tile * FORCE_TILE + lane;
     const bool pbc = fa.pbc != 0;
     double acc[D];
 #pragma unroll
@@ -91,35 +94,55 @@ k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f
         }
         __syncthreads();
     }
-    if (wave != 0 || i >= N) return;
-    if constexpr (KIND != POT_FREE) {
-        for (int w = 1; w < FORCE_WAVES; ++w) {
+    if (wave != 0) return;
+    double fe[D];
 #pragma unroll
-            for (int a = 0; a < D; ++a) acc[a] += red[((w - 1) * D + a) * FORCE_TILE + lane];
+    for (int a = 0; a < D; ++a) fe[a] = 0.0;
+    if (i < N) {
+        if constexpr (KIND != POT_FREE) {
+            for (int w = 1; w < FORCE_WAVES; ++w) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) acc[a] += red[((w - 1) * D + a) * FORCE_TILE + lane];
+            }
+        }
+        const bool exchange_bead = fa.bosonic && (b == 0 || b == P - 1);
+        const double* xprev = x + bs * ((b - 1 + P) % P);
+        const double* xnext = x + bs * ((b + 1) % P);
+        double xv[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) xv[a] = sx[a * N + i];
+        ext_force<D>(fa.ext, xv, fe);
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const size_t idx = bs * b + (size_t)a * N + i;
+            const double xi = xv[a];
+            const double phys = fe[a] + acc[a];
+            if (fext) fext[idx] = phys;
+            double spring = 0.0;
+            if (!exchange_bead) {
+                const double dp = disp(xi, xprev[(size_t)a * N + i], pbc, fa.L);
+                const double dn = disp(xi, xnext[(size_t)a * N + i], pbc, fa.L);
+                spring = fa.k_spring * (dp + dn);
+            }
+            // exchange beads get their spring part added later
+            f[idx] = exchange_bead ? phys : spring + phys;
         }
     }
-    const bool exchange_bead = fa.bosonic && (b == 0 || b == P - 1);
-    const double* xprev = x + bs * ((b - 1 + P) % P);
-    const double* xnext = x + bs * ((b + 1) % P);
-    double xv[D], fe[D];
+    if (fpart) {
+        const int nt = (N + FORCE_TILE - 1) / FORCE_TILE;
 #pragma unroll
-    for (int a = 0; a < D; ++a) xv[a] = sx[a * N + i];
-    ext_force<D>(fa.ext, xv, fe);
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        const size_t idx = bs * b + (size_t)a * N + i;
-        const double xi = xv[a];
-        const double phys = fe[a] + acc[a];
-        if (fext) fext[idx] = phys;
-        double spring = 0.0;
-        if (!exchange_bead) {
-            const double dp = disp(xi, xprev[(size_t)a * N + i], pbc, fa.L);
-            const double dn = disp(xi, xnext[(size_t)a * N + i], pbc, fa.L);
-            spring = fa.k_spring * (dp + dn);
+        for (int a = 0; a < D; ++a) {
+            const double s = wave_total(fe[a]);
+            if (lane == 0) fpart[((size_t)b * nt + tile) * D + a] = s;
         }
-        // exchange beads get their spring part added by k_exchange_forces
-        f[idx] = exchange_bead ? phys : spring + phys;
     }
+}
+
+template <int D, int KIND, bool GX = false>
+static __global__ void __launch_bounds__(FORCE_TILE * FORCE_WAVES)
+k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f, double* __restrict__ fext) {
+    extern __shared__ double smem[];
+    bead_forces_tile<D, KIND, GX>(fa, blockIdx.y, blockIdx.x, x, f, fext, nullptr, smem);
 }
 
 // Pair and external potential energies and virial per bead, for the energy

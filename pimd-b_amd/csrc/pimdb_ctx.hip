@@ -4,12 +4,13 @@
 // One MD step (Simulation::run body, src/simulation.cpp:246-259) is
 //   K1 k_momenta      O-step (+ deferred zeroMomentum of the previous step)
 //   K2 k_kick_drift   zeroMomentum, B, A          (or k_nm_propagate)
-//   K3 forces         s1: k_exchange_wide (cycle energies on the fly)
-//                     s0: k_bead_forces (all beads, all pairs)
-//                     s0 after join: k_exchange_forces (beads 1 and P)
+//   K3 k_step_forces  exchange recursions beside the bead forces, then
+//                     k_exchange_forces (beads 1 and P)
 //   K4 k_momenta      B, O-step, partial sums for zeroMomentum
-// The exchange chain (few long-latency workgroups) overlaps the pair forces
-// on a second stream of default priority.
+// and within a run of device-noise Langevin (or NVE) steps with the Cartesian
+// propagator K4, K1 and K2 are one k_step_integrate (steps.hpp).  Rings and
+// slices beyond a workgroup's LDS take the recursions and the bead forces as
+// two kernels on two streams.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +27,7 @@
 #include "nose_hoover.hpp"
 #include "integrator.hpp"
 #include "observables.hpp"
+#include "steps.hpp"
 
 using namespace pimdb;
 
@@ -46,6 +48,9 @@ struct pimdb_ctx {
     size_t noise_cap = 0;
     int* status = nullptr;
     unsigned long long* ctr = nullptr;
+    bool merged = false;           // recursions and bead forces in one k_step_forces
+    bool split = false;            // consecutive steps by k_step_forces and k_step_integrate
+    double *xc = nullptr, *H = nullptr, *fpart = nullptr, *hpart = nullptr;   // their workspace (StepArgs)
     int tc = 1, ntiles = 1;
     int ncom = 1;                  // rows of the partial momentum sums (com0 / com1)
     NhArgs nh{};                   // Nose-Hoover chains (thermostat >= 2)
@@ -160,9 +165,78 @@ static void launch_factorial(pimdb_ctx* ctx, hipStream_t s, double* f, double* f
     }
 }
 
+static StepArgs step_args(pimdb_ctx* ctx, bool noise) {
+    StepArgs a{};
+    a.fa = make_force_args(ctx->prm, ctx->dv);
+    a.bt = ctx->dv.bt;
+    const int N = ctx->N, P = ctx->P, D = ctx->D;
+    a.nx = ctx->dv.bosonic ? xw_grid(N) : 0;
+    a.nf = P * ((N + FORCE_TILE - 1) / FORCE_TILE);
+    a.thermostat = ctx->prm.thermostat;
+    a.nm = ctx->prm.nmthermostat;
+    a.fixcom = ctx->prm.fixcom;
+    a.nn = noise && (a.thermostat || a.fixcom) ? D * step_noise_tiles(N) : 0;
+    a.x = ctx->x; a.p = ctx->p; a.f = ctx->f;
+    a.fext = ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr;
+    a.V = ctx->V; a.Vb = ctx->Vb; a.Shi = ctx->Shi; a.Slo = ctx->Slo; a.xc = ctx->xc;
+    a.pub = ctx->pub; a.status = ctx->status;
+    a.c1 = a.thermostat ? ctx->dv.c1 : 1.0;
+    a.c2 = ctx->dv.c2;
+    a.half_dt = 0.5 * ctx->prm.dt;
+    a.dt_m = ctx->prm.dt / ctx->prm.mass;
+    a.CTt = ctx->CT;
+    a.H = ctx->H; a.hpart = ctx->hpart;
+    a.fpart = ctx->prm.ext_kind != PIMDB_POT_FREE && a.fixcom ? ctx->fpart : nullptr;
+    a.ctr = ctx->ctr;
+    a.seed = ctx->prm.seed;
+    return a;
+}
+
+static size_t tile_lds_bytes(int N, int D) {
+    return sizeof(double) * ((size_t)D * N + (size_t)(FORCE_WAVES - 1) * D * FORCE_TILE);
+}
+
+template <int D>
+static void launch_step_forces_d(pimdb_ctx* ctx, const StepArgs& a, hipStream_t s) {
+    size_t lds = tile_lds_bytes(ctx->N, D);
+    if (a.nx) lds = std::max(lds, xw_lds_bytes(ctx->N, D));
+    if (a.nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(ctx->P, a.thermostat && a.nm));
+    const dim3 grid(a.nx + a.nf + a.nn), blk(XW_THREADS);
+    switch (ctx->prm.int_kind) {
+    case POT_HARMONIC: hipLaunchKernelGGL((k_step_forces<D, POT_HARMONIC>), grid, blk, lds, s, a); break;
+    case POT_DIPOLE: hipLaunchKernelGGL((k_step_forces<D, POT_DIPOLE>), grid, blk, lds, s, a); break;
+    case POT_AZIZ: hipLaunchKernelGGL((k_step_forces<D, POT_AZIZ>), grid, blk, lds, s, a); break;
+    default: hipLaunchKernelGGL((k_step_forces<D, POT_FREE>), grid, blk, lds, s, a); break;
+    }
+}
+
+// Recursions, bead forces and (noise) the next integration's noise, all but
+// the exterior forces of beads 1 and P.
+static void launch_step_forces(pimdb_ctx* ctx, bool noise) {
+    const StepArgs a = step_args(ctx, noise);
+    switch (ctx->D) {
+    case 1: launch_step_forces_d<1>(ctx, a, ctx->s0); break;
+    case 2: launch_step_forces_d<2>(ctx, a, ctx->s0); break;
+    default: launch_step_forces_d<3>(ctx, a, ctx->s0); break;
+    }
+}
+
+static void launch_step_integrate(pimdb_ctx* ctx) {
+    const StepArgs a = step_args(ctx, true);
+    const dim3 grid((unsigned)(step_exterior_groups(a.fa) + (step_inner_elements(a.fa, ctx->D) + 255) / 256));
+    switch (ctx->D) {
+    case 1: hipLaunchKernelGGL(k_step_integrate<1>, grid, dim3(256), 0, ctx->s0, a); break;
+    case 2: hipLaunchKernelGGL(k_step_integrate<2>, grid, dim3(256), 0, ctx->s0, a); break;
+    default: hipLaunchKernelGGL(k_step_integrate<3>, grid, dim3(256), 0, ctx->s0, a); break;
+    }
+}
+
 // Forces of every bead (updateForces on all ranks); f and (NM propagator) fext.
 static int enqueue_forces(pimdb_ctx* ctx) {
-    if (factorial(ctx)) {
+    if (ctx->merged) {
+        launch_step_forces(ctx, false);
+        if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
+    } else if (factorial(ctx)) {
         launch_bead_forces(ctx, ctx->s0);
         launch_factorial(ctx, ctx->s0, ctx->f, nullptr, nullptr, nullptr);
     } else if (ctx->dv.bosonic) {
@@ -236,7 +310,8 @@ static void enqueue_nh_ostep(pimdb_ctx* ctx, const double* com_in, const double*
     hipLaunchKernelGGL(k_momenta, tgrid, dim3(256), momenta_lds(ctx), ctx->s0, m, ctx->p);
 }
 
-static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* noise1) {
+// Up to the drift: K1 and K2.
+static void enqueue_open(pimdb_ctx* ctx, const double* noise0) {
     const bool fixcom = ctx->prm.fixcom != 0;
     const int N = ctx->N, P = ctx->P, D = ctx->D;
     dim3 tgrid(ctx->ntiles, D);
@@ -269,10 +344,12 @@ static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* nois
         hipLaunchKernelGGL(k_kick_drift, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, d, ctx->x,
                            ctx->p, ctx->f);
     }
-    // K3: forces
-    int rc = enqueue_forces(ctx);
-    if (rc) return rc;
-    // K4: B + O-step + partial COM sums
+}
+
+// The closing half: K4 (B + O-step + partial COM sums).
+static void enqueue_close(pimdb_ctx* ctx, const double* noise1) {
+    const bool fixcom = ctx->prm.fixcom != 0;
+    dim3 tgrid(ctx->ntiles, ctx->D);
     const double* kick = ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : ctx->f;
     if (ctx->prm.thermostat >= PIMDB_THERMO_NOSE_HOOVER) {
         enqueue_nh_ostep(ctx, nullptr, kick, fixcom ? ctx->com1 : nullptr);
@@ -282,6 +359,39 @@ static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* nois
         m2.com_out = fixcom ? ctx->com1 : nullptr;
         hipLaunchKernelGGL(k_momenta, tgrid, dim3(256), momenta_lds(ctx), ctx->s0, m2, ctx->p);
     }
+}
+
+// One OBABO step; noise0/noise1: device noise of the two O-steps or null.
+static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* noise1) {
+    enqueue_open(ctx, noise0);
+    const int rc = enqueue_forces(ctx);
+    if (rc) return rc;
+    enqueue_close(ctx, noise1);
+    CK(hipGetLastError());
+    return PIMDB_OK;
+}
+
+// nsteps device-noise steps.
+static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
+    if (!ctx->split || nsteps < 2) {
+        for (int s = 0; s < nsteps; ++s) {
+            if (ctx->gexec) {
+                CK(hipGraphLaunch(ctx->gexec, ctx->s0));
+            } else {
+                const int rc = enqueue_step(ctx, nullptr, nullptr);
+                if (rc) return rc;
+            }
+        }
+        return PIMDB_OK;
+    }
+    enqueue_open(ctx, nullptr);
+    launch_step_forces(ctx, true);
+    for (int s = 1; s < nsteps; ++s) {
+        launch_step_integrate(ctx);
+        launch_step_forces(ctx, s + 1 < nsteps);
+    }
+    if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
+    enqueue_close(ctx, nullptr);
     CK(hipGetLastError());
     return PIMDB_OK;
 }
@@ -372,6 +482,16 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
             alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
         }
     }
+    const bool slice_fits = tile_lds_bytes(N, D) <= device_lds_limit();
+    ctx->merged = slice_fits && (!ctx->dv.bosonic || ctx->pub);
+    ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN && prm->propagator == PIMDB_PROP_CARTESIAN &&
+                 (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat || P <= STEP_NM_MAXP);
+    if (ctx->merged && ctx->dv.bosonic) alloc(&ctx->xc, sizeof(double) * 4 * (size_t)D * N);
+    if (ctx->split) {
+        alloc(&ctx->H, sizeof(double) * ctx->nbd);
+        alloc(&ctx->fpart, sizeof(double) * D * (size_t)P * ((N + FORCE_TILE - 1) / FORCE_TILE));
+        alloc(&ctx->hpart, sizeof(double) * D * (size_t)step_noise_tiles(N));
+    }
     alloc(&ctx->prob, sizeof(double) * (size_t)N * N);
     alloc(&ctx->fex, sizeof(double) * 2 * (size_t)D * N);
     alloc(&ctx->C, sizeof(double) * (size_t)P * P);
@@ -441,7 +561,8 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
     double* bufs[] = {ctx->x, ctx->p, ctx->f, ctx->fext, ctx->E, ctx->ET, ctx->V, ctx->Vb, ctx->prob, ctx->fex,
                       ctx->C, ctx->CT, ctx->rot, ctx->com0, ctx->com1, ctx->noise, ctx->obs, ctx->Shi, ctx->Slo,
-                      ctx->nh.eta, ctx->nh.eta_dot, ctx->nh.eta_dot_dot, ctx->modes, ctx->xws};
+                      ctx->nh.eta, ctx->nh.eta_dot, ctx->nh.eta_dot_dot, ctx->modes, ctx->xws, ctx->xc, ctx->H,
+                      ctx->fpart, ctx->hpart};
     for (double* b : bufs)
         if (b) (void)hipFree(b);
     if (ctx->pub) (void)hipFree(ctx->pub);
@@ -580,14 +701,8 @@ int pimdb_step(pimdb_ctx* ctx, int nsteps, const double* host_noise) {
             }
         }
     } else {
-        for (int s = 0; s < nsteps; ++s) {
-            if (ctx->gexec) {
-                CK(hipGraphLaunch(ctx->gexec, ctx->s0));
-            } else {
-                int rc = enqueue_step(ctx, nullptr, nullptr);
-                if (rc) return rc;
-            }
-        }
+        const int rc = enqueue_steps(ctx, nsteps);
+        if (rc) return rc;
     }
     int rc = finish_steps(ctx);
     if (rc) return rc;
@@ -596,7 +711,10 @@ int pimdb_step(pimdb_ctx* ctx, int nsteps, const double* host_noise) {
 
 int pimdb_graph_capture(pimdb_ctx* ctx) {
     if (!ctx) return PIMDB_E_ARG;
-    if (ctx->gexec) return PIMDB_OK;
+    // A step of one stream is launched faster than its graph is replayed (N=256,
+    // P=64 helium 36.9 against 41.1 us a step, N=8 Nose-Hoover 29.3 against
+    // 31.9): only the two-stream steps are captured.
+    if (ctx->gexec || ctx->merged || !ctx->dv.bosonic || factorial(ctx)) return PIMDB_OK;
     CK(hipStreamSynchronize(ctx->s0));
     CK(hipStreamBeginCapture(ctx->s0, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_step(ctx, nullptr, nullptr);
@@ -747,8 +865,12 @@ int pimdb_time_kernels(pimdb_ctx* ctx, int reps, double* ms_forces, double* ms_e
     if (ms_step) {
         // whole steps (device noise), as the benchmark replays them; this
         // advances the state by 2 * reps steps
-        rc = time_captured(ctx, reps, [&]() { return enqueue_step(ctx, nullptr, nullptr); }, ms_step);
+        hipGraphExec_t held = ctx->gexec;   // (a graph is not launched into a capture)
+        ctx->gexec = nullptr;
+        rc = time_captured(ctx, 1, [&]() { return enqueue_steps(ctx, reps); }, ms_step);
+        ctx->gexec = held;
         if (rc) return rc;
+        *ms_step /= reps;
         rc = finish_steps(ctx);
         if (rc) return rc;
     }
