@@ -238,16 +238,25 @@ int pimdb_batch_get_state(pimdb_batch* batch, int rep, double* x, double* p, dou
 int pimdb_batch_forces(pimdb_batch* batch);
 /* nsteps MD steps of every replica (pimdb_step with device noise for each). */
 int pimdb_batch_step(pimdb_batch* batch, int nsteps);
-/* Workgroup size of the persistent kernel (256, 512 or 1024; 0 keeps the
+/* A batch steps in one of two forms: the persistent kernel (a replica per
+ * workgroup) or, where that would leave compute units idle (few, uneven or
+ * small replicas with the Langevin or no thermostat and the Cartesian
+ * propagator), two kernels per step that spread every replica over the card.
+ * pimdb_batch_create chooses by an estimate of both; this call chooses the
+ * persistent kernel with the given shape.
+ * Workgroup size of the persistent kernel (256, 512 or 1024; 0 keeps the
  * current one) and number of workgroups (0 keeps the current one; default
- * one per compute unit).  More workgroups than compute units share each CU's
+ * one of 1024 threads per compute unit, or two of 512 where there are more
+ * replicas than compute units).  More workgroups than compute units share each CU's
  * LDS, and every replica's phases are planned for that share (an exchange
  * workspace that does not fit goes to device memory, allocated here);
  * PIMDB_E_ARG (the previous shape kept) when some replica does not fit it. */
 int pimdb_batch_configure(pimdb_batch* batch, int threads, int resident);
 /* Times trial_steps steps for each launch shape (256, 512 or 1024 threads,
  * 1, 2 or 4 workgroups per compute unit, at most 1024 threads per CU) whose
- * LDS plan fits, keeps the fastest and restores the state it started from. */
+ * LDS plan fits, and the two-kernel form where it applies, keeps the fastest
+ * and restores the state it started from.  The two-kernel form is reported as
+ * 256 threads and the number of workgroups of its forces kernel. */
 int pimdb_batch_autotune(pimdb_batch* batch, int trial_steps, int* threads_out, int* resident_out);
 /* nsteps MD steps of every replica, as pimdb_batch_step, with the device
  * time between events recorded on the batch's stream just before the first

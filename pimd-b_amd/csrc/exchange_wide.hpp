@@ -43,9 +43,10 @@
 
 namespace pimdb {
 
+// Threads of a workgroup (template parameter NT): 1024 where a ring has the
+// card to itself; 256 beside other rings' work, where the idle waves of a
+// waiting workgroup would hold registers that others could use.
 constexpr int XW_THREADS = 1024;
-constexpr int XW_WAVES = XW_THREADS / WAVE;
-constexpr int XW_SRC = REC_B / XW_WAVES;             // sources of a block per wave
 constexpr unsigned long long XW_EMPTY = ~0ull;
 constexpr long long XW_SPIN = 1ll << 22;             // polls of one wait (seconds)
 
@@ -56,23 +57,26 @@ __host__ __device__ inline int xw_grid(int N) { return 2 * rec_blocks(N); }
 // LDS doubles: the ring, the block's gauge and source logarithms, the
 // in-block matrix, per-wave partials, the substitution's results, the wave
 // totals of the prefix sums and a flag.
-__host__ __device__ inline size_t xw_shared_doubles(int N, int D) {
-    return (size_t)(2 * D + 2) * N + 2 * REC_B + (size_t)REC_TRI + 2 * (size_t)XW_WAVES * REC_B + 2 * REC_B +
-           2 * XW_WAVES + 2;
+__host__ __device__ inline size_t xw_shared_doubles(int N, int D, int nw) {
+    return (size_t)(2 * D + 2) * N + 2 * REC_B + (size_t)REC_TRI + 2 * (size_t)nw * REC_B + 2 * REC_B + 2 * (size_t)nw + 2;
 }
-inline size_t xw_lds_bytes(int N, int D) { return sizeof(double) * xw_shared_doubles(N, D); }
+inline size_t xw_lds_bytes(int N, int D, int threads = XW_THREADS) {
+    return sizeof(double) * xw_shared_doubles(N, D, threads / WAVE);
+}
 
 struct XwShared {
     double *x1, *xP, *Shi, *Slo;   // the ring [D][N], [D][N], [N], [N]
     double *g, *lgs;               // [REC_B] gauge; ln(N-q) of the block as sources (backward)
     double *a;                     // [REC_TRI] in-block matrix at rec_idx(j, t)
-    double *part, *psum;           // [XW_WAVES][REC_B]
+    double *part, *psum;           // [waves][REC_B]
     double *R, *z;                 // [REC_B]
-    double *tot;                   // [2 XW_WAVES] wave totals of the prefix sums
+    double *tot;                   // [2 waves] wave totals of the prefix sums
     int* flag;
 };
 
+template <int NT>
 __device__ __forceinline__ XwShared xw_carve(double* p, int N, int D) {
+    constexpr int NW = NT / WAVE;
     XwShared s;
     s.x1 = p; p += (size_t)D * N;
     s.xP = p; p += (size_t)D * N;
@@ -81,11 +85,11 @@ __device__ __forceinline__ XwShared xw_carve(double* p, int N, int D) {
     s.g = p; p += REC_B;
     s.lgs = p; p += REC_B;
     s.a = p; p += REC_TRI;
-    s.part = p; p += XW_WAVES * REC_B;
-    s.psum = p; p += XW_WAVES * REC_B;
+    s.part = p; p += NW * REC_B;
+    s.psum = p; p += NW * REC_B;
     s.R = p; p += REC_B;
     s.z = p; p += REC_B;
-    s.tot = p; p += 2 * XW_WAVES;
+    s.tot = p; p += 2 * NW;
     s.flag = (int*)p;
     return s;
 }
@@ -110,13 +114,14 @@ __device__ __forceinline__ DD dd_wave_scan(DD v) {
 // links, the waves scan their totals.  Every workgroup of a ring computes the
 // same values.  Shi_out / Slo_out / xc_out (may be null) receive the sums and
 // a copy [2][D][N] of the two beads.
-template <int D>
+template <int D, int NT>
 __device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, const double* __restrict__ x1,
                                          const double* __restrict__ xP, double k, bool pbc, double L,
                                          double* Shi_out, double* Slo_out, double* xc_out) {
+    constexpr int NW = NT / WAVE;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const Ring r = make_ring(sh.x1, sh.xP, sh.Shi, sh.Slo, k, pbc, L);
-    for (int e = tid; e < D * N; e += XW_THREADS) {
+    for (int e = tid; e < D * N; e += NT) {
         const double u = x1[e], v = xP[e];
         sh.x1[e] = u;
         sh.xP[e] = v;
@@ -125,7 +130,7 @@ __device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, const double
             xc_out[(size_t)D * N + e] = v;
         }
     }
-    const int c = (N + XW_THREADS - 1) / XW_THREADS, v0 = tid * c;
+    const int c = (N + NT - 1) / NT, v0 = tid * c;
     auto link = [&](int v) {
         double d[D];
 #pragma unroll
@@ -146,9 +151,9 @@ __device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, const double
     }
     __syncthreads();
     DD tw{0.0, 0.0};
-    if (lane < XW_WAVES) tw = DD{sh.tot[2 * lane], sh.tot[2 * lane + 1]};
+    if (lane < NW) tw = DD{sh.tot[2 * lane], sh.tot[2 * lane + 1]};
     tw = dd_wave_scan(tw);
-    const double total = wave_bcast_uniform(tw.hi, XW_WAVES - 1);
+    const double total = wave_bcast_uniform(tw.hi, NW - 1);
     DD ex{dpp_or_zero<0x138, 0xF>(inc.hi), dpp_or_zero<0x138, 0xF>(inc.lo)};   // wave_shr:1
     if (wave > 0) ex = dd_add(DD{wave_bcast_uniform(tw.hi, wave - 1), wave_bcast_uniform(tw.lo, wave - 1)}, ex);
     const double q = total > 0.0 ? ldexp(1.0, ilogb(total) - 40) : 1.0;
@@ -221,9 +226,10 @@ __device__ __forceinline__ double xw_wait(unsigned long long* p, int lane, int* 
 // One block with the exact min-plus shifts (exchange.hpp, steps (1)-(4)),
 // every earlier U being published: for blocks whose z left the range.  All
 // threads; U of the lane's target in every lane of wave 0.
-template <int DIR, int D>
+template <int DIR, int D, int NT>
 __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, double u0, const Ring r, const XwShared sh,
                                              unsigned long long* pub) {
+    constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // sources of a block per wave
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int n0 = 1 + I * REC_B;
     const RecTarget<D> tg = xw_target<DIR, D>(sh, N, n0 + min(lane, nb - 1));
@@ -242,7 +248,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
         }
     sh.part[wave * REC_B + lane] = lane < nb ? m : INFINITY;
     sh.psum[wave * REC_B + lane] = lane < nb ? s : 0.0;
-    for (int vr = wave; vr < REC_B / 2; vr += XW_WAVES) {
+    for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
         if (t < 0) continue;
@@ -253,7 +259,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
     __syncthreads();
     if (wave == 0) {
         double rr = INFINITY;
-        for (int w = 0; w < XW_WAVES; ++w) rr = fmin(rr, sh.part[w * REC_B + lane]);
+        for (int w = 0; w < NW; ++w) rr = fmin(rr, sh.part[w * REC_B + lane]);
         rec_inblock_seq<0>(sh.a, lane, rr, sh.R);
     }
     __syncthreads();
@@ -263,7 +269,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
         if (lane < nb && sw > 0.0) c = sw * exp_pair(sh.R[lane] - sh.part[wave * REC_B + lane]);
         sh.psum[wave * REC_B + lane] = c;
     }
-    for (int vr = wave; vr < REC_B / 2; vr += XW_WAVES) {
+    for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
         if (t >= 0) sh.a[rec_idx(j, t)] = t < nb ? exp_pair(-(sh.a[rec_idx(j, t)] + sh.R[j] - sh.R[t])) : 0.0;
@@ -272,7 +278,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
     double u = 0.0;
     if (wave == 0) {
         double z0 = 0.0;
-        for (int w = 0; w < XW_WAVES; ++w) z0 += sh.psum[w * REC_B + lane];
+        for (int w = 0; w < NW; ++w) z0 += sh.psum[w * REC_B + lane];
         rec_inblock_seq<1>(sh.a, lane, z0, sh.z);
         u = sh.R[lane] - log(sh.z[lane]);
     }
@@ -280,12 +286,13 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
     return u;
 }
 
-// Target block I of one recursion on one workgroup of XW_THREADS threads
+// Target block I of one recursion on one workgroup of NT threads
 // (the ring staged).  pub: this direction's published values [N+1].
-template <int DIR, int D>
+template <int DIR, int D, int NT>
 __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r, const XwShared& sh,
                                          unsigned long long* __restrict__ pub, double* __restrict__ V,
                                          double* __restrict__ Vb, int* __restrict__ status) {
+    constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // sources of a block per wave
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int ntarget = DIR == 0 ? N : N - 1;
     const int n0 = 1 + I * REC_B, nb = min(REC_B, ntarget - n0 + 1);
@@ -315,7 +322,7 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         sh.lgs[lane] = lgs;
     }
     __syncthreads();
-    for (int vr = wave; vr < REC_B / 2; vr += XW_WAVES) {
+    for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
         if (t < 0) continue;
@@ -332,29 +339,38 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         m = xw_w<DIR, D>(sh, r, bk, N, tg, 0) + u0;
         s = 1.0;
     }
+    // (four sources in registers at a time; the first four of a block are
+    // evaluated while their U are awaited)
+    constexpr int XQ = 4;
     for (int J = 0; J < I; ++J) {
-        const int qb = J * REC_B + 1;
-        double w[XW_SRC], uq[XW_SRC];
+        const int qb = J * REC_B + 1, q0 = wave * XW_SRC;
+        double w[XQ], uq[XQ];
 #pragma unroll
-        for (int u = 0; u < XW_SRC; ++u) w[u] = xw_w<DIR, D>(sh, r, bk, N, tg, qb + wave * XW_SRC + u);
+        for (int u = 0; u < XQ; ++u) w[u] = xw_w<DIR, D>(sh, r, bk, N, tg, qb + q0 + u);
         const double v = xw_wait(pub + qb, lane, status);
+        if (J == I - 1) sigma = wave_bcast_uniform(v, REC_B - 1);
+#pragma unroll 1
+        for (int c = 0; c < XW_SRC; c += XQ) {
 #pragma unroll
-        for (int u = 0; u < XW_SRC; ++u) uq[u] = wave_bcast_uniform(v, wave * XW_SRC + u);
-        if (J < I - 1) {
-            double mn = m;
-#pragma unroll
-            for (int u = 0; u < XW_SRC; ++u) {
-                w[u] += uq[u];
-                mn = fmin(mn, w[u]);
+            for (int u = 0; u < XQ; ++u) {
+                uq[u] = wave_bcast_uniform(v, q0 + c + u);
+                if (c > 0) w[u] = xw_w<DIR, D>(sh, r, bk, N, tg, qb + q0 + c + u);
             }
-            s *= exp_pair(mn - m);   // m = inf: s = 0 stays 0
-            m = mn;
+            if (J < I - 1) {
+                double mn = m;
 #pragma unroll
-            for (int u = 0; u < XW_SRC; ++u) s += exp_pair(mn - w[u]);
-        } else {
-            sigma = wave_bcast_uniform(v, REC_B - 1);
+                for (int u = 0; u < XQ; ++u) {
+                    w[u] += uq[u];
+                    mn = fmin(mn, w[u]);
+                }
+                s *= exp_pair(mn - m);   // m = inf: s = 0 stays 0
+                m = mn;
 #pragma unroll
-            for (int u = 0; u < XW_SRC; ++u) near += exp_pair((sigma - uq[u]) + (g - w[u]));
+                for (int u = 0; u < XQ; ++u) s += exp_pair(mn - w[u]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < XQ; ++u) near += exp_pair((sigma - uq[u]) + (g - w[u]));
+            }
         }
     }
     if (s > 0.0) near = fma(s, exp_pair((sigma - m) + g), near);
@@ -364,7 +380,7 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
     if (wave == 0) {
         double z0 = 0.0;
 #pragma unroll
-        for (int w = 0; w < XW_WAVES; ++w) z0 += sh.psum[w * REC_B + lane];
+        for (int w = 0; w < NW; ++w) z0 += sh.psum[w * REC_B + lane];
         rec_inblock_seq<1>(sh.a, lane, z0, sh.z);
         const double z = sh.z[lane];
         u = (sigma + g) - log(z);
@@ -375,7 +391,7 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
     }
     __syncthreads();
     if (*sh.flag) {
-        u = xw_block_safe<DIR, D>(I, N, nb, bk, u0, r, sh, pub);
+        u = xw_block_safe<DIR, D, NT>(I, N, nb, bk, u0, r, sh, pub);
         if (wave == 0) {
             if (lane < nb && !isfinite(u)) atomicOr(status, 1);
             if (!last) xw_publish(pub + n0 + lane, u + lgs);
@@ -391,7 +407,7 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         }
     }
     if (last) {   // every value has been read by every workgroup: empty for the next launch
-        for (int q = tid; q < n0; q += XW_THREADS)
+        for (int q = tid; q < n0; q += NT)
             __hip_atomic_store(pub + q, XW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
@@ -400,18 +416,18 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
 // lower blocks first.  pub: xw_pub_words(N) words, all XW_EMPTY on entry and
 // on return.  Block 0's forward workgroup writes the prefix sums and, where
 // asked, the beads' copy.
-template <int D>
+template <int D, int NT>
 __device__ __forceinline__ void xw_recursions(double* smem, int b, int N, double bt, double k, int pbc, double L,
                                               const double* __restrict__ x1, const double* __restrict__ xP,
                                               double* __restrict__ V, double* __restrict__ Vb, double* __restrict__ Shi,
                                               double* __restrict__ Slo, double* __restrict__ xc,
                                               unsigned long long* __restrict__ pub, int* __restrict__ status) {
-    const XwShared sh = xw_carve(smem, N, D);
+    const XwShared sh = xw_carve<NT>(smem, N, D);
     const bool first = b == 0;
-    const Ring r = xw_stage<D>(sh, N, x1, xP, k, pbc != 0, L, first ? Shi : nullptr, first ? Slo : nullptr,
+    const Ring r = xw_stage<D, NT>(sh, N, x1, xP, k, pbc != 0, L, first ? Shi : nullptr, first ? Slo : nullptr,
                                first ? xc : nullptr);
-    if ((b & 1) == 0) xw_block<0, D>(b >> 1, N, bt, r, sh, pub, V, Vb, status);
-    else xw_block<1, D>(b >> 1, N, bt, r, sh, pub + N + 1, V, Vb, status);
+    if ((b & 1) == 0) xw_block<0, D, NT>(b >> 1, N, bt, r, sh, pub, V, Vb, status);
+    else xw_block<1, D, NT>(b >> 1, N, bt, r, sh, pub + N + 1, V, Vb, status);
 }
 
 template <int D>
@@ -421,7 +437,7 @@ k_exchange_wide(int N, double bt, double k, int pbc, double L, const double* __r
                 double* __restrict__ Shi, double* __restrict__ Slo, unsigned long long* __restrict__ pub,
                 int* __restrict__ status) {
     extern __shared__ double smem[];
-    xw_recursions<D>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, nullptr, pub, status);
+    xw_recursions<D, XW_THREADS>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, nullptr, pub, status);
 }
 
 }  // namespace pimdb

@@ -449,25 +449,53 @@ struct SliceWalk {
         flush_row(ka, oka, ra);
         flush_row(kb, okb, rb);
     }
-    // row tiles A and B (B < 0: none) against column tile J, all distinct
-    __device__ __forceinline__ void off_tiles(int A, int B, int J) {
+    // offsets [lo, hi) of a diagonal tile's 0 .. 16 (diag_tile's, in the same
+    // order), for waves that share a slice
+    __device__ __forceinline__ void diag_part(int I, int lo, int hi) {
+        const int ka = I * PTILE + lane, kb = I * PTILE + ((lane + PTILE / 2) & (PTILE - 1));
+        double xa[D], xb[D], ra[D] = {}, rb[D] = {};
+        const bool oka = load_row(ka, xa), okb = load_row(kb, xb);
+        load_col(I * PTILE + ((lane + lo) & (PTILE - 1)));
+        const bool full = (I + 1) * PTILE <= N;
+        int s = lo;
+        if (s == 0) {
+            one(xb, rb, okb && lane < PTILE / 2 && col_ok());
+            rotate();
+            ++s;
+        }
+        for (; s < min(hi, PTILE / 4); ++s) {
+            if (full) {
+                two(xa, xb, ra, rb, true, true);
+            } else {
+                const bool c = col_ok();
+                two(xa, xb, ra, rb, oka && c, okb && c);
+            }
+            rotate();
+        }
+        if (s < hi) one(xa, ra, oka && col_ok());
+        flush_row(ka, oka, ra);
+        flush_row(kb, okb, rb);
+    }
+    // row tiles A and B (B < 0: none) against column tile J, all distinct;
+    // rotation offsets [s0, s1)
+    __device__ __forceinline__ void off_tiles(int A, int B, int J, int s0 = 0, int s1 = PTILE) {
         const int ka = A * PTILE + lane, kb = B * PTILE + lane;
         double xa[D], xb[D], ra[D] = {}, rb[D] = {};
         const bool oka = load_row(ka, xa), okb = B >= 0 && load_row(kb, xb);
-        load_col(J * PTILE + lane);
+        load_col(J * PTILE + ((lane + s0) & (PTILE - 1)));
         const bool full = (A + 1) * PTILE <= N && (J + 1) * PTILE <= N && (B < 0 || (B + 1) * PTILE <= N);
         if (B < 0) {
-            for (int s = 0; s < PTILE; ++s) {
+            for (int s = s0; s < s1; ++s) {
                 one(xa, ra, oka && col_ok());
                 rotate();
             }
         } else if (full) {
-            for (int s = 0; s < PTILE; ++s) {
+            for (int s = s0; s < s1; ++s) {
                 two(xa, xb, ra, rb, true, true);
                 rotate();
             }
         } else {
-            for (int s = 0; s < PTILE; ++s) {
+            for (int s = s0; s < s1; ++s) {
                 const bool c = col_ok();
                 two(xa, xb, ra, rb, oka && c, okb && c);
                 rotate();
@@ -489,6 +517,24 @@ __device__ __forceinline__ void slice_pair_forces_lds(const double* xs_, int N, 
     for (int J = 1; J < T; ++J)
         for (int A = J & 1; A < J; A += 2) w.off_tiles(A, A + 1, J);
     for (int A = 1; A < T; A += 4) w.off_tiles(A, A + 2 < T ? A + 2 : -1, 0);
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Share w of nw waves of the same pairs, every pass cut by its offsets, into
+// the wave's own force array F (zeroed here; the arrays of the waves are added
+// by the caller).
+template <int D, int KIND, int IMG>
+__device__ __forceinline__ void slice_pair_forces_part(const double* xs_, int N, const WalkGrad<D, KIND, IMG>& wg,
+                                                       int lane, lds_double* F, const lds_int* perm, int w, int nw) {
+    for (int e = lane; e < pair_fstride(D) * N; e += WAVE) F[e] = 0.0;
+    __builtin_amdgcn_wave_barrier();
+    SliceWalk<D, KIND, IMG> sw{(gbl_cdptr)xs_, N, wg, F, perm, lane, {}, 0u};
+    const int T = (N + PTILE - 1) / PTILE;
+    const int dlo = 17 * w / nw, dhi = 17 * (w + 1) / nw, s0 = PTILE * w / nw, s1 = PTILE * (w + 1) / nw;
+    for (int I = 0; I < T; ++I) sw.diag_part(I, dlo, dhi);
+    for (int J = 1; J < T; ++J)
+        for (int A = J & 1; A < J; A += 2) sw.off_tiles(A, A + 1, J, s0, s1);
+    for (int A = 1; A < T; A += 4) sw.off_tiles(A, A + 2 < T ? A + 2 : -1, 0, s0, s1);
     __builtin_amdgcn_wave_barrier();
 }
 

@@ -13,6 +13,7 @@
 
 #include "pimdb_gpu.h"
 #include "batch.hpp"
+#include "batch_split.hpp"
 #include "ctx_common.hpp"
 
 using namespace pimdb;
@@ -46,6 +47,15 @@ struct pimdb_batch {
     bool xdev_any = false;        // some replica's exchange workspace is in device memory
     bool ext_any = false;         // any of the three: the EXT kernels
     bool maybe_pending = false;   // a step ran since the last finishing launch
+    bool unsettled = false;       // cmp may hold what the two-kernel form does not keep (BatchPtrs)
+    // the two-kernel form (batch_split.hpp)
+    bool split = false;           // steps run in it
+    SplitPtrs sp{};
+    std::vector<StepArgs> hsteps;
+    double* d_split = nullptr;    // its workspace
+    unsigned long long* d_pub = nullptr;
+    StepArgs* d_steps = nullptr;
+    int2* d_maps = nullptr;
     std::string err;
     int fail(int code, const std::string& m) {
         err = m;
@@ -59,10 +69,25 @@ struct pimdb_batch {
         if (e_ != hipSuccess) return b->fail(PIMDB_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// Cost model for the schedule: ordered pairs dominate, the exchange adds N^2.
+// Microseconds of one compute unit that a replica's step takes, fitted to both
+// forms at N = 8 .. 256, P = 8 .. 64, free, dipole and helium pairs, with and
+// without normal-mode coupling (within about 15%).  Pairs: 64-particle tiles,
+// ns per pair; persistent: a fixed 55 us of barriers and phase starts; split:
+// the recursions' blocks and the noise tiles, each a workgroup with waits of
+// its own, instead.
+static double pair_us(const pimdb_params& p) {
+    static const double ns[4] = {0.0, 0.2, 0.3, 0.55};   // free, harmonic, dipole, Aziz
+    const double T = (p.natoms + PTILE - 1) / PTILE;
+    return p.nbeads * (T * PTILE) * (T * PTILE) * 0.5e-3 * ns[p.int_kind & 3];
+}
 static double rep_cost(const pimdb_params& p) {
-    const double N = p.natoms, P = p.nbeads;
-    return P * N * N + (p.bosonic && p.nbeads > 1 ? 8.0 * N * N : 0.0) + 4.0 * P * P * N;
+    const double N = p.natoms, nd = N * p.nbeads * p.ndim;
+    return 55.0 + 0.004 * nd + (p.bosonic && p.nbeads > 1 ? 10.0 + 9e-4 * N * N : 0.0) + pair_us(p);
+}
+static double rep_cost_split(const pimdb_params& p) {
+    const double T = (p.natoms + PTILE - 1) / PTILE, nd = (double)p.natoms * p.nbeads * p.ndim;
+    return 0.0064 * nd + (p.nmthermostat ? 0.005 * p.nbeads * p.ndim * PTILE * T : 0.0) +
+           (p.bosonic && p.nbeads > 1 ? 45.0 * T : 0.0) + 1.2 * pair_us(p);
 }
 
 // Longest-processing-time-first assignment of replicas to `grid` workgroups.
@@ -144,6 +169,23 @@ static size_t plan_lds(pimdb_batch* b, int threads, int per_cu, std::vector<RepD
         if (d.plds) need = std::max(need, pl);
     }
     return sizeof(double) * (16 + need);
+}
+
+// The largest load of a workgroup (us) in a schedule of `grid` workgroups.
+static double makespan(const pimdb_batch* b, int grid) {
+    std::vector<double> c;
+    for (const pimdb_params& p : b->prm) c.push_back(rep_cost(p));
+    std::sort(c.rbegin(), c.rend());
+    std::priority_queue<double, std::vector<double>, std::greater<double>> heap;
+    for (int g = 0; g < grid; ++g) heap.push(0.0);
+    double most = 0.0;
+    for (double x : c) {
+        const double t = heap.top() + x;
+        heap.pop();
+        heap.push(t);
+        most = std::max(most, t);
+    }
+    return most;
 }
 
 static int upload_schedule(pimdb_batch* b) {
@@ -241,6 +283,173 @@ static int launch_batch(pimdb_batch* b, int mode) {
     return PIMDB_OK;
 }
 
+// Whether every replica can take the two-kernel form: Langevin or no
+// thermostat, the Cartesian propagator, and parts that fit the LDS.
+static bool split_able(const pimdb_batch* b) {
+    const size_t lim = device_lds_limit();
+    for (int r = 0; r < b->R; ++r) {
+        const pimdb_params& p = b->prm[r];
+        const bool nm = p.thermostat == PIMDB_THERMO_LANGEVIN && p.nmthermostat;
+        if (p.thermostat > PIMDB_THERMO_LANGEVIN || p.propagator != PIMDB_PROP_CARTESIAN) return false;
+        if (nm && p.nbeads > STEP_NM_MAXP) return false;
+        if (b->desc[r].bosonic && xw_lds_bytes(p.natoms, p.ndim, SPLIT_THREADS) > lim) return false;
+        if (sizeof(double) * step_noise_lds_doubles(p.nbeads, nm) > lim) return false;
+    }
+    return true;
+}
+
+static void free_split(pimdb_batch* b) {
+    if (b->d_split) (void)hipFree(b->d_split);
+    if (b->d_pub) (void)hipFree(b->d_pub);
+    if (b->d_steps) (void)hipFree(b->d_steps);
+    if (b->d_maps) (void)hipFree(b->d_maps);
+    b->d_split = nullptr;
+    b->d_pub = nullptr;
+    b->d_steps = nullptr;
+    b->d_maps = nullptr;
+}
+
+static int build_split_buffers(pimdb_batch* b) {
+    const int D = b->D;
+    std::vector<size_t> off;
+    size_t nd = 0, nw = 0;
+    for (int r = 0; r < b->R; ++r) {
+        const pimdb_params& p = b->prm[r];
+        const size_t N = p.natoms, P = p.nbeads;
+        off.push_back(nd);
+        nd += 4 * D * N + (N + 1) + 2 * N + P * D * N + P * SPLIT_WAVES * D + D * (size_t)step_noise_tiles(p.natoms);
+        if (b->desc[r].bosonic) nw += xw_pub_words(p.natoms);
+    }
+    BCK(hipMalloc((void**)&b->d_split, nd * sizeof(double)));
+    if (nw) {
+        BCK(hipMalloc((void**)&b->d_pub, nw * 8));
+        BCK(hipMemset(b->d_pub, 0xFF, nw * 8));
+    }
+    // waves per slice: enough of them for four per SIMD, where the slices alone
+    // are fewer and their force arrays fit the LDS
+    size_t beads = 0;
+    bool fit = true;
+    for (const pimdb_params& p : b->prm) {
+        beads += p.nbeads;
+        fit = fit && split_slice_lds(p.natoms, D) <= device_lds_limit();
+    }
+    int share = 1;
+    while (fit && share < SPLIT_WAVES && beads * share < 8 * (size_t)b->cus) share *= 2;
+    std::vector<int2> slices;    // the long workgroups last
+    std::vector<int2> maps[4];   // forces, noise, full, open
+    size_t lds = 0, w = 0;
+    b->hsteps.clear();
+    for (int r = 0; r < b->R; ++r) {
+        const pimdb_params& p = b->prm[r];
+        const RepDesc& d = b->desc[r];
+        const Derived dv = derive(p);
+        const size_t N = p.natoms, P = p.nbeads;
+        StepArgs a{};
+        a.fa = make_force_args(p, dv);
+        a.bt = dv.bt;
+        a.thermostat = p.thermostat; a.nm = p.nmthermostat; a.fixcom = p.fixcom;
+        a.x = b->bp.x + d.off_x; a.p = b->bp.p + d.off_x; a.f = b->bp.f + d.off_x;
+        a.V = b->bp.V + d.off_V;
+        double* q = b->d_split + off[r];
+        a.xc = q; q += 4 * D * N;
+        a.Vb = q; q += N + 1;
+        a.Shi = q; q += N;
+        a.Slo = q; q += N;
+        a.H = q; q += P * D * N;
+        a.fpart = p.ext_kind != PIMDB_POT_FREE && p.fixcom ? q : nullptr; q += P * SPLIT_WAVES * D;
+        a.hpart = q;
+        a.frows = p.nbeads * share;
+        a.pub = d.bosonic ? b->d_pub + w : nullptr;
+        if (d.bosonic) w += xw_pub_words(p.natoms);
+        a.status = b->bp.status + r;
+        a.c1 = a.thermostat ? dv.c1 : 1.0;
+        a.c2 = dv.c2;
+        a.half_dt = 0.5 * p.dt;
+        a.dt_m = p.dt / p.mass;
+        a.CTt = b->bp.CTt + d.off_C;
+        a.ctr = b->bp.ctl;
+        a.seed = p.seed;
+        b->hsteps.push_back(a);
+        const int nx = d.bosonic ? xw_grid(p.natoms) : 0, ns = split_slices(p.nbeads, share), nn = step_noise_groups(a, D);
+        for (int i = 0; i < nx + nn; ++i) maps[0].push_back(int2{r, i});
+        for (int i = 0; i < ns; ++i) slices.push_back(int2{r, nx + nn + i});
+        for (int i = 0; i < nn; ++i) maps[1].push_back(int2{r, i});
+        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_FULL, SPLIT_EXT); ++i) maps[2].push_back(int2{r, i});
+        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_OPEN, SPLIT_EXT); ++i) maps[3].push_back(int2{r, i});
+        if (d.bosonic) lds = std::max(lds, xw_lds_bytes(p.natoms, D, SPLIT_THREADS));
+        const size_t sl = split_slice_lds(p.natoms, D);
+        if (sl <= device_lds_limit()) lds = std::max(lds, sl);
+        lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(p.nbeads, a.thermostat && a.nm));
+    }
+    maps[0].insert(maps[0].end(), slices.begin(), slices.end());
+    size_t nm = 0;
+    for (auto& m : maps) nm += m.size();
+    BCK(hipMalloc((void**)&b->d_maps, nm * sizeof(int2)));
+    BCK(hipMalloc((void**)&b->d_steps, b->R * sizeof(StepArgs)));
+    int2* at = b->d_maps;
+    const int2* ptr[4];
+    for (int k = 0; k < 4; ++k) {
+        if (!maps[k].empty()) BCK(hipMemcpy(at, maps[k].data(), maps[k].size() * sizeof(int2), hipMemcpyHostToDevice));
+        ptr[k] = at;
+        at += maps[k].size();
+    }
+    BCK(hipMemcpy(b->d_steps, b->hsteps.data(), b->R * sizeof(StepArgs), hipMemcpyHostToDevice));
+    BCK(hipStreamSynchronize(nullptr));
+    b->sp.steps = b->d_steps;
+    b->sp.forces_map = ptr[0]; b->sp.nforces = (int)maps[0].size();
+    b->sp.noise_map = ptr[1]; b->sp.nnoise = (int)maps[1].size();
+    b->sp.full_map = ptr[2]; b->sp.nfull = (int)maps[2].size();
+    b->sp.open_map = ptr[3]; b->sp.nopen = (int)maps[3].size();
+    b->sp.lds = lds;
+    b->sp.share = share;
+    return PIMDB_OK;
+}
+
+// The two-kernel form's workspace and maps (allocated once).
+static int build_split(pimdb_batch* b) {
+    if (b->d_steps) return PIMDB_OK;
+    const int rc = build_split_buffers(b);
+    if (rc) {
+        (void)hipGetLastError();
+        free_split(b);
+    }
+    return rc;
+}
+
+static int finish_pending(pimdb_batch* b);
+
+// nsteps steps in the two-kernel form; the state is complete afterwards.
+static int enqueue_split(pimdb_batch* b, int nsteps) {
+    if (nsteps < 1) return PIMDB_OK;
+    if (b->unsettled) {   // p from the persistent kernel: its owed half step, then its pending COM momentum
+        const int rc = finish_pending(b);
+        if (rc) return rc;
+        BCK(launch_split_settle(b->bp, b->D, b->R, b->s));
+        b->unsettled = false;
+    }
+    b->sp.bp = b->bp;
+    BCK(launch_split_forces(b->sp, b->D, b->kind, false, STEP_OPEN, b->s));
+    BCK(launch_split_integrate(b->sp, b->D, STEP_OPEN, b->s));
+    for (int s = 1; s <= nsteps; ++s) {
+        const int mode = s < nsteps ? STEP_FULL : STEP_CLOSE;
+        BCK(launch_split_forces(b->sp, b->D, b->kind, true, mode, b->s));
+        BCK(launch_split_integrate(b->sp, b->D, mode, b->s));
+    }
+    return PIMDB_OK;
+}
+
+static int capture(pimdb_batch* b);
+
+// nsteps steps of every replica on the batch's stream, in its current form.
+static int enqueue_batch_steps(pimdb_batch* b, int nsteps) {
+    if (b->split) return enqueue_split(b, nsteps);
+    const int rc = capture(b);
+    if (rc) return rc;
+    for (int s = 0; s < nsteps; ++s) BCK(hipGraphLaunch(b->gexec, b->s));
+    if (nsteps > 0) b->maybe_pending = b->unsettled = true;
+    return PIMDB_OK;
+}
+
 static int capture(pimdb_batch* b) {
     if (b->gexec) return PIMDB_OK;
     BCK(hipStreamSynchronize(b->s));
@@ -268,6 +477,40 @@ static int check_batch_status(pimdb_batch* b) {
             return b->fail(PIMDB_E_NONFINITE, "non-finite bosonic exchange potential in replica " + std::to_string(r));
         }
     }
+    return PIMDB_OK;
+}
+
+// Launch shape and form of a new batch.  More replicas than compute units: two
+// workgroups of 512 threads per CU overlap each other's latencies (512
+// replicas: 8 - 33% faster than one of 1024 at every size tried), where their
+// LDS plan keeps every exchange workspace and force array in LDS.  The
+// two-kernel form where its load over the whole card is below the persistent
+// kernel's longest workgroup: fewer replicas than compute units (16 helium
+// replicas of N=256, P=64: 162 against 1240 us a step, 128 of them 937 against
+// 1274, but 256 of them 1900 against 1345), uneven ones, and small ones (512
+// uneven dipole replicas 252 against 284 us).
+static int choose_form(pimdb_batch* b) {
+    double shape_gain = 1.0;
+    if (b->R > b->cus) {
+        std::vector<RepDesc> one = b->desc, two = b->desc;
+        std::vector<size_t> xdev(b->R, 0);
+        std::string why;
+        if (plan_lds(b, 1024, 1, one, &why) && plan_lds(b, 512, 2, two, &why, &xdev)) {
+            bool same = true;
+            for (int r = 0; r < b->R; ++r) same = same && !xdev[r] && two[r].plds == one[r].plds;
+            if (same) {
+                b->threads = 512;
+                b->resident = 2 * b->cus;
+                shape_gain = 0.85;
+            }
+        }
+    }
+    const int rc = upload_schedule(b);
+    if (rc || !split_able(b)) return rc;
+    double load = 0.0;
+    for (const pimdb_params& p : b->prm) load += rep_cost_split(p);
+    b->split = 20.0 + load / b->cus < 0.95 * shape_gain * makespan(b, std::min(b->R, b->cus));
+    if (b->split && build_split(b) != PIMDB_OK) b->split = false;   // (no memory for its workspace)
     return PIMDB_OK;
 }
 
@@ -416,7 +659,7 @@ int pimdb_batch_create(const pimdb_params* reps, int nrep, pimdb_batch** out) {
     if (!rc && (hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking) != hipSuccess ||
                 hipEventCreate(&b->t0) != hipSuccess || hipEventCreate(&b->t1) != hipSuccess))
         rc = b->fail(PIMDB_E_HIP, "stream/event creation failed");
-    if (!rc) rc = upload_schedule(b);
+    if (!rc) rc = choose_form(b);
     if (rc) {
         set_create_error(b->err);
         pimdb_batch_destroy(b);
@@ -441,6 +684,7 @@ void pimdb_batch_destroy(pimdb_batch* b) {
     if (b->d_desc) (void)hipFree(b->d_desc);
     if (b->d_sched) (void)hipFree(b->d_sched);
     if (b->d_sched_off) (void)hipFree(b->d_sched_off);
+    free_split(b);
     if (b->t0) (void)hipEventDestroy(b->t0);
     if (b->t1) (void)hipEventDestroy(b->t1);
     if (b->s) (void)hipStreamDestroy(b->s);
@@ -484,6 +728,7 @@ int pimdb_batch_set_state(pimdb_batch* b, int rep, const double* x, const double
         double cmp[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         for (size_t e = 0; e < n; ++e) cmp[4 + e % q.ndim] += p[e];
         BCK(hipMemcpy(b->bp.cmp + 8 * (size_t)rep, cmp, sizeof(cmp), hipMemcpyHostToDevice));
+        b->unsettled = true;
     }
     return PIMDB_OK;
 }
@@ -514,28 +759,32 @@ int pimdb_batch_get_state(pimdb_batch* b, int rep, double* x, double* p, double*
 
 int pimdb_batch_forces(pimdb_batch* b) {
     if (!b) return PIMDB_E_ARG;
-    int rc = launch_batch(b, BM_FORCES);
-    if (rc) return rc;
+    if (b->split) {
+        b->sp.bp = b->bp;
+        BCK(launch_split_forces(b->sp, b->D, b->kind, true, STEP_FORCES, b->s));
+        BCK(launch_split_integrate(b->sp, b->D, STEP_FORCES, b->s));
+    } else {
+        const int rc = launch_batch(b, BM_FORCES);
+        if (rc) return rc;
+    }
     return check_batch_status(b);
 }
 
 int pimdb_batch_step(pimdb_batch* b, int nsteps) {
     if (!b || nsteps < 0) return PIMDB_E_ARG;
-    int rc = capture(b);
+    const int rc = enqueue_batch_steps(b, nsteps);
     if (rc) return rc;
-    for (int s = 0; s < nsteps; ++s) BCK(hipGraphLaunch(b->gexec, b->s));
-    if (nsteps > 0) b->maybe_pending = true;
     return check_batch_status(b);
 }
 
 int pimdb_batch_step_timed(pimdb_batch* b, int nsteps, double* device_ms) {
     if (!b || nsteps < 1 || !device_ms) return PIMDB_E_ARG;
-    int rc = capture(b);
+    int rc = b->split ? PIMDB_OK : capture(b);
     if (rc) return rc;
     BCK(hipEventRecord(b->t0, b->s));
-    for (int s = 0; s < nsteps; ++s) BCK(hipGraphLaunch(b->gexec, b->s));
+    rc = enqueue_batch_steps(b, nsteps);
+    if (rc) return rc;
     BCK(hipEventRecord(b->t1, b->s));
-    b->maybe_pending = true;
     BCK(hipEventSynchronize(b->t1));
     float ms = 0.0f;
     BCK(hipEventElapsedTime(&ms, b->t0, b->t1));
@@ -552,11 +801,14 @@ int pimdb_batch_configure(pimdb_batch* b, int threads, int resident) {
     const int old_threads = b->threads, old_resident = b->resident;
     if (threads) b->threads = threads;
     if (resident) b->resident = resident;
+    const bool split = b->split;
+    b->split = false;   // an explicit shape is the persistent kernel's
     const int rc = upload_schedule(b);
     if (rc == PIMDB_E_ARG) {   // this shape's LDS plan does not fit: keep the previous one
         const std::string why = b->err;
         b->threads = old_threads;
         b->resident = old_resident;
+        b->split = split;
         const int rc2 = upload_schedule(b);
         if (rc2) return rc2;
         return b->fail(PIMDB_E_ARG, why);
@@ -566,12 +818,11 @@ int pimdb_batch_configure(pimdb_batch* b, int threads, int resident) {
 
 int pimdb_batch_time_step(pimdb_batch* b, int reps, double* ms_step) {
     if (!b || reps < 1 || !ms_step) return PIMDB_E_ARG;
-    int rc = capture(b);
+    int rc = enqueue_batch_steps(b, 1);
     if (rc) return rc;
-    BCK(hipGraphLaunch(b->gexec, b->s));
-    b->maybe_pending = true;
     BCK(hipEventRecord(b->t0, b->s));
-    for (int r = 0; r < reps; ++r) BCK(hipGraphLaunch(b->gexec, b->s));
+    rc = enqueue_batch_steps(b, reps);
+    if (rc) return rc;
     BCK(hipEventRecord(b->t1, b->s));
     BCK(hipEventSynchronize(b->t1));
     float ms = 0.0f;
@@ -667,6 +918,8 @@ int pimdb_batch_autotune(pimdb_batch* b, int trial_steps, int* threads_out, int*
     double best = 1e300;
     int bt = b->threads, br = b->resident;
     int rc = PIMDB_OK;
+    const bool pending = b->maybe_pending;
+    b->split = false;
     std::vector<std::pair<int, int>> tried;
     for (int ci = 0; ci < 6 && !rc; ++ci) {
         const int threads = cand[ci][0], per_cu = cand[ci][1], resident = b->cus * per_cu;
@@ -692,6 +945,14 @@ int pimdb_batch_autotune(pimdb_batch* b, int trial_steps, int* threads_out, int*
     b->threads = bt;
     b->resident = br;
     if (!rc) rc = upload_schedule(b);
+    // the two-kernel form (last: its steps leave nothing owed)
+    if (!rc && split_able(b) && build_split(b) == PIMDB_OK) {
+        b->split = true;
+        double ms = 0.0;
+        rc = pimdb_batch_time_step(b, trial_steps, &ms);
+        b->split = !rc && ms < best;
+    }
+    BCK(hipStreamSynchronize(b->s));
     BCK(hipMemcpy(b->bp.x, sx, sizeof(double) * b->nx, hipMemcpyDeviceToDevice));
     BCK(hipMemcpy(b->bp.p, sp, sizeof(double) * b->nx, hipMemcpyDeviceToDevice));
     BCK(hipMemcpy(b->bp.f, sf, sizeof(double) * b->nx, hipMemcpyDeviceToDevice));
@@ -703,8 +964,10 @@ int pimdb_batch_autotune(pimdb_batch* b, int trial_steps, int* threads_out, int*
     (void)hipFree(sp);
     (void)hipFree(sf);
     if (sfx) (void)hipFree(sfx);
-    if (threads_out) *threads_out = b->threads;
-    if (resident_out) *resident_out = b->resident;
+    b->maybe_pending = pending;   // as the restored momenta are
+    b->unsettled = true;
+    if (threads_out) *threads_out = b->split ? SPLIT_THREADS : b->threads;
+    if (resident_out) *resident_out = b->split ? b->sp.nforces : b->resident;
     return rc;
 }
 

@@ -7,8 +7,8 @@
 //   K3 k_step_forces  exchange recursions beside the bead forces, then
 //                     k_exchange_forces (beads 1 and P)
 //   K4 k_momenta      B, O-step, partial sums for zeroMomentum
-// and within a run of device-noise Langevin (or NVE) steps with the Cartesian
-// propagator K4, K1 and K2 are one k_step_integrate (steps.hpp).  Rings and
+// but device-noise Langevin (or NVE) steps with the Cartesian propagator take
+// k_step_forces and one k_step_integrate per step (steps.hpp).  Rings and
 // slices beyond a workgroup's LDS take the recursions and the bead forces as
 // two kernels on two streams.
 #include <hip/hip_runtime.h>
@@ -165,17 +165,13 @@ static void launch_factorial(pimdb_ctx* ctx, hipStream_t s, double* f, double* f
     }
 }
 
-static StepArgs step_args(pimdb_ctx* ctx, bool noise) {
+static StepArgs step_args(pimdb_ctx* ctx) {
     StepArgs a{};
     a.fa = make_force_args(ctx->prm, ctx->dv);
     a.bt = ctx->dv.bt;
-    const int N = ctx->N, P = ctx->P, D = ctx->D;
-    a.nx = ctx->dv.bosonic ? xw_grid(N) : 0;
-    a.nf = P * ((N + FORCE_TILE - 1) / FORCE_TILE);
     a.thermostat = ctx->prm.thermostat;
     a.nm = ctx->prm.nmthermostat;
     a.fixcom = ctx->prm.fixcom;
-    a.nn = noise && (a.thermostat || a.fixcom) ? D * step_noise_tiles(N) : 0;
     a.x = ctx->x; a.p = ctx->p; a.f = ctx->f;
     a.fext = ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr;
     a.V = ctx->V; a.Vb = ctx->Vb; a.Shi = ctx->Shi; a.Slo = ctx->Slo; a.xc = ctx->xc;
@@ -186,6 +182,7 @@ static StepArgs step_args(pimdb_ctx* ctx, bool noise) {
     a.dt_m = ctx->prm.dt / ctx->prm.mass;
     a.CTt = ctx->CT;
     a.H = ctx->H; a.hpart = ctx->hpart;
+    a.frows = ctx->P * ((ctx->N + FORCE_TILE - 1) / FORCE_TILE);
     a.fpart = ctx->prm.ext_kind != PIMDB_POT_FREE && a.fixcom ? ctx->fpart : nullptr;
     a.ctr = ctx->ctr;
     a.seed = ctx->prm.seed;
@@ -197,44 +194,49 @@ static size_t tile_lds_bytes(int N, int D) {
 }
 
 template <int D>
-static void launch_step_forces_d(pimdb_ctx* ctx, const StepArgs& a, hipStream_t s) {
-    size_t lds = tile_lds_bytes(ctx->N, D);
-    if (a.nx) lds = std::max(lds, xw_lds_bytes(ctx->N, D));
-    if (a.nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(ctx->P, a.thermostat && a.nm));
-    const dim3 grid(a.nx + a.nf + a.nn), blk(XW_THREADS);
+static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
+    const StepArgs a = step_args(ctx);
+    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = forces ? a.frows : 0;
+    const int nn = noise ? step_noise_groups(a, D) : 0;
+    if (nx + nf + nn == 0) return;
+    size_t lds = 0;
+    if (nf) lds = tile_lds_bytes(ctx->N, D);
+    if (nx) lds = std::max(lds, xw_lds_bytes(ctx->N, D));
+    if (nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(ctx->P, a.thermostat && a.nm));
+    const dim3 grid(nx + nf + nn), blk(XW_THREADS);
+    const hipStream_t s = ctx->s0;
     switch (ctx->prm.int_kind) {
-    case POT_HARMONIC: hipLaunchKernelGGL((k_step_forces<D, POT_HARMONIC>), grid, blk, lds, s, a); break;
-    case POT_DIPOLE: hipLaunchKernelGGL((k_step_forces<D, POT_DIPOLE>), grid, blk, lds, s, a); break;
-    case POT_AZIZ: hipLaunchKernelGGL((k_step_forces<D, POT_AZIZ>), grid, blk, lds, s, a); break;
-    default: hipLaunchKernelGGL((k_step_forces<D, POT_FREE>), grid, blk, lds, s, a); break;
+    case POT_HARMONIC: hipLaunchKernelGGL((k_step_forces<D, POT_HARMONIC>), grid, blk, lds, s, a, nx, nf, mode); break;
+    case POT_DIPOLE: hipLaunchKernelGGL((k_step_forces<D, POT_DIPOLE>), grid, blk, lds, s, a, nx, nf, mode); break;
+    case POT_AZIZ: hipLaunchKernelGGL((k_step_forces<D, POT_AZIZ>), grid, blk, lds, s, a, nx, nf, mode); break;
+    default: hipLaunchKernelGGL((k_step_forces<D, POT_FREE>), grid, blk, lds, s, a, nx, nf, mode); break;
     }
 }
 
-// Recursions, bead forces and (noise) the next integration's noise, all but
-// the exterior forces of beads 1 and P.
-static void launch_step_forces(pimdb_ctx* ctx, bool noise) {
-    const StepArgs a = step_args(ctx, noise);
+// The recursions and bead forces (forces: all but the exterior forces of beads
+// 1 and P) and the noise of the integration of this mode (noise).
+static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
     switch (ctx->D) {
-    case 1: launch_step_forces_d<1>(ctx, a, ctx->s0); break;
-    case 2: launch_step_forces_d<2>(ctx, a, ctx->s0); break;
-    default: launch_step_forces_d<3>(ctx, a, ctx->s0); break;
+    case 1: launch_step_forces_d<1>(ctx, forces, noise, mode); break;
+    case 2: launch_step_forces_d<2>(ctx, forces, noise, mode); break;
+    default: launch_step_forces_d<3>(ctx, forces, noise, mode); break;
     }
 }
 
-static void launch_step_integrate(pimdb_ctx* ctx) {
-    const StepArgs a = step_args(ctx, true);
-    const dim3 grid((unsigned)(step_exterior_groups(a.fa) + (step_inner_elements(a.fa, ctx->D) + 255) / 256));
+static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
+    const StepArgs a = step_args(ctx);
+    const dim3 grid(step_integrate_groups(a.fa, ctx->D, mode, 1));
     switch (ctx->D) {
-    case 1: hipLaunchKernelGGL(k_step_integrate<1>, grid, dim3(256), 0, ctx->s0, a); break;
-    case 2: hipLaunchKernelGGL(k_step_integrate<2>, grid, dim3(256), 0, ctx->s0, a); break;
-    default: hipLaunchKernelGGL(k_step_integrate<3>, grid, dim3(256), 0, ctx->s0, a); break;
+    case 1: hipLaunchKernelGGL(k_step_integrate<1>, grid, dim3(256), 0, ctx->s0, a, mode); break;
+    case 2: hipLaunchKernelGGL(k_step_integrate<2>, grid, dim3(256), 0, ctx->s0, a, mode); break;
+    default: hipLaunchKernelGGL(k_step_integrate<3>, grid, dim3(256), 0, ctx->s0, a, mode); break;
     }
 }
 
 // Forces of every bead (updateForces on all ranks); f and (NM propagator) fext.
 static int enqueue_forces(pimdb_ctx* ctx) {
     if (ctx->merged) {
-        launch_step_forces(ctx, false);
+        launch_step_forces(ctx, true, false, STEP_CLOSE);
         if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
     } else if (factorial(ctx)) {
         launch_bead_forces(ctx, ctx->s0);
@@ -373,7 +375,7 @@ static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* nois
 
 // nsteps device-noise steps.
 static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
-    if (!ctx->split || nsteps < 2) {
+    if (!ctx->split) {
         for (int s = 0; s < nsteps; ++s) {
             if (ctx->gexec) {
                 CK(hipGraphLaunch(ctx->gexec, ctx->s0));
@@ -384,21 +386,22 @@ static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
         }
         return PIMDB_OK;
     }
-    enqueue_open(ctx, nullptr);
-    launch_step_forces(ctx, true);
-    for (int s = 1; s < nsteps; ++s) {
-        launch_step_integrate(ctx);
-        launch_step_forces(ctx, s + 1 < nsteps);
+    if (nsteps == 0) return PIMDB_OK;
+    launch_step_forces(ctx, false, true, STEP_OPEN);
+    launch_step_integrate(ctx, STEP_OPEN);
+    for (int s = 1; s <= nsteps; ++s) {
+        const int mode = s < nsteps ? STEP_FULL : STEP_CLOSE;
+        launch_step_forces(ctx, true, true, mode);
+        launch_step_integrate(ctx, mode);
     }
-    if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
-    enqueue_close(ctx, nullptr);
     CK(hipGetLastError());
     return PIMDB_OK;
 }
 
 // Apply the pending zeroMomentum of the last O-step and clear the partials.
-static int finish_steps(pimdb_ctx* ctx) {
-    if (ctx->prm.fixcom) {
+// (Split steps leave neither.)
+static int finish_steps(pimdb_ctx* ctx, bool host_noise) {
+    if (ctx->prm.fixcom && (host_noise || !ctx->split)) {
         hipLaunchKernelGGL(k_com_subtract, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->N,
                            ctx->P, ctx->D, ctx->com1, ctx->ncom, ctx->p);
         CK(hipMemsetAsync(ctx->com1, 0, sizeof(double) * (size_t)ctx->ncom * ctx->D, ctx->s0));
@@ -704,7 +707,7 @@ int pimdb_step(pimdb_ctx* ctx, int nsteps, const double* host_noise) {
         const int rc = enqueue_steps(ctx, nsteps);
         if (rc) return rc;
     }
-    int rc = finish_steps(ctx);
+    int rc = finish_steps(ctx, host_noise != nullptr);
     if (rc) return rc;
     return check_status(ctx);
 }
@@ -871,7 +874,7 @@ int pimdb_time_kernels(pimdb_ctx* ctx, int reps, double* ms_forces, double* ms_e
         ctx->gexec = held;
         if (rc) return rc;
         *ms_step /= reps;
-        rc = finish_steps(ctx);
+        rc = finish_steps(ctx, false);
         if (rc) return rc;
     }
     CK(hipGetLastError());

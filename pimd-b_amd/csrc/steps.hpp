@@ -20,16 +20,18 @@
 //   (the momenta after a zeroMomentum sum to zero, so cm1 = mean(G1)).  H
 //   depends on no force, and neither does its sum: both are made beside the
 //   forces.  sum(f) is the sum of the external forces (pair, spring and
-//   exchange forces sum to zero up to rounding).
+//   exchange forces sum to zero up to rounding).  The first opening and the
+//   last closing half of a run are the same update with other coefficients
+//   (StepMode), so a run needs no other kernels.
 // * The exchange forces on beads 1 and P need the finished recursions, but
 //   only the integration needs them: it evaluates them itself.
 //
-// k_step_forces: workgroups of 1024 threads take one of three parts, in this
-// order: the recursions (exchange_wide.hpp), tiles of the bead forces
-// (forces.hpp), and tiles of H with the partial sums for the shift.  The
-// recursions' latency covers the rest up to about N = 500.
-// k_step_integrate: the exterior forces and update of beads 1 and P, one wave
-// per particle and bead, and the update of the others, elementwise.
+// Forces kernel: workgroups take one of three parts, in this order: the
+// recursions (exchange_wide.hpp), the bead forces (forces.hpp or, batched,
+// batch.hpp), and tiles of H with the partial sums for the shift.  The
+// recursions' latency covers the rest of a single system up to about N = 500.
+// Integration kernel: the exterior forces and update of beads 1 and P, one
+// wave per particle and bead, and the update of the others, elementwise.
 #pragma once
 
 #include "device_common.hpp"
@@ -41,10 +43,18 @@ namespace pimdb {
 constexpr int STEP_TILE = 64;         // columns (one axis) per noise workgroup
 constexpr int STEP_NM_MAXP = 64;      // beads of the matrix-core noise transform
 
+// What an integration does: p' = alpha (p + beta f) + H - mean(...) + gamma f,
+// then (but for CLOSE) x += dt/m p'.
+enum StepMode : int {
+    STEP_OPEN = 0,    // O, zeroMomentum, B, A with complete forces
+    STEP_FULL = 1,    // the closing half of a step and the opening half of the next
+    STEP_CLOSE = 2,   // B, O, zeroMomentum
+    STEP_FORCES = 3   // nothing but the exterior forces into f
+};
+
 struct StepArgs {
     ForceArgs fa;
     double bt;
-    int nx, nf, nn;                   // workgroups of the three parts
     double *x, *p, *f, *fext;
     // recursions
     double *V, *Vb, *Shi, *Slo, *xc;  // xc: copies [4][D][N] of beads 1, P, 2, P-1
@@ -52,58 +62,83 @@ struct StepArgs {
     int* status;
     // noise and the shift
     int thermostat, nm, fixcom;
-    double c1, c2, half_dt, dt_m;     // dt_m = dt / mass
+    double c1, c2, half_dt, dt_m;     // c1 = 1 without a thermostat; dt_m = dt / mass
     const double* CTt;                // nm -> cart transposed: CTt[k P + b]
     double* H;                        // [P][D][N]
-    double* fpart;                    // [P nt][D] external force sums of the force tiles (null: none)
-    double* hpart;                    // [noise tiles][D] sums of c1^2 p + H
+    double* fpart;                    // [frows][D] partial sums of the external forces (null: none)
+    double* hpart;                    // [noise tiles][D] sums of alpha p + H
+    int frows;
     unsigned long long* ctr;          // steps done
     uint32_t seed;
 };
 
+struct StepCoef {
+    double alpha, beta, gamma, k2, k1;   // H = c2 (k2 xi2 + k1 xi1)
+};
+__device__ __forceinline__ StepCoef step_coef(const StepArgs& s, int mode) {
+    if (mode == STEP_OPEN) return StepCoef{s.c1, 0.0, s.half_dt, 0.0, 1.0};
+    if (mode == STEP_FULL) return StepCoef{s.c1 * s.c1, s.half_dt, s.half_dt, s.c1, 1.0};
+    return StepCoef{s.c1, s.half_dt, 0.0, 1.0, 0.0};
+}
+
 __host__ __device__ inline int step_noise_tiles(int N) { return (N + STEP_TILE - 1) / STEP_TILE; }
+// Noise workgroups of a replica: none where nothing is drawn or summed.
+__host__ __device__ inline int step_noise_groups(const StepArgs& s, int D) {
+    return s.thermostat || s.fixcom ? D * step_noise_tiles(s.fa.N) : 0;
+}
 __host__ __device__ inline int step_pad16(int P) { return (P + 15) & ~15; }
 __host__ __device__ inline size_t step_noise_lds_doubles(int P, bool nm) {
     const size_t Pp = (size_t)step_pad16(P);
-    return XW_WAVES + (nm ? Pp * Pp + Pp * STEP_TILE : 0);
+    return XW_THREADS / WAVE + (nm ? Pp * Pp + Pp * STEP_TILE : 0);
 }
 
 typedef double step_v4d __attribute__((ext_vector_type(4)));
 
 // H of particles i0 .. i0+63 of axis a for all beads, and the tile's sum of
-// c1^2 p + H.  The noise has the keys of the single O-steps: modes (beads)
-// 2m and 2m+1 of column (a, i) from one Box-Muller pair, the closing O-step
-// of the step just made (O-step 1) and the opening one of the next (O-step
-// 0), both at the current step count.  Normal-mode coupling: H = C^T (c1 xi2 +
-// xi1) c2 on the matrix cores (v_mfma_f64_16x16x4f64; lane l, item v:
-// A[l%16][l/16], B[l/16][l%16], D[l/16 + 4v][l%16]).
-template <int D>
-__device__ __forceinline__ void step_noise(const StepArgs& s, int idx, double* smem) {
+// alpha p + H, by a workgroup of NT threads.  The noise has the keys of the
+// single O-steps: modes (beads) 2m and 2m+1 of column (a, i) from one
+// Box-Muller pair, at the current step count with O-step 1 for a closing half
+// (xi2) and 0 for an opening one (xi1).  Normal-mode coupling: C^T on the
+// matrix cores (v_mfma_f64_16x16x4f64; lane l, item v: A[l%16][l/16],
+// B[l/16][l%16], D[l/16 + 4v][l%16]).
+template <int D, int NT>
+__device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx, double* smem) {
+    constexpr int NW = NT / WAVE;
+    const StepCoef co = step_coef(s, mode);
     const int N = s.fa.N, P = s.fa.P, ncols = D * N;
     const int tiles = step_noise_tiles(N);
     const int a = idx / tiles, i0 = (idx % tiles) * STEP_TILE;
     const int nc = min(STEP_TILE, N - i0);
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const uint32_t step = (uint32_t)*s.ctr;
-    const double c1sq = s.c1 * s.c1;
     const int half = (P + 1) / 2;
     double* red = smem;
     double sum = 0.0;
     auto draw = [&](int m, int col, double& g0, double& g1) {
-        double h0, h1;
         const uint32_t key = (uint32_t)((size_t)m * ncols + col);
-        gauss2<true>(key, step, 1u, 0u, s.seed, h0, h1);
-        gauss2<true>(key, step, 0u, 0u, s.seed, g0, g1);
-        g0 = s.c2 * fma(s.c1, h0, g0);
-        g1 = s.c2 * fma(s.c1, h1, g1);
+        g0 = 0.0;
+        g1 = 0.0;
+        if (mode != STEP_OPEN) {
+            gauss2<true>(key, step, 1u, 0u, s.seed, g0, g1);
+            g0 *= co.k2;
+            g1 *= co.k2;
+        }
+        if (mode != STEP_CLOSE) {
+            double h0, h1;
+            gauss2<true>(key, step, 0u, 0u, s.seed, h0, h1);
+            g0 += h0;
+            g1 += h1;
+        }
+        g0 *= s.c2;
+        g1 *= s.c2;
     };
     if (s.thermostat == 0) {
-        for (int e = tid; e < P * STEP_TILE; e += XW_THREADS) {
+        for (int e = tid; e < P * STEP_TILE; e += NT) {
             const int b = e / STEP_TILE, c = e % STEP_TILE;
             if (c < nc) sum += s.p[(size_t)b * ncols + a * N + i0 + c];
         }
     } else if (!s.nm) {
-        for (int e = tid; e < half * STEP_TILE; e += XW_THREADS) {
+        for (int e = tid; e < half * STEP_TILE; e += NT) {
             const int m = e / STEP_TILE, c = e % STEP_TILE;
             if (c >= nc) continue;
             const int col = a * N + i0 + c;
@@ -114,19 +149,19 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int idx, double* s
                 if (2 * m + h < P) {
                     const size_t q = (size_t)(2 * m + h) * ncols + col;
                     s.H[q] = g[h];
-                    sum += fma(c1sq, s.p[q], g[h]);
+                    sum += fma(co.alpha, s.p[q], g[h]);
                 }
             }
         }
     } else {
         const int Pp = step_pad16(P), MB = Pp / 16, KK = Pp / 4;
-        double* CTl = smem + XW_WAVES;          // [k][b], zero padded
-        double* pn = CTl + (size_t)Pp * Pp;     // [column / 16][k][16]
-        for (int e = tid; e < Pp * Pp; e += XW_THREADS) {
+        double* CTl = smem + XW_THREADS / WAVE;   // [k][b], zero padded
+        double* pn = CTl + (size_t)Pp * Pp;       // [column / 16][k][16]
+        for (int e = tid; e < Pp * Pp; e += NT) {
             const int k = e / Pp, b = e % Pp;
             CTl[e] = (k < P && b < P) ? s.CTt[(size_t)k * P + b] : 0.0;
         }
-        for (int e = tid; e < (Pp / 2) * STEP_TILE; e += XW_THREADS) {
+        for (int e = tid; e < (Pp / 2) * STEP_TILE; e += NT) {
             const int m = e / STEP_TILE, c = e % STEP_TILE;
             double g0 = 0.0, g1 = 0.0;
             if (m < half && c < nc) draw(m, a * N + i0 + c, g0, g1);
@@ -136,7 +171,7 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int idx, double* s
         }
         __syncthreads();
         const int q4 = lane / 16, c16 = lane % 16;
-        for (int task = wave; task < MB * (STEP_TILE / 16); task += XW_WAVES) {
+        for (int task = wave; task < MB * (STEP_TILE / 16); task += NW) {
             const int bb = task % MB, g = task / MB, c = g * 16 + c16;
             step_v4d acc = {0.0, 0.0, 0.0, 0.0};
             const double* B = pn + (size_t)g * Pp * 16;
@@ -150,7 +185,7 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int idx, double* s
                 if (b < P && c < nc) {
                     const size_t q = (size_t)b * ncols + a * N + i0 + c;
                     s.H[q] = acc[v];
-                    sum += fma(c1sq, s.p[q], acc[v]);
+                    sum += fma(co.alpha, s.p[q], acc[v]);
                 }
             }
         }
@@ -161,117 +196,146 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int idx, double* s
         __syncthreads();
         if (tid == 0) {
             double t = 0.0;
-            for (int w = 0; w < XW_WAVES; ++w) t += red[w];
+            for (int w = 0; w < NW; ++w) t += red[w];
             s.hpart[(size_t)(idx % tiles) * D + a] = t;
         }
     }
 }
 
-// x, p, f: bead-major SoA [b][a][i].  Dynamic LDS: the largest part's need.
-template <int D, int KIND>
-static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s) {
-    extern __shared__ double smem[];
-    const int wg = blockIdx.x;
-    if (wg < s.nx) {
-        const int N = s.fa.N, P = s.fa.P;
-        const size_t bs = (size_t)D * N;
-        if (wg == 0) {   // beads 2 and P-1 for the exterior forces (the recursions copy beads 1 and P)
-            const double* x2 = s.x + bs * (1 % P);
-            const double* xPm1 = s.x + bs * ((P - 2 + P) % P);
-            for (int e = threadIdx.x; e < D * N; e += XW_THREADS) {
-                s.xc[2 * bs + e] = x2[e];
-                s.xc[3 * bs + e] = xPm1[e];
-            }
-        }
-        xw_recursions<D>(smem, wg, N, s.bt, s.fa.k_spring, s.fa.pbc, s.fa.L, s.x, s.x + bs * (P - 1), s.V, s.Vb, s.Shi,
-                         s.Slo, s.xc, s.pub, s.status);
-    } else if (wg < s.nx + s.nf) {
-        const int nt = (s.fa.N + FORCE_TILE - 1) / FORCE_TILE, id = wg - s.nx;
-        bead_forces_tile<D, KIND>(s.fa, id / nt, id % nt, s.x, s.f, s.fext, s.fpart, smem);
-    } else {
-        step_noise<D>(s, wg - s.nx - s.nf, smem);
-    }
-}
-
-// Workgroups of k_step_integrate: 4 (particle, bead) tasks of the exchange
-// beads each, then 256 elements of the other beads each.
-__host__ __device__ inline int step_exterior_groups(const ForceArgs& fa) { return fa.bosonic ? (2 * fa.N + 3) / 4 : 0; }
-__host__ __device__ inline size_t step_inner_elements(const ForceArgs& fa, int D) {
-    return (size_t)(fa.bosonic ? fa.P - 2 : fa.P) * D * fa.N;
-}
-
-// The closing half of a step and the opening half of the next (file header).
-// Leaves f complete.  The positions that other particles' exterior forces
-// need are read from the copies xc, so x is free to be written.
-template <int D>
-static __global__ void __launch_bounds__(256) k_step_integrate(StepArgs s) {
+// Workgroup wg of xw_grid(N): the recursions (exchange_wide.hpp), with copies
+// of the beads that the exterior forces read after the positions moved on.
+template <int D, int NT>
+__device__ __forceinline__ void step_recursions(const StepArgs& s, int wg, double* smem) {
     const int N = s.fa.N, P = s.fa.P;
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    __shared__ double shift[4];
-    const int ng = step_exterior_groups(s.fa);
-    const bool exterior = (int)blockIdx.x < ng;
     const size_t bs = (size_t)D * N;
-    const double c1sq = s.c1 * s.c1, h = s.half_dt;
+    if (wg == 0) {   // beads 2 and P-1 (the recursions copy beads 1 and P)
+        const double* x2 = s.x + bs * (1 % P);
+        const double* xPm1 = s.x + bs * ((P - 2 + P) % P);
+        for (int e = threadIdx.x; e < D * N; e += NT) {
+            s.xc[2 * bs + e] = x2[e];
+            s.xc[3 * bs + e] = xPm1[e];
+        }
+    }
+    xw_recursions<D, NT>(smem, wg, N, s.bt, s.fa.k_spring, s.fa.pbc, s.fa.L, s.x, s.x + bs * (P - 1), s.V, s.Vb, s.Shi,
+                         s.Slo, s.xc, s.pub, s.status);
+}
+
+// Workgroups of an integration: 4 tasks of M particles of an exchange bead each
+// (their forces are complete before an opening half), then 256 elements of the
+// other beads each.
+__host__ __device__ inline int step_exterior_tasks(int N, int M) { return (N + M - 1) / M; }   // per bead
+__host__ __device__ inline int step_exterior_groups(const ForceArgs& fa, int mode, int M) {
+    return fa.bosonic && mode != STEP_OPEN ? (2 * step_exterior_tasks(fa.N, M) + 3) / 4 : 0;   // (also STEP_FORCES)
+}
+__host__ __device__ inline size_t step_inner_elements(const ForceArgs& fa, int D, int mode) {
+    return (size_t)(fa.bosonic && mode != STEP_OPEN ? fa.P - 2 : fa.P) * D * fa.N;
+}
+__host__ __device__ inline int step_integrate_groups(const ForceArgs& fa, int D, int mode, int M) {
+    return step_exterior_groups(fa, mode, M) + (int)((step_inner_elements(fa, D, mode) + 255) / 256);
+}
+
+// Workgroup blk of an integration, 256 threads (file header).  Leaves f
+// complete.  The positions that other particles' exterior forces need are
+// read from the copies xc, so x is free to be written.
+// M: particles per wave of the exterior forces (1 for a single ring, where
+// latency counts; more where many rings share the card).
+template <int D, int M>
+__device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int blk) {
+    const StepCoef co = step_coef(s, mode);
+    const int N = s.fa.N, P = s.fa.P;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    __shared__ double shift[4];
+    const int ng = step_exterior_groups(s.fa, mode, M), nt = step_exterior_tasks(N, M);
+    const bool exterior = blk < ng;
+    const size_t bs = (size_t)D * N;
     // the element's (or, exterior, lane's) data first: the loads overlap the
     // reduction below
-    const int task = blockIdx.x * 4 + wave;
+    const int task = blk * 4 + wave;
     size_t e = 0;
     bool mine = false;
     int ax = 0;
     if (exterior) {
-        const int which = task / N, l = task % N;
-        if (task < 2 * N && lane < D) {
+        const int which = task / nt, l = (task % nt) * M + lane / D;   // lane: particle and axis
+        if (task < 2 * nt && lane < M * D && l < N) {
             mine = true;
-            ax = lane;
-            e = ((size_t)(which == 0 ? 0 : P - 1) * D + lane) * N + l;
+            ax = lane % D;
+            e = ((size_t)(which == 0 ? 0 : P - 1) * D + ax) * N + l;
         }
     } else {
-        const size_t o = (size_t)(blockIdx.x - ng) * 256 + tid;
-        mine = o < step_inner_elements(s.fa, D);
-        e = o + (s.fa.bosonic ? bs : 0);
+        const size_t o = (size_t)(blk - ng) * 256 + tid;
+        mine = o < step_inner_elements(s.fa, D, mode);
+        e = o + (ng ? bs : 0);
         ax = (int)((e / N) % D);
     }
     double pv = 0.0, fv = 0.0, xv = 0.0, hv = 0.0;
+    if (mode == STEP_FORCES && !exterior) return;
     if (mine) {
-        pv = s.p[e];
         fv = s.f[e];
-        xv = s.x[e];
-        if (s.thermostat) hv = s.H[e];
+        if (mode != STEP_FORCES) {
+            pv = s.p[e];
+            if (mode != STEP_CLOSE) xv = s.x[e];
+            if (s.thermostat) hv = s.H[e];
+        }
     }
-    if (s.fixcom) {
+    if (s.fixcom && mode != STEP_FORCES) {
         if (wave < D) {
             const int rows = step_noise_tiles(N);
             double t = 0.0;
             for (int r = lane; r < rows; r += WAVE) t += s.hpart[(size_t)r * D + wave];
-            if (s.fpart) {
-                const int nt = P * ((N + FORCE_TILE - 1) / FORCE_TILE);
+            if (s.fpart && mode != STEP_OPEN) {
                 double u = 0.0;
-                for (int r = lane; r < nt; r += WAVE) u += s.fpart[(size_t)r * D + wave];
-                t = fma(c1sq * h, u, t);
+                for (int r = lane; r < s.frows; r += WAVE) u += s.fpart[(size_t)r * D + wave];
+                t = fma(co.alpha * co.beta, u, t);
             }
             t = wave_total(t);
             if (lane == 0) shift[wave] = t / (double)(N * P);
         }
         __syncthreads();
     }
-    if (blockIdx.x == 0 && tid == 0) *s.ctr += 1;
     if (exterior) {
-        if (task >= 2 * N) return;
-        const int which = task / N, l = task % N;
+        if (task >= 2 * nt) return;
         const Ring r = make_ring(s.xc, s.xc + bs, s.Shi, s.Slo, s.fa.k_spring, s.fa.pbc != 0, s.fa.L);
-        double F[D];
-        exterior_force<D>(which, l, N, lane, s.bt, s.fa.k_spring, r, s.V, s.Vb, s.xc + 2 * bs, s.xc + 3 * bs, false, F);
+        double F[M][D];
+        exterior_force<D, M>(task / nt, (task % nt) * M, N, lane, s.bt, s.fa.k_spring, r, s.V, s.Vb, s.xc + 2 * bs,
+                             s.xc + 3 * bs, false, F);
 #pragma unroll
-        for (int a = 0; a < D; ++a)
-            if (lane == a) fv = F[a] + fv;
+        for (int q = 0; q < M * D; ++q)
+            if (lane == q) fv = F[q / D][q % D] + fv;
         if (mine) s.f[e] = fv;
     }
-    if (!mine) return;
-    const double hf = h * fv;
-    double v = fma(c1sq, pv + hf, hv) + hf;
+    if (!mine || mode == STEP_FORCES) return;
+    double v = fma(co.alpha, fma(co.beta, fv, pv), hv);
     if (s.fixcom) v -= shift[ax];
-    s.p[e] = v;
-    s.x[e] = fma(s.dt_m, v, xv);
+    if (mode == STEP_CLOSE) {
+        s.p[e] = v;
+    } else {
+        v = fma(co.gamma, fv, v);
+        s.p[e] = v;
+        s.x[e] = fma(s.dt_m, v, xv);
+    }
+}
+
+// ---- one system ----
+// nx, nf: workgroups of the recursions and of the force tiles; the rest make
+// noise.  x, p, f: bead-major SoA [b][a][i].  Dynamic LDS: the largest part's.
+template <int D, int KIND>
+static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, int nx, int nf, int mode) {
+    extern __shared__ double smem[];
+    const int wg = blockIdx.x;
+    if (wg < nx) {
+        step_recursions<D, XW_THREADS>(s, wg, smem);
+    } else if (wg < nx + nf) {
+        const int nt = (s.fa.N + FORCE_TILE - 1) / FORCE_TILE, id = wg - nx;
+        bead_forces_tile<D, KIND>(s.fa, id / nt, id % nt, s.x, s.f, s.fext, s.fpart, smem);
+    } else {
+        step_noise<D, XW_THREADS>(s, mode, wg - nx - nf, smem);
+    }
+}
+
+template <int D>
+static __global__ void __launch_bounds__(256) k_step_integrate(StepArgs s, int mode) {
+    if (blockIdx.x == 0 && threadIdx.x == 0 && mode != STEP_CLOSE) *s.ctr += 1;
+    step_integrate<D, 1>(s, mode, blockIdx.x);
 }
 
 }  // namespace pimdb
