@@ -196,6 +196,18 @@ void pimdb_xplan_destroy(pimdb_xplan* plan);
 int pimdb_xplan_forward(pimdb_xplan* plan, const double* x1, const double* xP, double* VB, double* V,
                         double* Vb, void* stream);
 int pimdb_xplan_vb_grad(pimdb_xplan* plan, const double* x1, const double* xP, double* grad, void* stream);
+/* The pair for reverse-mode differentiation.  forward_saved reads particle i,
+ * axis a of bead 1 at x1[i s1n + a s1d] (strides in doubles; xP alike), writes
+ * V_B to VB and what the backward pass needs (V, Vb, the ring's prefix sums and
+ * its own copy of the beads) to saved, pimdb_xplan_saved_doubles() doubles, and
+ * returns after `stream` is done.  backward_saved writes scale dV_B/dx1 and
+ * scale dV_B/dxP as [particle][axis] (scale: one device double, or NULL for 1)
+ * from saved alone; it is ordered by `stream` and does not wait for it. */
+long long pimdb_xplan_saved_doubles(const pimdb_xplan* plan);
+int pimdb_xplan_forward_saved(pimdb_xplan* plan, const double* x1, long long s1n, long long s1d, const double* xP,
+                              long long sPn, long long sPd, double* VB, double* saved, void* stream);
+int pimdb_xplan_backward_saved(pimdb_xplan* plan, const double* saved, const double* scale, double* d1, double* dP,
+                               void* stream);
 
 /* pimdb_xplan_create + pimdb_xplan_forward (VB only) + pimdb_xplan_vb_grad in
  * one call that allocates nothing: the same kernels, with their workspace

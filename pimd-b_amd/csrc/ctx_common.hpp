@@ -6,7 +6,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <mutex>
 #include <string>
+#include <vector>
 
 #include "pimdb_gpu.h"
 #include "exchange.hpp"
@@ -210,19 +212,29 @@ inline size_t device_lds_limit() {
 // take k_exchange_recursions_gws.
 inline bool exchange_wide(int N, int D) { return xw_lds_bytes(N, D) <= device_lds_limit(); }
 
-// Both recursions of one ring.  pub: xw_pub_words(N) words holding XW_EMPTY
-// (exchange_wide rings); ws: 2 rec_lds_bytes(N, D) bytes (the others).
+// The recursions of a ring for which exchange_wide holds.  VB and xc may be
+// null (xw_recursions).
+inline void launch_exchange_wide(int D, int N, double bt, double k, int pbc, double L, BeadView x1, BeadView xP,
+                                 double* V, double* Vb, double* VB, double* Shi, double* Slo, double* xc,
+                                 unsigned long long* pub, int* status, hipStream_t s) {
+    const dim3 grid(xw_grid(N)), blk(XW_THREADS);
+    const size_t lds = xw_lds_bytes(N, D);
+    switch (D) {
+    case 1: hipLaunchKernelGGL(k_exchange_wide<1>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status); break;
+    case 2: hipLaunchKernelGGL(k_exchange_wide<2>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status); break;
+    default: hipLaunchKernelGGL(k_exchange_wide<3>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status); break;
+    }
+}
+
+// Both recursions of one ring, x1 and xP SoA [a][i].  pub: xw_pub_words(N)
+// words holding XW_EMPTY (exchange_wide rings); ws: 2 rec_lds_bytes(N, D)
+// bytes (the others).
 inline void launch_exchange_recursions(int D, int N, double bt, double k, int pbc, double L, const double* x1,
                                        const double* xP, double* V, double* Vb, double* Shi, double* Slo,
                                        unsigned long long* pub, double* ws, int* status, hipStream_t s) {
     if (exchange_wide(N, D)) {
-        const dim3 grid(xw_grid(N)), blk(XW_THREADS);
-        const size_t lds = xw_lds_bytes(N, D);
-        switch (D) {
-        case 1: hipLaunchKernelGGL(k_exchange_wide<1>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
-        case 2: hipLaunchKernelGGL(k_exchange_wide<2>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
-        default: hipLaunchKernelGGL(k_exchange_wide<3>, grid, blk, lds, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, pub, status); break;
-        }
+        launch_exchange_wide(D, N, bt, k, pbc, L, BeadView{x1, N, 1}, BeadView{xP, N, 1}, V, Vb, nullptr, Shi, Slo,
+                             nullptr, pub, status, s);
         return;
     }
     switch (D) {
@@ -230,6 +242,48 @@ inline void launch_exchange_recursions(int D, int N, double bt, double k, int pb
     case 2: hipLaunchKernelGGL(k_exchange_recursions_gws<2>, dim3(2), dim3(1024), 0, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status, ws); break;
     default: hipLaunchKernelGGL(k_exchange_recursions_gws<3>, dim3(2), dim3(1024), 0, s, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, status, ws); break;
     }
+}
+
+// Status flags in pinned host memory (the host pointer serves the kernels
+// too), one per context or plan: slots of one page that the process keeps,
+// since a pinned allocation of its own costs 0.1 ms, and an allocation each
+// beyond its 1024 slots.  Any thread.
+class StatusPool {
+    static constexpr int SLOTS = 1024;
+    std::mutex mu;
+    int* page = nullptr;
+    std::vector<int> free_slots;
+
+public:
+    int* take() {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!page) {
+            if (hipHostMalloc((void**)&page, SLOTS * sizeof(int), hipHostMallocPortable) != hipSuccess) {
+                page = nullptr;
+                return nullptr;
+            }
+            for (int i = SLOTS - 1; i >= 0; --i) free_slots.push_back(i);
+        }
+        int* p = nullptr;
+        if (free_slots.empty()) {
+            if (hipHostMalloc((void**)&p, sizeof(int), hipHostMallocPortable) != hipSuccess) return nullptr;
+        } else {
+            p = page + free_slots.back();
+            free_slots.pop_back();
+        }
+        *p = 0;
+        return p;
+    }
+    void give(int* p) {   // its kernels are done
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        if (page && p >= page && p < page + SLOTS) free_slots.push_back((int)(p - page));
+        else (void)hipHostFree(p);
+    }
+};
+inline StatusPool& status_pool() {
+    static StatusPool* pool = new StatusPool();   // (never destroyed: objects may be released at process end)
+    return *pool;
 }
 
 inline void launch_cycle_energies(int D, int N, const double* x1, const double* xP, double k, int pbc, double L,
@@ -285,8 +339,23 @@ inline void launch_bead_energies(int D, const pimdb_params& p, const Derived& d,
     }
 }
 
+// k_ring_estimator's sums -> {primitive estimator, distinct and longest
+// probabilities} (quadratic_bosonic_exchange.cpp:222-279).
+inline void combine_estimators(int N, int P, double bt, const double* est, double* out) {
+    double mean = 0.0, ones = 0.0;
+    for (int l = 0; l < N; ++l) {
+        mean += est[l];
+        ones += est[N + l];
+    }
+    const double VN = est[2 * (size_t)N + 1];
+    out[0] = -mean / P;
+    out[1] = std::exp(-bt * (ones - VN) - std::lgamma((double)N + 1.0));
+    out[2] = std::exp(-bt * (est[2 * (size_t)N] - VN));
+}
+
 // Per-bead sums -> the observables the reference's ObservablesLogger prints
 // after its MPI_Allreduce over beads (observable.cpp:92-116), in atomic units.
+// prim: {primitive estimator, distinct and longest probabilities} (bosonic).
 inline void combine_observables(const pimdb_params& p, const Derived& d, const double* sums, const double* epart,
                                 int nt, const double* prim, double VN, double* out) {
     const int N = p.natoms, P = p.nbeads, D = p.ndim;

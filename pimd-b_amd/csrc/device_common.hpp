@@ -30,6 +30,9 @@ struct Aziz {
 };
 constexpr double HARD_CORE_EPS = 1.0E-7;   // include/common.h:193
 
+// Raises an error flag (device or pinned host memory; every writer stores 1).
+__device__ __forceinline__ void raise_status(int* status) { *(volatile int*)status = 1; }
+
 // dx - L floor(dx/L + 1/2), src/common.cpp:41-43.
 __device__ __forceinline__ double min_image(double dx, double L) {
 #pragma clang fp contract(off)
@@ -187,48 +190,8 @@ __device__ __forceinline__ double exp2_pair(double x) {
 }
 
 // Scalar factor g(r) of the interaction gradient, gradV(d) = g * d
-// (harmonic.cpp:21-23, dipole.cpp:24-45, aziz.cpp:56-106).  `norm` is |d|.
-template <int KIND>
-__device__ __forceinline__ double pair_grad_factor(double norm, double kpair, double strength) {
-    if constexpr (KIND == POT_HARMONIC) {
-        return kpair;
-    } else if constexpr (KIND == POT_DIPOLE) {
-        return -3.0 * strength / (norm * norm * norm * norm * norm);
-    } else if constexpr (KIND == POT_AZIZ) {
-        const double r = norm / Aziz::rm;
-        const double T1 = -Aziz::A * Aziz::alpha * exp(-Aziz::alpha * r);
-        double g;
-        if (r > HARD_CORE_EPS && r < 0.01) {
-            g = T1 * (Aziz::epsilon / Aziz::rm);
-        } else {
-            const double ix = 1.0 / r;
-            const double ix2 = ix * ix;
-            const double ix6 = ix2 * ix2 * ix2;
-            const double ix7 = ix6 * ix;
-            const double ix8 = ix6 * ix2;
-            const double ix9 = ix8 * ix;
-            const double ix10 = ix8 * ix2;
-            const double ix11 = ix10 * ix;
-            double F = 1.0, dF = 0.0;
-            if (r < Aziz::D) {
-                // aziz.h:25-43: F uses D/x, dF uses D*(1/x); one exponential
-                // serves both (the two arguments differ by at most an ulp).
-                const double t = Aziz::D * ix - 1.0;
-                const double ex = exp(-t * t);
-                F = ex;
-                dF = 2.0 * Aziz::D * ix * ix * t * ex;
-            }
-            const double T2 = (6.0 * Aziz::C6 * ix7 + 8.0 * Aziz::C8 * ix9 + 10.0 * Aziz::C10 * ix11) * F;
-            const double T3 = -(Aziz::C6 * ix6 + Aziz::C8 * ix8 + Aziz::C10 * ix10) * dF;
-            g = (Aziz::epsilon / Aziz::rm) * (T1 + T2 + T3);
-        }
-        return g / norm;
-    } else {
-        return 0.0;
-    }
-}
-
-// g(r) as above from |d| and 1/|d| with products in place of the
+// (harmonic.cpp:21-23, dipole.cpp:24-45, aziz.cpp:56-106), from |d| and 1/|d|
+// with products in place of the
 // reference's divisions (norm/rm, 1/r, g/norm), the dispersion terms
 // factored as polynomials in ix^2, and exp_pair in place of the library exp:
 // within a few 1e-14 relative.  For Aziz the factor epsilon/rm is folded into the
@@ -329,29 +292,6 @@ __device__ __forceinline__ double ext_energy(const ExtPot& e, const double (&x)[
         return s * e.d;
     }
     return 0.0;
-}
-
-// Pair potential energy V(d) (harmonic.cpp:9-19, dipole.cpp:5-22, aziz.cpp:18-54).
-template <int KIND>
-__device__ __forceinline__ double pair_energy(double norm, double r2, double kpair, double strength) {
-    if constexpr (KIND == POT_HARMONIC) {
-        return 0.5 * kpair * r2;
-    } else if constexpr (KIND == POT_DIPOLE) {
-        return strength / (norm * norm * norm);
-    } else if constexpr (KIND == POT_AZIZ) {
-        const double r = norm / Aziz::rm;
-        const double Urep = Aziz::A * exp(-Aziz::alpha * r);
-        if (r > HARD_CORE_EPS && r < 0.01) return Aziz::epsilon * Urep;
-        const double ix2 = 1.0 / (r * r);
-        const double ix6 = ix2 * ix2 * ix2;
-        const double ix8 = ix6 * ix2;
-        const double ix10 = ix8 * ix2;
-        const double F = (r < Aziz::D) ? exp(-(Aziz::D / r - 1.0) * (Aziz::D / r - 1.0)) : 1.0;
-        const double Uatt = -(Aziz::C6 * ix6 + Aziz::C8 * ix8 + Aziz::C10 * ix10) * F;
-        return Aziz::epsilon * (Urep + Uatt);
-    } else {
-        return 0.0;
-    }
 }
 
 // ---- wave-level reductions (DPP/permute through the compiler's shuffles) ----

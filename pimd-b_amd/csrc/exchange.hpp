@@ -499,7 +499,7 @@ __device__ void exchange_recursion(int N, double bt, const Ring& r, double* __re
             if (t < nb) {
                 const double u = sh.R[t] - log(z);
                 sh.U[n0 + t] = u;
-                if (!isfinite(u)) atomicOr(status, 1);
+                if (!isfinite(u)) raise_status(status);
             }
         }
         __syncthreads();
@@ -709,6 +709,33 @@ static __global__ void __launch_bounds__(256) k_exchange_vb_grad(int N, double b
     if (lane == 0) {
 #pragma unroll
         for (int a = 0; a < D; ++a) out[((size_t)which * D + a) * N + l] = F[0][a];
+    }
+}
+
+// scale dV_B/dx1 and scale dV_B/dxP from what a forward pass left (V, Vb, the
+// prefix sums and the beads, SoA), as d1, dP [N][D]; scale: a device value or
+// null (1).
+template <int D>
+static __global__ void __launch_bounds__(256) k_exchange_backward(int N, double bt, double k, int pbc, double L,
+                                                           const double* __restrict__ Shi,
+                                                           const double* __restrict__ Slo,
+                                                           const double* __restrict__ V,
+                                                           const double* __restrict__ Vb, const double* __restrict__ xc,
+                                                           const double* __restrict__ scale, double* __restrict__ d1,
+                                                           double* __restrict__ dP) {
+    const int task = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+    if (task >= 2 * N) return;
+    const int which = task / N, l = task % N;
+    const int lane = threadIdx.x % WAVE;
+    const double* xP = xc + (size_t)D * N;
+    const Ring r = make_ring(xc, xP, Shi, Slo, k, pbc != 0, L);
+    const double g = scale ? *scale : 1.0;
+    double F[1][D];
+    exterior_force<D>(which, l, N, lane, bt, k, r, V, Vb, xc, xP, true, F);
+    if (lane == 0) {
+        double* out = (which == 0 ? d1 : dP) + (size_t)l * D;
+#pragma unroll
+        for (int a = 0; a < D; ++a) out[a] = -F[0][a] * g;   // (F is -dV_B/dx)
     }
 }
 

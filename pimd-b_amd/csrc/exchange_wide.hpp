@@ -109,20 +109,27 @@ __device__ __forceinline__ DD dd_wave_scan(DD v) {
     return v;
 }
 
+// One bead's positions: axis a of particle i at p[a sa + i si].
+struct BeadView {
+    const double* p;
+    long long sa, si;
+    __device__ __forceinline__ double at(int a, int i) const { return p[a * sa + i * si]; }
+};
+
 // Beads 1 and P into LDS and the split prefix sums of the ring's links
 // (exchange.hpp, Ring), by the whole workgroup: every thread sums a run of
 // links, the waves scan their totals.  Every workgroup of a ring computes the
 // same values.  Shi_out / Slo_out / xc_out (may be null) receive the sums and
 // a copy [2][D][N] of the two beads.
 template <int D, int NT>
-__device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, const double* __restrict__ x1,
-                                         const double* __restrict__ xP, double k, bool pbc, double L,
+__device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, BeadView x1, BeadView xP, double k, bool pbc, double L,
                                          double* Shi_out, double* Slo_out, double* xc_out) {
     constexpr int NW = NT / WAVE;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const Ring r = make_ring(sh.x1, sh.xP, sh.Shi, sh.Slo, k, pbc, L);
     for (int e = tid; e < D * N; e += NT) {
-        const double u = x1[e], v = xP[e];
+        const int a = D == 1 ? 0 : e / N, i = e - a * N;
+        const double u = x1.at(a, i), v = xP.at(a, i);
         sh.x1[e] = u;
         sh.xP[e] = v;
         if (xc_out) {
@@ -134,7 +141,7 @@ __device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, const double
     auto link = [&](int v) {
         double d[D];
 #pragma unroll
-        for (int ax = 0; ax < D; ++ax) d[ax] = ring_image(x1[ax * N + v + 1] - xP[ax * N + v], r);
+        for (int ax = 0; ax < D; ++ax) d[ax] = ring_image(x1.at(ax, v + 1) - xP.at(ax, v), r);
         return norm2_fma<D>(d);
     };
     DD sum{0.0, 0.0};
@@ -215,7 +222,7 @@ __device__ __forceinline__ double xw_wait(unsigned long long* p, int lane, int* 
         b = __hip_atomic_load(p + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__all(b != XW_EMPTY)) break;
         if (++spin >= XW_SPIN) {
-            if (lane == 0) atomicOr(status, 1);
+            if (lane == 0) raise_status(status);
             break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -291,7 +298,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, do
 template <int DIR, int D, int NT>
 __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r, const XwShared& sh,
                                          unsigned long long* __restrict__ pub, double* __restrict__ V,
-                                         double* __restrict__ Vb, int* __restrict__ status) {
+                                         double* __restrict__ Vb, double* __restrict__ VB, int* __restrict__ status) {
     constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // sources of a block per wave
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int ntarget = DIR == 0 ? N : N - 1;
@@ -393,7 +400,7 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
     if (*sh.flag) {
         u = xw_block_safe<DIR, D, NT>(I, N, nb, bk, u0, r, sh, pub);
         if (wave == 0) {
-            if (lane < nb && !isfinite(u)) atomicOr(status, 1);
+            if (lane < nb && !isfinite(u)) raise_status(status);
             if (!last) xw_publish(pub + n0 + lane, u + lgs);
         }
     }
@@ -401,7 +408,10 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         const int n = n0 + lane;
         if (DIR == 0) {
             V[n] = u / bt;
-            if (n == N) Vb[0] = u / bt;   // V_backwards[0] = V[N], :127
+            if (n == N) {
+                Vb[0] = u / bt;   // V_backwards[0] = V[N], :127
+                if (VB) *VB = u / bt;
+            }
         } else {
             Vb[N - n] = u / bt;
         }
@@ -415,29 +425,28 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
 // Workgroup b of xw_grid(N): block b / 2, forward (even) or backward (odd);
 // lower blocks first.  pub: xw_pub_words(N) words, all XW_EMPTY on entry and
 // on return.  Block 0's forward workgroup writes the prefix sums and, where
-// asked, the beads' copy.
+// asked (xc, VB not null), the beads' copy and V[N].
 template <int D, int NT>
 __device__ __forceinline__ void xw_recursions(double* smem, int b, int N, double bt, double k, int pbc, double L,
-                                              const double* __restrict__ x1, const double* __restrict__ xP,
-                                              double* __restrict__ V, double* __restrict__ Vb, double* __restrict__ Shi,
-                                              double* __restrict__ Slo, double* __restrict__ xc,
+                                              BeadView x1, BeadView xP, double* __restrict__ V,
+                                              double* __restrict__ Vb, double* __restrict__ VB,
+                                              double* __restrict__ Shi, double* __restrict__ Slo, double* __restrict__ xc,
                                               unsigned long long* __restrict__ pub, int* __restrict__ status) {
     const XwShared sh = xw_carve<NT>(smem, N, D);
     const bool first = b == 0;
     const Ring r = xw_stage<D, NT>(sh, N, x1, xP, k, pbc != 0, L, first ? Shi : nullptr, first ? Slo : nullptr,
                                first ? xc : nullptr);
-    if ((b & 1) == 0) xw_block<0, D, NT>(b >> 1, N, bt, r, sh, pub, V, Vb, status);
-    else xw_block<1, D, NT>(b >> 1, N, bt, r, sh, pub + N + 1, V, Vb, status);
+    if ((b & 1) == 0) xw_block<0, D, NT>(b >> 1, N, bt, r, sh, pub, V, Vb, VB, status);
+    else xw_block<1, D, NT>(b >> 1, N, bt, r, sh, pub + N + 1, V, Vb, nullptr, status);
 }
 
 template <int D>
 static __global__ void __launch_bounds__(XW_THREADS)
-k_exchange_wide(int N, double bt, double k, int pbc, double L, const double* __restrict__ x1,
-                const double* __restrict__ xP, double* __restrict__ V, double* __restrict__ Vb,
-                double* __restrict__ Shi, double* __restrict__ Slo, unsigned long long* __restrict__ pub,
-                int* __restrict__ status) {
+k_exchange_wide(int N, double bt, double k, int pbc, double L, BeadView x1, BeadView xP, double* __restrict__ V,
+                double* __restrict__ Vb, double* __restrict__ VB, double* __restrict__ Shi, double* __restrict__ Slo,
+                double* __restrict__ xc, unsigned long long* __restrict__ pub, int* __restrict__ status) {
     extern __shared__ double smem[];
-    xw_recursions<D, XW_THREADS>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, Shi, Slo, nullptr, pub, status);
+    xw_recursions<D, XW_THREADS>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status);
 }
 
 }  // namespace pimdb

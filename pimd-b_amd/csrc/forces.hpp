@@ -145,16 +145,54 @@ k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f
     bead_forces_tile<D, KIND, GX>(fa, blockIdx.y, blockIdx.x, x, f, fext, nullptr, smem);
 }
 
-// Pair and external potential energies and virial per bead, for the energy
-// observable (src/observables/energy.cpp:56-111): out[b] = {ext_pot, int_pot,
-// virial_sum} (un-normalised sums of the reference).
-// GX as for k_bead_forces.
+// Pair energy V and g with gradV = g d (harmonic.cpp:9-23, dipole.cpp:5-45,
+// aziz.cpp:18-106) from r^2, sharing the root, the exponentials and the
+// reciprocal powers; each elementary function within an ulp or so.
+template <int KIND>
+__device__ __forceinline__ void pair_energy_grad(double r2, double kpair, double strength, double& e, double& g) {
+    const double inv = rsqrt_refined(r2), norm = r2 * inv;
+    if constexpr (KIND == POT_HARMONIC) {
+        e = 0.5 * kpair * r2;
+        g = kpair;
+    } else if constexpr (KIND == POT_DIPOLE) {
+        const double i2 = inv * inv;
+        e = strength * (i2 * inv);
+        g = -3.0 * strength * (i2 * i2 * inv);
+    } else if constexpr (KIND == POT_AZIZ) {
+        const double ix = Aziz::rm * inv, ix2 = ix * ix, ix6 = ix2 * ix2 * ix2;
+        const double rep = Aziz::A * exp_minimax((-Aziz::alpha / Aziz::rm) * norm);
+        const double pe = fma(fma(Aziz::C10, ix2, Aziz::C8), ix2, Aziz::C6);
+        double F = 1.0, att = ix6 * pe;
+        double datt = ix6 * ix * fma(fma(10.0 * Aziz::C10, ix2, 8.0 * Aziz::C8), ix2, 6.0 * Aziz::C6);
+        if (norm < Aziz::D * Aziz::rm) {
+            if (norm > HARD_CORE_EPS * Aziz::rm && norm < 0.01 * Aziz::rm) {   // the repulsion alone
+                att = 0.0;
+                datt = 0.0;
+            } else {
+                const double t = fma(Aziz::D, ix, -1.0);
+                F = exp_minimax(-t * t);
+                datt = F * fma(-2.0 * Aziz::D * ix2 * t, att, datt);
+                att *= F;
+            }
+        }
+        e = Aziz::epsilon * (rep - att);
+        g = (Aziz::epsilon / Aziz::rm) * (datt - Aziz::alpha * rep) * inv;
+    } else {
+        e = 0.0;
+        g = 0.0;
+    }
+}
+
+// Pair and external potential energies and virial of particles tile*64 .. +63
+// of bead b, by a workgroup of 1024 threads, for the energy observable
+// (src/observables/energy.cpp:56-111): part[(b nt + tile)] = {ext_pot, int_pot,
+// virial_sum} (un-normalised sums of the reference; pairs (i, j > i), the
+// virial with r_i alone).  The waves take the partners j > i in turn.  GX and
+// smem as for bead_forces_tile.
 template <int D, int KIND, bool GX = false>
-static __global__ void __launch_bounds__(FORCE_TILE * FORCE_WAVES)
-k_bead_energies(ForceArgs fa, const double* __restrict__ x, double* __restrict__ part) {
-    extern __shared__ double smem[];
+__device__ __forceinline__ void bead_energies_tile(const ForceArgs& fa, int b, int tile, const double* __restrict__ x,
+                                                   double* __restrict__ part, double* smem) {
     const int N = fa.N;
-    const int b = blockIdx.y;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     const size_t bs = (size_t)D * N;
     const double* xb = x + bs * b;
@@ -162,12 +200,13 @@ k_bead_energies(ForceArgs fa, const double* __restrict__ x, double* __restrict__
     if constexpr (GX) {
         sx = xb;
     } else {
-        for (int e = tid; e < D * N; e += blockDim.x) smem[e] = xb[e];
+        for (int e = tid; e < D * N; e += FORCE_TILE * FORCE_WAVES) smem[e] = xb[e];
         __syncthreads();
         sx = smem;
     }
-    const int i = blockIdx.x * FORCE_TILE + lane;
+    const int i = tile * FORCE_TILE + lane;
     const bool pbc = fa.pbc != 0;
+    const double invL = pbc ? 1.0 / fa.L : 0.0;
     double ext = 0.0, ipot = 0.0, vir = 0.0;
     if (i < N) {
         double xi[D];
@@ -182,28 +221,27 @@ k_bead_energies(ForceArgs fa, const double* __restrict__ x, double* __restrict__
         }
         if constexpr (KIND != POT_FREE) {
             if (fa.cutoff != 0.0) {
-                // pairs (i, j > i): energy.cpp:76-94, virial uses r_i only (i < j)
-                const int chunk = (N + FORCE_WAVES - 1) / FORCE_WAVES;
-                const int jlo = max(i + 1, wave * chunk), jhi = min(N, wave * chunk + chunk);
-                for (int j = jlo; j < jhi; ++j) {
+                const bool all = fa.cutoff < 0.0;
+                for (int j = tile * FORCE_TILE + 1 + wave; j < N; j += FORCE_WAVES) {
                     double d[D];
 #pragma unroll
-                    for (int a = 0; a < D; ++a) d[a] = disp(sx[a * N + j], xi[a], pbc, fa.L);
+                    for (int a = 0; a < D; ++a) d[a] = disp_fast(sx[a * N + j], xi[a], pbc, fa.L, invL);
                     const double r2 = norm2<D>(d);
-                    const double norm = sqrt(r2);
-                    if (norm < fa.cutoff || fa.cutoff < 0.0) {
-                        const double g = pair_grad_factor<KIND>(norm, fa.int_k, fa.strength);
-                        ipot += pair_energy<KIND>(norm, r2, fa.int_k, fa.strength);
+                    if (j > i && (all || r2 < fa.cut2)) {
+                        double e, g, xd = 0.0;
+                        pair_energy_grad<KIND>(r2, fa.int_k, fa.strength, e, g);
+                        ipot += e;
 #pragma unroll
-                        for (int a = 0; a < D; ++a) vir -= xi[a] * (-(g * d[a]));
+                        for (int a = 0; a < D; ++a) xd = fma(xi[a], d[a], xd);
+                        vir = fma(g, xd, vir);
                     }
                 }
             }
         }
     }
-    ext = wave_sum(ext);
-    ipot = wave_sum(ipot);
-    vir = wave_sum(vir);
+    ext = wave_total(ext);
+    ipot = wave_total(ipot);
+    vir = wave_total(vir);
     double* red = smem + (GX ? 0 : (size_t)D * N);
     if (lane == 0) {
         red[wave * 3 + 0] = ext;
@@ -214,9 +252,17 @@ k_bead_energies(ForceArgs fa, const double* __restrict__ x, double* __restrict__
     if (tid == 0) {
         double e = 0, ip = 0, v = 0;
         for (int w = 0; w < FORCE_WAVES; ++w) { e += red[w * 3]; ip += red[w * 3 + 1]; v += red[w * 3 + 2]; }
-        double* o = part + ((size_t)b * gridDim.x + blockIdx.x) * 3;
+        const int nt = (N + FORCE_TILE - 1) / FORCE_TILE;
+        double* o = part + ((size_t)b * nt + tile) * 3;
         o[0] = e; o[1] = ip; o[2] = v;
     }
+}
+
+template <int D, int KIND, bool GX = false>
+static __global__ void __launch_bounds__(FORCE_TILE * FORCE_WAVES)
+k_bead_energies(ForceArgs fa, const double* __restrict__ x, double* __restrict__ part) {
+    extern __shared__ double smem[];
+    bead_energies_tile<D, KIND, GX>(fa, blockIdx.y, blockIdx.x, x, part, smem);
 }
 
 }  // namespace pimdb

@@ -410,13 +410,68 @@ static int finish_steps(pimdb_ctx* ctx, bool host_noise) {
     return PIMDB_OK;
 }
 
+// Layout of ctx->obs: bead sums [P][2], energies [P][tiles][3], then the
+// estimators: k_ring_estimator's 2N + 2 values, or of the factorial exchange
+// the triple (and V_eff at 2N + 1); then the Nose-Hoover energy.
+static size_t obs_tail(int N, int P) { return 2 * (size_t)P + 3 * (size_t)P * ((N + FORCE_TILE - 1) / FORCE_TILE); }
+static size_t obs_doubles(int N, int P) { return obs_tail(N, P) + std::max<size_t>(2 * (size_t)N + 2, 5) + 1; }
+
+static double* pinned_buffer(pimdb_ctx* ctx, size_t n);
+
+// Copies n doubles of ctx->obs from offset `from` and waits; null on failure.
+static const double* read_obs(pimdb_ctx* ctx, size_t from, size_t n) {
+    double* h = pinned_buffer(ctx, n);
+    if (!h) return nullptr;
+    if (hipMemcpyAsync(h, ctx->obs + from, n * sizeof(double), hipMemcpyDeviceToHost, ctx->s0) != hipSuccess) return nullptr;
+    return hipStreamSynchronize(ctx->s0) == hipSuccess ? h : nullptr;
+}
+
+static void launch_estimators(pimdb_ctx* ctx) {
+    const int N = ctx->N, D = ctx->D;
+    const double* xP = ctx->x + (size_t)(ctx->P - 1) * D * N;
+    double* out = ctx->obs + obs_tail(N, ctx->P);
+    const dim3 grid((N + 3) / 4), blk(256);
+    switch (D) {
+    case 1: hipLaunchKernelGGL(k_ring_estimator<1>, grid, blk, 0, ctx->s0, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x, xP, ctx->Shi, ctx->Slo, ctx->V, ctx->Vb, out); break;
+    case 2: hipLaunchKernelGGL(k_ring_estimator<2>, grid, blk, 0, ctx->s0, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x, xP, ctx->Shi, ctx->Slo, ctx->V, ctx->Vb, out); break;
+    default: hipLaunchKernelGGL(k_ring_estimator<3>, grid, blk, 0, ctx->s0, N, ctx->dv.bt, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x, xP, ctx->Shi, ctx->Slo, ctx->V, ctx->Vb, out); break;
+    }
+}
+
+// Natoms that the reference-order estimator's workgroup held.
+static bool estimator_fits(int N) { return sizeof(double) * ((size_t)N + 1 + 16) <= device_lds_limit(); }
+
+template <int D>
+static void launch_observe_d(pimdb_ctx* ctx) {
+    ObserveArgs o{};
+    const int N = ctx->N, P = ctx->P;
+    o.fa = make_force_args(ctx->prm, ctx->dv);
+    o.bt = ctx->dv.bt;
+    o.nx = ctx->dv.bosonic ? xw_grid(N) : 0;
+    o.nf = P * ((N + FORCE_TILE - 1) / FORCE_TILE);
+    o.x = ctx->x; o.p = ctx->p;
+    o.V = ctx->V; o.Vb = ctx->Vb; o.Shi = ctx->Shi; o.Slo = ctx->Slo;
+    o.pub = ctx->pub; o.status = ctx->status;
+    o.sums = ctx->obs;
+    o.epart = ctx->obs + 2 * (size_t)P;
+    const size_t red = std::max<size_t>(3 * FORCE_WAVES, 2 * XW_THREADS / WAVE);
+    size_t lds = sizeof(double) * ((size_t)D * N + red);
+    if (o.nx) lds = std::max(lds, xw_lds_bytes(N, D));
+    const dim3 grid(o.nx + o.nf + P), blk(XW_THREADS);
+    switch (ctx->prm.int_kind) {
+    case POT_HARMONIC: hipLaunchKernelGGL((k_observe<D, POT_HARMONIC>), grid, blk, lds, ctx->s0, o); break;
+    case POT_DIPOLE: hipLaunchKernelGGL((k_observe<D, POT_DIPOLE>), grid, blk, lds, ctx->s0, o); break;
+    case POT_AZIZ: hipLaunchKernelGGL((k_observe<D, POT_AZIZ>), grid, blk, lds, ctx->s0, o); break;
+    default: hipLaunchKernelGGL((k_observe<D, POT_FREE>), grid, blk, lds, ctx->s0, o); break;
+    }
+}
+
+// Waits for the stream.  The flag is pinned host memory that the kernels write
+// through, so looking at it takes no copy.
 static int check_status(pimdb_ctx* ctx) {
-    int st = 0;
-    CK(hipMemcpyAsync(&st, ctx->status, sizeof(int), hipMemcpyDeviceToHost, ctx->s0));
     CK(hipStreamSynchronize(ctx->s0));
-    if (st) {
-        CK(hipMemsetAsync(ctx->status, 0, sizeof(int), ctx->s0));
-        CK(hipStreamSynchronize(ctx->s0));
+    if (*(volatile int*)ctx->status) {
+        *(volatile int*)ctx->status = 0;
         return ctx->fail(PIMDB_E_NONFINITE, "Invalid sig_denom in bosonic exchange potential (non-finite V)");
     }
     return PIMDB_OK;
@@ -523,8 +578,8 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
         alloc(&h.eta_dot_dot, sizeof(double) * nch);
         if (prm->nmthermostat) alloc(&ctx->modes, sizeof(double) * ctx->nbd);
     }
-    alloc(&ctx->obs, sizeof(double) * (2 * (size_t)P + 3 * (size_t)P * ((N + FORCE_TILE - 1) / FORCE_TILE) + 5));
-    alloc(&ctx->status, sizeof(int));
+    alloc(&ctx->obs, sizeof(double) * obs_doubles(N, P));
+    if (!rc && !(ctx->status = status_pool().take())) rc = ctx->fail(PIMDB_E_HIP, "pinned allocation failed");
     alloc(&ctx->ctr, sizeof(unsigned long long));
     if (!rc && (hipStreamCreateWithFlags(&ctx->s0, hipStreamNonBlocking) != hipSuccess ||
                 hipStreamCreateWithFlags(&ctx->s1, hipStreamNonBlocking) != hipSuccess ||
@@ -569,7 +624,7 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
     for (double* b : bufs)
         if (b) (void)hipFree(b);
     if (ctx->pub) (void)hipFree(ctx->pub);
-    if (ctx->status) (void)hipFree(ctx->status);
+    status_pool().give(ctx->status);
     if (ctx->ctr) (void)hipFree(ctx->ctr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
@@ -737,36 +792,42 @@ int pimdb_observables(pimdb_ctx* ctx, double* out) {
     if (!ctx || !out) return PIMDB_E_ARG;
     const int N = ctx->N, P = ctx->P, D = ctx->D;
     const int nt = (N + FORCE_TILE - 1) / FORCE_TILE;
-    double* sums = ctx->obs;                 // [P][2]
-    double* epart = ctx->obs + 2 * (size_t)P;    // [P][nt][3]
-    double* prim = epart + 3 * (size_t)P * nt;   // [3]
-    launch_bead_sums(D, N, P, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x, ctx->p, sums, ctx->s0);
-    launch_bead_energies(D, ctx->prm, ctx->dv, ctx->x, epart, ctx->s0);
-    if (factorial(ctx)) {
-        launch_factorial(ctx, ctx->s0, nullptr, nullptr, ctx->V + N, prim);
-    } else if (ctx->dv.bosonic) {
-        launch_exchange_forward(ctx, ctx->s0);
-        launch_cycle_energies_ctx(ctx, ctx->s0);
-        if (sizeof(double) * (N + 1 + 16) > device_lds_limit())
-            return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
-        hipLaunchKernelGGL(k_prim_estimator, dim3(1), dim3(1024), sizeof(double) * (N + 1 + 16), ctx->s0, N, P,
-                           ctx->dv.bt, ctx->E, ctx->V, prim);
+    const size_t tail = obs_tail(N, P), all = obs_doubles(N, P);
+    double* est = ctx->obs + tail;
+    const bool ring = ctx->dv.bosonic && !factorial(ctx);
+    if (ring && !estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
+    if (ctx->merged) {
+        switch (D) {
+        case 1: launch_observe_d<1>(ctx); break;
+        case 2: launch_observe_d<2>(ctx); break;
+        default: launch_observe_d<3>(ctx); break;
+        }
+    } else {
+        launch_bead_sums(D, N, P, ctx->dv.k, ctx->prm.pbc, ctx->prm.size, ctx->x, ctx->p, ctx->obs, ctx->s0);
+        launch_bead_energies(D, ctx->prm, ctx->dv, ctx->x, ctx->obs + 2 * (size_t)P, ctx->s0);
+        if (ring) launch_exchange_forward(ctx, ctx->s0);
     }
-    double* nh_out = prim + 3;   // [1]
+    if (ring) launch_estimators(ctx);
+    if (factorial(ctx)) launch_factorial(ctx, ctx->s0, nullptr, nullptr, est + std::max(2 * N + 1, 4), est);
     if (ctx->prm.thermostat >= PIMDB_THERMO_NOSE_HOOVER) {
         const int ndof = ctx->nh.kind == PIMDB_THERMO_NOSE_HOOVER ? D * N : ctx->nh.kind == PIMDB_THERMO_NOSE_HOOVER_NP ? D : 1;
-        hipLaunchKernelGGL(k_nh_energy, dim3(1), dim3(256), 0, ctx->s0, ctx->nh, ndof, nh_out);
+        hipLaunchKernelGGL(k_nh_energy, dim3(1), dim3(256), 0, ctx->s0, ctx->nh, ndof, ctx->obs + all - 1);
     }
     CK(hipGetLastError());
+    const double* h = read_obs(ctx, 0, all);
+    if (!h) return ctx->fail(PIMDB_E_HIP, "reading the observables failed");
     int rc = check_status(ctx);
     if (rc) return rc;
-    std::vector<double> h(2 * (size_t)P + 3 * (size_t)P * nt + 4);
-    CK(hipMemcpy(h.data(), ctx->obs, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
-    double VN = 0.0;
-    if (ctx->dv.bosonic) CK(hipMemcpy(&VN, ctx->V + N, sizeof(double), hipMemcpyDeviceToHost));
-    combine_observables(ctx->prm, ctx->dv, h.data(), h.data() + 2 * (size_t)P, nt, h.data() + 2 * (size_t)P + 3 * (size_t)P * nt,
-                        VN, out);
-    out[10] = ctx->prm.thermostat >= PIMDB_THERMO_NOSE_HOOVER ? h[2 * (size_t)P + 3 * (size_t)P * nt + 3] : 0.0;
+    double prim[3] = {0.0, 0.0, 0.0}, VN = 0.0;
+    if (ring) {
+        combine_estimators(N, P, ctx->dv.bt, h + tail, prim);
+        VN = h[tail + 2 * (size_t)N + 1];
+    } else if (factorial(ctx)) {
+        std::copy(h + tail, h + tail + 3, prim);
+        VN = h[tail + std::max(2 * N + 1, 4)];
+    }
+    combine_observables(ctx->prm, ctx->dv, h, h + 2 * (size_t)P, nt, prim, VN, out);
+    out[10] = ctx->prm.thermostat >= PIMDB_THERMO_NOSE_HOOVER ? h[all - 1] : 0.0;
     return PIMDB_OK;
 }
 
@@ -774,26 +835,25 @@ int pimdb_exchange_estimators(pimdb_ctx* ctx, double* prim, double* prob_distinc
     if (!ctx) return PIMDB_E_ARG;
     if (!ctx->dv.bosonic) return ctx->fail(PIMDB_E_STATE, "exchange estimators need a bosonic system");
     const int N = ctx->N, P = ctx->P;
-    const int nt = (N + FORCE_TILE - 1) / FORCE_TILE;
-    double* out = ctx->obs + 2 * (size_t)P + 3 * (size_t)P * nt;   // [3], as pimdb_observables
+    const size_t tail = obs_tail(N, P);
     if (factorial(ctx)) {
-        launch_factorial(ctx, ctx->s0, nullptr, nullptr, nullptr, out);
+        launch_factorial(ctx, ctx->s0, nullptr, nullptr, nullptr, ctx->obs + tail);
     } else {
+        if (!estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
         launch_exchange_forward(ctx, ctx->s0);
-        launch_cycle_energies_ctx(ctx, ctx->s0);
-        if (sizeof(double) * (N + 1 + 16) > device_lds_limit())
-            return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
-        hipLaunchKernelGGL(k_prim_estimator, dim3(1), dim3(1024), sizeof(double) * (N + 1 + 16), ctx->s0, N, P,
-                           ctx->dv.bt, ctx->E, ctx->V, out);
+        launch_estimators(ctx);
     }
     CK(hipGetLastError());
+    const double* h = read_obs(ctx, tail, obs_doubles(N, P) - tail);
+    if (!h) return ctx->fail(PIMDB_E_HIP, "reading the estimators failed");
     int rc = check_status(ctx);
     if (rc) return rc;
-    double h[3];
-    CK(hipMemcpy(h, out, sizeof(h), hipMemcpyDeviceToHost));
-    if (prim) *prim = h[0];
-    if (prob_distinct) *prob_distinct = h[1];
-    if (prob_longest) *prob_longest = h[2];
+    double e[3];
+    if (factorial(ctx)) std::copy(h, h + 3, e);
+    else combine_estimators(N, P, ctx->dv.bt, h, e);
+    if (prim) *prim = e[0];
+    if (prob_distinct) *prob_distinct = e[1];
+    if (prob_longest) *prob_longest = e[2];
     return PIMDB_OK;
 }
 

@@ -216,8 +216,8 @@ __device__ __forceinline__ void step_recursions(const StepArgs& s, int wg, doubl
             s.xc[3 * bs + e] = xPm1[e];
         }
     }
-    xw_recursions<D, NT>(smem, wg, N, s.bt, s.fa.k_spring, s.fa.pbc, s.fa.L, s.x, s.x + bs * (P - 1), s.V, s.Vb, s.Shi,
-                         s.Slo, s.xc, s.pub, s.status);
+    xw_recursions<D, NT>(smem, wg, N, s.bt, s.fa.k_spring, s.fa.pbc, s.fa.L, BeadView{s.x, N, 1},
+                         BeadView{s.x + bs * (P - 1), N, 1}, s.V, s.Vb, nullptr, s.Shi, s.Slo, s.xc, s.pub, s.status);
 }
 
 // Workgroups of an integration: 4 tasks of M particles of an exchange bead each

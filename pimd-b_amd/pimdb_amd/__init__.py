@@ -79,7 +79,7 @@ def lib():
         raise RuntimeError("libpimdb_gpu.so is not built: run __graft_entry__.build() "
                            "(there is no CPU fallback)")
     L = C.CDLL(LIB_PATH)
-    vp, i, d = C.c_void_p, C.c_int, C.c_double
+    vp, i, d, ll = C.c_void_p, C.c_int, C.c_double, C.c_longlong
     sigs = {
         "pimdb_ctx_create": (i, [C.POINTER(Params), C.POINTER(vp)]),
         "pimdb_ctx_destroy": (None, [vp]),
@@ -101,6 +101,9 @@ def lib():
         "pimdb_xplan_destroy": (None, [vp]),
         "pimdb_xplan_forward": (i, [vp, vp, vp, vp, vp, vp, vp]),
         "pimdb_xplan_vb_grad": (i, [vp, vp, vp, vp, vp]),
+        "pimdb_xplan_saved_doubles": (ll, [vp]),
+        "pimdb_xplan_forward_saved": (i, [vp, vp, ll, ll, vp, ll, ll, vp, vp, vp]),
+        "pimdb_xplan_backward_saved": (i, [vp, vp, vp, vp, vp, vp]),
         "pimdb_exchange_vb_grad_noalloc": (i, [i, i, d, d, i, d, vp, vp, vp, vp, vp]),
         "pimdb_batch_create": (i, [C.POINTER(Params), i, C.POINTER(vp)]),
         "pimdb_batch_destroy": (None, [vp]),
@@ -344,6 +347,8 @@ class XPlan:
             _raise(rc, "pimdb_xplan_create failed")
         self.h = h
         self.natoms, self.ndim = natoms, ndim
+        # doubles of the record that forward_saved leaves for backward_saved
+        self.saved_doubles = int(lib().pimdb_xplan_saved_doubles(h))
 
     def close(self):
         if getattr(self, "h", None):
@@ -361,6 +366,19 @@ class XPlan:
         rc = lib().pimdb_xplan_vb_grad(self.h, x1_ptr, xP_ptr, grad_ptr, stream)
         if rc != OK:
             _raise(rc, "pimdb_xplan_vb_grad failed")
+
+    def forward_saved(self, x1_ptr, x1_strides, xP_ptr, xP_strides, VB_ptr, saved_ptr, stream=None):
+        """V_B of beads given with (particle, axis) strides in doubles, and the record for backward_saved."""
+        rc = lib().pimdb_xplan_forward_saved(self.h, x1_ptr, x1_strides[0], x1_strides[1], xP_ptr, xP_strides[0],
+                                             xP_strides[1], VB_ptr, saved_ptr, stream)
+        if rc != OK:
+            _raise(rc, "pimdb_xplan_forward_saved failed")
+
+    def backward_saved(self, saved_ptr, scale_ptr, d1_ptr, dP_ptr, stream=None):
+        """scale dV_B/dx1 and scale dV_B/dxP ([particle][axis]) from a forward pass's record; does not wait."""
+        rc = lib().pimdb_xplan_backward_saved(self.h, saved_ptr, scale_ptr, d1_ptr, dP_ptr, stream)
+        if rc != OK:
+            _raise(rc, "pimdb_xplan_backward_saved failed")
 
 
 def exchange_vb_grad_noalloc(natoms, ndim, beta_t, spring_k, pbc, size, x1_ptr, xP_ptr, VB_ptr=None,

@@ -1,9 +1,10 @@
 """torch.autograd harness over the exchange kernels (test harness, not the
-driver): the forward kernel chain computes V_B = V[N] from beads 1 and P
-(quadratic_bosonic_exchange.cpp:34-132) and the backward is the hand-written
-adjoint kernel, -dV_B/dx for both beads (the exterior spring forces of
-:159-215 without the interior links).  Tensors are float64 CUDA tensors of
-shape (N, D); the kernels read them as SoA copies on torch's current stream.
+driver): the forward kernel computes V_B = V[N] from beads 1 and P
+(quadratic_bosonic_exchange.cpp:34-132) and leaves both recursions for the
+backward, the hand-written adjoint kernel: -dV_B/dx for both beads (the
+exterior spring forces of :159-215 without the interior links).  Tensors are
+float64 CUDA tensors of shape (N, D), read with whatever strides they have on
+torch's current stream.
 """
 import torch
 
@@ -19,26 +20,24 @@ class ExchangeVB(torch.autograd.Function):
             raise TypeError("ExchangeVB takes float64 CUDA tensors")
         if x1.shape != xP.shape or x1.dim() != 2 or x1.shape != (plan.natoms, plan.ndim):
             raise ValueError("x1 and xP must both have shape (%d, %d)" % (plan.natoms, plan.ndim))
-        x1s = x1.detach().t().contiguous()
-        xPs = xP.detach().t().contiguous()
-        vb = torch.empty(1, dtype=torch.float64, device=x1.device)
+        vb = torch.empty((), dtype=torch.float64, device=x1.device)
+        saved = torch.empty(plan.saved_doubles, dtype=torch.float64, device=x1.device)
         stream = torch.cuda.current_stream(x1.device).cuda_stream
-        plan.forward(x1s.data_ptr(), xPs.data_ptr(), vb.data_ptr(), None, None, stream)
+        plan.forward_saved(x1.data_ptr(), x1.stride(), xP.data_ptr(), xP.stride(), vb.data_ptr(), saved.data_ptr(), stream)
         ctx.plan = plan
-        ctx.save_for_backward(x1s, xPs)
-        return vb.reshape(())
+        ctx.save_for_backward(saved)
+        return vb
 
     @staticmethod
     def backward(ctx, g):
-        x1s, xPs = ctx.saved_tensors
-        D, N = x1s.shape
-        grad = torch.empty((2, D, N), dtype=torch.float64, device=x1s.device)
-        stream = torch.cuda.current_stream(x1s.device).cuda_stream
-        ctx.plan.vb_grad(x1s.data_ptr(), xPs.data_ptr(), grad.data_ptr(), stream)
-        # the kernel returns -dV_B/dx (a force)
-        dx1 = grad[0].t().neg() * g
-        dxP = grad[1].t().neg() * g
-        return dx1, dxP, None
+        (saved,) = ctx.saved_tensors
+        plan = ctx.plan
+        d1, dP = (torch.empty((plan.natoms, plan.ndim), dtype=torch.float64, device=saved.device) for _ in range(2))
+        stream = torch.cuda.current_stream(saved.device).cuda_stream
+        # the product with g stays a torch operation where it is to be differentiated itself
+        inside = not torch.is_grad_enabled()
+        plan.backward_saved(saved.data_ptr(), g.data_ptr() if inside else None, d1.data_ptr(), dP.data_ptr(), stream)
+        return (d1, dP, None) if inside else (d1 * g, dP * g, None)
 
 
 def exchange_potential(x1, xP, plan):
