@@ -56,6 +56,7 @@ struct pimdb_batch {
     unsigned long long* d_pub = nullptr;
     StepArgs* d_steps = nullptr;
     int2* d_maps = nullptr;
+    HostStage stage;
     std::string err;
     int fail(int code, const std::string& m) {
         err = m;
@@ -685,6 +686,7 @@ void pimdb_batch_destroy(pimdb_batch* b) {
     if (b->d_sched) (void)hipFree(b->d_sched);
     if (b->d_sched_off) (void)hipFree(b->d_sched_off);
     free_split(b);
+    b->stage.free();
     if (b->t0) (void)hipEventDestroy(b->t0);
     if (b->t1) (void)hipEventDestroy(b->t1);
     if (b->s) (void)hipStreamDestroy(b->s);
@@ -714,15 +716,17 @@ int pimdb_batch_set_state(pimdb_batch* b, int rep, const double* x, const double
     if (frc) return frc;
     const pimdb_params& q = b->prm[rep];
     const size_t n = (size_t)q.nbeads * q.ndim * q.natoms;
-    std::vector<double> st(n);
+    const RepDesc& d = b->desc[rep];
     const double* src[2] = {x, p};
-    double* dst[2] = {b->bp.x, b->bp.p};
-    for (int k = 0; k < 2; ++k) {
-        if (!src[k]) continue;
-        to_soa(src[k], st.data(), q.natoms, q.nbeads, q.ndim);
-        BCK(hipMemcpyAsync(dst[k] + b->desc[rep].off_x, st.data(), sizeof(double) * n, hipMemcpyHostToDevice, b->s));
-        BCK(hipStreamSynchronize(b->s));
-    }
+    double* dst[2] = {b->bp.x + d.off_x, b->bp.p + d.off_x};
+    StateArrays a{{nullptr, nullptr, nullptr}, 0, q.natoms, q.ndim, n, nullptr, 0};
+    double* host[3];
+    for (int k = 0; k < 2; ++k)
+        if (src[k]) {
+            host[a.count] = const_cast<double*>(src[k]);
+            a.dev[a.count++] = dst[k];
+        }
+    if (a.count) BCK(copy_state<true>(b->stage, a, host, b->s));
     if (p) {
         // no COM pending; the sum of p per axis for the next first O-step
         double cmp[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -739,21 +743,22 @@ int pimdb_batch_get_state(pimdb_batch* b, int rep, double* x, double* p, double*
     if (frc) return frc;
     const pimdb_params& q = b->prm[rep];
     const size_t n = (size_t)q.nbeads * q.ndim * q.natoms;
-    std::vector<double> st(n);
+    const RepDesc& d = b->desc[rep];
     double* dst[3] = {x, p, f};
-    const double* src[3] = {b->bp.x, b->bp.p, b->bp.f};
-    for (int k = 0; k < 3; ++k) {
-        if (!dst[k]) continue;
-        BCK(hipMemcpyAsync(st.data(), src[k] + b->desc[rep].off_x, sizeof(double) * n, hipMemcpyDeviceToHost, b->s));
-        BCK(hipStreamSynchronize(b->s));
-        from_soa(st.data(), dst[k], q.natoms, q.nbeads, q.ndim);
-    }
-    if (p) {
-        // the COM momentum still pending from the last O-step
-        double cmp[8];
-        BCK(hipMemcpy(cmp, b->bp.cmp + 8 * (size_t)rep, sizeof(cmp), hipMemcpyDeviceToHost));
-        for (size_t e = 0; e < n; ++e) p[e] -= cmp[e % q.ndim];
-    }
+    double* src[3] = {b->bp.x + d.off_x, b->bp.p + d.off_x, b->bp.f + d.off_x};
+    // p without the COM momentum still pending from the last O-step
+    StateArrays a{{nullptr, nullptr, nullptr}, 0, q.natoms, q.ndim, n, nullptr, 0};
+    double* host[3];
+    for (int k = 0; k < 3; ++k)
+        if (dst[k]) {
+            if (k == 1) {
+                a.cm = b->bp.cmp + 8 * (size_t)rep;
+                a.cm_of = a.count;
+            }
+            host[a.count] = dst[k];
+            a.dev[a.count++] = src[k];
+        }
+    if (a.count) BCK(copy_state<false>(b->stage, a, host, b->s));
     return PIMDB_OK;
 }
 

@@ -57,7 +57,7 @@ struct pimdb_ctx {
     double* modes = nullptr;       // normal modes of p, [k][a][i] (Nose-Hoover with nmthermostat)
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    std::vector<double> stage;
+    HostStage stage;
     double* pinned = nullptr;
     size_t pinned_cap = 0;
     std::string err;
@@ -627,6 +627,7 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
     status_pool().give(ctx->status);
     if (ctx->ctr) (void)hipFree(ctx->ctr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+    ctx->stage.free();
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->t0) (void)hipEventDestroy(ctx->t0);
@@ -642,29 +643,29 @@ int pimdb_set_state(pimdb_ctx* ctx, const double* x, const double* p) {
     if (!ctx) return PIMDB_E_ARG;
     const double* src[2] = {x, p};
     double* dst[2] = {ctx->x, ctx->p};
-    for (int k = 0; k < 2; ++k) {
-        if (!src[k]) continue;
-        double* st = pinned_buffer(ctx, ctx->nbd);
-        if (!st) return ctx->fail(PIMDB_E_HIP, "pinned allocation failed");
-        to_soa(src[k], st, ctx->N, ctx->P, ctx->D);
-        CK(hipMemcpyAsync(dst[k], st, sizeof(double) * ctx->nbd, hipMemcpyHostToDevice, ctx->s0));
-        CK(hipStreamSynchronize(ctx->s0));
-    }
+    StateArrays a{{nullptr, nullptr, nullptr}, 0, ctx->N, ctx->D, ctx->nbd, nullptr, 0};
+    double* host[3];
+    for (int k = 0; k < 2; ++k)
+        if (src[k]) {
+            host[a.count] = const_cast<double*>(src[k]);
+            a.dev[a.count++] = dst[k];
+        }
+    if (a.count) CK(copy_state<true>(ctx->stage, a, host, ctx->s0));
     return PIMDB_OK;
 }
 
 int pimdb_get_state(pimdb_ctx* ctx, double* x, double* p, double* f) {
     if (!ctx) return PIMDB_E_ARG;
     double* dst[3] = {x, p, f};
-    const double* src[3] = {ctx->x, ctx->p, ctx->f};
-    for (int k = 0; k < 3; ++k) {
-        if (!dst[k]) continue;
-        double* st = pinned_buffer(ctx, ctx->nbd);
-        if (!st) return ctx->fail(PIMDB_E_HIP, "pinned allocation failed");
-        CK(hipMemcpyAsync(st, src[k], sizeof(double) * ctx->nbd, hipMemcpyDeviceToHost, ctx->s0));
-        CK(hipStreamSynchronize(ctx->s0));
-        from_soa(st, dst[k], ctx->N, ctx->P, ctx->D);
-    }
+    double* src[3] = {ctx->x, ctx->p, ctx->f};
+    StateArrays a{{nullptr, nullptr, nullptr}, 0, ctx->N, ctx->D, ctx->nbd, nullptr, 0};
+    double* host[3];
+    for (int k = 0; k < 3; ++k)
+        if (dst[k]) {
+            host[a.count] = dst[k];
+            a.dev[a.count++] = src[k];
+        }
+    if (a.count) CK(copy_state<false>(ctx->stage, a, host, ctx->s0));
     return PIMDB_OK;
 }
 

@@ -172,7 +172,7 @@ class Context:
         self._chk(lib().pimdb_set_state(self.h, _p(x), _p(p)))
 
     def state(self):
-        x, p, f = (np.zeros(self.shape) for _ in range(3))
+        x, p, f = (np.empty(self.shape) for _ in range(3))
         self._chk(lib().pimdb_get_state(self.h, _p(x), _p(p), _p(f)))
         return x, p, f
 
@@ -262,7 +262,7 @@ class Batch:
         self._chk(lib().pimdb_batch_set_state(self.h, int(r), _p(x), _p(p)))
 
     def state(self, r):
-        x, p, f = (np.zeros(self.shape(r)) for _ in range(3))
+        x, p, f = (np.empty(self.shape(r)) for _ in range(3))
         self._chk(lib().pimdb_batch_get_state(self.h, int(r), _p(x), _p(p), _p(f)))
         return x, p, f
 
