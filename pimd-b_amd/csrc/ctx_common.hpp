@@ -194,40 +194,77 @@ static __global__ void __launch_bounds__(256) k_state_copy(StateArrays s, size_t
     }
 }
 
-// The pinned buffer of one context or batch: grown to a state, at most CAP
-// doubles (larger states pass through it in parts).
-struct HostStage {
+// Pinned buffers for calls that move data to or from the host and wait for
+// it: taken for one call, so a process holds as many as calls overlapped (at
+// most KEEP of them between calls).  A buffer per context would cost each new
+// one 0.4 - 0.8 ms, the mapping and the device's first accesses to it.  Sizes
+// are powers of two up to CAP doubles; larger states pass through in parts.
+// Any thread.
+class StagePool {
+    static constexpr size_t KEEP = 4, LEAST = (size_t)1 << 16;
+    std::mutex mu;
+    std::vector<std::pair<double*, size_t>> idle;
+
+public:
     static constexpr size_t CAP = (size_t)1 << 20;
-    double* buf = nullptr;
-    size_t cap = 0;
-    double* get(size_t n) {
-        n = std::min(n, CAP);
-        if (cap < n) {
-            free();
-            if (hipHostMalloc((void**)&buf, n * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-                buf = nullptr;
-                return nullptr;
+    // a buffer of at least min(n, CAP) doubles and its size, or null
+    std::pair<double*, size_t> take(size_t n) {
+        size_t cap = LEAST;
+        while (cap < n && cap < CAP) cap *= 2;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            size_t best = idle.size();
+            for (size_t i = 0; i < idle.size(); ++i)
+                if (idle[i].second >= cap && (best == idle.size() || idle[i].second < idle[best].second)) best = i;
+            if (best < idle.size()) {
+                const auto got = idle[best];
+                idle.erase(idle.begin() + best);
+                return got;
             }
-            cap = n;
         }
-        return buf;
+        double* p = nullptr;
+        if (hipHostMalloc((void**)&p, cap * sizeof(double), hipHostMallocPortable) != hipSuccess) return {nullptr, 0};
+        return {p, cap};
     }
-    void free() {
-        if (buf) (void)hipHostFree(buf);
-        buf = nullptr;
-        cap = 0;
+    void give(std::pair<double*, size_t> b) {   // nothing on the device uses it
+        if (!b.first) return;
+        std::pair<double*, size_t> out = b;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            idle.push_back(b);
+            if (idle.size() <= KEEP) return;
+            size_t least = 0;   // the smallest goes
+            for (size_t i = 1; i < idle.size(); ++i)
+                if (idle[i].second < idle[least].second) least = i;
+            out = idle[least];
+            idle.erase(idle.begin() + least);
+        }
+        (void)hipHostFree(out.first);
     }
+};
+inline StagePool& stage_pool() {
+    static StagePool* pool = new StagePool();   // (never destroyed, as status_pool)
+    return *pool;
+}
+// A buffer for one call.
+struct Stage {
+    std::pair<double*, size_t> b;
+    explicit Stage(size_t n) : b(stage_pool().take(n)) {}
+    ~Stage() { stage_pool().give(b); }
+    Stage(const Stage&) = delete;
+    Stage& operator=(const Stage&) = delete;
 };
 
 // Copies the arrays to (IN) or from the device; host[k] is array k's host
 // memory.  Returns when the copy is complete.
 template <bool IN>
-inline hipError_t copy_state(HostStage& st, const StateArrays& s, double* const* host, hipStream_t stream) {
+inline hipError_t copy_state(const StateArrays& s, double* const* host, hipStream_t stream) {
     const size_t all = s.n * s.count;
-    double* buf = st.get(all);
+    const Stage st(all);
+    double* const buf = st.b.first;
     if (!buf) return hipErrorOutOfMemory;
-    for (size_t first = 0; first < all; first += st.cap) {
-        const size_t total = std::min(st.cap, all - first);
+    for (size_t first = 0; first < all; first += st.b.second) {
+        const size_t total = std::min(st.b.second, all - first);
         auto pieces = [&](bool in) {
             for (size_t q = 0; q < total;) {
                 const size_t e = first + q, k = e / s.n, t = e % s.n, m = std::min(total - q, s.n - t);
@@ -239,7 +276,8 @@ inline hipError_t copy_state(HostStage& st, const StateArrays& s, double* const*
         if (IN) pieces(true);
         hipLaunchKernelGGL(k_state_copy<IN>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, s, first, total, buf);
         hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        const hipError_t w = hipStreamSynchronize(stream);   // (also on an error: the buffer goes back)
+        if (e == hipSuccess) e = w;
         if (e != hipSuccess) return e;
         if (!IN) pieces(false);
     }

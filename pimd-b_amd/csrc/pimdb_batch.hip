@@ -56,7 +56,6 @@ struct pimdb_batch {
     unsigned long long* d_pub = nullptr;
     StepArgs* d_steps = nullptr;
     int2* d_maps = nullptr;
-    HostStage stage;
     std::string err;
     int fail(int code, const std::string& m) {
         err = m;
@@ -686,7 +685,6 @@ void pimdb_batch_destroy(pimdb_batch* b) {
     if (b->d_sched) (void)hipFree(b->d_sched);
     if (b->d_sched_off) (void)hipFree(b->d_sched_off);
     free_split(b);
-    b->stage.free();
     if (b->t0) (void)hipEventDestroy(b->t0);
     if (b->t1) (void)hipEventDestroy(b->t1);
     if (b->s) (void)hipStreamDestroy(b->s);
@@ -726,7 +724,7 @@ int pimdb_batch_set_state(pimdb_batch* b, int rep, const double* x, const double
             host[a.count] = const_cast<double*>(src[k]);
             a.dev[a.count++] = dst[k];
         }
-    if (a.count) BCK(copy_state<true>(b->stage, a, host, b->s));
+    if (a.count) BCK(copy_state<true>(a, host, b->s));
     if (p) {
         // no COM pending; the sum of p per axis for the next first O-step
         double cmp[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -758,7 +756,7 @@ int pimdb_batch_get_state(pimdb_batch* b, int rep, double* x, double* p, double*
             host[a.count] = dst[k];
             a.dev[a.count++] = src[k];
         }
-    if (a.count) BCK(copy_state<false>(b->stage, a, host, b->s));
+    if (a.count) BCK(copy_state<false>(a, host, b->s));
     return PIMDB_OK;
 }
 

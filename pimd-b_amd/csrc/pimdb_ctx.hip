@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "pimdb_gpu.h"
@@ -36,6 +37,7 @@ struct pimdb_ctx {
     Derived dv{};
     int N = 0, P = 0, D = 0;
     size_t nbd = 0;
+    char* arena = nullptr;         // holds every device buffer but E, ET, prob and noise
     hipStream_t s0 = nullptr, s1 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, t0 = nullptr, t1 = nullptr;
     double *x = nullptr, *p = nullptr, *f = nullptr, *fext = nullptr;
@@ -57,7 +59,6 @@ struct pimdb_ctx {
     double* modes = nullptr;       // normal modes of p, [k][a][i] (Nose-Hoover with nmthermostat)
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    HostStage stage;
     double* pinned = nullptr;
     size_t pinned_cap = 0;
     std::string err;
@@ -116,8 +117,14 @@ static void launch_exchange_forward(pimdb_ctx* ctx, hipStream_t s) {
                                ctx->pub, ctx->xws, ctx->status, s);
 }
 
-// The stored triangle E (and its row-major copy), for the outputs and
-// estimators that take E itself.
+// Buffers of the outputs that take the energies or probabilities themselves,
+// allocated when first asked for.
+static int need_buffer(pimdb_ctx* ctx, double** buf, size_t n) {
+    if (!*buf) CK(hipMalloc((void**)buf, sizeof(double) * n));
+    return PIMDB_OK;
+}
+
+// The stored triangle E (and its row-major copy).
 static void launch_cycle_energies_ctx(pimdb_ctx* ctx, hipStream_t s) {
     const int N = ctx->N, P = ctx->P;
     const double* x1 = ctx->x;
@@ -416,14 +423,20 @@ static int finish_steps(pimdb_ctx* ctx, bool host_noise) {
 static size_t obs_tail(int N, int P) { return 2 * (size_t)P + 3 * (size_t)P * ((N + FORCE_TILE - 1) / FORCE_TILE); }
 static size_t obs_doubles(int N, int P) { return obs_tail(N, P) + std::max<size_t>(2 * (size_t)N + 2, 5) + 1; }
 
-static double* pinned_buffer(pimdb_ctx* ctx, size_t n);
-
-// Copies n doubles of ctx->obs from offset `from` and waits; null on failure.
-static const double* read_obs(pimdb_ctx* ctx, size_t from, size_t n) {
-    double* h = pinned_buffer(ctx, n);
-    if (!h) return nullptr;
-    if (hipMemcpyAsync(h, ctx->obs + from, n * sizeof(double), hipMemcpyDeviceToHost, ctx->s0) != hipSuccess) return nullptr;
-    return hipStreamSynchronize(ctx->s0) == hipSuccess ? h : nullptr;
+// Copies n doubles of ctx->obs from offset `from` to h (may be larger than a
+// pinned buffer) and waits.
+static hipError_t read_obs(pimdb_ctx* ctx, size_t from, std::vector<double>& h) {
+    const Stage st(h.size());
+    if (!st.b.first) return hipErrorOutOfMemory;
+    for (size_t o = 0; o < h.size(); o += st.b.second) {
+        const size_t n = std::min(st.b.second, h.size() - o);
+        hipError_t e = hipMemcpyAsync(st.b.first, ctx->obs + from + o, n * sizeof(double), hipMemcpyDeviceToHost, ctx->s0);
+        const hipError_t w = hipStreamSynchronize(ctx->s0);
+        if (e == hipSuccess) e = w;
+        if (e != hipSuccess) return e;
+        std::memcpy(h.data() + o, st.b.first, n * sizeof(double));
+    }
+    return hipSuccess;
 }
 
 static void launch_estimators(pimdb_ctx* ctx) {
@@ -514,34 +527,29 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     ctx->ntiles = (ctx->N + ctx->tc - 1) / ctx->tc;
     const int N = ctx->N, P = ctx->P, D = ctx->D;
     int rc = PIMDB_OK;
+    // one device allocation for all buffers (each of its own costs 10 us or more)
+    std::vector<std::pair<void**, size_t>> want;   // pointer, offset
+    size_t arena = 0;
     auto alloc = [&](auto** ptr, size_t bytes) {
-        if (rc) return;
-        if (hipMalloc((void**)ptr, bytes) != hipSuccess || hipMemset(*ptr, 0, bytes) != hipSuccess)
-            rc = ctx->fail(PIMDB_E_HIP, "device allocation failed");
+        want.push_back({(void**)ptr, arena});
+        arena += (bytes + 255) & ~(size_t)255;
     };
     alloc(&ctx->x, sizeof(double) * ctx->nbd);
     alloc(&ctx->p, sizeof(double) * ctx->nbd);
     alloc(&ctx->f, sizeof(double) * ctx->nbd);
     alloc(&ctx->fext, sizeof(double) * ctx->nbd);
-    alloc(&ctx->E, sizeof(double) * ((size_t)N * (N + 1) / 2));
-    alloc(&ctx->ET, sizeof(double) * ((size_t)N * (N + 1) / 2));
     alloc(&ctx->V, sizeof(double) * (N + 1));
     alloc(&ctx->Vb, sizeof(double) * (N + 1));
     alloc(&ctx->Shi, sizeof(double) * N);
     alloc(&ctx->Slo, sizeof(double) * N);
-    if (ctx->dv.bosonic && prm->exchange_algo != PIMDB_EXCHANGE_FACTORIAL) {
-        // the recursions' published values, or both workspaces in device
-        // memory when the ring exceeds the LDS of a workgroup
-        if (exchange_wide(N, D)) {
-            alloc(&ctx->pub, 8 * xw_pub_words(N));
-            if (!rc && hipMemset(ctx->pub, 0xFF, 8 * xw_pub_words(N)) != hipSuccess)
-                rc = ctx->fail(PIMDB_E_HIP, "device initialisation failed");
-        } else {
-            alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
-        }
-    }
+    // the recursions' published values, or both workspaces in device memory
+    // when the ring exceeds the LDS of a workgroup
+    const bool ring = ctx->dv.bosonic && prm->exchange_algo != PIMDB_EXCHANGE_FACTORIAL;
+    const bool wide = ring && exchange_wide(N, D);
+    if (wide) alloc(&ctx->pub, 8 * xw_pub_words(N));
+    else if (ring) alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
     const bool slice_fits = tile_lds_bytes(N, D) <= device_lds_limit();
-    ctx->merged = slice_fits && (!ctx->dv.bosonic || ctx->pub);
+    ctx->merged = slice_fits && (!ctx->dv.bosonic || wide);
     ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN && prm->propagator == PIMDB_PROP_CARTESIAN &&
                  (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat || P <= STEP_NM_MAXP);
     if (ctx->merged && ctx->dv.bosonic) alloc(&ctx->xc, sizeof(double) * 4 * (size_t)D * N);
@@ -550,7 +558,6 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
         alloc(&ctx->fpart, sizeof(double) * D * (size_t)P * ((N + FORCE_TILE - 1) / FORCE_TILE));
         alloc(&ctx->hpart, sizeof(double) * D * (size_t)step_noise_tiles(N));
     }
-    alloc(&ctx->prob, sizeof(double) * (size_t)N * N);
     alloc(&ctx->fex, sizeof(double) * 2 * (size_t)D * N);
     alloc(&ctx->C, sizeof(double) * (size_t)P * P);
     alloc(&ctx->CT, sizeof(double) * (size_t)P * P);
@@ -579,13 +586,22 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
         if (prm->nmthermostat) alloc(&ctx->modes, sizeof(double) * ctx->nbd);
     }
     alloc(&ctx->obs, sizeof(double) * obs_doubles(N, P));
-    if (!rc && !(ctx->status = status_pool().take())) rc = ctx->fail(PIMDB_E_HIP, "pinned allocation failed");
     alloc(&ctx->ctr, sizeof(unsigned long long));
+    if (hipMalloc((void**)&ctx->arena, arena) != hipSuccess || hipMemset(ctx->arena, 0, arena) != hipSuccess)
+        rc = ctx->fail(PIMDB_E_HIP, "device allocation failed");
+    if (!rc)
+        for (auto& w : want) *w.first = ctx->arena + w.second;
+    if (!rc && wide && hipMemset(ctx->pub, 0xFF, 8 * xw_pub_words(N)) != hipSuccess)
+        rc = ctx->fail(PIMDB_E_HIP, "device initialisation failed");
+    if (!rc && !(ctx->status = status_pool().take())) rc = ctx->fail(PIMDB_E_HIP, "pinned allocation failed");
     if (!rc && (hipStreamCreateWithFlags(&ctx->s0, hipStreamNonBlocking) != hipSuccess ||
-                hipStreamCreateWithFlags(&ctx->s1, hipStreamNonBlocking) != hipSuccess ||
-                hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
-                hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess ||
                 hipEventCreate(&ctx->t0) != hipSuccess || hipEventCreate(&ctx->t1) != hipSuccess))
+        rc = ctx->fail(PIMDB_E_HIP, "stream/event creation failed");
+    // the second stream of steps whose recursions are a kernel of their own
+    if (!rc && ring && !ctx->merged &&
+        (hipStreamCreateWithFlags(&ctx->s1, hipStreamNonBlocking) != hipSuccess ||
+         hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
+         hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess))
         rc = ctx->fail(PIMDB_E_HIP, "stream/event creation failed");
     if (!rc) {
         std::vector<double> C0((size_t)P * P), CT0((size_t)P * P), Cm((size_t)P * P), CTm((size_t)P * P),
@@ -617,17 +633,11 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
     if (ctx->s1) (void)hipStreamSynchronize(ctx->s1);
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-    double* bufs[] = {ctx->x, ctx->p, ctx->f, ctx->fext, ctx->E, ctx->ET, ctx->V, ctx->Vb, ctx->prob, ctx->fex,
-                      ctx->C, ctx->CT, ctx->rot, ctx->com0, ctx->com1, ctx->noise, ctx->obs, ctx->Shi, ctx->Slo,
-                      ctx->nh.eta, ctx->nh.eta_dot, ctx->nh.eta_dot_dot, ctx->modes, ctx->xws, ctx->xc, ctx->H,
-                      ctx->fpart, ctx->hpart};
-    for (double* b : bufs)
+    void* bufs[] = {ctx->arena, ctx->E, ctx->ET, ctx->prob, ctx->noise};
+    for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (ctx->pub) (void)hipFree(ctx->pub);
     status_pool().give(ctx->status);
-    if (ctx->ctr) (void)hipFree(ctx->ctr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
-    ctx->stage.free();
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->t0) (void)hipEventDestroy(ctx->t0);
@@ -650,7 +660,7 @@ int pimdb_set_state(pimdb_ctx* ctx, const double* x, const double* p) {
             host[a.count] = const_cast<double*>(src[k]);
             a.dev[a.count++] = dst[k];
         }
-    if (a.count) CK(copy_state<true>(ctx->stage, a, host, ctx->s0));
+    if (a.count) CK(copy_state<true>(a, host, ctx->s0));
     return PIMDB_OK;
 }
 
@@ -665,7 +675,7 @@ int pimdb_get_state(pimdb_ctx* ctx, double* x, double* p, double* f) {
             host[a.count] = dst[k];
             a.dev[a.count++] = src[k];
         }
-    if (a.count) CK(copy_state<false>(ctx->stage, a, host, ctx->s0));
+    if (a.count) CK(copy_state<false>(a, host, ctx->s0));
     return PIMDB_OK;
 }
 
@@ -690,6 +700,14 @@ int pimdb_exchange_forward(pimdb_ctx* ctx, double* VB, double* V, double* Vb, do
         if (VB) CK(hipMemcpy(VB, ctx->V + N, sizeof(double), hipMemcpyDeviceToHost));
         return PIMDB_OK;
     }
+    const size_t tri = (size_t)N * (N + 1) / 2;
+    int rc = PIMDB_OK;
+    if (prob || E) {
+        rc = need_buffer(ctx, &ctx->E, tri);
+        if (!rc) rc = need_buffer(ctx, &ctx->ET, tri);
+    }
+    if (!rc && prob) rc = need_buffer(ctx, &ctx->prob, (size_t)N * N);
+    if (rc) return rc;
     launch_exchange_forward(ctx, ctx->s0);
     if (prob || E) launch_cycle_energies_ctx(ctx, ctx->s0);
     if (prob) {
@@ -698,7 +716,7 @@ int pimdb_exchange_forward(pimdb_ctx* ctx, double* VB, double* V, double* Vb, do
                            ctx->dv.bt, ctx->E, ctx->V, ctx->Vb, ctx->prob);
     }
     CK(hipGetLastError());
-    int rc = check_status(ctx);
+    rc = check_status(ctx);
     if (rc) return rc;
     if (VB) CK(hipMemcpy(VB, ctx->V + N, sizeof(double), hipMemcpyDeviceToHost));
     if (V) CK(hipMemcpy(V, ctx->V, sizeof(double) * (N + 1), hipMemcpyDeviceToHost));
@@ -815,8 +833,9 @@ int pimdb_observables(pimdb_ctx* ctx, double* out) {
         hipLaunchKernelGGL(k_nh_energy, dim3(1), dim3(256), 0, ctx->s0, ctx->nh, ndof, ctx->obs + all - 1);
     }
     CK(hipGetLastError());
-    const double* h = read_obs(ctx, 0, all);
-    if (!h) return ctx->fail(PIMDB_E_HIP, "reading the observables failed");
+    std::vector<double> obs(all);
+    CK(read_obs(ctx, 0, obs));
+    const double* h = obs.data();
     int rc = check_status(ctx);
     if (rc) return rc;
     double prim[3] = {0.0, 0.0, 0.0}, VN = 0.0;
@@ -845,8 +864,9 @@ int pimdb_exchange_estimators(pimdb_ctx* ctx, double* prim, double* prob_distinc
         launch_estimators(ctx);
     }
     CK(hipGetLastError());
-    const double* h = read_obs(ctx, tail, obs_doubles(N, P) - tail);
-    if (!h) return ctx->fail(PIMDB_E_HIP, "reading the estimators failed");
+    std::vector<double> est(obs_doubles(N, P) - tail);
+    CK(read_obs(ctx, tail, est));
+    const double* h = est.data();
     int rc = check_status(ctx);
     if (rc) return rc;
     double e[3];
