@@ -212,7 +212,7 @@ int pimdb_xplan_backward_saved(pimdb_xplan* plan, const double* saved, const dou
 /* pimdb_xplan_create + pimdb_xplan_forward (VB only) + pimdb_xplan_vb_grad in
  * one call that allocates nothing: the same kernels, with their workspace
  * (V, Vb, the ring's link prefix sums, the recursions' published values, the
- * overflow flag) in a fixed device array of the library (96 KB per GPU, held until the process ends).  x1, xP,
+ * overflow flag) in a fixed device array of the library (128 KB per GPU, held until the process ends).  x1, xP,
  * VB (may be NULL) and grad (may be NULL: forward only) are device arrays as
  * above.  natoms <= 2048 (and within the recursion's LDS workspace), else
  * PIMDB_E_ARG; the message of any failure is pimdb_last_error(NULL).  Every

@@ -10,33 +10,53 @@
 // idle and one CU's vector units carry a direction's N^2/2 terms: N=256 took
 // 36.8 us and N=1000 271 us.  The terms of target block I over the sources of
 // block J < I depend on earlier blocks only through the 64 values U of block
-// J, so block I's workgroup evaluates everything else ahead of time and waits
-// for those values.  What is left on the chain from one block to the next:
-// the 64 x 64 exponentials against the previous block, one reduction, the
-// in-block substitution and the publication of 64 doubles.
+// J, so block I's workgroup prepares everything else and waits for those.
 //
-// Publication.  U (plus, backward, the source's ln(N-q) term) goes to a
-// global array by relaxed device-scope atomic stores and is read by relaxed
-// device-scope atomic loads until it differs from XW_EMPTY (a NaN pattern no
-// result carries): the value is its own flag, so no fence is needed.  A
-// workgroup waits only for lower-numbered ones, which are dispatched first,
-// and a wait ends after XW_SPIN polls at the latest (the status flag is then
-// set).  The last block's workgroup has read every value once all others have
-// (block J publishes only after its own reads), so it puts XW_EMPTY back for
-// the next launch.
+// Scaling.  No running minimum is needed between neighbours.  Let
+//     G_t = sum_{r <= t} (e_r + l_r / 2)
+// over a block's targets, e_r = beta~ ecyc(r) the one-particle cycle's energy
+// and l_r the logarithm its term carries (ln n forward, ln(N-q) backward; a
+// scale only, so the hardware's single-precision logarithm serves), and
+//     z_t = exp(-(U_t - G_t - sigma)),   sigma = U of the last earlier target
+// (plus, backward, its logarithm as a source; 0 in block 0).  Then
+//     z_t = s_t + sum_{j<t} B(j,t) z_j,      B(j,t) = c(j,t) exp(G_t - G_j - w'(t,j)),
+//     s_t = [ sum_{j in J} E(j,t) z_j + f_t ] / z_last,
+//     E(j,t) = c(j,t) exp(G_t + G^J_last - G^J_j - w'(t,j)),   J the block before,
+// w' being w without its logarithm and c the factor that stands for it (1/n
+// forward; backward 1/(N-j), and in E (N-last)/(N-j)), f_t the farther sources
+// in J's scale (an online log-sum-exp, finished a block earlier).  B, E and f
+// are known before block J's z arrive, so the chain from block to block is
+// 64 x 64 multiply-adds on four waves, a reduction, the in-block substitution
+// (row by row of 16 lanes, xw_substitute) and the publication of 64 values: no
+// exponential or logarithm, and no minimum.
 //
-// Scaling.  The in-block part needs no min-plus pass.  With the one-particle
-// cycles' energies e_r = beta~ ecyc(r) and their running sum
-// g_t = sum_{r <= t} e_r over the block's targets,
-//     z_t = exp(-(U_t - g_t - sigma)),  sigma = U of the last earlier target,
-// obeys  z_t = s_t + sum_{j<t} B(j,t) z_j,  B(j,t) = exp(g_t - g_j - w(t,j)),
-//     s_t = sum_{q earlier} exp(sigma + g_t - w(t,q) - U_q):
-// B is known before any U arrives and s needs no running minimum for the
-// sources of the previous block (farther ones keep their online log-sum-exp,
-// off the chain).  z_t is at least the one-particle path's product of 1/n,
-// e^-621 for N = 2^14, and it overflows only where longer cycles are favoured
-// by e^700 within one block; such a block (z not in [1e-290, 1e290]) is taken
-// again by the exact min-plus form (xw_block_safe).
+// What bounds it: instructions on the chain.  One wave issues a dependent
+// instruction every 8 cycles (measured, single and double precision alike), so
+// the substitution's 60 dependent steps and their operands' addressing, the
+// prefix sums' scans and every logarithm (470 cycles) show.  Hence the dense
+// in-block matrix (xw_b), sums split before they are scanned (xw_stage), and
+// work off the chain on other waves.  Both recursions with the exterior force
+// took 10.9, 12.7, 25.2, 42.4 and 76.8 us at N = 4, 64, 256, 500 and 1000 with
+// the block's exponentials, its logarithm and a substitution through scalar
+// registers on the chain, and take 8.0, 9.5, 19.3, 31.1 and 54.1 us so.
+//
+// Range.  z stays near exp(-+ sum l_r / 2), 1e-116 .. 1e116 for the largest
+// rings here, between one-particle and freely exchanging cycles.  A block with
+// z outside 1e-140 .. 1e140, or after one whose z falls below 1e-140 of its
+// largest (an entry of B or E that underflowed could count then; one that
+// overflowed makes z infinite or NaN), is taken again by the exact min-plus
+// form (xw_block_safe) and publishes XW_BAD, on which the next block takes its
+// U like a farther block's.
+//
+// Publication.  z, and off the chain U (plus, backward, the source's ln(N-q)),
+// go to global arrays by relaxed device-scope atomic stores and are read by
+// relaxed device-scope atomic loads until they differ from XW_EMPTY (NaN
+// patterns that no result carries): the value is its own flag, so no fence is
+// needed.  A workgroup waits only for lower-numbered ones, which are
+// dispatched first, and a wait ends after XW_SPIN polls at the latest (the
+// status flag is then set).  The last block's workgroup reads U of every block
+// before it, each published after that block's own reads, so it puts XW_EMPTY
+// back for the next launch.
 #pragma once
 
 #include "exchange.hpp"
@@ -47,66 +67,66 @@ namespace pimdb {
 // card to itself; 256 beside other rings' work, where the idle waves of a
 // waiting workgroup would hold registers that others could use.
 constexpr int XW_THREADS = 1024;
-constexpr unsigned long long XW_EMPTY = ~0ull;
+constexpr unsigned long long XW_EMPTY = ~0ull, XW_BAD = ~1ull;
+constexpr double XW_RANGE = 1e140;
 constexpr long long XW_SPIN = 1ll << 22;             // polls of one wait (seconds)
 
-// Global workspace of one ring: the published values of both directions.
-__host__ __device__ inline size_t xw_pub_words(int N) { return 2 * ((size_t)N + 1); }
+// Global workspace of one ring: z and U of both directions.
+__host__ __device__ inline size_t xw_pub_words(int N) { return 4 * ((size_t)N + 1); }
 __host__ __device__ inline int xw_grid(int N) { return 2 * rec_blocks(N); }
 
-// LDS doubles: the ring, the block's gauge and source logarithms, the
-// in-block matrix, per-wave partials, the substitution's results, the wave
-// totals of the prefix sums and a flag.
+// The in-block matrix by rows of 16 sources and, in a row, by target: entry
+// (j, t), 16 R <= j < 16 R + 16, t >= 16 R, at xw_b(j, t), so that a target's
+// 16 coefficients are contiguous and, 18 apart, meet every bank alike; entries
+// j >= t of the diagonal parts are 0.
+constexpr int XW_BS = 18;
+__host__ __device__ __forceinline__ constexpr int xw_brow(int R) { return XW_BS * (REC_B * R - 8 * R * (R - 1)); }
+__device__ __forceinline__ int xw_b(int j, int t) {
+    const int R = j / 16;
+    return xw_brow(R) + (t - 16 * R) * XW_BS + (j - 16 * R);
+}
+constexpr int XW_MAT = xw_brow(4);
+constexpr int XW_SAFE_WAVES = 8;   // waves that take sources in the safe form
+static_assert(XW_MAT >= REC_TRI + XW_SAFE_WAVES * REC_B + 3 * REC_B, "the safe form's arrays lie in the matrix's place");
+
+// LDS doubles: the ring, the in-block matrix, the per-wave partials, the
+// block's gauge, the previous block's gauge and factors as sources, the
+// targets' logarithms as sources, the prefix sums' wave totals, the flags.
 __host__ __device__ inline size_t xw_shared_doubles(int N, int D, int nw) {
-    return (size_t)(2 * D + 2) * N + 2 * REC_B + (size_t)REC_TRI + 2 * (size_t)nw * REC_B + 2 * REC_B + 2 * (size_t)nw + 2;
+    return (size_t)(2 * D + 2) * N + (size_t)XW_MAT + (size_t)nw * REC_B + 4 * REC_B + 3 * (size_t)nw + 1 + 2;
 }
 inline size_t xw_lds_bytes(int N, int D, int threads = XW_THREADS) {
     return sizeof(double) * xw_shared_doubles(N, D, threads / WAVE);
 }
 
 struct XwShared {
+    double *a;                     // [XW_MAT] in-block matrix B
+    double *psum;                  // [waves][REC_B]
+    double *g;                     // [REC_B] gauge
+    double *off, *rat;             // [REC_B] the previous block's: G_last - G_j, and backward (N-last)/(N-j)
+    double *lq;                    // [REC_B] backward, ln(N-q) of the targets as sources
+    double *tot;                   // [3 waves] wave totals: links, their split sums; then G_last of the previous block
+    int* flag;                     // [0] the block left the range, [1] the previous one did, [2] its z fall too far
     double *x1, *xP, *Shi, *Slo;   // the ring [D][N], [D][N], [N], [N]
-    double *g, *lgs;               // [REC_B] gauge; ln(N-q) of the block as sources (backward)
-    double *a;                     // [REC_TRI] in-block matrix at rec_idx(j, t)
-    double *part, *psum;           // [waves][REC_B]
-    double *R, *z;                 // [REC_B]
-    double *tot;                   // [2 waves] wave totals of the prefix sums
-    int* flag;
 };
 
 template <int NT>
 __device__ __forceinline__ XwShared xw_carve(double* p, int N, int D) {
     constexpr int NW = NT / WAVE;
     XwShared s;
+    s.a = p; p += XW_MAT;
+    s.psum = p; p += NW * REC_B;
+    s.g = p; p += REC_B;
+    s.off = p; p += REC_B;
+    s.rat = p; p += REC_B;
+    s.lq = p; p += REC_B;
+    s.tot = p; p += 3 * NW + 1;
+    s.flag = (int*)p; p += 2;
     s.x1 = p; p += (size_t)D * N;
     s.xP = p; p += (size_t)D * N;
     s.Shi = p; p += N;
-    s.Slo = p; p += N;
-    s.g = p; p += REC_B;
-    s.lgs = p; p += REC_B;
-    s.a = p; p += REC_TRI;
-    s.part = p; p += NW * REC_B;
-    s.psum = p; p += NW * REC_B;
-    s.R = p; p += REC_B;
-    s.z = p; p += REC_B;
-    s.tot = p; p += 2 * NW;
-    s.flag = (int*)p;
+    s.Slo = p;
     return s;
-}
-
-template <int CTRL, int ROWS>
-__device__ __forceinline__ DD dd_scan_step(DD v) {
-    return dd_add(DD{dpp_or_zero<CTRL, ROWS>(v.hi), dpp_or_zero<CTRL, ROWS>(v.lo)}, v);
-}
-// Inclusive sums over the lanes of a wave (wave_scan's steps).
-__device__ __forceinline__ DD dd_wave_scan(DD v) {
-    v = dd_scan_step<0x111, 0xF>(v);
-    v = dd_scan_step<0x112, 0xF>(v);
-    v = dd_scan_step<0x114, 0xF>(v);
-    v = dd_scan_step<0x118, 0xF>(v);
-    v = dd_scan_step<0x142, 0xA>(v);
-    v = dd_scan_step<0x143, 0xC>(v);
-    return v;
 }
 
 // One bead's positions: axis a of particle i at p[a sa + i si].
@@ -116,71 +136,184 @@ struct BeadView {
     __device__ __forceinline__ double at(int a, int i) const { return p[a * sa + i * si]; }
 };
 
-// Beads 1 and P into LDS and the split prefix sums of the ring's links
-// (exchange.hpp, Ring), by the whole workgroup: every thread sums a run of
-// links, the waves scan their totals.  Every workgroup of a ring computes the
-// same values.  Shi_out / Slo_out / xc_out (may be null) receive the sums and
-// a copy [2][D][N] of the two beads.
-template <int D, int NT>
-__device__ __forceinline__ Ring xw_stage(const XwShared& sh, int N, BeadView x1, BeadView xP, double k, bool pbc, double L,
-                                         double* Shi_out, double* Slo_out, double* xc_out) {
+// 1 / x within an ulp (x normal).
+__device__ __forceinline__ double rcp_newton(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
+// The gauge of target block I over the ring's particles, one target per lane
+// (whole wave): positions loaded ahead (get), then the scan.
+template <int DIR, int D>
+struct XwGauge {
+    double u[D], v[D];
+    __device__ __forceinline__ void get(int I, int N, int lane, BeadView x1, BeadView xP) {
+        const int n = 1 + I * REC_B + lane, idx = DIR == 0 ? min(n, N) - 1 : max(N - n, 0);
+#pragma unroll
+        for (int ax = 0; ax < D; ++ax) {
+            u[ax] = x1.at(ax, idx);
+            v[ax] = xP.at(ax, idx);
+        }
+    }
+    __device__ __forceinline__ double scan(int I, int N, int lane, double bk, const Ring& r) const {
+        const int n = 1 + I * REC_B + lane;
+        double d[D];
+#pragma unroll
+        for (int ax = 0; ax < D; ++ax) d[ax] = ring_image(u[ax] - v[ax], r);
+        // l / 2 = ln 2 / 2 log2(n) or log2(N - n + 1)
+        const float c = (float)max(1, DIR == 0 ? n : N - n + 1);
+        return wave_scan(fma(bk, norm2_fma<D>(d), (double)(0.34657359f * __builtin_amdgcn_logf(c))));
+    }
+};
+
+// Beads 1 and P into LDS, the split prefix sums of the ring's links
+// (exchange.hpp, Ring), the gauges of target block I (wave 1) and of the block
+// before it (wave 2), the latter's factors and the targets' logarithms (wave
+// 3), by the whole workgroup.  The links are split into multiples of
+// q = 2^(e-40) and remainders before they are summed, 2^e <= their total <
+// 2^(e+1): the multiples add exactly (at most 42 bits) in any order and the
+// remainders' sums stay below N q / 2, so plain sums keep what a sum in double
+// double kept, in a tenth of the instructions.  Every workgroup of a ring
+// computes the same values.  Shi_out / Slo_out / xc_out (may be null) receive
+// the sums and a copy [2][D][N] of the two beads.
+template <int DIR, int D, int NT>
+__device__ __forceinline__ Ring xw_stage(const XwShared& sh, int I, int N, double bt, BeadView x1, BeadView xP, double k,
+                                         bool pbc, double L, double* Shi_out, double* Slo_out, double* xc_out) {
     constexpr int NW = NT / WAVE;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const Ring r = make_ring(sh.x1, sh.xP, sh.Shi, sh.Slo, k, pbc, L);
-    for (int e = tid; e < D * N; e += NT) {
-        const int a = D == 1 ? 0 : e / N, i = e - a * N;
-        const double u = x1.at(a, i), v = xP.at(a, i);
+    const double bk = bt * r.halfk;
+    const int c = (N + NT - 1) / NT, v0 = tid * c;
+    auto keep = [&](int a, int i, double u, double v) {
+        const int e = a * N + i;
         sh.x1[e] = u;
         sh.xP[e] = v;
         if (xc_out) {
             xc_out[e] = u;
             xc_out[(size_t)D * N + e] = v;
         }
-    }
-    const int c = (N + NT - 1) / NT, v0 = tid * c;
-    auto link = [&](int v) {
+    };
+    auto split_link = [&](int v) {   // (more than one link per thread: from LDS)
         double d[D];
 #pragma unroll
-        for (int ax = 0; ax < D; ++ax) d[ax] = ring_image(x1.at(ax, v + 1) - xP.at(ax, v), r);
+        for (int ax = 0; ax < D; ++ax) d[ax] = ring_image(sh.x1[ax * N + v + 1] - sh.xP[ax * N + v], r);
         return norm2_fma<D>(d);
     };
-    DD sum{0.0, 0.0};
-    double first = 0.0;   // the thread's first link, kept for the running sums of runs of one
-    for (int v = v0; v < min(v0 + c, N - 1); ++v) {
-        const double l = link(v);
-        if (v == v0) first = l;
-        sum = dd_add(sum, DD{l, 0.0});
-    }
-    const DD inc = dd_wave_scan(sum);
-    if (lane == WAVE - 1) {
-        sh.tot[2 * wave] = inc.hi;
-        sh.tot[2 * wave + 1] = inc.lo;
-    }
-    __syncthreads();
-    DD tw{0.0, 0.0};
-    if (lane < NW) tw = DD{sh.tot[2 * lane], sh.tot[2 * lane + 1]};
-    tw = dd_wave_scan(tw);
-    const double total = wave_bcast_uniform(tw.hi, NW - 1);
-    DD ex{dpp_or_zero<0x138, 0xF>(inc.hi), dpp_or_zero<0x138, 0xF>(inc.lo)};   // wave_shr:1
-    if (wave > 0) ex = dd_add(DD{wave_bcast_uniform(tw.hi, wave - 1), wave_bcast_uniform(tw.lo, wave - 1)}, ex);
-    const double q = total > 0.0 ? ldexp(1.0, ilogb(total) - 40) : 1.0;
-    const double invq = 1.0 / q;
-    for (int v = v0; v < min(v0 + c, N); ++v) {
-        const double h = rint(ex.hi * invq) * q, l = (ex.hi - h) + ex.lo;
+    auto put = [&](int v, double h, double l) {
         sh.Shi[v] = h;
         sh.Slo[v] = l;
         if (Shi_out) {
             Shi_out[v] = h;
             Slo_out[v] = l;
         }
-        if (v + 1 < v0 + c && v < N - 1) ex = dd_add(ex, DD{v == v0 ? first : link(v), 0.0});
+    };
+    XwGauge<DIR, D> ga;
+    const bool gauges = wave == 1 || (wave == 2 && I > 0);
+    if (gauges) ga.get(I - (wave - 1), N, lane, x1, xP);
+    double sum = 0.0;   // the thread's links
+    if (c == 1) {       // a particle and its link per thread, all loads together
+        if (tid < N) {
+            double u[D], v[D], w[D], d[D];
+#pragma unroll
+            for (int ax = 0; ax < D; ++ax) {
+                u[ax] = x1.at(ax, tid);
+                v[ax] = xP.at(ax, tid);
+                w[ax] = x1.at(ax, min(tid + 1, N - 1));
+            }
+#pragma unroll
+            for (int ax = 0; ax < D; ++ax) {
+                keep(ax, tid, u[ax], v[ax]);
+                d[ax] = ring_image(w[ax] - v[ax], r);
+            }
+            if (tid < N - 1) sum = norm2_fma<D>(d);
+        }
+    } else {
+        for (int e = tid; e < D * N; e += NT) {
+            const int a = D == 1 ? 0 : e / N, i = e - a * N;
+            keep(a, i, x1.at(a, i), xP.at(a, i));
+        }
+        __syncthreads();
+        for (int v = v0; v < min(v0 + c, N - 1); ++v) sum += split_link(v);
+    }
+    if (tid < 4) sh.flag[tid] = 0;
+    if (gauges) {
+        const double g = ga.scan(I - (wave - 1), N, lane, bk, r);
+        if (wave == 1) sh.g[lane] = g;
+        if (wave == 2) {
+            const double gl = wave_bcast_uniform(g, WAVE - 1);
+            sh.off[lane] = gl - g;
+            sh.tot[3 * NW] = gl;
+        }
+    }
+    if (DIR == 1 && wave == 3) {
+        const int n0 = 1 + I * REC_B;
+        if (I > 0) sh.rat[lane] = (double)(N - n0 + 1) * rcp_newton((double)(N - n0 + REC_B - lane));   // j = n0 - 64 + lane
+        sh.lq[lane] = log((double)max(1, N - n0 - lane));
+    }
+    // the quantum from the links' total, the same bits in every wave
+    auto quantum = [](double total) { return total > 0.0 ? __builtin_amdgcn_frexp_exp(total) - 41 : 0; };
+    if (N <= WAVE && c == 1) {   // one wave has every link
+        if (wave == 0) {
+            const int qe = quantum(wave_total(sum));
+            const double h = ldexp(rint(ldexp(sum, -qe)), qe), l = sum - h;
+            const double hs = wave_scan(h) - h, ls = wave_scan(l) - l;
+            if (lane < N) put(lane, hs, ls);
+        }
+        __syncthreads();
+        return r;
+    }
+    const double wt = wave_scan(sum);
+    if (lane == WAVE - 1) sh.tot[wave] = wt;
+    __syncthreads();
+    auto row_scan = [](double v) {   // (at most 16 waves)
+        v += dpp_or_zero<0x111, 0xF>(v);
+        v += dpp_or_zero<0x112, 0xF>(v);
+        v += dpp_or_zero<0x114, 0xF>(v);
+        v += dpp_or_zero<0x118, 0xF>(v);
+        return v;
+    };
+    const int qe = quantum(wave_bcast_uniform(row_scan(lane < NW ? sh.tot[lane] : 0.0), NW - 1));
+    double h = 0.0, l = 0.0;
+    auto add = [&](double x) {
+        const double m = ldexp(rint(ldexp(x, -qe)), qe);
+        h += m;
+        l += x - m;
+    };
+    if (c == 1) add(sum);
+    else
+        for (int v = v0; v < min(v0 + c, N - 1); ++v) add(split_link(v));
+    const double hi = wave_scan(h), li = wave_scan(l);
+    if (lane == WAVE - 1) {
+        sh.tot[NW + wave] = hi;
+        sh.tot[2 * NW + wave] = li;
+    }
+    __syncthreads();
+    double hs = hi - h, ls = li - l;
+    if (wave > 0) {
+        hs += wave_bcast_uniform(row_scan(lane < NW ? sh.tot[NW + lane] : 0.0), wave - 1);
+        ls += wave_bcast_uniform(row_scan(lane < NW ? sh.tot[2 * NW + lane] : 0.0), wave - 1);
+    }
+    if (c == 1) {
+        if (tid < N) put(tid, hs, ls);
+    } else {
+        for (int v = v0; v < min(v0 + c, N); ++v) {
+            put(v, hs, ls);
+            if (v < N - 1) {
+                h = hs;
+                l = ls;
+                add(split_link(v));
+                hs = h;
+                ls = l;
+            }
+        }
     }
     __syncthreads();
     return r;
 }
 
-// The target side of w(n,q) of one lane, and w(n,q) without the source's
-// logarithm (backward: ln(N-q) travels with the published U).
+// The target side of w(n,q) of one lane, and w(n,q) without its logarithm
+// (forward ln n, backward ln(N-q)).
 template <int DIR, int D>
 __device__ __forceinline__ RecTarget<D> xw_target(const XwShared& sh, int N, int n) {
     RecTarget<D> t;
@@ -190,7 +323,7 @@ __device__ __forceinline__ RecTarget<D> xw_target(const XwShared& sh, int N, int
     for (int a = 0; a < D; ++a) t.x[a] = xs[a * N + idx];
     t.shi = sh.Shi[idx];
     t.slo = sh.Slo[idx];
-    t.lg = DIR == 0 ? log((double)n) : 0.0;
+    t.lg = 0.0;
     return t;
 }
 template <int DIR, int D>
@@ -203,7 +336,7 @@ __device__ __forceinline__ double xw_w(const XwShared& sh, const Ring& r, double
     for (int a = 0; a < D; ++a) d[a] = ring_image(xs[a * N + idx] - t.x[a], r);
     const double sd = DIR == 0 ? ring_sdiff(t.shi, t.slo, sh.Shi[idx], sh.Slo[idx])
                                : ring_sdiff(sh.Shi[idx], sh.Slo[idx], t.shi, t.slo);
-    return fma(bk, sd + norm2_fma<D>(d), t.lg);
+    return bk * (sd + norm2_fma<D>(d));
 }
 
 __device__ __forceinline__ unsigned long long xw_bits(double v) { return (unsigned long long)__double_as_longlong(v); }
@@ -214,92 +347,199 @@ __device__ __forceinline__ void xw_publish(unsigned long long* p, double v) {
     if (b == XW_EMPTY) b = 0x7FF8000000000000ull;
     __hip_atomic_store(p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The 64 values of a finished block, one per lane (whole wave).
-__device__ __forceinline__ double xw_wait(unsigned long long* p, int lane, int* status) {
+// The 64 values of a finished block from p, one per lane (whole wave; p[at]
+// for the lane).
+__device__ __forceinline__ double xw_wait(unsigned long long* p, int at, int* status) {
+    // (asleep between polls: what is awaited here is off the chain, and the polls
+    // of the whole card share the caches with those that are on it)
     unsigned long long b = XW_EMPTY;
     long long spin = 0;
     for (;;) {
-        b = __hip_atomic_load(p + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        b = __hip_atomic_load(p + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__all(b != XW_EMPTY)) break;
         if (++spin >= XW_SPIN) {
-            if (lane == 0) raise_status(status);
+            raise_status(status);
             break;
         }
-        __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_s_sleep(4);
     }
     return __longlong_as_double((long long)b);
 }
 
-// One block with the exact min-plus shifts (exchange.hpp, steps (1)-(4)),
-// every earlier U being published: for blocks whose z left the range.  All
-// threads; U of the lane's target in every lane of wave 0.
+// One block with the exact min-plus shifts (exchange.hpp, steps (1)-(4)) from
+// every earlier U: for blocks whose z left the range.  All threads; U of the
+// lane's target in every lane of wave 0.
 template <int DIR, int D, int NT>
-__device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, double u0, const Ring r, const XwShared sh,
-                                             unsigned long long* pub) {
-    constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // sources of a block per wave
+__device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, const Ring r, const XwShared sh,
+                                             unsigned long long* upub, int* status) {
+    constexpr int NW = NT / WAVE, SW = NW < XW_SAFE_WAVES ? NW : XW_SAFE_WAVES, SRC = REC_B / SW;
+    double *part = sh.a + REC_TRI, *R = part + SW * REC_B, *z = R + REC_B, *lt = z + REC_B;   // (in the matrix's place)
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const int n0 = 1 + I * REC_B;
-    const RecTarget<D> tg = xw_target<DIR, D>(sh, N, n0 + min(lane, nb - 1));
+    const int n0 = 1 + I * REC_B, tl = min(lane, nb - 1);
+    __syncthreads();   // (the matrix is no longer read)
+    // the logarithm of the lane's target: as a target forward, as a source backward
+    if (wave == 0) lt[lane] = DIR == 0 ? log((double)(n0 + tl)) : sh.lq[lane];
+    const double u0 = DIR == 0 ? 0.0 : log((double)N);
+    const RecTarget<D> tg = xw_target<DIR, D>(sh, N, n0 + tl);
+    __syncthreads();
+    const double lg = DIR == 0 ? lt[lane] : 0.0;
     double m = INFINITY, s = 0.0;
     auto add = [&](int q, double uq) {
-        const double y = xw_w<DIR, D>(sh, r, bk, N, tg, q) + uq;
+        const double y = xw_w<DIR, D>(sh, r, bk, N, tg, q) + lg + uq;
         const double mn = fmin(m, y);
         s = fma(s, exp_pair(mn - m), exp_pair(mn - y));   // m = inf (first source): s = 0 stays 0
         m = mn;
     };
+    auto inblock = [&](int j, int t) {
+        const double w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j);
+        return w + lt[DIR == 0 ? t : j];
+    };
     if (wave == 0) add(0, u0);
-    for (int J = 0; J < I; ++J)
-        for (int u = 0; u < XW_SRC; ++u) {
-            const int q = J * REC_B + 1 + wave * XW_SRC + u;
-            add(q, __longlong_as_double((long long)__hip_atomic_load(pub + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+    if (wave < SW) {
+        for (int J = 0; J < I; ++J) {
+            const double v = xw_wait(upub + J * REC_B + 1, lane, status);
+            for (int u = 0; u < SRC; ++u) add(J * REC_B + 1 + wave * SRC + u, wave_bcast_uniform(v, wave * SRC + u));
         }
-    sh.part[wave * REC_B + lane] = lane < nb ? m : INFINITY;
-    sh.psum[wave * REC_B + lane] = lane < nb ? s : 0.0;
+        part[wave * REC_B + lane] = lane < nb ? m : INFINITY;
+    }
     for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
-        if (t < 0) continue;
-        double w = INFINITY;
-        if (t < nb) w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j) + sh.lgs[j];
-        sh.a[rec_idx(j, t)] = w;
+        if (t >= 0) sh.a[rec_idx(j, t)] = t < nb ? inblock(j, t) : INFINITY;
     }
     __syncthreads();
     if (wave == 0) {
         double rr = INFINITY;
-        for (int w = 0; w < NW; ++w) rr = fmin(rr, sh.part[w * REC_B + lane]);
-        rec_inblock_seq<0>(sh.a, lane, rr, sh.R);
+        for (int w = 0; w < SW; ++w) rr = fmin(rr, part[w * REC_B + lane]);
+        rec_inblock_seq<0>(sh.a, lane, rr, R);
     }
     __syncthreads();
-    {
-        const double sw = sh.psum[wave * REC_B + lane];
-        double c = 0.0;
-        if (lane < nb && sw > 0.0) c = sw * exp_pair(sh.R[lane] - sh.part[wave * REC_B + lane]);
-        sh.psum[wave * REC_B + lane] = c;
-    }
+    if (wave < SW) sh.psum[wave * REC_B + lane] = lane < nb && s > 0.0 ? s * exp_pair(R[lane] - m) : 0.0;
     for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
-        if (t >= 0) sh.a[rec_idx(j, t)] = t < nb ? exp_pair(-(sh.a[rec_idx(j, t)] + sh.R[j] - sh.R[t])) : 0.0;
+        if (t >= 0) sh.a[rec_idx(j, t)] = t < nb ? exp_pair(-(sh.a[rec_idx(j, t)] + R[j] - R[t])) : 0.0;
     }
     __syncthreads();
     double u = 0.0;
     if (wave == 0) {
         double z0 = 0.0;
-        for (int w = 0; w < NW; ++w) z0 += sh.psum[w * REC_B + lane];
-        rec_inblock_seq<1>(sh.a, lane, z0, sh.z);
-        u = sh.R[lane] - log(sh.z[lane]);
+        for (int w = 0; w < SW; ++w) z0 += sh.psum[w * REC_B + lane];
+        rec_inblock_seq<1>(sh.a, lane, z0, z);
+        u = R[lane] - log(z[lane]);
     }
     __syncthreads();
     return u;
 }
 
-// Target block I of one recursion on one workgroup of NT threads
-// (the ring staged).  pub: this direction's published values [N+1].
+// Row R (lanes 16R .. 16R+15) of v in every row.
+template <int R>
+__device__ __forceinline__ unsigned row_everywhere(unsigned v) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    const unsigned x = h[R / 2];
+    const auto q = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return q[R % 2];
+}
+template <int R>
+__device__ __forceinline__ double row_everywhere(double v) {
+    return __hiloint2double((int)row_everywhere<R>((unsigned)__double2hiint(v)),
+                            (int)row_everywhere<R>((unsigned)__double2loint(v)));
+}
+// w += c * (lane J of the row's w), and acc += c * (lane J of the row's w):
+// one instruction, the broadcast being its DPP operand (two wait states after
+// the write of w).
+template <int J>
+__device__ __forceinline__ void row_step(double& w, double c) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(w) : "v"(c), "n"(J));
+}
+template <int J>
+__device__ __forceinline__ void row_add(double& acc, double w, double c) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc)
+        : "v"(w), "v"(c), "n"(J));
+}
+// 16 contiguous coefficients (16-byte aligned).
+__device__ __forceinline__ void xw_coefs(const double* a, double (&d)[16]) {
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) {
+        const double2 v = *(const double2*)(a + j);
+        d[j] = v.x;
+        d[j + 1] = v.y;
+    }
+}
+template <int J>
+__device__ __forceinline__ void row_steps(double& w, const double (&d)[16]) {
+    if constexpr (J < 15) {
+        row_step<J>(w, d[J]);
+        row_steps<J + 1>(w, d);
+    }
+}
+template <int J>
+__device__ __forceinline__ void row_adds(double& v0, double& v1, double w, const double (&u)[16]) {
+    if constexpr (J < 16) {
+        row_add<J>(v0, w, u[J]);
+        row_add<J + 1>(v1, w, u[J + 1]);
+        row_adds<J + 2>(v0, v1, w, u);
+    }
+}
+// One row of 16 targets: its own substitution in every row at once, then its
+// share of the later rows' sums.  d: the row's own coefficients, replaced by
+// the next row's.
+template <int R>
+__device__ __forceinline__ void xw_row(const double* a, int lane, int nb, double& v, double& z, double (&d)[16]) {
+    if (16 * R >= nb) return;   // (uniform)
+    double u[16];
+    if constexpr (R < 3) xw_coefs(a + xw_brow(R) + max(lane - 16 * R, 0) * XW_BS, u);
+    double w = row_everywhere<R>(v);
+    row_steps<0>(w, d);
+    z = lane / 16 == R ? w : z;
+    if constexpr (R < 3) {
+        xw_coefs(a + xw_brow(R + 1) + lane % 16 * XW_BS, d);
+        double v1 = 0.0;
+        row_adds<0>(v, v1, w, u);
+        v += v1;
+        xw_row<R + 1>(a, lane, nb, v, z, d);
+    }
+}
+// The substitution z_t = s_t + sum_{j<t} B(j,t) z_j of one wave, lane t
+// holding s_t, for a block of nb targets.  Values of rows already done are not
+// used again, so the later sums run over all rows without a mask.  A step is
+// one multiply-add with the broadcast in it (16 cycles) instead of two
+// cross-lane reads through scalar registers and a multiply-add (52).
+__device__ __forceinline__ double xw_substitute(const double* a, int lane, int nb, double v) {
+    double d[16], z = 0.0;
+    xw_coefs(a + lane % 16 * XW_BS, d);
+    xw_row<0>(a, lane, nb, v, z, d);
+    return z;
+}
+
+// The 16 z of a row of the previous block in every row of lanes and its last
+// one, zl (XW_BAD in place of both if that block left the range).
+__device__ __forceinline__ void xw_wait_z(unsigned long long* p, int row, int lane, int* status, double& z, double& zl) {
+    unsigned long long b = XW_EMPTY, e = XW_EMPTY;
+    for (long long spin = 0;; ++spin) {
+        b = __hip_atomic_load(p + 16 * row + lane % 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        e = __hip_atomic_load(p + REC_B - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__all(b != XW_EMPTY && e != XW_EMPTY)) break;
+        if (spin >= XW_SPIN) {
+            raise_status(status);
+            b = e = XW_BAD;
+            break;
+        }
+    }
+    z = __longlong_as_double((long long)b);
+    zl = __longlong_as_double((long long)e);
+}
+
+// Target block I of one recursion on one workgroup of NT threads (the ring
+// staged).  zpub, upub: this direction's published values [N+1].
 template <int DIR, int D, int NT>
 __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r, const XwShared& sh,
-                                         unsigned long long* __restrict__ pub, double* __restrict__ V,
-                                         double* __restrict__ Vb, double* __restrict__ VB, int* __restrict__ status) {
-    constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // sources of a block per wave
+                                         unsigned long long* __restrict__ zpub, unsigned long long* __restrict__ upub,
+                                         double* __restrict__ V, double* __restrict__ Vb, double* __restrict__ VB,
+                                         int* __restrict__ status) {
+    constexpr int NW = NT / WAVE, XW_SRC = REC_B / NW;   // farther sources of a block per wave
+    constexpr int ZW = 4;                                // waves that take the previous block's z, a row each
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int ntarget = DIR == 0 ? N : N - 1;
     const int n0 = 1 + I * REC_B, nb = min(REC_B, ntarget - n0 + 1);
@@ -310,98 +550,139 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
     if (nb <= 0) return;   // (the backward recursion's empty last block)
     const bool last = n0 + nb > ntarget;
     const double bk = bt * r.halfk;
-    const int tn = n0 + min(lane, nb - 1);
+    const int tl = min(lane, nb - 1), tn = n0 + tl;   // the lane's target (clamped)
+    const int qn = n0 - REC_B;                        // the previous block's first target (I > 0)
+    const double g = sh.g[lane];
+    const double cn = DIR == 0 ? rcp_newton((double)tn) : 1.0;       // the target's factor
+    const double c0 = DIR == 0 ? cn : rcp_newton((double)N);         // source 0's
     const RecTarget<D> tg = xw_target<DIR, D>(sh, N, tn);
-    const double u0 = DIR == 0 ? 0.0 : log((double)N);   // source 0
-    // the gauge: running sum of the one-particle cycles' energies
-    double e1;
-    {
-        const int idx = DIR == 0 ? tn - 1 : N - tn;
-        double d[D];
+    // the z waves' coefficients of the previous block
+    double E[16];
+    if (I > 0 && wave < ZW) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) d[a] = ring_image(sh.x1[a * N + idx] - sh.xP[a * N + idx], r);
-        e1 = bk * norm2_fma<D>(d);
-    }
-    const double g = wave_scan(e1);
-    const double lgs = DIR == 0 ? 0.0 : log((double)max(1, N - (n0 + lane)));   // the lane's target as a source
-    if (wave == 0) {
-        sh.g[lane] = g;
-        sh.lgs[lane] = lgs;
-    }
-    __syncthreads();
-    for (int vr = wave; vr < REC_B / 2; vr += NW) {
-        int t, j;
-        rec_tri(vr, lane, t, j);
-        if (t < 0) continue;
-        double c = 0.0;
-        if (t < nb) {
-            const double w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j) + sh.lgs[j];
-            c = exp_pair((sh.g[t] - sh.g[j]) - w);
+        for (int u = 0; u < 16; ++u) {
+            const int j = 16 * wave + u;
+            E[u] = exp_pair((g + sh.off[j]) - xw_w<DIR, D>(sh, r, bk, N, tg, qn + j)) * (DIR == 0 ? cn : sh.rat[j]);
         }
-        sh.a[rec_idx(j, t)] = c;
     }
-    // earlier sources: source 0 on wave 0, then XW_SRC of every block per wave
-    double m = INFINITY, s = 0.0, near = 0.0, sigma = u0;
-    if (wave == 0) {
-        m = xw_w<DIR, D>(sh, r, bk, N, tg, 0) + u0;
-        s = 1.0;
+    // the in-block matrix, by the other waves if there are any and E was to do
+    const int w0 = NW > ZW && I > 0 ? ZW : 0;
+    if (wave >= w0) {
+        for (int e = tid - w0 * WAVE; e < 4 * 256; e += NT - w0 * WAVE) {   // zeros of the diagonal parts
+            const int t = e / 16, j = t / 16 * 16 + e % 16;
+            if (j >= t) sh.a[xw_b(j, t)] = 0.0;
+        }
+        for (int vr = wave - w0; vr < REC_B / 2; vr += NW - w0) {
+            int t, j;
+            rec_tri(vr, lane, t, j);
+            if (t < 0) continue;
+            double c = 0.0;
+            if (t < nb) {
+                const double w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j);
+                c = exp_pair((sh.g[t] - sh.g[j]) - w) * rcp_newton((double)(DIR == 0 ? n0 + t : N - n0 - j));
+            }
+            sh.a[xw_b(j, t)] = c;
+        }
     }
-    // (four sources in registers at a time; the first four of a block are
-    // evaluated while their U are awaited)
-    constexpr int XQ = 4;
-    for (int J = 0; J < I; ++J) {
-        const int qb = J * REC_B + 1, q0 = wave * XW_SRC;
-        double w[XQ], uq[XQ];
+    // farther sources: source 0 on wave 0, then XW_SRC of every block per
+    // wave, four in registers at a time
+    const int q0 = wave * XW_SRC;
+    double m = INFINITY, s = 0.0, before = 0.0;   // before: the scale of the previous block's z
+    auto far = [&](int J) {
+        constexpr int XQ = 4;
+        const int qb = J * REC_B + 1;
+        double w[XQ];
 #pragma unroll
         for (int u = 0; u < XQ; ++u) w[u] = xw_w<DIR, D>(sh, r, bk, N, tg, qb + q0 + u);
-        const double v = xw_wait(pub + qb, lane, status);
-        if (J == I - 1) sigma = wave_bcast_uniform(v, REC_B - 1);
+        const double v = xw_wait(upub + qb, lane, status);
 #pragma unroll 1
         for (int c = 0; c < XW_SRC; c += XQ) {
+            double mn = m;
 #pragma unroll
             for (int u = 0; u < XQ; ++u) {
-                uq[u] = wave_bcast_uniform(v, q0 + c + u);
                 if (c > 0) w[u] = xw_w<DIR, D>(sh, r, bk, N, tg, qb + q0 + c + u);
+                w[u] += wave_bcast_uniform(v, q0 + c + u);
+                mn = fmin(mn, w[u]);
             }
-            if (J < I - 1) {
-                double mn = m;
+            s *= exp_pair(mn - m);   // m = inf: s = 0 stays 0
+            m = mn;
 #pragma unroll
-                for (int u = 0; u < XQ; ++u) {
-                    w[u] += uq[u];
-                    mn = fmin(mn, w[u]);
-                }
-                s *= exp_pair(mn - m);   // m = inf: s = 0 stays 0
-                m = mn;
-#pragma unroll
-                for (int u = 0; u < XQ; ++u) s += exp_pair(mn - w[u]);
-            } else {
-#pragma unroll
-                for (int u = 0; u < XQ; ++u) near += exp_pair((sigma - uq[u]) + (g - w[u]));
-            }
+            for (int u = 0; u < XQ; ++u) s += exp_pair(mn - w[u]);
         }
+        return wave_bcast_uniform(v, REC_B - 1);
+    };
+    if (wave == 0) {
+        m = xw_w<DIR, D>(sh, r, bk, N, tg, 0);
+        s = DIR == 0 ? 1.0 : c0;   // (forward the target's factor comes last)
     }
-    if (s > 0.0) near = fma(s, exp_pair((sigma - m) + g), near);
-    sh.psum[wave * REC_B + lane] = lane < nb ? near : 0.0;
-    __syncthreads();
+    double z, sigma = 0.0;      // wave 0: the lane's s_t, then z_t
+    bool known = I == 0;        // sigma is known
+    if (I == 0) {
+        z = s * cn * exp_pair(g - m);
+        __syncthreads();
+    } else {
+        for (int J = 0; J < I - 1; ++J) before = far(J);
+        const double cf = DIR == 0 ? cn : (double)(N - n0 + 1);
+        double acc = s > 0.0 ? s * cf * exp_pair((before + (sh.tot[3 * NW] + g)) - m) : 0.0;
+        if (NW > ZW) {
+            sh.psum[wave * REC_B + lane] = acc;
+        }
+        __syncthreads();   // (the matrix is complete, too)
+        if (wave < ZW) {
+            if (NW > ZW) {   // the slots of waves wave, wave + 4, ...; the first is then written
+                acc = 0.0;
+#pragma unroll
+                for (int w = 0; w < NW / ZW; ++w) acc += sh.psum[(wave + w * ZW) * REC_B + lane];
+            }
+            // (in registers before the wait: the compiler would move them into the branch)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) asm volatile("" : "+v"(E[u]));
+            asm volatile("" : "+v"(acc));
+            double zv, zl;
+            xw_wait_z(zpub + qn, wave, lane, status, zv, zl);
+            if (xw_bits(zl) != XW_BAD) {
+                double v1 = 0.0;
+                row_adds<0>(acc, v1, zv, E);
+                acc = (acc + v1) * rcp_newton(zl);
+                if (!__all(zl * XW_RANGE >= zv) && lane == 0) sh.flag[2] = 1;
+            } else if (lane == 0) {
+                sh.flag[1] = 1;
+            }
+            sh.psum[wave * REC_B + lane] = acc;
+        }
+        __syncthreads();
+        if (sh.flag[1]) {   // (uniform) the block before as a farther one
+            sigma = far(I - 1);
+            known = true;
+            sh.psum[wave * REC_B + lane] = s > 0.0 ? s * cn * exp_pair((sigma + g) - m) : 0.0;
+            __syncthreads();
+        }
+        const double* ps = sh.psum + lane;
+        z = (ps[0] + ps[REC_B]) + (ps[2 * REC_B] + ps[3 * REC_B]);
+        if (NW > ZW && sh.flag[1])
+            for (int w = ZW; w < NW; ++w) z += ps[w * REC_B];
+    }
     double u = 0.0;
     if (wave == 0) {
-        double z0 = 0.0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) z0 += sh.psum[w * REC_B + lane];
-        rec_inblock_seq<1>(sh.a, lane, z0, sh.z);
-        const double z = sh.z[lane];
-        u = (sigma + g) - log(z);
-        const bool ok = lane >= nb || (z >= 1e-290 && z <= 1e290);
-        const bool all = __all(ok);
-        if (all && !last) xw_publish(pub + n0 + lane, u + lgs);
-        if (lane == 0) *sh.flag = all ? 0 : 1;
+        z = xw_substitute(sh.a, lane, nb, lane < nb ? z : 0.0);
+        const bool all = __all(lane >= nb || (z >= 1.0 / XW_RANGE && z <= XW_RANGE)) && !sh.flag[2];
+        if (!last) {
+            const unsigned long long b = all ? xw_bits(z) : XW_BAD;
+            __hip_atomic_store(zpub + n0 + lane, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (!known) sigma = wave_bcast_uniform(xw_wait(upub + qn, lane, status), REC_B - 1);   // (all 64: see the reset below)
+        if (all) {
+            u = (sigma + g) - log(z);
+            if (!last) xw_publish(upub + n0 + lane, DIR == 0 ? u : u + sh.lq[lane]);
+        }
+        if (lane == 0) sh.flag[0] = all ? 0 : 1;
     }
     __syncthreads();
-    if (*sh.flag) {
-        u = xw_block_safe<DIR, D, NT>(I, N, nb, bk, u0, r, sh, pub);
+    if (sh.flag[0]) {
+        u = xw_block_safe<DIR, D, NT>(I, N, nb, bk, r, sh, upub, status);
         if (wave == 0) {
             if (lane < nb && !isfinite(u)) raise_status(status);
-            if (!last) xw_publish(pub + n0 + lane, u + lgs);
+            if (!last) xw_publish(upub + n0 + lane, DIR == 0 ? u : u + sh.lq[lane]);
         }
     }
     if (wave == 0 && lane < nb) {
@@ -417,8 +698,10 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         }
     }
     if (last) {   // every value has been read by every workgroup: empty for the next launch
-        for (int q = tid; q < n0; q += NT)
-            __hip_atomic_store(pub + q, XW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int q = tid; q < n0; q += NT) {
+            __hip_atomic_store(zpub + q, XW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(upub + q, XW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
@@ -433,11 +716,16 @@ __device__ __forceinline__ void xw_recursions(double* smem, int b, int N, double
                                               double* __restrict__ Shi, double* __restrict__ Slo, double* __restrict__ xc,
                                               unsigned long long* __restrict__ pub, int* __restrict__ status) {
     const XwShared sh = xw_carve<NT>(smem, N, D);
-    const bool first = b == 0;
-    const Ring r = xw_stage<D, NT>(sh, N, x1, xP, k, pbc != 0, L, first ? Shi : nullptr, first ? Slo : nullptr,
-                               first ? xc : nullptr);
-    if ((b & 1) == 0) xw_block<0, D, NT>(b >> 1, N, bt, r, sh, pub, V, Vb, VB, status);
-    else xw_block<1, D, NT>(b >> 1, N, bt, r, sh, pub + N + 1, V, Vb, nullptr, status);
+    const bool first = b == 0, fwd = (b & 1) == 0;
+    const int I = b >> 1;
+    double *sh_out = first ? Shi : nullptr, *sl_out = first ? Slo : nullptr, *x_out = first ? xc : nullptr;
+    if (fwd) {
+        const Ring r = xw_stage<0, D, NT>(sh, I, N, bt, x1, xP, k, pbc != 0, L, sh_out, sl_out, x_out);
+        xw_block<0, D, NT>(I, N, bt, r, sh, pub, pub + N + 1, V, Vb, VB, status);
+    } else {
+        const Ring r = xw_stage<1, D, NT>(sh, I, N, bt, x1, xP, k, pbc != 0, L, nullptr, nullptr, nullptr);
+        xw_block<1, D, NT>(I, N, bt, r, sh, pub + 2 * (N + 1), pub + 3 * (N + 1), V, Vb, nullptr, status);
+    }
 }
 
 template <int D>
@@ -445,7 +733,7 @@ static __global__ void __launch_bounds__(XW_THREADS)
 k_exchange_wide(int N, double bt, double k, int pbc, double L, BeadView x1, BeadView xP, double* __restrict__ V,
                 double* __restrict__ Vb, double* __restrict__ VB, double* __restrict__ Shi, double* __restrict__ Slo,
                 double* __restrict__ xc, unsigned long long* __restrict__ pub, int* __restrict__ status) {
-    extern __shared__ double smem[];
+    extern __shared__ __align__(16) double smem[];
     xw_recursions<D, XW_THREADS>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status);
 }
 

@@ -80,7 +80,7 @@ struct ObserveArgs {
 
 template <int D, int KIND>
 static __global__ void __launch_bounds__(XW_THREADS) k_observe(ObserveArgs o) {
-    extern __shared__ double smem[];
+    extern __shared__ __align__(16) double smem[];
     const int wg = blockIdx.x, N = o.fa.N, P = o.fa.P;
     if (wg < o.nx) {
         xw_recursions<D, XW_THREADS>(smem, wg, N, o.bt, o.fa.k_spring, o.fa.pbc, o.fa.L, BeadView{o.x, N, 1},

@@ -141,7 +141,7 @@ __device__ __noinline__ void split_slice(const RepDesc& r_, const BatchPtrs& bp,
 template <int D, int KIND>
 static __global__ void __launch_bounds__(SPLIT_THREADS, 4) k_split_forces(SplitPtrs sp, const int2* __restrict__ map,
                                                                         int only_noise, int mode) {
-    extern __shared__ double smem[];
+    extern __shared__ __align__(16) double smem[];
     const int2 m = map[blockIdx.x];
     const int ri = uni(m.x), id = uni(m.y);
     const StepArgs s = sp.steps[ri];   // (a copy: stores through it would make every use a load)

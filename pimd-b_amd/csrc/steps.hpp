@@ -320,7 +320,7 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
 // noise.  x, p, f: bead-major SoA [b][a][i].  Dynamic LDS: the largest part's.
 template <int D, int KIND>
 static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, int nx, int nf, int mode) {
-    extern __shared__ double smem[];
+    extern __shared__ __align__(16) double smem[];
     const int wg = blockIdx.x;
     if (wg < nx) {
         step_recursions<D, XW_THREADS>(s, wg, smem);
