@@ -123,6 +123,7 @@ static __global__ void __launch_bounds__(256) k_momenta(MomentaArgs m, double* _
         }
     } else if (m.thermostat == 1) {
         const int half = (P + 1) / 2;
+        __syncthreads();   // beads 2mp and 2mp + 1 were staged by other threads
         if (!m.nm) {
             for (int e = tid; e < half * TC; e += blockDim.x) {
                 const int mp = e / TC, c = e % TC;
@@ -136,7 +137,6 @@ static __global__ void __launch_bounds__(256) k_momenta(MomentaArgs m, double* _
                 }
             }
         } else {
-            __syncthreads();
             // noise of modes 2mp, 2mp+1 (one Box-Muller pair) into pn
             for (int e = tid; e < half * TC; e += blockDim.x) {
                 const int mp = e / TC, c = e % TC;
