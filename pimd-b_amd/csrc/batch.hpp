@@ -80,22 +80,6 @@ __device__ __forceinline__ double wg_sum(double v, double* red) {
     return s;
 }
 
-// Wave-uniform copies (v_readfirstlane) of values that reach a non-inlined
-// function in vector registers.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ double uni(double v) {
-    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
-    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
-    return __hiloint2double(hi, lo);
-}
-template <typename T>
-__device__ __forceinline__ T* uni(T* p) {
-    const unsigned long long u = (unsigned long long)p;
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32));
-    return (T*)(((unsigned long long)hi << 32) | lo);
-}
-
 // Wave-uniform copy of a replica descriptor.  The phases below are kept out
 // of line (each one's registers would otherwise add to the others'); their
 // arguments arrive in vector registers, and these copies put the replica's

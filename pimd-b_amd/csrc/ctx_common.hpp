@@ -326,6 +326,15 @@ inline size_t device_lds_limit() {
     return lim;
 }
 
+inline int device_cus() {
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) v = 256;
+        return v;
+    }();
+    return n;
+}
+
 // Whether a ring's recursions run with one workgroup per block of targets
 // (k_exchange_wide: the ring staged in every workgroup's LDS); larger rings
 // take k_exchange_recursions_gws.

@@ -73,6 +73,22 @@ __device__ __forceinline__ double norm2(const double (&d)[D]) {
     return s;
 }
 
+// Wave-uniform copies (v_readfirstlane) of values that reach a non-inlined
+// function in vector registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uni(double v) {
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+template <typename T>
+__device__ __forceinline__ T* uni(T* p) {
+    const unsigned long long u = (unsigned long long)p;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32));
+    return (T*)(((unsigned long long)hi << 32) | lo);
+}
+
 // Lane l receives what lane (l+1) mod 64 held (DPP wave_rol:1).  Call with
 // the whole wave active.
 __device__ __forceinline__ int lane_rotate(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x134, 0xF, 0xF, false); }

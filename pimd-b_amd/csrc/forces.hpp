@@ -11,7 +11,8 @@
 // partial forces are reduced in LDS.  Every ordered pair
 // (i,j) evaluates gradV(r_i - r_j); for central potentials this is bitwise
 // the negation of gradV(r_j - r_i), so the result equals the reference's
-// Newton's-third-law loop up to summation order.
+// Newton's-third-law loop up to summation order.  Up to 128 particles; larger
+// single systems take slice_groups.hpp.
 #pragma once
 
 #include "device_common.hpp"
@@ -30,6 +31,38 @@ struct ForceArgs {
 
 constexpr int FORCE_TILE = 64;
 constexpr int FORCE_WAVES = 16;
+
+// The external and spring forces of particle i of bead b and its pair forces
+// `pair` into f (and fext: external and pair alone); fe receives the external
+// force.  Exchange beads get no spring part (added later).
+template <int D>
+__device__ __forceinline__ void row_forces(const ForceArgs& fa, int b, int i, const double* __restrict__ x,
+                                           const double (&pair)[D], double* __restrict__ f, double* __restrict__ fext,
+                                           double (&fe)[D]) {
+    const int N = fa.N, P = fa.P;
+    const size_t bs = (size_t)D * N;
+    const bool exchange_bead = fa.bosonic && (b == 0 || b == P - 1), pbc = fa.pbc != 0;
+    const double* xprev = x + bs * ((b - 1 + P) % P);
+    const double* xnext = x + bs * ((b + 1) % P);
+    double xv[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) xv[a] = x[bs * b + (size_t)a * N + i];
+    ext_force<D>(fa.ext, xv, fe);
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const size_t idx = bs * b + (size_t)a * N + i;
+        const double xi = xv[a];
+        const double phys = fe[a] + pair[a];
+        if (fext) fext[idx] = phys;
+        double spring = 0.0;
+        if (!exchange_bead) {
+            const double dp = disp(xi, xprev[(size_t)a * N + i], pbc, fa.L);
+            const double dn = disp(xi, xnext[(size_t)a * N + i], pbc, fa.L);
+            spring = fa.k_spring * (dp + dn);
+        }
+        f[idx] = exchange_bead ? phys : spring + phys;
+    }
+}
 
 // The forces of particles tile*64 .. +63 of bead b by a workgroup of 1024
 // threads.  smem: the staged slice (GX: none) and the reduction.  Exchange
@@ -71,12 +104,13 @@ __device__ __forceinline__ void bead_forces_tile(const ForceArgs& fa, int b, int
             const PairParams pp = make_pair_params(fa.L, fa.pbc, fa.cutoff, fa.cut2, fa.int_k, fa.strength);
             auto run = [&](auto img) {
                 constexpr int IMG = decltype(img)::value;
+                const ImageGrad<D, KIND, IMG> grad{pp, image_params<KIND, IMG>(pp)};
                 for (int j = jlo; j < jhi; ++j) {
                     if (j == i) continue;
                     double xj[D], d[D], g;
 #pragma unroll
                     for (int a = 0; a < D; ++a) xj[a] = sx[a * N + j];
-                    if (pair_grad<D, KIND, IMG>(xi, xj, pp, d, g)) {
+                    if (grad(xi, xj, d, g)) {
 #pragma unroll
                         for (int a = 0; a < D; ++a) acc[a] = fma(-g, d[a], acc[a]);
                     }
@@ -105,28 +139,7 @@ __device__ __forceinline__ void bead_forces_tile(const ForceArgs& fa, int b, int
                 for (int a = 0; a < D; ++a) acc[a] += red[((w - 1) * D + a) * FORCE_TILE + lane];
             }
         }
-        const bool exchange_bead = fa.bosonic && (b == 0 || b == P - 1);
-        const double* xprev = x + bs * ((b - 1 + P) % P);
-        const double* xnext = x + bs * ((b + 1) % P);
-        double xv[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) xv[a] = sx[a * N + i];
-        ext_force<D>(fa.ext, xv, fe);
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const size_t idx = bs * b + (size_t)a * N + i;
-            const double xi = xv[a];
-            const double phys = fe[a] + acc[a];
-            if (fext) fext[idx] = phys;
-            double spring = 0.0;
-            if (!exchange_bead) {
-                const double dp = disp(xi, xprev[(size_t)a * N + i], pbc, fa.L);
-                const double dn = disp(xi, xnext[(size_t)a * N + i], pbc, fa.L);
-                spring = fa.k_spring * (dp + dn);
-            }
-            // exchange beads get their spring part added later
-            f[idx] = exchange_bead ? phys : spring + phys;
-        }
+        row_forces<D>(fa, b, i, x, acc, f, fext, fe);
     }
     if (fpart) {
         const int nt = (N + FORCE_TILE - 1) / FORCE_TILE;

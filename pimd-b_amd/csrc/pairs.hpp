@@ -175,21 +175,10 @@ __device__ __forceinline__ double frac_exp2(double f) {
     return p;
 }
 
-// gradV = g d for the pair (i, j) in fractional coordinates (xi, xj = x / L):
-// d = min-imaged s_i - s_j and g = g_s as above when the pair is inside the
-// cutoff (the return value), g = 0 otherwise.  Branch-free but for the
-// damping range: outside the cutoff r > L/2 and every term is finite, and in
-// the hard-core range the damped terms are finite with F = 0.
-template <int D, int KIND>
-__device__ __forceinline__ bool pair_grad_frac(const double (&xi)[D], const double (&xj)[D], const FracParams& fp,
-                                               double (&d)[D], double& g) {
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        const double t = xi[a] - xj[a];
-        d[a] = t - rint(t);
-    }
-    const double s = norm2_fma<D>(d);
-    const bool in = s < fp.cut2;
+// g_s from |d_s|^2 (above), for a pair inside the cutoff; finite outside it.
+template <int KIND>
+__device__ __forceinline__ double frac_factor(double s, const FracParams& fp) {
+    double g;
     if constexpr (KIND == POT_HARMONIC) {
         g = fp.kh;
     } else if constexpr (KIND == POT_DIPOLE) {
@@ -220,6 +209,40 @@ __device__ __forceinline__ bool pair_grad_frac(const double (&xi)[D], const doub
     } else {
         g = 0.0;
     }
+    return g;
+}
+
+// gradV = g d for the pair (i, j) in fractional coordinates (xi, xj = x / L):
+// d = min-imaged s_i - s_j and g = g_s as above when the pair is inside the
+// cutoff (the return value), g = 0 otherwise.  Branch-free but for the
+// damping range: outside the cutoff r > L/2 and every term is finite, and in
+// the hard-core range the damped terms are finite with F = 0.
+template <int D, int KIND>
+__device__ __forceinline__ bool pair_grad_frac(const double (&xi)[D], const double (&xj)[D], const FracParams& fp,
+                                               double (&d)[D], double& g) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const double t = xi[a] - xj[a];
+        d[a] = t - rint(t);
+    }
+    const double s = norm2_fma<D>(d);
+    const bool in = s < fp.cut2;
+    g = frac_factor<KIND>(s, fp);
+    g = in ? g : 0.0;
+    return in;
+}
+
+// The same from positions in length units (fp for a box of 1: y = 1 / r), the
+// image taken on their difference: three operations more, without the rounding
+// of x / L, which a close pair's steep repulsion would amplify.
+template <int D, int KIND>
+__device__ __forceinline__ bool pair_grad_image(const double (&xi)[D], const double (&xj)[D], const PairParams& pp,
+                                                const FracParams& fp, double (&d)[D], double& g) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) d[a] = min_image_pair<1>(xi[a] - xj[a], pp);
+    const double s = norm2_fma<D>(d);
+    const bool in = s < fp.cut2;
+    g = frac_factor<KIND>(s, fp);
     g = in ? g : 0.0;
     return in;
 }
@@ -311,6 +334,32 @@ struct WalkGrad {
         else return pair_grad<D, KIND, IMG>(xi, xj, pp, d, g);
     }
 };
+
+// The same on positions in length units (pair_grad_image), for single systems.
+template <int D, int KIND, int IMG>
+struct ImageGrad {
+    PairParams pp;
+    FracParams fp;   // of a box of 1
+    __device__ __forceinline__ bool operator()(const double (&xi)[D], const double (&xj)[D], double (&d)[D],
+                                               double& g) const {
+        if constexpr (IMG == 1) return pair_grad_image<D, KIND>(xi, xj, pp, fp, d, g);
+        else return pair_grad<D, KIND, IMG>(xi, xj, pp, d, g);
+    }
+};
+// Its parameters, uniform in the wave (IMG 1; the others use none).
+template <int KIND, int IMG>
+__device__ __forceinline__ FracParams image_params(PairParams pp) {
+    FracParams fp{};
+    if constexpr (IMG != 1) return fp;
+    pp.L = pp.invL = 1.0;
+    fp = make_frac_params(pp);
+    if constexpr (KIND != POT_AZIZ) return fp;
+    fp.cut2 = uni(fp.cut2); fp.kh = uni(fp.kh); fp.kd = uni(fp.kd); fp.ex = uni(fp.ex);
+    fp.b0 = uni(fp.b0); fp.b1 = uni(fp.b1); fp.b2 = uni(fp.b2); fp.dl = uni(fp.dl);
+    fp.b1v = vgpr_copy(fp.b1);
+    fp.b2v = vgpr_copy(fp.b2);
+    return fp;
+}
 
 // Doubles per tile position in the LDS force arrays of the slice walk: D
 // rounded up to odd, so that 32 consecutive positions (64-bit LDS accesses

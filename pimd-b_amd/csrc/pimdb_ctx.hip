@@ -51,6 +51,7 @@ struct pimdb_ctx {
     int* status = nullptr;
     unsigned long long* ctr = nullptr;
     bool merged = false;           // recursions and bead forces in one k_step_forces
+    PairGroups pg{};               // pair forces by groups of 128 (slice_groups.hpp)
     bool split = false;            // consecutive steps by k_step_forces and k_step_integrate
     double *xc = nullptr, *H = nullptr, *fpart = nullptr, *hpart = nullptr;   // their workspace (StepArgs)
     int tc = 1, ntiles = 1;
@@ -172,6 +173,40 @@ static void launch_factorial(pimdb_ctx* ctx, hipStream_t s, double* f, double* f
     }
 }
 
+// How the pair forces of a merged step are cut (PairGroups; G = 0 for one tile
+// of 64 rows per workgroup).
+static PairGroups plan_pair_groups(const pimdb_params& p, const Derived& d, int nx) {
+    PairGroups pg{};
+    const int N = p.natoms;
+    if (p.int_kind == PIMDB_POT_FREE || d.cutoff == 0.0 || N <= GROUP_MIN) return pg;
+    const int G = (N + GROUP - 1) / GROUP;
+    // A workgroup takes about 4 us and 1 us per 16 steps (Aziz), and each of the
+    // recursions' holds a compute unit for as long as they take (8 us and 4.6 us
+    // per 100 particles).  More parts, which the integration reads, only for a
+    // tenth less: N=1000, P=4 without exchange 44.0, 28.6, 25.0, 21.3 us a step
+    // with 1 .. 4 parts (64 us at P=8 with exchange whatever the parts), N=256,
+    // P=64 25.5, 31.7, 30.7, 42.9.
+    const int steps = GROUP_OWN + group_seg_start(G, group_segments(G)), cus = std::max(1, device_cus() - nx);
+    double best = 0.0;
+    int parts = 0;
+    for (int q = 1; q <= GROUP_PARTS; ++q) {
+        if (sizeof(double) * group_lds_doubles(p.ndim, group_kslots(G, q)) > device_lds_limit()) continue;
+        const int rounds = (p.nbeads * G * q + cus - 1) / cus;
+        const double t = std::max(rounds * (4.0 + steps / (16.0 * q)), nx ? 8.0 + 0.046 * N : 0.0);
+        if (!parts || t < 0.9 * best) {
+            best = t;
+            parts = q;
+        }
+    }
+    if (!parts) return pg;
+    const int k = group_kslots(G, parts);
+    pg.G = G;
+    pg.parts = parts;
+    pg.kslots = k;
+    pg.nslots = G / 2 + parts - 1;
+    return pg;
+}
+
 static StepArgs step_args(pimdb_ctx* ctx) {
     StepArgs a{};
     a.fa = make_force_args(ctx->prm, ctx->dv);
@@ -191,6 +226,7 @@ static StepArgs step_args(pimdb_ctx* ctx) {
     a.H = ctx->H; a.hpart = ctx->hpart;
     a.frows = ctx->P * ((ctx->N + FORCE_TILE - 1) / FORCE_TILE);
     a.fpart = ctx->prm.ext_kind != PIMDB_POT_FREE && a.fixcom ? ctx->fpart : nullptr;
+    a.pg = ctx->pg;
     a.ctr = ctx->ctr;
     a.seed = ctx->prm.seed;
     return a;
@@ -203,20 +239,20 @@ static size_t tile_lds_bytes(int N, int D) {
 template <int D>
 static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
     const StepArgs a = step_args(ctx);
-    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = forces ? a.frows : 0;
+    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = !forces ? 0 : a.pg.G ? ctx->P * a.pg.G * a.pg.parts : a.frows;
     const int nn = noise ? step_noise_groups(a, D) : 0;
     if (nx + nf + nn == 0) return;
     size_t lds = 0;
-    if (nf) lds = tile_lds_bytes(ctx->N, D);
+    if (nf) lds = a.pg.G ? sizeof(double) * group_lds_doubles(D, a.pg.kslots) : tile_lds_bytes(ctx->N, D);
     if (nx) lds = std::max(lds, xw_lds_bytes(ctx->N, D));
     if (nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(ctx->P, a.thermostat && a.nm));
     const dim3 grid(nx + nf + nn), blk(XW_THREADS);
     const hipStream_t s = ctx->s0;
     switch (ctx->prm.int_kind) {
-    case POT_HARMONIC: hipLaunchKernelGGL((k_step_forces<D, POT_HARMONIC>), grid, blk, lds, s, a, nx, nf, mode); break;
-    case POT_DIPOLE: hipLaunchKernelGGL((k_step_forces<D, POT_DIPOLE>), grid, blk, lds, s, a, nx, nf, mode); break;
-    case POT_AZIZ: hipLaunchKernelGGL((k_step_forces<D, POT_AZIZ>), grid, blk, lds, s, a, nx, nf, mode); break;
-    default: hipLaunchKernelGGL((k_step_forces<D, POT_FREE>), grid, blk, lds, s, a, nx, nf, mode); break;
+    case POT_HARMONIC: hipLaunchKernelGGL((k_step_forces<D, POT_HARMONIC>), grid, blk, lds, s, a, nx, nn, mode); break;
+    case POT_DIPOLE: hipLaunchKernelGGL((k_step_forces<D, POT_DIPOLE>), grid, blk, lds, s, a, nx, nn, mode); break;
+    case POT_AZIZ: hipLaunchKernelGGL((k_step_forces<D, POT_AZIZ>), grid, blk, lds, s, a, nx, nn, mode); break;
+    default: hipLaunchKernelGGL((k_step_forces<D, POT_FREE>), grid, blk, lds, s, a, nx, nn, mode); break;
     }
 }
 
@@ -244,6 +280,9 @@ static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
 static int enqueue_forces(pimdb_ctx* ctx) {
     if (ctx->merged) {
         launch_step_forces(ctx, true, false, STEP_CLOSE);
+        if (ctx->pg.nslots)
+            hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->nbd,
+                               ctx->pg, ctx->f, ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr);
         if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
     } else if (factorial(ctx)) {
         launch_bead_forces(ctx, ctx->s0);
@@ -552,6 +591,10 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     ctx->merged = slice_fits && (!ctx->dv.bosonic || wide);
     ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN && prm->propagator == PIMDB_PROP_CARTESIAN &&
                  (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat || P <= STEP_NM_MAXP);
+    if (ctx->merged) {
+        ctx->pg = plan_pair_groups(*prm, ctx->dv, wide ? xw_grid(N) : 0);
+        if (ctx->pg.nslots) alloc(&ctx->pg.cpart, sizeof(double) * ctx->nbd * ctx->pg.nslots);
+    }
     if (ctx->merged && ctx->dv.bosonic) alloc(&ctx->xc, sizeof(double) * 4 * (size_t)D * N);
     if (ctx->split) {
         alloc(&ctx->H, sizeof(double) * ctx->nbd);

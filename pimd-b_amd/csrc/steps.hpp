@@ -37,6 +37,7 @@
 #include "device_common.hpp"
 #include "exchange_wide.hpp"
 #include "forces.hpp"
+#include "slice_groups.hpp"
 
 namespace pimdb {
 
@@ -68,6 +69,7 @@ struct StepArgs {
     double* fpart;                    // [frows][D] partial sums of the external forces (null: none)
     double* hpart;                    // [noise tiles][D] sums of alpha p + H
     int frows;
+    PairGroups pg;                    // G > 0: the pair forces by groups, f to be completed from pg.cpart
     unsigned long long* ctr;          // steps done
     uint32_t seed;
 };
@@ -276,6 +278,12 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
             if (mode != STEP_CLOSE) xv = s.x[e];
             if (s.thermostat) hv = s.H[e];
         }
+        if (mode != STEP_OPEN) {
+            const size_t n = (size_t)P * bs;
+            double c = 0.0;
+            for (int k = 0; k < s.pg.nslots; ++k) c += s.pg.cpart[k * n + e];
+            fv += c;
+        }
     }
     if (s.fixcom && mode != STEP_FORCES) {
         if (wave < D) {
@@ -302,6 +310,8 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
         for (int q = 0; q < M * D; ++q)
             if (lane == q) fv = F[q / D][q % D] + fv;
         if (mine) s.f[e] = fv;
+    } else if (mine && s.pg.nslots && mode != STEP_OPEN) {
+        s.f[e] = fv;
     }
     if (!mine || mode == STEP_FORCES) return;
     double v = fma(co.alpha, fma(co.beta, fv, pv), hv);
@@ -316,19 +326,25 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
 }
 
 // ---- one system ----
-// nx, nf: workgroups of the recursions and of the force tiles; the rest make
-// noise.  x, p, f: bead-major SoA [b][a][i].  Dynamic LDS: the largest part's.
+// nx, nn: workgroups of the recursions and of the noise; the rest are the pair
+// groups or force tiles.  x, p, f: bead-major SoA [b][a][i].  Dynamic LDS: the largest part's.
 template <int D, int KIND>
-static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, int nx, int nf, int mode) {
+static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, int nx, int nn, int mode) {
     extern __shared__ __align__(16) double smem[];
     const int wg = blockIdx.x;
     if (wg < nx) {
         step_recursions<D, XW_THREADS>(s, wg, smem);
-    } else if (wg < nx + nf) {
-        const int nt = (s.fa.N + FORCE_TILE - 1) / FORCE_TILE, id = wg - nx;
-        bead_forces_tile<D, KIND>(s.fa, id / nt, id % nt, s.x, s.f, s.fext, s.fpart, smem);
+    } else if (wg < nx + nn) {
+        step_noise<D, XW_THREADS>(s, mode, wg - nx, smem);
     } else {
-        step_noise<D, XW_THREADS>(s, mode, wg - nx - nf, smem);
+        const int nt = (s.fa.N + FORCE_TILE - 1) / FORCE_TILE, id = wg - nx - nn;
+        if constexpr (KIND != POT_FREE) {
+            if (s.pg.G) {
+                group_forces<D, KIND>(s.fa, s.pg, id, s.x, s.f, s.fext, s.fpart, smem);
+                return;
+            }
+        }
+        bead_forces_tile<D, KIND>(s.fa, id / nt, id % nt, s.x, s.f, s.fext, s.fpart, smem);
     }
 }
 
