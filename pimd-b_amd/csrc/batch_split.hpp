@@ -10,11 +10,9 @@
 
 namespace pimdb {
 
-// Threads of a workgroup of either kernel, and particles per wave of the
-// exterior forces.
+// Threads of a workgroup of either kernel.
 constexpr int SPLIT_THREADS = 256;
 constexpr int SPLIT_WAVES = SPLIT_THREADS / WAVE;
-constexpr int SPLIT_EXT = 4;
 
 // A workgroup's part of a forces launch: its replica and its index among the
 // replica's workgroups (recursions first, then slices, then noise).

@@ -585,77 +585,58 @@ static __global__ void __launch_bounds__(256) k_exchange_probabilities(int N, do
 // energy (ecyc(l,j) for bead 1, ecyc(j,l) for bead P).  x2 / xPm1 hold the
 // interior neighbours; with grad_only the interior link is left out and the
 // result is -dV_B/dx (the adjoint of V_B alone, used by the autograd harness).
-// A wave takes particles l .. l + M-1 (those below N), whose terms share the
-// partners' data: with many rings the passes over it are what bounds this (256
-// rings of N=256: one particle a wave moves 1.8 GB through L2).
-template <int D, int M = 1>
+// Four terms a lane are in flight, which hides more than sharing the partners'
+// data between the particles of a wave did (128 rings of N=256, four particles
+// a wave: 802 us a step, one: 748).
+template <int D>
 __device__ __forceinline__ void exterior_force(int which, int l, int N, int lane, double bt, double k, const Ring& r,
                                                const double* __restrict__ V, const double* __restrict__ Vb,
                                                const double* __restrict__ x2, const double* __restrict__ xPm1,
-                                               bool grad_only, double (&F)[M][D]) {
+                                               bool grad_only, double (&F)[D]) {
     const double* self = which == 0 ? r.x1 : r.xP;
     const double* other = which == 0 ? r.xP : r.x1;
     // U terms: bead 1, exp(-bt (V[l] + e + Vb[j+1] - V[N])) / (j+1); bead P, exp(-bt (V[j] + e + Vb[l+1] - V[N])) / (l+1)
-    double xs[M][D], shl[M], sll[M], ul[M], inv[M], S[M][D];
+    double xs[D], S[D];
     const double VN = V[N];
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        const int lm = min(l + m, N - 1);
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            xs[m][a] = self[a * N + lm];
-            S[m][a] = 0.0;
-        }
-        shl[m] = r.Shi[lm];
-        sll[m] = r.Slo[lm];
-        ul[m] = which == 0 ? V[lm] : Vb[lm + 1];
-        inv[m] = 1.0 / (lm + 1);
+    for (int a = 0; a < D; ++a) {
+        xs[a] = self[a * N + l];
+        S[a] = 0.0;
     }
+    const double shl = r.Shi[l], sll = r.Slo[l], ul = which == 0 ? V[l] : Vb[l + 1], inv = 1.0 / (l + 1);
     const int jlo = which == 0 ? max(0, l - 1) : 0;
-    const int jhi = which == 0 ? N - 1 : min(l + M, N - 1);
+    const int jhi = which == 0 ? N - 1 : min(l + 1, N - 1);
     const double* uo = which == 0 ? Vb + 1 : V;
-#pragma unroll(M == 1 ? 4 : 1)
+#pragma unroll 4
     for (int j = jlo + lane; j <= jhi; j += WAVE) {
-        double xo[D];
+        double d[D];
 #pragma unroll
-        for (int a = 0; a < D; ++a) xo[a] = other[a * N + j];
+        for (int a = 0; a < D; ++a) d[a] = ring_image(other[a * N + j] - xs[a], r);
         const double shj = r.Shi[j], slj = r.Slo[j], uj = uo[j];
         const double linkarg = which == 0 ? (V[j + 1] + uj) - VN : 0.0;   // bead 1's link: row j
         // 1/(j+1): the reciprocal estimate and two Newton steps (within an ulp)
         double rc = __builtin_amdgcn_rcp((double)(j + 1));
         rc = fma(rc, fma(-(double)(j + 1), rc, 1.0), rc);
         rc = fma(rc, fma(-(double)(j + 1), rc, 1.0), rc);
+        const int row = which == 0 ? j : l, col = which == 0 ? l : j;
+        const bool link = col == row + 1 && row < N - 1;
+        // ecyc(col, row): u = col, v = row
+        const double e = which == 0 ? ring_ecyc<D>(r, d, shl, sll, shj, slj) : ring_ecyc<D>(r, d, shj, slj, shl, sll);
+        double arg = (ul + e + uj) - VN;
+        if (link) arg = which == 0 ? linkarg : (V[l + 1] + ul) - VN;
+        const double ex = exp_minimax(-bt * arg);
+        double pr = (which == 0 ? rc : inv) * ex;
+        if (link) pr = 1.0 - ex;
+        else if (col > row) pr = 0.0;
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const int lm = l + m;
-            double d[D];
-#pragma unroll
-            for (int a = 0; a < D; ++a) d[a] = ring_image(xo[a] - xs[m][a], r);
-            const int row = which == 0 ? j : lm, col = which == 0 ? lm : j;
-            const bool link = col == row + 1 && row < N - 1;
-            // ecyc(col, row): u = col, v = row
-            const double e = which == 0 ? ring_ecyc<D>(r, d, shl[m], sll[m], shj, slj)
-                                        : ring_ecyc<D>(r, d, shj, slj, shl[m], sll[m]);
-            double arg = (ul[m] + e + uj) - VN;
-            if (link) arg = which == 0 ? linkarg : (V[lm + 1] + ul[m]) - VN;
-            const double ex = exp_minimax(-bt * arg);
-            double pr = (which == 0 ? rc : inv[m]) * ex;
-            if (link) pr = 1.0 - ex;
-            else if (col > row) pr = 0.0;
-#pragma unroll
-            for (int a = 0; a < D; ++a) S[m][a] = fma(pr, d[a], S[m][a]);
-        }
+        for (int a = 0; a < D; ++a) S[a] = fma(pr, d[a], S[a]);
     }
     const double* link = which == 0 ? x2 : xPm1;
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        const int lm = min(l + m, N - 1);
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            double s = wave_total(S[m][a]);
-            if (!grad_only) s += ring_image(link[a * N + lm] - xs[m][a], r);
-            F[m][a] = s * k;
-        }
+    for (int a = 0; a < D; ++a) {
+        double s = wave_total(S[a]);
+        if (!grad_only) s += ring_image(link[a * N + l] - xs[a], r);
+        F[a] = s * k;
     }
 }
 
@@ -677,15 +658,15 @@ static __global__ void __launch_bounds__(256) k_exchange_forces(int N, int P, do
     const double* x2 = x + bs * (1 % P);
     const double* xPm1 = x + bs * ((P - 2 + P) % P);
     const Ring r = make_ring(x, x + bs * (P - 1), Shi, Slo, k, pbc != 0, L);
-    double F[1][D];
+    double F[D];
     exterior_force<D>(which, l, N, lane, bt, k, r, V, Vb, x2, xPm1, false, F);
     if (lane == 0) {
         const size_t b = which == 0 ? 0 : (size_t)(P - 1);
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             const size_t idx = (b * D + a) * N + l;
-            if (fex) fex[((size_t)which * D + a) * N + l] = F[0][a];
-            if (f) f[idx] = F[0][a] + f[idx];
+            if (fex) fex[((size_t)which * D + a) * N + l] = F[a];
+            if (f) f[idx] = F[a] + f[idx];
         }
     }
 }
@@ -704,11 +685,11 @@ static __global__ void __launch_bounds__(256) k_exchange_vb_grad(int N, double b
     const int which = task / N, l = task % N;
     const int lane = threadIdx.x % WAVE;
     const Ring r = make_ring(x1, xP, Shi, Slo, k, pbc != 0, L);
-    double F[1][D];
+    double F[D];
     exterior_force<D>(which, l, N, lane, bt, k, r, V, Vb, x1, xP, true, F);
     if (lane == 0) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) out[((size_t)which * D + a) * N + l] = F[0][a];
+        for (int a = 0; a < D; ++a) out[((size_t)which * D + a) * N + l] = F[a];
     }
 }
 
@@ -730,12 +711,12 @@ static __global__ void __launch_bounds__(256) k_exchange_backward(int N, double 
     const double* xP = xc + (size_t)D * N;
     const Ring r = make_ring(xc, xP, Shi, Slo, k, pbc != 0, L);
     const double g = scale ? *scale : 1.0;
-    double F[1][D];
+    double F[D];
     exterior_force<D>(which, l, N, lane, bt, k, r, V, Vb, xc, xP, true, F);
     if (lane == 0) {
         double* out = (which == 0 ? d1 : dP) + (size_t)l * D;
 #pragma unroll
-        for (int a = 0; a < D; ++a) out[a] = -F[0][a] * g;   // (F is -dV_B/dx)
+        for (int a = 0; a < D; ++a) out[a] = -F[a] * g;   // (F is -dV_B/dx)
     }
 }
 

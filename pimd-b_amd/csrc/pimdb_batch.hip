@@ -71,10 +71,10 @@ struct pimdb_batch {
 
 // Microseconds of one compute unit that a replica's step takes, fitted to both
 // forms at N = 8 .. 256, P = 8 .. 64, free, dipole and helium pairs, with and
-// without normal-mode coupling (within about 15%).  Pairs: 64-particle tiles,
-// ns per pair; persistent: a fixed 55 us of barriers and phase starts; split:
-// the recursions' blocks and the noise tiles, each a workgroup with waits of
-// its own, instead.
+// without normal-mode coupling (split within about 15%, persistent 25%).
+// Pairs: 64-particle tiles, ns per pair; persistent: a fixed 55 us of barriers
+// and phase starts; split: the recursions' blocks, each a workgroup with waits
+// of its own, instead.
 static double pair_us(const pimdb_params& p) {
     static const double ns[4] = {0.0, 0.2, 0.3, 0.55};   // free, harmonic, dipole, Aziz
     const double T = (p.natoms + PTILE - 1) / PTILE;
@@ -84,10 +84,19 @@ static double rep_cost(const pimdb_params& p) {
     const double N = p.natoms, nd = N * p.nbeads * p.ndim;
     return 55.0 + 0.004 * nd + (p.bosonic && p.nbeads > 1 ? 10.0 + 9e-4 * N * N : 0.0) + pair_us(p);
 }
+// Steps of the pair walk (two rows per lane) over one slice, and the
+// microseconds that a step costs one compute unit when the card is full.
+static double walk_steps(const pimdb_params& p) {
+    const int T = (p.natoms + PTILE - 1) / PTILE;
+    return 17.0 * T + PTILE / 4 * T * (T - 1);
+}
+static double walk_step_us(const pimdb_params& p) {
+    return p.int_kind == PIMDB_POT_FREE ? 0.0 : p.int_kind == PIMDB_POT_AZIZ ? 0.06 : 0.018;
+}
 static double rep_cost_split(const pimdb_params& p) {
     const double T = (p.natoms + PTILE - 1) / PTILE, nd = (double)p.natoms * p.nbeads * p.ndim;
-    return 0.0064 * nd + (p.nmthermostat ? 0.005 * p.nbeads * p.ndim * PTILE * T : 0.0) +
-           (p.bosonic && p.nbeads > 1 ? 45.0 * T : 0.0) + 1.2 * pair_us(p);
+    return 0.0079 * nd + (p.nmthermostat ? 0.0013 * p.nbeads * p.ndim * PTILE * T : 0.0) +
+           (p.bosonic && p.nbeads > 1 ? 14.0 * T : 0.0) + p.nbeads * walk_steps(p) * walk_step_us(p);
 }
 
 // Longest-processing-time-first assignment of replicas to `grid` workgroups.
@@ -293,7 +302,7 @@ static bool split_able(const pimdb_batch* b) {
         if (p.thermostat > PIMDB_THERMO_LANGEVIN || p.propagator != PIMDB_PROP_CARTESIAN) return false;
         if (nm && p.nbeads > STEP_NM_MAXP) return false;
         if (b->desc[r].bosonic && xw_lds_bytes(p.natoms, p.ndim, SPLIT_THREADS) > lim) return false;
-        if (sizeof(double) * step_noise_lds_doubles(p.nbeads, nm) > lim) return false;
+        if (sizeof(double) * step_noise_lds_doubles<SPLIT_THREADS>(p.nbeads, nm) > lim) return false;
     }
     return true;
 }
@@ -308,6 +317,13 @@ static void free_split(pimdb_batch* b) {
     b->d_steps = nullptr;
     b->d_maps = nullptr;
 }
+
+// About how long a slice and a noise workgroup of the two-kernel form take (a
+// walk step of one of twelve waves on a compute unit, two draws per four beads).
+static double slice_wg_us(const pimdb_params& p, int share) {
+    return 3.0 + 12.0 * walk_step_us(p) * walk_steps(p) / share;
+}
+static double noise_wg_us(const pimdb_params& p) { return 2.0 + 0.2 * p.nbeads; }
 
 static int build_split_buffers(pimdb_batch* b) {
     const int D = b->D;
@@ -335,7 +351,8 @@ static int build_split_buffers(pimdb_batch* b) {
     }
     int share = 1;
     while (fit && share < SPLIT_WAVES && beads * share < 8 * (size_t)b->cus) share *= 2;
-    std::vector<int2> slices;    // the long workgroups last
+    using Work = std::pair<double, int2>;
+    std::vector<Work> rest;      // slices and noise, the longest first
     std::vector<int2> maps[4];   // forces, noise, full, open
     size_t lds = 0, w = 0;
     b->hsteps.clear();
@@ -371,17 +388,19 @@ static int build_split_buffers(pimdb_batch* b) {
         a.seed = p.seed;
         b->hsteps.push_back(a);
         const int nx = d.bosonic ? xw_grid(p.natoms) : 0, ns = split_slices(p.nbeads, share), nn = step_noise_groups(a, D);
-        for (int i = 0; i < nx + nn; ++i) maps[0].push_back(int2{r, i});
-        for (int i = 0; i < ns; ++i) slices.push_back(int2{r, nx + nn + i});
+        for (int i = 0; i < nx; ++i) maps[0].push_back(int2{r, i});
+        for (int i = nx; i < nx + nn; ++i) rest.push_back({noise_wg_us(p), int2{r, i}});
+        for (int i = 0; i < ns; ++i) rest.push_back({slice_wg_us(p, share), int2{r, nx + nn + i}});
         for (int i = 0; i < nn; ++i) maps[1].push_back(int2{r, i});
-        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_FULL, SPLIT_EXT); ++i) maps[2].push_back(int2{r, i});
-        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_OPEN, SPLIT_EXT); ++i) maps[3].push_back(int2{r, i});
+        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_FULL); ++i) maps[2].push_back(int2{r, i});
+        for (int i = 0; i < step_integrate_groups(a.fa, D, STEP_OPEN); ++i) maps[3].push_back(int2{r, i});
         if (d.bosonic) lds = std::max(lds, xw_lds_bytes(p.natoms, D, SPLIT_THREADS));
         const size_t sl = split_slice_lds(p.natoms, D);
         if (sl <= device_lds_limit()) lds = std::max(lds, sl);
-        lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(p.nbeads, a.thermostat && a.nm));
+        lds = std::max(lds, sizeof(double) * step_noise_lds_doubles<SPLIT_THREADS>(p.nbeads, a.thermostat && a.nm));
     }
-    maps[0].insert(maps[0].end(), slices.begin(), slices.end());
+    std::stable_sort(rest.begin(), rest.end(), [](const Work& a, const Work& c) { return a.first > c.first; });
+    for (const Work& v : rest) maps[0].push_back(v.second);
     size_t nm = 0;
     for (auto& m : maps) nm += m.size();
     BCK(hipMalloc((void**)&b->d_maps, nm * sizeof(int2)));
@@ -486,9 +505,10 @@ static int check_batch_status(pimdb_batch* b) {
 // LDS plan keeps every exchange workspace and force array in LDS.  The
 // two-kernel form where its load over the whole card is below the persistent
 // kernel's longest workgroup: fewer replicas than compute units (16 helium
-// replicas of N=256, P=64: 162 against 1240 us a step, 128 of them 937 against
-// 1274, but 256 of them 1900 against 1345), uneven ones, and small ones (512
-// uneven dipole replicas 252 against 284 us).
+// replicas of N=256, P=64: 122 against 1240 us a step, 128 of them 716 against
+// 1278, but 256 of them 1486 against 1335), uneven ones, and small ones (512
+// uneven dipole replicas 210 against 277 us, 256 helium replicas of N=30, P=32
+// 104 against 133).
 static int choose_form(pimdb_batch* b) {
     double shape_gain = 1.0;
     if (b->R > b->cus) {
@@ -509,7 +529,7 @@ static int choose_form(pimdb_batch* b) {
     if (rc || !split_able(b)) return rc;
     double load = 0.0;
     for (const pimdb_params& p : b->prm) load += rep_cost_split(p);
-    b->split = 20.0 + load / b->cus < 0.95 * shape_gain * makespan(b, std::min(b->R, b->cus));
+    b->split = 22.0 + load / b->cus < 0.95 * shape_gain * makespan(b, std::min(b->R, b->cus));
     if (b->split && build_split(b) != PIMDB_OK) b->split = false;   // (no memory for its workspace)
     return PIMDB_OK;
 }

@@ -245,7 +245,7 @@ static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mo
     size_t lds = 0;
     if (nf) lds = a.pg.G ? sizeof(double) * group_lds_doubles(D, a.pg.kslots) : tile_lds_bytes(ctx->N, D);
     if (nx) lds = std::max(lds, xw_lds_bytes(ctx->N, D));
-    if (nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles(ctx->P, a.thermostat && a.nm));
+    if (nn) lds = std::max(lds, sizeof(double) * step_noise_lds_doubles<XW_THREADS>(ctx->P, a.thermostat && a.nm));
     const dim3 grid(nx + nf + nn), blk(XW_THREADS);
     const hipStream_t s = ctx->s0;
     switch (ctx->prm.int_kind) {
@@ -268,7 +268,7 @@ static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode
 
 static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
     const StepArgs a = step_args(ctx);
-    const dim3 grid(step_integrate_groups(a.fa, ctx->D, mode, 1));
+    const dim3 grid(step_integrate_groups(a.fa, ctx->D, mode));
     switch (ctx->D) {
     case 1: hipLaunchKernelGGL(k_step_integrate<1>, grid, dim3(256), 0, ctx->s0, a, mode); break;
     case 2: hipLaunchKernelGGL(k_step_integrate<2>, grid, dim3(256), 0, ctx->s0, a, mode); break;

@@ -10,9 +10,13 @@
 // exchange term (the recursions and the exterior forces do not share them,
 // about 80 us of one CU per replica against 1090 for its pairs).
 //
-// Workgroups are ordered replica by replica with the recursions first, so a
-// recursion waits only for earlier workgroups of its own replica, and every
-// compute unit holds a mix of latency-bound recursions and issue-bound slices.
+// The recursions of all replicas come first, so that one waits only for
+// earlier workgroups of its own replica, then slices and noise tiles, the
+// longest first, so that the last round over the card is a short one.  Three
+// workgroups share a compute unit (44 KB of LDS, the ring of N=256), since the
+// noise no longer stages C^T (66 KB).  With these two and one particle a wave in
+// the exterior forces, helium N=256, P=64: 4 replicas 64.4 -> 58.2 us a step, 16
+// 148.5 -> 121.6, 40 335 -> 268, 128 875 -> 718.
 #include "batch_split.hpp"
 
 namespace pimdb {
@@ -162,7 +166,7 @@ static __global__ void __launch_bounds__(SPLIT_THREADS) k_split_integrate(SplitP
     const int2 m = map[blockIdx.x];
     const StepArgs s = sp.steps[uni(m.x)];
     if (blockIdx.x == 0 && threadIdx.x == 0 && mode <= STEP_FULL) *s.ctr += 1;
-    step_integrate<D, SPLIT_EXT>(s, mode, uni(m.y));
+    step_integrate<D>(s, mode, uni(m.y));
 }
 
 template <int D>

@@ -89,9 +89,10 @@ __host__ __device__ inline int step_noise_groups(const StepArgs& s, int D) {
     return s.thermostat || s.fixcom ? D * step_noise_tiles(s.fa.N) : 0;
 }
 __host__ __device__ inline int step_pad16(int P) { return (P + 15) & ~15; }
+template <int NT>
 __host__ __device__ inline size_t step_noise_lds_doubles(int P, bool nm) {
     const size_t Pp = (size_t)step_pad16(P);
-    return XW_THREADS / WAVE + (nm ? Pp * Pp + Pp * STEP_TILE : 0);
+    return XW_THREADS / WAVE + (nm ? (NT == XW_THREADS ? Pp * Pp : 0) + Pp * STEP_TILE : 0);
 }
 
 typedef double step_v4d __attribute__((ext_vector_type(4)));
@@ -156,13 +157,35 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
             }
         }
     } else {
+        // C^T is staged in LDS where the workgroup has the compute unit to
+        // itself (N=128, P=64: 18.5 us a step, 21.5 without); beside other
+        // workgroups, which the 32 KB would keep out, a wave holds its rows of it.
+        constexpr int KMAX = STEP_NM_MAXP / 4;
+        constexpr bool STAGED = NT == XW_THREADS;
         const int Pp = step_pad16(P), MB = Pp / 16, KK = Pp / 4;
-        double* CTl = smem + XW_THREADS / WAVE;   // [k][b], zero padded
-        double* pn = CTl + (size_t)Pp * Pp;       // [column / 16][k][16]
-        for (int e = tid; e < Pp * Pp; e += NT) {
-            const int k = e / Pp, b = e % Pp;
-            CTl[e] = (k < P && b < P) ? s.CTt[(size_t)k * P + b] : 0.0;
+        double* CTl = smem + XW_THREADS / WAVE;                     // [k][b], zero padded
+        double* pn = CTl + (STAGED ? (size_t)Pp * Pp : 0);          // [column / 16][k][16]
+        if constexpr (STAGED) {
+            for (int e = tid; e < Pp * Pp; e += NT) {
+                const int k = e / Pp, b = e % Pp;
+                CTl[e] = (k < P && b < P) ? s.CTt[(size_t)k * P + b] : 0.0;
+            }
         }
+        const int q4 = lane / 16, c16 = lane % 16;
+        const int ntask = MB * (STEP_TILE / 16);
+        double A[KMAX];
+        int held = -1;
+        auto rows = [&](int bb) {
+            held = bb;
+            const int b = bb * 16 + c16;
+#pragma unroll
+            for (int kk = 0; kk < KMAX; ++kk) {
+                const int k = 4 * kk + q4;
+                const double v = s.CTt[(size_t)min(k, P - 1) * P + min(b, P - 1)];
+                A[kk] = k < P && b < P ? v : 0.0;
+            }
+        };
+        if (!STAGED && wave < ntask) rows(wave % MB);
         for (int e = tid; e < (Pp / 2) * STEP_TILE; e += NT) {
             const int m = e / STEP_TILE, c = e % STEP_TILE;
             double g0 = 0.0, g1 = 0.0;
@@ -172,14 +195,20 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
             out[(2 * m + 1) * 16] = 2 * m + 1 < P ? g1 : 0.0;
         }
         __syncthreads();
-        const int q4 = lane / 16, c16 = lane % 16;
-        for (int task = wave; task < MB * (STEP_TILE / 16); task += NW) {
+        for (int task = wave; task < ntask; task += NW) {
             const int bb = task % MB, g = task / MB, c = g * 16 + c16;
+            if (!STAGED && bb != held) rows(bb);
             step_v4d acc = {0.0, 0.0, 0.0, 0.0};
             const double* B = pn + (size_t)g * Pp * 16;
-            for (int kk = 0; kk < KK; ++kk) {
-                const int k = 4 * kk + q4;
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(CTl[(size_t)k * Pp + bb * 16 + c16], B[k * 16 + c16], acc, 0, 0, 0);
+            if constexpr (STAGED) {
+                for (int kk = 0; kk < KK; ++kk) {
+                    const int k = 4 * kk + q4;
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(CTl[(size_t)k * Pp + bb * 16 + c16], B[k * 16 + c16], acc, 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < KMAX; ++kk)
+                    if (kk < KK) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[kk], B[(4 * kk + q4) * 16 + c16], acc, 0, 0, 0);
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -222,32 +251,29 @@ __device__ __forceinline__ void step_recursions(const StepArgs& s, int wg, doubl
                          BeadView{s.x + bs * (P - 1), N, 1}, s.V, s.Vb, nullptr, s.Shi, s.Slo, s.xc, s.pub, s.status);
 }
 
-// Workgroups of an integration: 4 tasks of M particles of an exchange bead each
-// (their forces are complete before an opening half), then 256 elements of the
-// other beads each.
-__host__ __device__ inline int step_exterior_tasks(int N, int M) { return (N + M - 1) / M; }   // per bead
-__host__ __device__ inline int step_exterior_groups(const ForceArgs& fa, int mode, int M) {
-    return fa.bosonic && mode != STEP_OPEN ? (2 * step_exterior_tasks(fa.N, M) + 3) / 4 : 0;   // (also STEP_FORCES)
+// Workgroups of an integration: 4 particles of an exchange bead each (their
+// forces are complete before an opening half), then 256 elements of the other
+// beads each.
+__host__ __device__ inline int step_exterior_groups(const ForceArgs& fa, int mode) {
+    return fa.bosonic && mode != STEP_OPEN ? (2 * fa.N + 3) / 4 : 0;   // (also STEP_FORCES)
 }
 __host__ __device__ inline size_t step_inner_elements(const ForceArgs& fa, int D, int mode) {
     return (size_t)(fa.bosonic && mode != STEP_OPEN ? fa.P - 2 : fa.P) * D * fa.N;
 }
-__host__ __device__ inline int step_integrate_groups(const ForceArgs& fa, int D, int mode, int M) {
-    return step_exterior_groups(fa, mode, M) + (int)((step_inner_elements(fa, D, mode) + 255) / 256);
+__host__ __device__ inline int step_integrate_groups(const ForceArgs& fa, int D, int mode) {
+    return step_exterior_groups(fa, mode) + (int)((step_inner_elements(fa, D, mode) + 255) / 256);
 }
 
 // Workgroup blk of an integration, 256 threads (file header).  Leaves f
 // complete.  The positions that other particles' exterior forces need are
 // read from the copies xc, so x is free to be written.
-// M: particles per wave of the exterior forces (1 for a single ring, where
-// latency counts; more where many rings share the card).
-template <int D, int M>
+template <int D>
 __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int blk) {
     const StepCoef co = step_coef(s, mode);
     const int N = s.fa.N, P = s.fa.P;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     __shared__ double shift[4];
-    const int ng = step_exterior_groups(s.fa, mode, M), nt = step_exterior_tasks(N, M);
+    const int ng = step_exterior_groups(s.fa, mode);
     const bool exterior = blk < ng;
     const size_t bs = (size_t)D * N;
     // the element's (or, exterior, lane's) data first: the loads overlap the
@@ -257,11 +283,10 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
     bool mine = false;
     int ax = 0;
     if (exterior) {
-        const int which = task / nt, l = (task % nt) * M + lane / D;   // lane: particle and axis
-        if (task < 2 * nt && lane < M * D && l < N) {
+        if (task < 2 * N && lane < D) {   // a wave per particle, its first lanes an axis each
             mine = true;
-            ax = lane % D;
-            e = ((size_t)(which == 0 ? 0 : P - 1) * D + ax) * N + l;
+            ax = lane;
+            e = ((size_t)(task < N ? 0 : P - 1) * D + ax) * N + task % N;
         }
     } else {
         const size_t o = (size_t)(blk - ng) * 256 + tid;
@@ -301,14 +326,14 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
         __syncthreads();
     }
     if (exterior) {
-        if (task >= 2 * nt) return;
+        if (task >= 2 * N) return;
         const Ring r = make_ring(s.xc, s.xc + bs, s.Shi, s.Slo, s.fa.k_spring, s.fa.pbc != 0, s.fa.L);
-        double F[M][D];
-        exterior_force<D, M>(task / nt, (task % nt) * M, N, lane, s.bt, s.fa.k_spring, r, s.V, s.Vb, s.xc + 2 * bs,
-                             s.xc + 3 * bs, false, F);
+        double F[D];
+        exterior_force<D>(task / N, task % N, N, lane, s.bt, s.fa.k_spring, r, s.V, s.Vb, s.xc + 2 * bs, s.xc + 3 * bs,
+                          false, F);
 #pragma unroll
-        for (int q = 0; q < M * D; ++q)
-            if (lane == q) fv = F[q / D][q % D] + fv;
+        for (int a = 0; a < D; ++a)
+            if (lane == a) fv = F[a] + fv;
         if (mine) s.f[e] = fv;
     } else if (mine && s.pg.nslots && mode != STEP_OPEN) {
         s.f[e] = fv;
@@ -351,7 +376,7 @@ static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, i
 template <int D>
 static __global__ void __launch_bounds__(256) k_step_integrate(StepArgs s, int mode) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && mode != STEP_CLOSE) *s.ctr += 1;
-    step_integrate<D, 1>(s, mode, blockIdx.x);
+    step_integrate<D>(s, mode, blockIdx.x);
 }
 
 }  // namespace pimdb
