@@ -7,8 +7,8 @@
 //   K3 k_step_forces  exchange recursions beside the bead forces, then
 //                     k_exchange_forces (beads 1 and P)
 //   K4 k_momenta      B, O-step, partial sums for zeroMomentum
-// but device-noise Langevin (or NVE) steps with the Cartesian propagator take
-// k_step_forces and one k_step_integrate per step (steps.hpp).  Rings and
+// but device-noise Langevin (or NVE) steps take k_step_forces and one
+// k_step_integrate (normal-mode propagator: k_step_modes) per step (steps.hpp).  Rings and
 // slices beyond a workgroup's LDS take the recursions and the bead forces as
 // two kernels on two streams.
 #include <hip/hip_runtime.h>
@@ -222,7 +222,7 @@ static StepArgs step_args(pimdb_ctx* ctx) {
     a.c2 = ctx->dv.c2;
     a.half_dt = 0.5 * ctx->prm.dt;
     a.dt_m = ctx->prm.dt / ctx->prm.mass;
-    a.CTt = ctx->CT;
+    a.Ct = ctx->C; a.CTt = ctx->CT; a.rot = ctx->rot;
     a.H = ctx->H; a.hpart = ctx->hpart;
     a.frows = ctx->P * ((ctx->N + FORCE_TILE - 1) / FORCE_TILE);
     a.fpart = ctx->prm.ext_kind != PIMDB_POT_FREE && a.fixcom ? ctx->fpart : nullptr;
@@ -266,8 +266,29 @@ static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode
     }
 }
 
+// f (and fext) completed with the group pair forces' slots.
+static void launch_pair_sum(pimdb_ctx* ctx) {
+    if (ctx->pg.nslots)
+        hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->nbd, ctx->pg,
+                           ctx->f, ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr);
+}
+
 static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
-    const StepArgs a = step_args(ctx);
+    StepArgs a = step_args(ctx);
+    if (ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES) {
+        if (mode != STEP_CLOSE) {
+            const dim3 mgrid(step_modes_groups(ctx->N, ctx->D));
+            const size_t lds = sizeof(double) * step_modes_lds_doubles(ctx->P);
+            switch (ctx->D) {
+            case 1: hipLaunchKernelGGL(k_step_modes<1>, mgrid, dim3(256), lds, ctx->s0, a, mode); break;
+            case 2: hipLaunchKernelGGL(k_step_modes<2>, mgrid, dim3(256), lds, ctx->s0, a, mode); break;
+            default: hipLaunchKernelGGL(k_step_modes<3>, mgrid, dim3(256), lds, ctx->s0, a, mode); break;
+            }
+            return;
+        }
+        a.f = a.fext;   // the closing kick (f and fext are complete)
+        a.pg = PairGroups{};
+    }
     const dim3 grid(step_integrate_groups(a.fa, ctx->D, mode));
     switch (ctx->D) {
     case 1: hipLaunchKernelGGL(k_step_integrate<1>, grid, dim3(256), 0, ctx->s0, a, mode); break;
@@ -280,9 +301,7 @@ static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
 static int enqueue_forces(pimdb_ctx* ctx) {
     if (ctx->merged) {
         launch_step_forces(ctx, true, false, STEP_CLOSE);
-        if (ctx->pg.nslots)
-            hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->nbd,
-                               ctx->pg, ctx->f, ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr);
+        launch_pair_sum(ctx);
         if (ctx->dv.bosonic) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
     } else if (factorial(ctx)) {
         launch_bead_forces(ctx, ctx->s0);
@@ -438,6 +457,7 @@ static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
     for (int s = 1; s <= nsteps; ++s) {
         const int mode = s < nsteps ? STEP_FULL : STEP_CLOSE;
         launch_step_forces(ctx, true, true, mode);
+        if (ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES) launch_pair_sum(ctx);
         launch_step_integrate(ctx, mode);
     }
     CK(hipGetLastError());
@@ -589,8 +609,9 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     else if (ring) alloc(&ctx->xws, 2 * rec_lds_bytes(N, D));
     const bool slice_fits = tile_lds_bytes(N, D) <= device_lds_limit();
     ctx->merged = slice_fits && (!ctx->dv.bosonic || wide);
-    ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN && prm->propagator == PIMDB_PROP_CARTESIAN &&
-                 (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat || P <= STEP_NM_MAXP);
+    ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN &&
+                 (P <= STEP_NM_MAXP || (prm->propagator == PIMDB_PROP_CARTESIAN &&
+                                        (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat)));
     if (ctx->merged) {
         ctx->pg = plan_pair_groups(*prm, ctx->dv, wide ? xw_grid(N) : 0);
         if (ctx->pg.nslots) alloc(&ctx->pg.cpart, sizeof(double) * ctx->nbd * ctx->pg.nslots);

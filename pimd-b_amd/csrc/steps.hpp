@@ -64,7 +64,7 @@ struct StepArgs {
     // noise and the shift
     int thermostat, nm, fixcom;
     double c1, c2, half_dt, dt_m;     // c1 = 1 without a thermostat; dt_m = dt / mass
-    const double* CTt;                // nm -> cart transposed: CTt[k P + b]
+    const double *Ct, *CTt, *rot;     // cart -> nm and nm -> cart transposed (CTt[k P + b]); free-ring rotation
     double* H;                        // [P][D][N]
     double* fpart;                    // [frows][D] partial sums of the external forces (null: none)
     double* hpart;                    // [noise tiles][D] sums of alpha p + H
@@ -264,6 +264,24 @@ __host__ __device__ inline int step_integrate_groups(const ForceArgs& fa, int D,
     return step_exterior_groups(fa, mode) + (int)((step_inner_elements(fa, D, mode) + 255) / 256);
 }
 
+// The momentum per particle and axis that an integration takes out, into
+// shift[0 .. D-1] (wave a for axis a; a barrier is the caller's).
+template <int D>
+__device__ __forceinline__ void step_shift(const StepArgs& s, int mode, int wave, int lane, double* shift) {
+    if (wave >= D) return;
+    const StepCoef co = step_coef(s, mode);
+    const int rows = step_noise_tiles(s.fa.N);
+    double t = 0.0;
+    for (int r = lane; r < rows; r += WAVE) t += s.hpart[(size_t)r * D + wave];
+    if (s.fpart && mode != STEP_OPEN) {
+        double u = 0.0;
+        for (int r = lane; r < s.frows; r += WAVE) u += s.fpart[(size_t)r * D + wave];
+        t = fma(co.alpha * co.beta, u, t);
+    }
+    t = wave_total(t);
+    if (lane == 0) shift[wave] = t / (double)(s.fa.N * s.fa.P);
+}
+
 // Workgroup blk of an integration, 256 threads (file header).  Leaves f
 // complete.  The positions that other particles' exterior forces need are
 // read from the copies xc, so x is free to be written.
@@ -311,18 +329,7 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
         }
     }
     if (s.fixcom && mode != STEP_FORCES) {
-        if (wave < D) {
-            const int rows = step_noise_tiles(N);
-            double t = 0.0;
-            for (int r = lane; r < rows; r += WAVE) t += s.hpart[(size_t)r * D + wave];
-            if (s.fpart && mode != STEP_OPEN) {
-                double u = 0.0;
-                for (int r = lane; r < s.frows; r += WAVE) u += s.fpart[(size_t)r * D + wave];
-                t = fma(co.alpha * co.beta, u, t);
-            }
-            t = wave_total(t);
-            if (lane == 0) shift[wave] = t / (double)(N * P);
-        }
+        step_shift<D>(s, mode, wave, lane, shift);
         __syncthreads();
     }
     if (exterior) {
@@ -377,6 +384,122 @@ template <int D>
 static __global__ void __launch_bounds__(256) k_step_integrate(StepArgs s, int mode) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && mode != STEP_CLOSE) *s.ctr += 1;
     step_integrate<D>(s, mode, blockIdx.x);
+}
+
+// ---- the normal-mode propagator (distinguishable particles) ----
+// What k_step_integrate does, with the kicks on the physical forces fext and
+// the free ring polymer's rotation of the modes for the drift
+// (normal_modes_propagator.cpp:19-53): 16 columns (one axis) of all beads per
+// workgroup, the four P x P products on the matrix cores (step_noise's lane
+// layout).  OPEN and FULL; a closing half is step_integrate's.  What bounds it
+// is latency (21 workgroups for N=101): a step of N=101, P=24 took 25.8 us as
+// k_momenta, k_nm_propagate, forces and k_momenta and takes 16.3 so, half of it
+// this kernel.
+constexpr int MODE_COLS = 16;
+__host__ __device__ inline int step_modes_groups(int N, int D) { return D * ((N + MODE_COLS - 1) / MODE_COLS); }
+__host__ __device__ inline size_t step_modes_lds_doubles(int P) { return (size_t)step_pad16(P) * (4 * MODE_COLS + 4); }
+
+template <int D>
+static __global__ void __launch_bounds__(256) k_step_modes(StepArgs s, int mode) {
+    extern __shared__ __align__(16) double smem[];
+    __shared__ double shift[4];
+    constexpr int NW = 256 / WAVE, KMAX = STEP_NM_MAXP / 4, EMAX = STEP_NM_MAXP * MODE_COLS / 256;
+    const StepCoef co = step_coef(s, mode);
+    const int N = s.fa.N, P = s.fa.P, tiles = (N + MODE_COLS - 1) / MODE_COLS;
+    const int a = blockIdx.x / tiles, i0 = (blockIdx.x % tiles) * MODE_COLS, nc = min(MODE_COLS, N - i0);
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int q4 = lane / 16, c16 = lane % 16;
+    const int Pp = step_pad16(P), MB = Pp / 16, KK = Pp / 4, ntask = 2 * MB;   // task: 16 rows of x or of p
+    if (blockIdx.x == 0 && tid == 0) *s.ctr += 1;
+    double* in = smem;                                // [x, p'][bead][16]
+    double* md = in + 2 * (size_t)Pp * MODE_COLS;     // [x, p'][mode][16]
+    double* rc = md + 2 * (size_t)Pp * MODE_COLS;     // [mode][4]: x = xx q + xp p, p = px q + pp p
+    // all loads first: the elements, then a wave's rows of both matrices
+    double xv[EMAX], pv[EMAX], fv[EMAX], hv[EMAX];
+#pragma unroll
+    for (int u = 0; u < EMAX; ++u) {
+        const int e = tid + u * 256, b = e / MODE_COLS, c = e % MODE_COLS;
+        xv[u] = pv[u] = fv[u] = hv[u] = 0.0;
+        if (b < P && c < nc) {
+            const size_t g = ((size_t)b * D + a) * N + i0 + c;
+            xv[u] = s.x[g];
+            pv[u] = s.p[g];
+            fv[u] = s.fext[g];
+            if (s.thermostat) hv[u] = s.H[g];
+        }
+    }
+    double A[KMAX], B[KMAX];
+    auto rows = [&](const double* M, int bb, double (&R)[KMAX]) {
+        const int m = bb * 16 + c16;
+#pragma unroll
+        for (int kk = 0; kk < KMAX; ++kk) {
+            if (kk >= KK) break;
+            const int k = 4 * kk + q4;
+            const double v = M[(size_t)min(k, P - 1) * P + min(m, P - 1)];
+            R[kk] = k < P && m < P ? v : 0.0;
+        }
+    };
+    if (wave < ntask) {
+        rows(s.Ct, wave % MB, A);
+        rows(s.CTt, wave % MB, B);
+    }
+    if (tid < Pp) {
+        double xx = 0.0, xp = 0.0, px = 0.0, pp = 0.0;
+        if (tid < P) {
+            const double cs = s.rot[4 * tid], sn = s.rot[4 * tid + 1], mw = s.rot[4 * tid + 2], w = s.rot[4 * tid + 3];
+            xx = w == 0 ? 1.0 : cs;
+            xp = w == 0 ? s.dt_m : sn / mw;
+            px = w == 0 ? 0.0 : (-1) * mw * sn;
+            pp = w == 0 ? 1.0 : cs;
+        }
+        rc[4 * tid] = xx;
+        rc[4 * tid + 1] = xp;
+        rc[4 * tid + 2] = px;
+        rc[4 * tid + 3] = pp;
+    }
+    if (s.fixcom) {
+        step_shift<D>(s, mode, wave, lane, shift);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < EMAX; ++u) {
+        const int e = tid + u * 256;
+        if (e < Pp * MODE_COLS) {
+            double v = fma(co.alpha, fma(co.beta, fv[u], pv[u]), hv[u]);
+            if (s.fixcom) v -= shift[a];
+            in[e] = xv[u];
+            in[Pp * MODE_COLS + e] = e / MODE_COLS < P ? fma(co.gamma, fv[u], v) : 0.0;
+        }
+    }
+    __syncthreads();
+    auto product = [&](int t, const double* M, double (&R)[KMAX], auto&& operand, auto&& store) {
+        const int bb = t % MB;
+        if (t != wave && bb != wave % MB) rows(M, bb, R);
+        step_v4d acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};   // (two chains; KK is a multiple of 4)
+#pragma unroll
+        for (int kk = 0; kk < KMAX; ++kk)
+            if (kk < KK) acc[kk % 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(R[kk], operand(4 * kk + q4), acc[kk % 2], 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) store(bb * 16 + q4 + 4 * v, acc[0][v] + acc[1][v]);
+    };
+    for (int t = wave; t < ntask; t += NW) {
+        const size_t o = (size_t)(t / MB) * Pp * MODE_COLS + c16;
+        product(t, s.Ct, A, [&](int k) { return in[o + k * MODE_COLS]; },
+                [&](int k, double v) { md[o + k * MODE_COLS] = v; });
+    }
+    __syncthreads();
+    for (int t = wave; t < ntask; t += NW) {
+        const int w = t / MB;
+        double* out = w == 0 ? s.x : s.p;
+        product(t, s.CTt, B,
+                [&](int k) {
+                    const double q = md[k * MODE_COLS + c16], pm = md[(Pp + k) * MODE_COLS + c16];
+                    return fma(rc[4 * k + 2 * w], q, rc[4 * k + 2 * w + 1] * pm);
+                },
+                [&](int b, double v) {
+                    if (b < P && c16 < nc) out[((size_t)b * D + a) * N + i0 + c16] = v;
+                });
+    }
 }
 
 }  // namespace pimdb
