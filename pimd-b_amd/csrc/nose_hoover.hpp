@@ -37,13 +37,16 @@ struct NhArgs {
     double *eta, *eta_dot, *eta_dot_dot;   // [P][groups][nc]
 };
 
-// singleChainStep on one chain; returns the momentum scale.
-__device__ inline double nh_chain_step(const NhArgs& h, double* e, double* ed, double* edd, double current_energy) {
-    const int nc = h.nc;
+// singleChainStep on one chain of NC components; returns the momentum scale.
+template <int NC>
+__device__ __forceinline__ double nh_chain_core(const NhArgs& h, const int nc_, double* e, double* ed, double* edd,
+                                                double current_energy) {
+    const int nc = NC > 0 ? NC : nc_;
     const double dt2 = 0.5 * h.dt, dt4 = 0.25 * h.dt, dt8 = 0.125 * h.dt;
     double exp_factor = 0.0;
     edd[0] = (current_energy - h.required) / h.Q1;
     ed[nc - 1] += edd[nc - 1] * dt4;
+#pragma unroll
     for (int i = nc - 2; i >= 0; i--) {
         exp_factor = exp(-dt8 * ed[i + 1]);
         ed[i] *= exp_factor;
@@ -51,12 +54,14 @@ __device__ inline double nh_chain_step(const NhArgs& h, double* e, double* ed, d
         ed[i] *= exp_factor;
     }
     const double scale = exp(-dt2 * ed[0]);
+#pragma unroll
     for (int i = 0; i < nc; i++) e[i] += dt2 * ed[i];
     edd[0] = (current_energy * scale * scale - h.required) / h.Q1;
     ed[0] *= exp_factor;
     ed[0] += edd[0] * dt4;
     ed[0] *= exp_factor;
     double Q_former = h.Q1;
+#pragma unroll
     for (int i = 1; i < nc - 1; i++) {
         exp_factor = exp(-dt8 * ed[i + 1]);
         ed[i] *= exp_factor;
@@ -68,6 +73,29 @@ __device__ inline double nh_chain_step(const NhArgs& h, double* e, double* ed, d
     edd[nc - 1] = (h.Qi * ed[nc - 2] * ed[nc - 2] - 1 / h.thermo_beta) / h.Qi;
     ed[nc - 1] += edd[nc - 1] * dt4;
     return scale;
+}
+
+// A chain of four (the default) in registers; others in place, every access a
+// load or a store that the next one waits for.
+__device__ inline double nh_chain_step(const NhArgs& h, double* e, double* ed, double* edd, double current_energy) {
+    if (h.nc == 4) {
+        double x[4], v[4], a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = e[i];
+            v[i] = ed[i];
+            a[i] = edd[i];
+        }
+        const double scale = nh_chain_core<4>(h, 4, x, v, a, current_energy);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            e[i] = x[i];
+            ed[i] = v[i];
+            edd[i] = a[i];
+        }
+        return scale;
+    }
+    return nh_chain_core<0>(h, h.nc, e, ed, edd, current_energy);
 }
 
 // One Nose-Hoover O-step on p [b][a][i] (Cartesian momenta, or the modes

@@ -29,6 +29,7 @@
 #include "integrator.hpp"
 #include "observables.hpp"
 #include "steps.hpp"
+#include "nh_steps.hpp"
 
 using namespace pimdb;
 
@@ -52,6 +53,8 @@ struct pimdb_ctx {
     unsigned long long* ctr = nullptr;
     bool merged = false;           // recursions and bead forces in one k_step_forces
     PairGroups pg{};               // pair forces by groups of 128 (slice_groups.hpp)
+    bool nh_whole = false;         // consecutive Nose-Hoover steps by k_step_forces and k_nh_steps
+    bool nh_close = false;         // closing halves with the exchange forces by k_nh_steps
     bool split = false;            // consecutive steps by k_step_forces and k_step_integrate
     double *xc = nullptr, *H = nullptr, *fpart = nullptr, *hpart = nullptr;   // their workspace (StepArgs)
     int tc = 1, ntiles = 1;
@@ -413,6 +416,26 @@ static void enqueue_open(pimdb_ctx* ctx, const double* noise0) {
     }
 }
 
+template <int D>
+static void launch_nh_steps_d(pimdb_ctx* ctx, int mode) {
+    const StepArgs a = step_args(ctx);
+    NhArgs h = ctx->nh;
+    h.half_dt = 0.5 * ctx->prm.dt;
+    if (!ctx->nh_whole && ctx->prm.fixcom) h.com_out = ctx->com1;
+    const int nb = ctx->prm.fixcom && ctx->nh_whole ? ctx->P : 1;
+    const bool ext = ctx->dv.bosonic && ctx->N <= NH_EXT;
+    hipLaunchKernelGGL(k_nh_steps<D>, dim3(ctx->P / nb), dim3(NH_THREADS),
+                       sizeof(double) * nh_step_lds_doubles(ctx->N, D, nb, ext), ctx->s0, a, h, nb, ext ? 1 : 0, mode);
+}
+
+static void launch_nh_steps(pimdb_ctx* ctx, int mode) {
+    switch (ctx->D) {
+    case 1: launch_nh_steps_d<1>(ctx, mode); break;
+    case 2: launch_nh_steps_d<2>(ctx, mode); break;
+    default: launch_nh_steps_d<3>(ctx, mode); break;
+    }
+}
+
 // The closing half: K4 (B + O-step + partial COM sums).
 static void enqueue_close(pimdb_ctx* ctx, const double* noise1) {
     const bool fixcom = ctx->prm.fixcom != 0;
@@ -431,15 +454,35 @@ static void enqueue_close(pimdb_ctx* ctx, const double* noise1) {
 // One OBABO step; noise0/noise1: device noise of the two O-steps or null.
 static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* noise1) {
     enqueue_open(ctx, noise0);
-    const int rc = enqueue_forces(ctx);
-    if (rc) return rc;
-    enqueue_close(ctx, noise1);
+    if (ctx->nh_close) {
+        launch_step_forces(ctx, true, false, STEP_CLOSE);
+        launch_nh_steps(ctx, STEP_CLOSE);
+    } else {
+        const int rc = enqueue_forces(ctx);
+        if (rc) return rc;
+        enqueue_close(ctx, noise1);
+    }
+    CK(hipGetLastError());
+    return PIMDB_OK;
+}
+
+// nsteps Nose-Hoover steps by k_step_forces and k_nh_steps.
+static int enqueue_nh_steps(pimdb_ctx* ctx, int nsteps) {
+    if (nsteps == 0) return PIMDB_OK;
+    launch_nh_steps(ctx, STEP_OPEN);
+    for (int s = 1; s <= nsteps; ++s) {
+        launch_step_forces(ctx, true, false, STEP_CLOSE);
+        launch_pair_sum(ctx);
+        if (ctx->dv.bosonic && ctx->N > NH_EXT) launch_exchange_forces(ctx, ctx->s0, ctx->f, nullptr);
+        launch_nh_steps(ctx, s < nsteps ? STEP_FULL : STEP_CLOSE);
+    }
     CK(hipGetLastError());
     return PIMDB_OK;
 }
 
 // nsteps device-noise steps.
 static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
+    if (ctx->nh_whole) return enqueue_nh_steps(ctx, nsteps);
     if (!ctx->split) {
         for (int s = 0; s < nsteps; ++s) {
             if (ctx->gexec) {
@@ -465,9 +508,9 @@ static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
 }
 
 // Apply the pending zeroMomentum of the last O-step and clear the partials.
-// (Split steps leave neither.)
+// (Split and whole Nose-Hoover steps leave neither.)
 static int finish_steps(pimdb_ctx* ctx, bool host_noise) {
-    if (ctx->prm.fixcom && (host_noise || !ctx->split)) {
+    if (ctx->prm.fixcom && (host_noise || !(ctx->split || ctx->nh_whole))) {
         hipLaunchKernelGGL(k_com_subtract, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->N,
                            ctx->P, ctx->D, ctx->com1, ctx->ncom, ctx->p);
         CK(hipMemsetAsync(ctx->com1, 0, sizeof(double) * (size_t)ctx->ncom * ctx->D, ctx->s0));
@@ -612,6 +655,17 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN &&
                  (P <= STEP_NM_MAXP || (prm->propagator == PIMDB_PROP_CARTESIAN &&
                                         (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat)));
+    if (ctx->merged && prm->thermostat >= PIMDB_THERMO_NOSE_HOOVER && !prm->nmthermostat &&
+        prm->propagator == PIMDB_PROP_CARTESIAN) {
+        const int groups = prm->thermostat == PIMDB_THERMO_NOSE_HOOVER ? 1 : prm->thermostat == PIMDB_THERMO_NOSE_HOOVER_NP ? N : N * D;
+        const bool fits = sizeof(double) * nh_step_lds_doubles(N, D, prm->fixcom ? P : 1, ctx->dv.bosonic && N <= NH_EXT) + 1024 <=
+                          device_lds_limit();
+        // with zeroMomentum one workgroup: two chains a thread or beads a wave
+        // in turn already cost more than the kernels they replace (nh_steps.hpp)
+        const bool few = groups == 1 ? P <= NH_WAVES && ctx->nbd <= NH_THREADS : (size_t)P * groups <= NH_THREADS / 2;
+        ctx->nh_whole = fits && (!prm->fixcom || few);
+        ctx->nh_close = !ctx->nh_whole && ctx->dv.bosonic && N <= NH_EXT / 2;
+    }
     if (ctx->merged) {
         ctx->pg = plan_pair_groups(*prm, ctx->dv, wide ? xw_grid(N) : 0);
         if (ctx->pg.nslots) alloc(&ctx->pg.cpart, sizeof(double) * ctx->nbd * ctx->pg.nslots);
