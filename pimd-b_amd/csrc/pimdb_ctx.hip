@@ -177,36 +177,41 @@ static void launch_factorial(pimdb_ctx* ctx, hipStream_t s, double* f, double* f
 }
 
 // How the pair forces of a merged step are cut (PairGroups; G = 0 for one tile
-// of 64 rows per workgroup).
-static PairGroups plan_pair_groups(const pimdb_params& p, const Derived& d, int nx) {
+// of 64 rows per workgroup).  nx, nn: workgroups of the recursions, which hold a
+// compute unit each for as long as they take (8 us and 4.6 us per 100
+// particles), and of the noise.
+//
+// A workgroup takes about 4 us and 1 us per 16 steps (Aziz).  Whole rounds over
+// the card take groups whole (or in q1 parts); the beads that are left over
+// would take as long again on a part of the card and are cut finer (N=400, P=64
+// 56.7 -> 46.1 us a step, N=1000, P=32 85 -> 79.5, P=64 133 -> 119; too few
+// workgroups to fill the card: N=1000, P=4 without exchange 44.0, 28.6, 25.0, 21.3
+// with 1 .. 4 parts).  Finer only for a tenth less, since the integration reads
+// the sums of every part.
+static PairGroups plan_pair_groups(const pimdb_params& p, const Derived& d, int nx, int nn) {
     PairGroups pg{};
-    const int N = p.natoms;
+    const int N = p.natoms, P = p.nbeads;
     if (p.int_kind == PIMDB_POT_FREE || d.cutoff == 0.0 || N <= GROUP_MIN) return pg;
     const int G = (N + GROUP - 1) / GROUP;
-    // A workgroup takes about 4 us and 1 us per 16 steps (Aziz), and each of the
-    // recursions' holds a compute unit for as long as they take (8 us and 4.6 us
-    // per 100 particles).  More parts, which the integration reads, only for a
-    // tenth less: N=1000, P=4 without exchange 44.0, 28.6, 25.0, 21.3 us a step
-    // with 1 .. 4 parts (64 us at P=8 with exchange whatever the parts), N=256,
-    // P=64 25.5, 31.7, 30.7, 42.9.
     const int steps = GROUP_OWN + group_seg_start(G, group_segments(G)), cus = std::max(1, device_cus() - nx);
+    const double rec = nx ? 8.0 + 0.046 * N : 0.0;
+    auto us = [&](int q) { return 4.0 + steps / (16.0 * q); };
     double best = 0.0;
-    int parts = 0;
-    for (int q = 1; q <= GROUP_PARTS; ++q) {
-        if (sizeof(double) * group_lds_doubles(p.ndim, group_kslots(G, q)) > device_lds_limit()) continue;
-        const int rounds = (p.nbeads * G * q + cus - 1) / cus;
-        const double t = std::max(rounds * (4.0 + steps / (16.0 * q)), nx ? 8.0 + 0.046 * N : 0.0);
-        if (!parts || t < 0.9 * best) {
-            best = t;
-            parts = q;
+    for (int q1 = 1; q1 <= GROUP_PARTS; ++q1) {
+        for (int q2 = q1; q2 <= GROUP_PARTS; ++q2) {
+            const int k = std::max(group_kslots(G, q1), group_kslots(G, q2));
+            if (sizeof(double) * group_lds_doubles(p.ndim, k) > device_lds_limit()) continue;
+            const int rounds = P * G * q1 / cus;
+            const int b1 = q1 == q2 ? 0 : std::min(P, std::max(0, rounds * cus - nn) / (G * q1));
+            const int left = (P - b1) * G * q2;
+            const double t = std::max((b1 ? rounds * us(q1) : 0.0) + (left + cus - 1) / cus * us(q2), rec);
+            if (!pg.G || t < 0.9 * best) {
+                best = t;
+                pg.G = G; pg.kslots = k;
+                pg.b1 = b1; pg.q1 = q1; pg.q2 = q2;
+            }
         }
     }
-    if (!parts) return pg;
-    const int k = group_kslots(G, parts);
-    pg.G = G;
-    pg.parts = parts;
-    pg.kslots = k;
-    pg.nslots = G / 2 + parts - 1;
     return pg;
 }
 
@@ -242,7 +247,7 @@ static size_t tile_lds_bytes(int N, int D) {
 template <int D>
 static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
     const StepArgs a = step_args(ctx);
-    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = !forces ? 0 : a.pg.G ? ctx->P * a.pg.G * a.pg.parts : a.frows;
+    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = !forces ? 0 : a.pg.G ? a.pg.groups_of(ctx->P) : a.frows;
     const int nn = noise ? step_noise_groups(a, D) : 0;
     if (nx + nf + nn == 0) return;
     size_t lds = 0;
@@ -271,9 +276,9 @@ static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode
 
 // f (and fext) completed with the group pair forces' slots.
 static void launch_pair_sum(pimdb_ctx* ctx) {
-    if (ctx->pg.nslots)
-        hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->nbd, ctx->pg,
-                           ctx->f, ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr);
+    if (ctx->pg.G)
+        hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((ctx->nbd + 255) / 256)), dim3(256), 0, ctx->s0, ctx->nbd,
+                           (size_t)ctx->D * ctx->N, ctx->pg, ctx->f, ctx->prm.propagator == PIMDB_PROP_NORMAL_MODES ? ctx->fext : nullptr);
 }
 
 static void launch_step_integrate(pimdb_ctx* ctx, int mode) {
@@ -667,8 +672,8 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
         ctx->nh_close = !ctx->nh_whole && ctx->dv.bosonic && N <= NH_EXT / 2;
     }
     if (ctx->merged) {
-        ctx->pg = plan_pair_groups(*prm, ctx->dv, wide ? xw_grid(N) : 0);
-        if (ctx->pg.nslots) alloc(&ctx->pg.cpart, sizeof(double) * ctx->nbd * ctx->pg.nslots);
+        ctx->pg = plan_pair_groups(*prm, ctx->dv, wide ? xw_grid(N) : 0, D * step_noise_tiles(N));
+        if (ctx->pg.G && ctx->pg.max_slots(P)) alloc(&ctx->pg.cpart, sizeof(double) * ctx->nbd * ctx->pg.max_slots(P));
     }
     if (ctx->merged && ctx->dv.bosonic) alloc(&ctx->xc, sizeof(double) * 4 * (size_t)D * N);
     if (ctx->split) {

@@ -10,8 +10,8 @@
 // often.  What bounds these: vector issue, 36 us for the 33 steps per wave of
 // N=1000 (four waves a SIMD, 2 x 83 issue slots of 4 cycles a step).  A whole
 // Langevin step, both with pair_grad_image: N=256, P=64 39.7 -> 25.3 us, N=500,
-// P=32 63.6 -> 35.7, N=1000, P=32 159 -> 85 and P=64 257 -> 133; without exchange
-// N=1000, P=4 54.8 -> 21.2, N=300, P=4 25.2 -> 17.1.
+// P=32 63.6 -> 35.7, N=1000, P=32 159 -> 79 and P=64 257 -> 120; without exchange
+// N=1000, P=4 54.8 -> 21.3, N=300, P=4 25.2 -> 17.1.
 //
 // Work.  Group g meets itself and, of the other G - 1 groups on a ring, those
 // at distances 1 .. (G-1)/2 ahead, and for even G half of the pairs with the
@@ -23,8 +23,9 @@
 //   tile A with itself, tile B with itself (17 steps each: SliceWalk's
 //   diagonal tile, pairs.hpp), rows l and l+32 of A against B (32 steps),
 //   then A and B against one tile of another group (64 steps; 32 opposite),
-// cut evenly over the waves, and over `parts` workgroups at segment bounds
-// where whole groups would leave the last wave of workgroups nearly empty.
+// cut evenly over the waves, and over several workgroups ("parts") at segment
+// bounds: for the beads of the last round over the card, which whole groups
+// would leave nearly empty, or for all where they are too few to fill it.
 //
 // Sums.  A wave accumulates its rows, and the columns of the group's own
 // tiles, in an LDS array of its own, and every other column tile in a slot of
@@ -50,8 +51,13 @@ constexpr int GROUP_PARTS = 4;  // parts at most
 constexpr int GROUP_OWN = 17 + 17 + 32;   // steps of a group with itself
 
 struct PairGroups {
-    int G, parts, nslots, kslots;   // groups (0: bead_forces_tile), parts per group, slots of cpart, LDS slots per wave
-    double* cpart;                  // [nslots][P][D][N]
+    int G, kslots;      // groups (0: bead_forces_tile), LDS slots per wave
+    int b1, q1, q2;     // parts per group: q1 for beads below b1, q2 for the others
+    double* cpart;      // [slots][P][D][N]
+    __host__ __device__ int parts(int b) const { return b < b1 ? q1 : q2; }
+    __host__ __device__ int slots(int b) const { return G ? G / 2 + parts(b) - 1 : 0; }   // those of bead b
+    __host__ __device__ int max_slots(int P) const { return b1 < P ? slots(P - 1) : slots(0); }   // (q1 <= q2)
+    __host__ __device__ int groups_of(int P) const { return G * (b1 * q1 + (P - b1) * q2); }      // workgroups
 };
 
 // Segments of a group with others, their first steps, and a part's first segment.
@@ -213,9 +219,9 @@ __device__ __forceinline__ void group_walk(const double* xs, int N, const ImageG
     }
 }
 
-// The forces of group id / parts % G of bead id / parts / G, part id % parts,
-// by a workgroup of 1024 threads: as bead_forces_tile, with the pair forces of
-// other workgroups' rows and of other parts left in pg.cpart.
+// Workgroup id of pg.groups_of(P): the forces of one part of one group of one
+// bead, by 1024 threads: as bead_forces_tile, with the pair forces of other
+// workgroups' rows and of other parts left in pg.cpart.
 template <int D, int KIND>
 __device__ __forceinline__ void group_forces(const ForceArgs& fa, const PairGroups& pg, int id, const double* __restrict__ x,
                                              double* __restrict__ f, double* __restrict__ fext,
@@ -223,10 +229,11 @@ __device__ __forceinline__ void group_forces(const ForceArgs& fa, const PairGrou
     constexpr int S = pair_fstride(D);
     const int N = fa.N, P = fa.P, G = pg.G;
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-    const int part = id % pg.parts, bg = id / pg.parts, g = bg % G, b = bg / G;
+    const int n1 = G * pg.b1 * pg.q1, at = id < n1 ? id : id - n1, parts = id < n1 ? pg.q1 : pg.q2;
+    const int part = at % parts, bg = at / parts, g = bg % G, b = bg / G + (id < n1 ? 0 : pg.b1);
     const size_t bs = (size_t)D * N;
     const double* xb = x + bs * b;
-    const GroupPart gp(G, pg.parts, part);
+    const GroupPart gp(G, parts, part);
     lds_double* R0 = (lds_double*)smem;
     lds_double* slots0 = R0 + GROUP_WAVES * GROUP * S;
     lds_double* R = R0 + wave * GROUP * S;
@@ -302,12 +309,12 @@ __device__ __forceinline__ void group_forces(const ForceArgs& fa, const PairGrou
 }
 
 // The slots' sum into f (and fext), for readers of f that do not add them.
-static __global__ void __launch_bounds__(256) k_pair_sum(size_t n, PairGroups pg, double* __restrict__ f,
-                                                  double* __restrict__ fext) {
+static __global__ void __launch_bounds__(256) k_pair_sum(size_t n, size_t bs, PairGroups pg,
+                                                  double* __restrict__ f, double* __restrict__ fext) {
     const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= n) return;
     double s = 0.0;
-    for (int k = 0; k < pg.nslots; ++k) s += pg.cpart[k * n + e];
+    for (int k = 0, m = pg.slots((int)(e / bs)); k < m; ++k) s += pg.cpart[k * n + e];
     f[e] += s;
     if (fext) fext[e] += s;
 }

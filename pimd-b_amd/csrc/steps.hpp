@@ -321,10 +321,10 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
             if (mode != STEP_CLOSE) xv = s.x[e];
             if (s.thermostat) hv = s.H[e];
         }
-        if (mode != STEP_OPEN) {
+        if (mode != STEP_OPEN && s.pg.G) {
             const size_t n = (size_t)P * bs;
             double c = 0.0;
-            for (int k = 0; k < s.pg.nslots; ++k) c += s.pg.cpart[k * n + e];
+            for (int k = 0, m = s.pg.slots((int)(e / bs)); k < m; ++k) c += s.pg.cpart[k * n + e];
             fv += c;
         }
     }
@@ -342,7 +342,7 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
         for (int a = 0; a < D; ++a)
             if (lane == a) fv = F[a] + fv;
         if (mine) s.f[e] = fv;
-    } else if (mine && s.pg.nslots && mode != STEP_OPEN) {
+    } else if (mine && s.pg.G && mode != STEP_OPEN) {
         s.f[e] = fv;
     }
     if (!mine || mode == STEP_FORCES) return;
