@@ -8,7 +8,9 @@
 //                     k_exchange_forces (beads 1 and P)
 //   K4 k_momenta      B, O-step, partial sums for zeroMomentum
 // but device-noise Langevin (or NVE) steps take k_step_forces and one
-// k_step_integrate (normal-mode propagator: k_step_modes) per step (steps.hpp).  Rings and
+// k_step_integrate (normal-mode propagator: k_step_modes) per step (steps.hpp),
+// or a handful of particles one k_small_steps for many (small_steps.hpp), and
+// Nose-Hoover ones k_step_forces and k_nh_steps (nh_steps.hpp).  Rings and
 // slices beyond a workgroup's LDS take the recursions and the bead forces as
 // two kernels on two streams.
 #include <hip/hip_runtime.h>
@@ -30,6 +32,7 @@
 #include "observables.hpp"
 #include "steps.hpp"
 #include "nh_steps.hpp"
+#include "small_steps.hpp"
 
 using namespace pimdb;
 
@@ -53,6 +56,7 @@ struct pimdb_ctx {
     unsigned long long* ctr = nullptr;
     bool merged = false;           // recursions and bead forces in one k_step_forces
     PairGroups pg{};               // pair forces by groups of 128 (slice_groups.hpp)
+    bool small = false;            // split steps, many in one k_small_steps
     bool nh_whole = false;         // consecutive Nose-Hoover steps by k_step_forces and k_nh_steps
     bool nh_close = false;         // closing halves with the exchange forces by k_nh_steps
     bool split = false;            // consecutive steps by k_step_forces and k_step_integrate
@@ -485,8 +489,34 @@ static int enqueue_nh_steps(pimdb_ctx* ctx, int nsteps) {
     return PIMDB_OK;
 }
 
+template <int D>
+static void launch_small_steps_d(pimdb_ctx* ctx, int nsteps) {
+    const StepArgs a = step_args(ctx);
+    const size_t lds = sizeof(double) * small_lds_doubles(ctx->N, ctx->P, D, a.thermostat && a.nm);
+    const dim3 grid(1), blk(SMALL_THREADS);
+    switch (ctx->prm.int_kind) {
+    case POT_HARMONIC: hipLaunchKernelGGL((k_small_steps<D, POT_HARMONIC>), grid, blk, lds, ctx->s0, a, nsteps); break;
+    case POT_DIPOLE: hipLaunchKernelGGL((k_small_steps<D, POT_DIPOLE>), grid, blk, lds, ctx->s0, a, nsteps); break;
+    default: hipLaunchKernelGGL((k_small_steps<D, POT_FREE>), grid, blk, lds, ctx->s0, a, nsteps); break;
+    }
+}
+
+static int enqueue_small_steps(pimdb_ctx* ctx, int nsteps) {
+    for (int s = 0; s < nsteps; s += SMALL_STEPS) {
+        const int n = std::min(SMALL_STEPS, nsteps - s);
+        switch (ctx->D) {
+        case 1: launch_small_steps_d<1>(ctx, n); break;
+        case 2: launch_small_steps_d<2>(ctx, n); break;
+        default: launch_small_steps_d<3>(ctx, n); break;
+        }
+    }
+    CK(hipGetLastError());
+    return PIMDB_OK;
+}
+
 // nsteps device-noise steps.
 static int enqueue_steps(pimdb_ctx* ctx, int nsteps) {
+    if (ctx->small) return enqueue_small_steps(ctx, nsteps);
     if (ctx->nh_whole) return enqueue_nh_steps(ctx, nsteps);
     if (!ctx->split) {
         for (int s = 0; s < nsteps; ++s) {
@@ -660,6 +690,8 @@ int pimdb_ctx_create(const pimdb_params* prm, pimdb_ctx** out) {
     ctx->split = ctx->merged && prm->thermostat <= PIMDB_THERMO_LANGEVIN &&
                  (P <= STEP_NM_MAXP || (prm->propagator == PIMDB_PROP_CARTESIAN &&
                                         (prm->thermostat == PIMDB_THERMO_NONE || !prm->nmthermostat)));
+    ctx->small = ctx->split && prm->propagator == PIMDB_PROP_CARTESIAN && prm->int_kind != PIMDB_POT_AZIZ &&
+                 N <= (ctx->dv.bosonic ? SMALL_RING : SMALL_N) && ctx->nbd <= SMALL_E && P <= STEP_NM_MAXP;
     if (ctx->merged && prm->thermostat >= PIMDB_THERMO_NOSE_HOOVER && !prm->nmthermostat &&
         prm->propagator == PIMDB_PROP_CARTESIAN) {
         const int groups = prm->thermostat == PIMDB_THERMO_NOSE_HOOVER ? 1 : prm->thermostat == PIMDB_THERMO_NOSE_HOOVER_NP ? N : N * D;
