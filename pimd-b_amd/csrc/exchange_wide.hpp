@@ -46,7 +46,12 @@
 // largest (an entry of B or E that underflowed could count then; one that
 // overflowed makes z infinite or NaN), is taken again by the exact min-plus
 // form (xw_block_safe) and publishes XW_BAD, on which the next block takes its
-// U like a farther block's.
+// U like a farther block's and the exact form at once.  Rings that exchange
+// strongly take it throughout, at about 7 us a block: a step of helium whose
+// bead P of each particle lies at its neighbour's bead 1 takes 29.6 us at N=64,
+// P=64, 64.6 at N=256 and 201 at N=1000, P=32 (18.9, 26.8 and 82 without
+// exchange; 60, 100 and 359 with one workgroup per direction; 26.8, 99.5 and 628
+// when the exact form took every earlier source again).
 //
 // Publication.  z, and off the chain U (plus, backward, the source's ln(N-q)),
 // go to global arrays by relaxed device-scope atomic stores and are read by
@@ -86,8 +91,7 @@ __device__ __forceinline__ int xw_b(int j, int t) {
     return xw_brow(R) + (t - 16 * R) * XW_BS + (j - 16 * R);
 }
 constexpr int XW_MAT = xw_brow(4);
-constexpr int XW_SAFE_WAVES = 8;   // waves that take sources in the safe form
-static_assert(XW_MAT >= REC_TRI + XW_SAFE_WAVES * REC_B + 3 * REC_B, "the safe form's arrays lie in the matrix's place");
+static_assert(XW_MAT >= REC_TRI + 2 * REC_B, "the safe form's arrays lie in the matrix's place");
 
 // LDS doubles: the ring, the in-block matrix, the per-wave partials, the
 // block's gauge, the previous block's gauge and factors as sources, the
@@ -104,7 +108,7 @@ struct XwShared {
     double *psum;                  // [waves][REC_B]
     double *g;                     // [REC_B] gauge
     double *off, *rat;             // [REC_B] the previous block's: G_last - G_j, and backward (N-last)/(N-j)
-    double *lq;                    // [REC_B] backward, ln(N-q) of the targets as sources
+    double *lq;                    // [REC_B] ln n of the targets; backward, ln(N-q) of them as sources
     double *tot;                   // [3 waves] wave totals: links, their split sums; then G_last of the previous block
     int* flag;                     // [0] the block left the range, [1] the previous one did, [2] its z fall too far
     double *x1, *xP, *Shi, *Slo;   // the ring [D][N], [D][N], [N], [N]
@@ -246,10 +250,10 @@ __device__ __forceinline__ Ring xw_stage(const XwShared& sh, int I, int N, doubl
             sh.tot[3 * NW] = gl;
         }
     }
-    if (DIR == 1 && wave == 3) {
+    if (wave == 3) {
         const int n0 = 1 + I * REC_B;
-        if (I > 0) sh.rat[lane] = (double)(N - n0 + 1) * rcp_newton((double)(N - n0 + REC_B - lane));   // j = n0 - 64 + lane
-        sh.lq[lane] = log((double)max(1, N - n0 - lane));
+        if (DIR == 1 && I > 0) sh.rat[lane] = (double)(N - n0 + 1) * rcp_newton((double)(N - n0 + REC_B - lane));   // j = n0 - 64 + lane
+        sh.lq[lane] = log((double)(DIR == 0 ? n0 + lane : max(1, N - n0 - lane)));
     }
     // the quantum from the links' total, the same bits in every wave
     auto quantum = [](double total) { return total > 0.0 ? __builtin_amdgcn_frexp_exp(total) - 41 : 0; };
@@ -366,55 +370,44 @@ __device__ __forceinline__ double xw_wait(unsigned long long* p, int at, int* st
     return __longlong_as_double((long long)b);
 }
 
-// One block with the exact min-plus shifts (exchange.hpp, steps (1)-(4)) from
-// every earlier U: for blocks whose z left the range.  All threads; U of the
-// lane's target in every lane of wave 0.
+// One block with the exact min-plus shifts (exchange.hpp, steps (1)-(4)), for
+// blocks whose z left the range: rings that exchange strongly (a two-particle
+// cycle that is favoured by e^10 moves z by that).  Every earlier source is in
+// the waves' online sums m, s already, all but the previous block's since
+// before the wait; the in-block weights (xw_safe_weights) need no U at all.  All
+// threads; U of the lane's target in every lane of wave 0.
 template <int DIR, int D, int NT>
-__device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, const Ring r, const XwShared sh,
-                                             unsigned long long* upub, int* status) {
-    constexpr int NW = NT / WAVE, SW = NW < XW_SAFE_WAVES ? NW : XW_SAFE_WAVES, SRC = REC_B / SW;
-    double *part = sh.a + REC_TRI, *R = part + SW * REC_B, *z = R + REC_B, *lt = z + REC_B;   // (in the matrix's place)
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const int n0 = 1 + I * REC_B, tl = min(lane, nb - 1);
+__device__ __noinline__ void xw_safe_weights(int N, int n0, int nb, double bk, const Ring r, const XwShared sh) {
+    constexpr int NW = NT / WAVE;
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
     __syncthreads();   // (the matrix is no longer read)
-    // the logarithm of the lane's target: as a target forward, as a source backward
-    if (wave == 0) lt[lane] = DIR == 0 ? log((double)(n0 + tl)) : sh.lq[lane];
-    const double u0 = DIR == 0 ? 0.0 : log((double)N);
-    const RecTarget<D> tg = xw_target<DIR, D>(sh, N, n0 + tl);
-    __syncthreads();
-    const double lg = DIR == 0 ? lt[lane] : 0.0;
-    double m = INFINITY, s = 0.0;
-    auto add = [&](int q, double uq) {
-        const double y = xw_w<DIR, D>(sh, r, bk, N, tg, q) + lg + uq;
-        const double mn = fmin(m, y);
-        s = fma(s, exp_pair(mn - m), exp_pair(mn - y));   // m = inf (first source): s = 0 stays 0
-        m = mn;
-    };
-    auto inblock = [&](int j, int t) {
-        const double w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j);
-        return w + lt[DIR == 0 ? t : j];
-    };
-    if (wave == 0) add(0, u0);
-    if (wave < SW) {
-        for (int J = 0; J < I; ++J) {
-            const double v = xw_wait(upub + J * REC_B + 1, lane, status);
-            for (int u = 0; u < SRC; ++u) add(J * REC_B + 1 + wave * SRC + u, wave_bcast_uniform(v, wave * SRC + u));
-        }
-        part[wave * REC_B + lane] = lane < nb ? m : INFINITY;
-    }
     for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
-        if (t >= 0) sh.a[rec_idx(j, t)] = t < nb ? inblock(j, t) : INFINITY;
+        if (t < 0) continue;
+        double w = INFINITY;
+        if (t < nb) w = xw_w<DIR, D>(sh, r, bk, N, xw_target<DIR, D>(sh, N, n0 + t), n0 + j) + sh.lq[DIR == 0 ? t : j];
+        sh.a[rec_idx(j, t)] = w;
     }
+}
+// forward: sh.lq holds the targets' logarithms.
+template <int NT>
+__device__ __noinline__ double xw_block_safe(bool forward, int nb, const XwShared sh, double m, double s) {
+    constexpr int NW = NT / WAVE;
+    double *R = sh.a + REC_TRI, *z = R + REC_B;   // (the triangle and these in the matrix's place)
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int tl = min(lane, nb - 1);
+    __syncthreads();   // (the partials are no longer read)
+    m += forward ? sh.lq[tl] : 0.0;
+    sh.psum[wave * REC_B + lane] = lane < nb ? m : INFINITY;
     __syncthreads();
     if (wave == 0) {
         double rr = INFINITY;
-        for (int w = 0; w < SW; ++w) rr = fmin(rr, part[w * REC_B + lane]);
+        for (int w = 0; w < NW; ++w) rr = fmin(rr, sh.psum[w * REC_B + lane]);
         rec_inblock_seq<0>(sh.a, lane, rr, R);
     }
     __syncthreads();
-    if (wave < SW) sh.psum[wave * REC_B + lane] = lane < nb && s > 0.0 ? s * exp_pair(R[lane] - m) : 0.0;
+    sh.psum[wave * REC_B + lane] = lane < nb && s > 0.0 ? s * exp_pair(R[lane] - m) : 0.0;
     for (int vr = wave; vr < REC_B / 2; vr += NW) {
         int t, j;
         rec_tri(vr, lane, t, j);
@@ -424,7 +417,7 @@ __device__ __noinline__ double xw_block_safe(int I, int N, int nb, double bk, co
     double u = 0.0;
     if (wave == 0) {
         double z0 = 0.0;
-        for (int w = 0; w < SW; ++w) z0 += sh.psum[w * REC_B + lane];
+        for (int w = 0; w < NW; ++w) z0 += sh.psum[w * REC_B + lane];
         rec_inblock_seq<1>(sh.a, lane, z0, z);
         u = R[lane] - log(z[lane]);
     }
@@ -615,8 +608,8 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
         m = xw_w<DIR, D>(sh, r, bk, N, tg, 0);
         s = DIR == 0 ? 1.0 : c0;   // (forward the target's factor comes last)
     }
-    double z, sigma = 0.0;      // wave 0: the lane's s_t, then z_t
-    bool known = I == 0;        // sigma is known
+    double z = 0.0, sigma = 0.0;   // wave 0: the lane's s_t, then z_t
+    bool safe = false;             // (uniform) the exact form
     if (I == 0) {
         z = s * cn * exp_pair(g - m);
         __syncthreads();
@@ -651,35 +644,41 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
             sh.psum[wave * REC_B + lane] = acc;
         }
         __syncthreads();
-        if (sh.flag[1]) {   // (uniform) the block before as a farther one
-            sigma = far(I - 1);
-            known = true;
-            sh.psum[wave * REC_B + lane] = s > 0.0 ? s * cn * exp_pair((sigma + g) - m) : 0.0;
-            __syncthreads();
+        if (sh.flag[1]) {   // (uniform) the block before left the range: this one will, too
+            if (wave == 0 && !last) __hip_atomic_store(zpub + n0 + lane, XW_BAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            xw_safe_weights<DIR, D, NT>(N, n0, nb, bk, r, sh);
+            far(I - 1);
+            safe = true;
+        } else {
+            const double* ps = sh.psum + lane;
+            z = (ps[0] + ps[REC_B]) + (ps[2 * REC_B] + ps[3 * REC_B]);
         }
-        const double* ps = sh.psum + lane;
-        z = (ps[0] + ps[REC_B]) + (ps[2 * REC_B] + ps[3 * REC_B]);
-        if (NW > ZW && sh.flag[1])
-            for (int w = ZW; w < NW; ++w) z += ps[w * REC_B];
     }
     double u = 0.0;
-    if (wave == 0) {
-        z = xw_substitute(sh.a, lane, nb, lane < nb ? z : 0.0);
-        const bool all = __all(lane >= nb || (z >= 1.0 / XW_RANGE && z <= XW_RANGE)) && !sh.flag[2];
-        if (!last) {
-            const unsigned long long b = all ? xw_bits(z) : XW_BAD;
-            __hip_atomic_store(zpub + n0 + lane, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!safe) {
+        if (wave == 0) {
+            z = xw_substitute(sh.a, lane, nb, lane < nb ? z : 0.0);
+            const bool all = __all(lane >= nb || (z >= 1.0 / XW_RANGE && z <= XW_RANGE)) && !sh.flag[2];
+            if (!last) {
+                const unsigned long long b = all ? xw_bits(z) : XW_BAD;
+                __hip_atomic_store(zpub + n0 + lane, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (I > 0) sigma = wave_bcast_uniform(xw_wait(upub + qn, lane, status), REC_B - 1);   // (all 64: see the reset below)
+            if (all) {
+                u = (sigma + g) - log(z);
+                if (!last) xw_publish(upub + n0 + lane, DIR == 0 ? u : u + sh.lq[lane]);
+            }
+            if (lane == 0) sh.flag[0] = all ? 0 : 1;
         }
-        if (!known) sigma = wave_bcast_uniform(xw_wait(upub + qn, lane, status), REC_B - 1);   // (all 64: see the reset below)
-        if (all) {
-            u = (sigma + g) - log(z);
-            if (!last) xw_publish(upub + n0 + lane, DIR == 0 ? u : u + sh.lq[lane]);
+        __syncthreads();
+        safe = sh.flag[0] != 0;
+        if (safe) {
+            xw_safe_weights<DIR, D, NT>(N, n0, nb, bk, r, sh);
+            if (I > 0) far(I - 1);
         }
-        if (lane == 0) sh.flag[0] = all ? 0 : 1;
     }
-    __syncthreads();
-    if (sh.flag[0]) {
-        u = xw_block_safe<DIR, D, NT>(I, N, nb, bk, r, sh, upub, status);
+    if (safe) {
+        u = xw_block_safe<NT>(DIR == 0, nb, sh, m, s);
         if (wave == 0) {
             if (lane < nb && !isfinite(u)) raise_status(status);
             if (!last) xw_publish(upub + n0 + lane, DIR == 0 ? u : u + sh.lq[lane]);
