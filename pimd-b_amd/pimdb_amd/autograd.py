@@ -11,6 +11,13 @@ import torch
 from . import XPlan
 
 
+def _in_memory(t):
+    """t with its values in its memory: a lazily negated view (the imaginary part of a conjugate) holds the opposite
+    ones there, and zeros that autograd makes may have no memory at all."""
+    t = t.resolve_neg()
+    return t.clone() if t._is_zerotensor() else t
+
+
 class ExchangeVB(torch.autograd.Function):
     """V_B(x1, xP) with its gradient from the adjoint kernel."""
 
@@ -20,6 +27,7 @@ class ExchangeVB(torch.autograd.Function):
             raise TypeError("ExchangeVB takes float64 CUDA tensors")
         if x1.shape != xP.shape or x1.dim() != 2 or x1.shape != (plan.natoms, plan.ndim):
             raise ValueError("x1 and xP must both have shape (%d, %d)" % (plan.natoms, plan.ndim))
+        x1, xP = _in_memory(x1), _in_memory(xP)
         vb = torch.empty((), dtype=torch.float64, device=x1.device)
         saved = torch.empty(plan.saved_doubles, dtype=torch.float64, device=x1.device)
         stream = torch.cuda.current_stream(x1.device).cuda_stream
@@ -36,6 +44,8 @@ class ExchangeVB(torch.autograd.Function):
         stream = torch.cuda.current_stream(saved.device).cuda_stream
         # the product with g stays a torch operation where it is to be differentiated itself
         inside = not torch.is_grad_enabled()
+        if inside:
+            g = _in_memory(g)
         plan.backward_saved(saved.data_ptr(), g.data_ptr() if inside else None, d1.data_ptr(), dP.data_ptr(), stream)
         return (d1, dP, None) if inside else (d1 * g, dP * g, None)
 
