@@ -42,12 +42,17 @@ class ExchangeVB(torch.autograd.Function):
         plan = ctx.plan
         d1, dP = (torch.empty((plan.natoms, plan.ndim), dtype=torch.float64, device=saved.device) for _ in range(2))
         stream = torch.cuda.current_stream(saved.device).cuda_stream
-        # the product with g stays a torch operation where it is to be differentiated itself
-        inside = not torch.is_grad_enabled()
-        if inside:
+        # the product with g stays a torch operation where it is to be differentiated itself, and where g is many
+        # gradients at once (is_grads_batched), which have no memory to read
+        scale = None
+        if not torch.is_grad_enabled():
             g = _in_memory(g)
-        plan.backward_saved(saved.data_ptr(), g.data_ptr() if inside else None, d1.data_ptr(), dP.data_ptr(), stream)
-        return (d1, dP, None) if inside else (d1 * g, dP * g, None)
+            try:
+                scale = g.data_ptr()
+            except RuntimeError:
+                pass
+        plan.backward_saved(saved.data_ptr(), scale, d1.data_ptr(), dP.data_ptr(), stream)
+        return (d1, dP, None) if scale is not None else (d1 * g, dP * g, None)
 
 
 def exchange_potential(x1, xP, plan):
