@@ -30,7 +30,8 @@ enum pimdb_status {
     PIMDB_OK = 0,
     PIMDB_E_NONFINITE = 1, /* exchange potential not finite (overflow_error) */
     PIMDB_E_ARG = 2,       /* invalid argument (invalid_argument)            */
-    PIMDB_E_HIP = 3,       /* HIP runtime failure or no GPU                   */
+    PIMDB_E_HIP = 3,       /* HIP runtime failure, no GPU, or a wait between
+                              workgroups of a kernel that ran out             */
     PIMDB_E_STATE = 4      /* call not valid in the current state             */
 };
 
@@ -181,6 +182,13 @@ int pimdb_device_info(int* compute_units, long long* lds_bytes);
  * C library's exp and sqrt, aziz.cpp:56-106, and draws its noise on the host,
  * random_mars.cpp:83-103). */
 int pimdb_math_probe(int fn, const double* x, double* y, long long n);
+/* For tests of the recovery from a wait between workgroups that ran out (the
+ * exchange recursions' blocks wait for each other, a few seconds at most):
+ * leave the object as such a kernel would and return what its call would,
+ * PIMDB_E_HIP. */
+int pimdb_test_lost_wait(pimdb_ctx* ctx);
+int pimdb_xplan_test_lost_wait(struct pimdb_xplan* plan);
+int pimdb_batch_test_lost_wait(struct pimdb_batch* batch);
 
 /* ---------------------------------------------------------------------- */
 /* Exchange on caller-provided device arrays (the autograd harness).       */

@@ -63,7 +63,7 @@ struct BatchPtrs {
     const RepDesc* reps;
     const int* sched;          // replicas of workgroup g: sched[sched_off[g] .. sched_off[g+1])
     const int* sched_off;
-    int* status;               // per replica: 1 when the exchange overflowed
+    int* status;               // per replica (raise_status)
     unsigned long long* ctl;   // [0] step counter, [1] finished-workgroup counter
     double* cmp;               // per replica [8]: pending COM momentum [0..3], known sum of p [4..7]
 };

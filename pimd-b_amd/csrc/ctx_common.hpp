@@ -372,6 +372,27 @@ inline void launch_exchange_recursions(int D, int N, double bt, double k, int pb
     }
 }
 
+// A raised flag (device_common.hpp) whose first byte tells a lost wait.
+inline bool lost_wait(int status) { return (status & 0xFF00) != 0; }
+constexpr int LOST_WAIT = 0x0100;
+constexpr const char* LOST_WAIT_MESSAGE = "the exchange recursions' wait for an earlier block of the ring ran out";
+
+// Puts XW_EMPTY back into published words after a raised flag: a lost wait
+// leaves some of them filled, which the next launch would take for its own.
+// The stream is idle and is waited for.
+inline hipError_t empty_published(unsigned long long* pub, size_t words, hipStream_t s) {
+    if (!pub) return hipSuccess;
+    const hipError_t e = hipMemsetAsync(pub, 0xFF, 8 * words, s), w = hipStreamSynchronize(s);
+    return e == hipSuccess ? w : e;
+}
+// Published words as a lost wait may leave them, for tests of the recovery: of
+// other positions (0).
+inline hipError_t fill_published(unsigned long long* pub, size_t words, hipStream_t s) {
+    if (!pub) return hipSuccess;
+    const hipError_t e = hipMemsetAsync(pub, 0, 8 * words, s), w = hipStreamSynchronize(s);
+    return e == hipSuccess ? w : e;
+}
+
 // Status flags in pinned host memory (the host pointer serves the kernels
 // too), one per context or plan: slots of one page that the process keeps,
 // since a pinned allocation of its own costs 0.1 ms, and an allocation each

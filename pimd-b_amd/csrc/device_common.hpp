@@ -30,8 +30,10 @@ struct Aziz {
 };
 constexpr double HARD_CORE_EPS = 1.0E-7;   // include/common.h:193
 
-// Raises an error flag (device or pinned host memory; every writer stores 1).
-__device__ __forceinline__ void raise_status(int* status) { *(volatile int*)status = 1; }
+// Raises an error flag (device or pinned host memory), a byte per error: the
+// exchange potential is not finite, or a wait for another workgroup ran out.
+__device__ __forceinline__ void raise_status(int* status) { ((volatile unsigned char*)status)[0] = 1; }
+__device__ __forceinline__ void raise_lost_wait(int* status) { ((volatile unsigned char*)status)[1] = 1; }
 
 // dx - L floor(dx/L + 1/2), src/common.cpp:41-43.
 __device__ __forceinline__ double min_image(double dx, double L) {

@@ -59,7 +59,8 @@
 // patterns that no result carries): the value is its own flag, so no fence is
 // needed.  A workgroup waits only for lower-numbered ones, which are
 // dispatched first, and a wait ends after XW_SPIN polls at the latest (the
-// status flag is then set).  The last block's workgroup reads U of every block
+// flag of a lost wait is then set, and the host puts XW_EMPTY back,
+// empty_published).  The last block's workgroup reads U of every block
 // before it, each published after that block's own reads, so it puts XW_EMPTY
 // back for the next launch.
 #pragma once
@@ -351,6 +352,15 @@ __device__ __forceinline__ void xw_publish(unsigned long long* p, double v) {
     if (b == XW_EMPTY) b = 0x7FF8000000000000ull;
     __hip_atomic_store(p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Whether a wait ends after this many polls without its values: its own bound,
+// or the flag of another one that did (looked at every 1024 polls).
+__device__ __forceinline__ bool xw_give_up(long long polls, int* status) {
+    if (polls >= XW_SPIN) {
+        raise_lost_wait(status);
+        return true;
+    }
+    return polls % 1024 == 0 && (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) & 0xFF00) != 0;
+}
 // The 64 values of a finished block from p, one per lane (whole wave; p[at]
 // for the lane).
 __device__ __forceinline__ double xw_wait(unsigned long long* p, int at, int* status) {
@@ -361,10 +371,7 @@ __device__ __forceinline__ double xw_wait(unsigned long long* p, int at, int* st
     for (;;) {
         b = __hip_atomic_load(p + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__all(b != XW_EMPTY)) break;
-        if (++spin >= XW_SPIN) {
-            raise_status(status);
-            break;
-        }
+        if (xw_give_up(++spin, status)) break;
         __builtin_amdgcn_s_sleep(4);
     }
     return __longlong_as_double((long long)b);
@@ -514,8 +521,7 @@ __device__ __forceinline__ void xw_wait_z(unsigned long long* p, int row, int la
         b = __hip_atomic_load(p + 16 * row + lane % 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         e = __hip_atomic_load(p + REC_B - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__all(b != XW_EMPTY && e != XW_EMPTY)) break;
-        if (spin >= XW_SPIN) {
-            raise_status(status);
+        if (xw_give_up(spin + 1, status)) {
             b = e = XW_BAD;
             break;
         }

@@ -53,7 +53,8 @@ struct pimdb_batch {
     SplitPtrs sp{};
     std::vector<StepArgs> hsteps;
     double* d_split = nullptr;    // its workspace
-    unsigned long long* d_pub = nullptr;
+    unsigned long long* d_pub = nullptr;   // the recursions' published values of all replicas
+    size_t npub = 0;
     StepArgs* d_steps = nullptr;
     int2* d_maps = nullptr;
     std::string err;
@@ -337,6 +338,7 @@ static int build_split_buffers(pimdb_batch* b) {
         if (b->desc[r].bosonic) nw += xw_pub_words(p.natoms);
     }
     BCK(hipMalloc((void**)&b->d_split, nd * sizeof(double)));
+    b->npub = nw;
     if (nw) {
         BCK(hipMalloc((void**)&b->d_pub, nw * 8));
         BCK(hipMemset(b->d_pub, 0xFF, nw * 8));
@@ -492,7 +494,11 @@ static int check_batch_status(pimdb_batch* b) {
     BCK(hipMemcpy(st.data(), b->bp.status, sizeof(int) * b->R, hipMemcpyDeviceToHost));
     for (int r = 0; r < b->R; ++r) {
         if (st[r]) {
+            bool lost = false;
+            for (int s : st) lost = lost || lost_wait(s);
             BCK(hipMemset(b->bp.status, 0, sizeof(int) * b->R));
+            BCK(empty_published(b->d_pub, b->npub, b->s));
+            if (lost) return b->fail(PIMDB_E_HIP, LOST_WAIT_MESSAGE);
             return b->fail(PIMDB_E_NONFINITE, "non-finite bosonic exchange potential in replica " + std::to_string(r));
         }
     }
@@ -727,6 +733,14 @@ static int finish_pending(pimdb_batch* b) {
 }
 
 extern "C" {
+
+int pimdb_batch_test_lost_wait(pimdb_batch* b) {
+    if (!b) return PIMDB_E_ARG;
+    BCK(fill_published(b->d_pub, b->npub, b->s));
+    const int st = LOST_WAIT;
+    BCK(hipMemcpy(b->bp.status, &st, sizeof(int), hipMemcpyHostToDevice));
+    return check_batch_status(b);
+}
 
 int pimdb_batch_set_state(pimdb_batch* b, int rep, const double* x, const double* p) {
     if (!b || rep < 0 || rep >= b->R) return PIMDB_E_ARG;

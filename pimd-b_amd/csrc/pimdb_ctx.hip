@@ -620,8 +620,10 @@ static void launch_observe_d(pimdb_ctx* ctx) {
 // through, so looking at it takes no copy.
 static int check_status(pimdb_ctx* ctx) {
     CK(hipStreamSynchronize(ctx->s0));
-    if (*(volatile int*)ctx->status) {
+    if (const int st = *(volatile int*)ctx->status) {
         *(volatile int*)ctx->status = 0;
+        CK(empty_published(ctx->pub, xw_pub_words(ctx->N), ctx->s0));
+        if (lost_wait(st)) return ctx->fail(PIMDB_E_HIP, LOST_WAIT_MESSAGE);
         return ctx->fail(PIMDB_E_NONFINITE, "Invalid sig_denom in bosonic exchange potential (non-finite V)");
     }
     return PIMDB_OK;
@@ -803,6 +805,13 @@ void pimdb_ctx_destroy(pimdb_ctx* ctx) {
 }
 
 const char* pimdb_last_error(const pimdb_ctx* ctx) { return ctx ? ctx->err.c_str() : create_error(); }
+
+int pimdb_test_lost_wait(pimdb_ctx* ctx) {
+    if (!ctx) return PIMDB_E_ARG;
+    CK(fill_published(ctx->pub, xw_pub_words(ctx->N), ctx->s0));
+    *(volatile int*)ctx->status = LOST_WAIT;
+    return check_status(ctx);
+}
 
 int pimdb_set_state(pimdb_ctx* ctx, const double* x, const double* p) {
     if (!ctx) return PIMDB_E_ARG;

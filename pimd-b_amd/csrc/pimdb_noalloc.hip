@@ -114,6 +114,10 @@ extern "C" int pimdb_exchange_vb_grad_noalloc(int natoms, int ndim, double beta_
     int st = 0;
     if (hipMemcpyAsync(&st, flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess) return PIMDB_E_HIP;
     if (hipStreamSynchronize(s) != hipSuccess) return PIMDB_E_HIP;
+    if (lost_wait(st)) {
+        set_create_error(std::string("pimdb_exchange_vb_grad_noalloc: ") + LOST_WAIT_MESSAGE);
+        return PIMDB_E_HIP;
+    }
     if (st) {
         set_create_error("pimdb_exchange_vb_grad_noalloc: non-finite bosonic exchange potential");
         return PIMDB_E_NONFINITE;

@@ -29,9 +29,10 @@ static int xplan_recursions(pimdb_xplan* pl, const double* x1, const double* xP,
 // Waits for the stream and looks at the overflow flag (pinned host memory).
 static int xplan_finish(pimdb_xplan* pl, hipStream_t s) {
     if (hipStreamSynchronize(s) != hipSuccess) return PIMDB_E_HIP;
-    if (*(volatile int*)pl->status) {
+    if (const int st = *(volatile int*)pl->status) {
         *(volatile int*)pl->status = 0;
-        return PIMDB_E_NONFINITE;
+        if (empty_published(pl->pub, xw_pub_words(pl->N), s) != hipSuccess) return PIMDB_E_HIP;
+        return lost_wait(st) ? PIMDB_E_HIP : PIMDB_E_NONFINITE;
     }
     return PIMDB_OK;
 }
@@ -88,6 +89,13 @@ void pimdb_xplan_destroy(pimdb_xplan* pl) {
     if (pl->V) (void)hipFree(pl->V);
     status_pool().give(pl->status);
     delete pl;
+}
+
+int pimdb_xplan_test_lost_wait(pimdb_xplan* pl) {
+    if (!pl) return PIMDB_E_ARG;
+    if (fill_published(pl->pub, xw_pub_words(pl->N), nullptr) != hipSuccess) return PIMDB_E_HIP;
+    *(volatile int*)pl->status = LOST_WAIT;
+    return xplan_finish(pl, nullptr);
 }
 
 int pimdb_xplan_forward(pimdb_xplan* pl, const double* x1, const double* xP, double* VB, double* V, double* Vb,

@@ -97,6 +97,9 @@ def lib():
         "pimdb_peak_probe": (i, [_DP, _DP, _DP, C.c_longlong]),
         "pimdb_math_probe": (i, [i, _DP, _DP, C.c_longlong]),
         "pimdb_device_info": (i, [C.POINTER(i), C.POINTER(C.c_longlong)]),
+        "pimdb_test_lost_wait": (i, [vp]),
+        "pimdb_xplan_test_lost_wait": (i, [vp]),
+        "pimdb_batch_test_lost_wait": (i, [vp]),
         "pimdb_xplan_create": (i, [i, i, d, d, i, d, C.POINTER(vp)]),
         "pimdb_xplan_destroy": (None, [vp]),
         "pimdb_xplan_forward": (i, [vp, vp, vp, vp, vp, vp, vp]),
