@@ -57,12 +57,22 @@
 // go to global arrays by relaxed device-scope atomic stores and are read by
 // relaxed device-scope atomic loads until they differ from XW_EMPTY (NaN
 // patterns that no result carries): the value is its own flag, so no fence is
-// needed.  A workgroup waits only for lower-numbered ones, which are
-// dispatched first, and a wait ends after XW_SPIN polls at the latest (the
-// flag of a lost wait is then set, and the host puts XW_EMPTY back,
-// empty_published).  The last block's workgroup reads U of every block
+// needed.  A wait ends after XW_SPIN polls at the latest (the flag of a lost
+// wait is then set, and the host puts XW_EMPTY back, empty_published).  The last
+// block's workgroup reads U of every block
 // before it, each published after that block's own reads, so it puts XW_EMPTY
 // back for the next launch.
+//
+// Progress.  A workgroup's block is its place in the order in which the
+// workgroups started (xw_place), not its index in the grid, and it waits only for
+// lower places.  So whatever it waits for is running already and waits only for
+// still lower ones: launches of other streams or processes that hold compute
+// units can delay a ring, but no set of waiting workgroups can keep each other's
+// predecessors out, as they could where the dies start a grid's workgroups
+// independently of each other.  The place costs an atomic per workgroup, 1 - 2 us
+// where the chain is the longest part (the differentiable exchange of N=500 140.7
+// -> 143.5 us a call, the observables of N=256 50.1 -> 50.9) and nothing where
+// other work covers it (a helium step of N=256 or N=1000).
 #pragma once
 
 #include "exchange.hpp"
@@ -77,9 +87,26 @@ constexpr unsigned long long XW_EMPTY = ~0ull, XW_BAD = ~1ull;
 constexpr double XW_RANGE = 1e140;
 constexpr long long XW_SPIN = 1ll << 22;             // polls of one wait (seconds)
 
-// Global workspace of one ring: z and U of both directions.
-__host__ __device__ inline size_t xw_pub_words(int N) { return 4 * ((size_t)N + 1); }
+// Global workspace of one ring: z and U of both directions, then the counter of
+// xw_place.
+__host__ __device__ inline size_t xw_places_word(int N) { return 4 * ((size_t)N + 1); }
+__host__ __device__ inline size_t xw_pub_words(int N) { return xw_places_word(N) + 1; }
 __host__ __device__ inline int xw_grid(int N) { return 2 * rec_blocks(N); }
+
+// The place of this workgroup, one of n, among those of the launch in the order
+// of their start.  counter: all bits set (XW_EMPTY) or as n such workgroups leave
+// it (each launch of n counts from n - 1 round to n - 1).  lds: any word, free
+// again on return.
+__device__ __forceinline__ int xw_place(unsigned long long* counter, int n, double* lds) {
+    if (threadIdx.x == 0) {
+        const unsigned c = atomicInc((unsigned*)counter, (unsigned)(n - 1));
+        *(volatile int*)lds = c >= (unsigned)(n - 1) ? 0 : (int)c + 1;
+    }
+    __syncthreads();
+    const int place = uni(*(volatile int*)lds);
+    __syncthreads();
+    return place;
+}
 
 // The in-block matrix by rows of 16 sources and, in a row, by target: entry
 // (j, t), 16 R <= j < 16 R + 16, t >= 16 R, at xw_b(j, t), so that a target's
@@ -710,9 +737,9 @@ __device__ __forceinline__ void xw_block(int I, int N, double bt, const Ring& r,
     }
 }
 
-// Workgroup b of xw_grid(N): block b / 2, forward (even) or backward (odd);
-// lower blocks first.  pub: xw_pub_words(N) words, all XW_EMPTY on entry and
-// on return.  Block 0's forward workgroup writes the prefix sums and, where
+// The workgroup in place b of xw_grid(N): block b / 2, forward (even) or backward
+// (odd); lower blocks first.  pub: xw_pub_words(N) words, all but the counter
+// XW_EMPTY on entry and on return.  Block 0's forward workgroup writes the prefix sums and, where
 // asked (xc, VB not null), the beads' copy and V[N].
 template <int D, int NT>
 __device__ __forceinline__ void xw_recursions(double* smem, int b, int N, double bt, double k, int pbc, double L,
@@ -733,13 +760,21 @@ __device__ __forceinline__ void xw_recursions(double* smem, int b, int N, double
     }
 }
 
+// The place of workgroup wg of a launch that xw_grid(N) workgroups of one ring
+// take part in (a single block waits for nothing).
+__device__ __forceinline__ int xw_ring_place(unsigned long long* pub, int N, int wg, double* lds) {
+    const int n = xw_grid(N);
+    return n > 2 ? xw_place(pub + xw_places_word(N), n, lds) : wg;
+}
+
 template <int D>
 static __global__ void __launch_bounds__(XW_THREADS)
 k_exchange_wide(int N, double bt, double k, int pbc, double L, BeadView x1, BeadView xP, double* __restrict__ V,
                 double* __restrict__ Vb, double* __restrict__ VB, double* __restrict__ Shi, double* __restrict__ Slo,
                 double* __restrict__ xc, unsigned long long* __restrict__ pub, int* __restrict__ status) {
     extern __shared__ __align__(16) double smem[];
-    xw_recursions<D, XW_THREADS>(smem, blockIdx.x, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status);
+    const int b = xw_ring_place(pub, N, blockIdx.x, smem);
+    xw_recursions<D, XW_THREADS>(smem, b, N, bt, k, pbc, L, x1, xP, V, Vb, VB, Shi, Slo, xc, pub, status);
 }
 
 }  // namespace pimdb

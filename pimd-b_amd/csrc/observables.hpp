@@ -83,7 +83,8 @@ static __global__ void __launch_bounds__(XW_THREADS) k_observe(ObserveArgs o) {
     extern __shared__ __align__(16) double smem[];
     const int wg = blockIdx.x, N = o.fa.N, P = o.fa.P;
     if (wg < o.nx) {
-        xw_recursions<D, XW_THREADS>(smem, wg, N, o.bt, o.fa.k_spring, o.fa.pbc, o.fa.L, BeadView{o.x, N, 1},
+        const int b = xw_ring_place(o.pub, N, wg, smem);
+        xw_recursions<D, XW_THREADS>(smem, b, N, o.bt, o.fa.k_spring, o.fa.pbc, o.fa.L, BeadView{o.x, N, 1},
                                      BeadView{o.x + (size_t)(P - 1) * D * N, N, 1}, o.V, o.Vb, nullptr, o.Shi, o.Slo,
                                      nullptr, o.pub, o.status);
     } else if (wg < o.nx + o.nf) {

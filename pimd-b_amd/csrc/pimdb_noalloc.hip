@@ -25,7 +25,7 @@ namespace {
 constexpr int NOALLOC_MAX_N = 2048;
 constexpr size_t NOALLOC_FLAG = 4 * (size_t)(NOALLOC_MAX_N + 1);
 constexpr size_t NOALLOC_PUB = NOALLOC_FLAG + 1;
-constexpr size_t NOALLOC_DOUBLES = NOALLOC_PUB + 4 * (size_t)(NOALLOC_MAX_N + 1);
+constexpr size_t NOALLOC_DOUBLES = NOALLOC_PUB + 4 * (size_t)(NOALLOC_MAX_N + 1) + 1;   // (xw_pub_words)
 
 __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 

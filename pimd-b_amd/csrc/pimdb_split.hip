@@ -10,8 +10,9 @@
 // exchange term (the recursions and the exterior forces do not share them,
 // about 80 us of one CU per replica against 1090 for its pairs).
 //
-// The recursions of all replicas come first, so that one waits only for
-// earlier workgroups of its own replica, then slices and noise tiles, the
+// The recursions of all replicas come first, those of several blocks in the
+// order of their start (xw_place), so that one waits only for running workgroups
+// of its own replica, then slices and noise tiles, the
 // longest first, so that the last round over the card is a short one.  Three
 // workgroups share a compute unit (44 KB of LDS, the ring of N=256), since the
 // noise no longer stages C^T (66 KB).  With these two and one particle a wave in
@@ -146,7 +147,9 @@ template <int D, int KIND>
 static __global__ void __launch_bounds__(SPLIT_THREADS, 4) k_split_forces(SplitPtrs sp, const int2* __restrict__ map,
                                                                         int only_noise, int mode) {
     extern __shared__ __align__(16) double smem[];
-    const int2 m = map[blockIdx.x];
+    int at = blockIdx.x;
+    if (!only_noise && at < sp.nwait) at = xw_place(sp.places, sp.nwait, smem);
+    const int2 m = map[at];
     const int ri = uni(m.x), id = uni(m.y);
     const StepArgs s = sp.steps[ri];   // (a copy: stores through it would make every use a load)
     const int N = s.fa.N, P = s.fa.P;

@@ -233,7 +233,7 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
     }
 }
 
-// Workgroup wg of xw_grid(N): the recursions (exchange_wide.hpp), with copies
+// The workgroup in place wg of xw_grid(N): the recursions (exchange_wide.hpp), with copies
 // of the beads that the exterior forces read after the positions moved on.
 template <int D, int NT>
 __device__ __forceinline__ void step_recursions(const StepArgs& s, int wg, double* smem) {
@@ -365,7 +365,7 @@ static __global__ void __launch_bounds__(XW_THREADS) k_step_forces(StepArgs s, i
     extern __shared__ __align__(16) double smem[];
     const int wg = blockIdx.x;
     if (wg < nx) {
-        step_recursions<D, XW_THREADS>(s, wg, smem);
+        step_recursions<D, XW_THREADS>(s, xw_ring_place(s.pub, s.fa.N, wg, smem), smem);
     } else if (wg < nx + nn) {
         step_noise<D, XW_THREADS>(s, mode, wg - nx, smem);
     } else {
