@@ -245,7 +245,7 @@ static __global__ void __launch_bounds__(SMALL_THREADS) k_small_steps(StepArgs s
         for (int k = 0; k < SMALL_EACH; ++k) {
             const int e = tid + k * SMALL_THREADS;
             if (e >= E) continue;
-            v[k] = fma(co.alpha, fma(co.beta, f[e], p[e]), H[e]);
+            v[k] = step_kept(co, fma(co.beta, f[e], p[e]), H[e]);
             const int ax = e % nc / N;
 #pragma unroll
             for (int a = 0; a < D; ++a) c[a] += a == ax ? v[k] : 0.0;

@@ -44,7 +44,7 @@ namespace pimdb {
 constexpr int STEP_TILE = 64;         // columns (one axis) per noise workgroup
 constexpr int STEP_NM_MAXP = 64;      // beads of the matrix-core noise transform
 
-// What an integration does: p' = alpha (p + beta f) + H - mean(...) + gamma f,
+// What an integration does: p' = a1 a2 (p + beta f) + H - mean(...) + gamma f,
 // then (but for CLOSE) x += dt/m p'.
 enum StepMode : int {
     STEP_OPEN = 0,    // O, zeroMomentum, B, A with complete forces
@@ -67,21 +67,25 @@ struct StepArgs {
     const double *Ct, *CTt, *rot;     // cart -> nm and nm -> cart transposed (CTt[k P + b]); free-ring rotation
     double* H;                        // [P][D][N]
     double* fpart;                    // [frows][D] partial sums of the external forces (null: none)
-    double* hpart;                    // [noise tiles][D] sums of alpha p + H
+    double* hpart;                    // [noise tiles][D] sums of a1 a2 p + H
     int frows;
     PairGroups pg;                    // G > 0: the pair forces by groups, f to be completed from pg.cpart
     unsigned long long* ctr;          // steps done
     uint32_t seed;
 };
 
+// a1, a2: the two O-steps' factors (1 for one that is not there), applied one
+// after the other: c1 c1 rounded once would be the same error in every step, and
+// add up over the momenta's memory of 2 / (gamma dt) steps.
 struct StepCoef {
-    double alpha, beta, gamma, k2, k1;   // H = c2 (k2 xi2 + k1 xi1)
+    double a1, a2, beta, gamma, k2, k1;   // H = c2 (k2 xi2 + k1 xi1)
 };
 __device__ __forceinline__ StepCoef step_coef(const StepArgs& s, int mode) {
-    if (mode == STEP_OPEN) return StepCoef{s.c1, 0.0, s.half_dt, 0.0, 1.0};
-    if (mode == STEP_FULL) return StepCoef{s.c1 * s.c1, s.half_dt, s.half_dt, s.c1, 1.0};
-    return StepCoef{s.c1, s.half_dt, 0.0, 1.0, 0.0};
+    if (mode == STEP_OPEN) return StepCoef{s.c1, 1.0, 0.0, s.half_dt, 0.0, 1.0};
+    if (mode == STEP_FULL) return StepCoef{s.c1, s.c1, s.half_dt, s.half_dt, s.c1, 1.0};
+    return StepCoef{s.c1, 1.0, s.half_dt, 0.0, 1.0, 0.0};
 }
+__device__ __forceinline__ double step_kept(const StepCoef& co, double p, double h) { return fma(co.a1, co.a2 * p, h); }
 
 __host__ __device__ inline int step_noise_tiles(int N) { return (N + STEP_TILE - 1) / STEP_TILE; }
 // Noise workgroups of a replica: none where nothing is drawn or summed.
@@ -98,7 +102,7 @@ __host__ __device__ inline size_t step_noise_lds_doubles(int P, bool nm) {
 typedef double step_v4d __attribute__((ext_vector_type(4)));
 
 // H of particles i0 .. i0+63 of axis a for all beads, and the tile's sum of
-// alpha p + H, by a workgroup of NT threads.  The noise has the keys of the
+// a1 a2 p + H, by a workgroup of NT threads.  The noise has the keys of the
 // single O-steps: modes (beads) 2m and 2m+1 of column (a, i) from one
 // Box-Muller pair, at the current step count with O-step 1 for a closing half
 // (xi2) and 0 for an opening one (xi1).  Normal-mode coupling: C^T on the
@@ -152,7 +156,7 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
                 if (2 * m + h < P) {
                     const size_t q = (size_t)(2 * m + h) * ncols + col;
                     s.H[q] = g[h];
-                    sum += fma(co.alpha, s.p[q], g[h]);
+                    sum += step_kept(co, s.p[q], g[h]);
                 }
             }
         }
@@ -216,7 +220,7 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
                 if (b < P && c < nc) {
                     const size_t q = (size_t)b * ncols + a * N + i0 + c;
                     s.H[q] = acc[v];
-                    sum += fma(co.alpha, s.p[q], acc[v]);
+                    sum += step_kept(co, s.p[q], acc[v]);
                 }
             }
         }
@@ -276,7 +280,7 @@ __device__ __forceinline__ void step_shift(const StepArgs& s, int mode, int wave
     if (s.fpart && mode != STEP_OPEN) {
         double u = 0.0;
         for (int r = lane; r < s.frows; r += WAVE) u += s.fpart[(size_t)r * D + wave];
-        t = fma(co.alpha * co.beta, u, t);
+        t = step_kept(co, co.beta * u, t);
     }
     t = wave_total(t);
     if (lane == 0) shift[wave] = t / (double)(s.fa.N * s.fa.P);
@@ -346,7 +350,7 @@ __device__ __forceinline__ void step_integrate(const StepArgs& s, int mode, int 
         s.f[e] = fv;
     }
     if (!mine || mode == STEP_FORCES) return;
-    double v = fma(co.alpha, fma(co.beta, fv, pv), hv);
+    double v = step_kept(co, fma(co.beta, fv, pv), hv);
     if (s.fixcom) v -= shift[ax];
     if (mode == STEP_CLOSE) {
         s.p[e] = v;
@@ -465,7 +469,7 @@ static __global__ void __launch_bounds__(256) k_step_modes(StepArgs s, int mode)
     for (int u = 0; u < EMAX; ++u) {
         const int e = tid + u * 256;
         if (e < Pp * MODE_COLS) {
-            double v = fma(co.alpha, fma(co.beta, fv[u], pv[u]), hv[u]);
+            double v = step_kept(co, fma(co.beta, fv[u], pv[u]), hv[u]);
             if (s.fixcom) v -= shift[a];
             in[e] = xv[u];
             in[Pp * MODE_COLS + e] = e / MODE_COLS < P ? fma(co.gamma, fv[u], v) : 0.0;
