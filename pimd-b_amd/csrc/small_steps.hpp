@@ -142,12 +142,12 @@ static __global__ void __launch_bounds__(SMALL_THREADS) k_small_steps(StepArgs s
             const int m = e / nc, col = e - m * nc;
             double g0 = 0.0, g1 = 0.0, h0, h1;
             if (mode != STEP_OPEN) {
-                gauss2<true>((uint32_t)e, step, 1u, 0u, s.seed, g0, g1);
+                gauss2<false>((uint32_t)e, step, 1u, 0u, s.seed, g0, g1);
                 g0 *= co.k2;
                 g1 *= co.k2;
             }
             if (mode != STEP_CLOSE) {
-                gauss2<true>((uint32_t)e, step, 0u, 0u, s.seed, h0, h1);
+                gauss2<false>((uint32_t)e, step, 0u, 0u, s.seed, h0, h1);
                 g0 += h0;
                 g1 += h1;
             }

@@ -111,6 +111,10 @@ typedef double step_v4d __attribute__((ext_vector_type(4)));
 template <int D, int NT>
 __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx, double* smem) {
     constexpr int NW = NT / WAVE;
+    // a single system's deviates are k_momenta's, with the correctly rounded
+    // quotient and root (N=64, P=64: 14.6 -> 14.9 us a step, N=256 the same), a
+    // batch's the persistent kernel's
+    constexpr bool FAST = NT != XW_THREADS;
     const StepCoef co = step_coef(s, mode);
     const int N = s.fa.N, P = s.fa.P, ncols = D * N;
     const int tiles = step_noise_tiles(N);
@@ -126,13 +130,13 @@ __device__ __forceinline__ void step_noise(const StepArgs& s, int mode, int idx,
         g0 = 0.0;
         g1 = 0.0;
         if (mode != STEP_OPEN) {
-            gauss2<true>(key, step, 1u, 0u, s.seed, g0, g1);
+            gauss2<FAST>(key, step, 1u, 0u, s.seed, g0, g1);
             g0 *= co.k2;
             g1 *= co.k2;
         }
         if (mode != STEP_CLOSE) {
             double h0, h1;
-            gauss2<true>(key, step, 0u, 0u, s.seed, h0, h1);
+            gauss2<FAST>(key, step, 0u, 0u, s.seed, h0, h1);
             g0 += h0;
             g1 += h1;
         }
