@@ -262,8 +262,12 @@ int pimdb_batch_step(pimdb_batch* batch, int nsteps);
  * workgroup) or, where that would leave compute units idle (few, uneven or
  * small replicas with the Langevin or no thermostat and the Cartesian
  * propagator), two kernels per step that spread every replica over the card.
- * pimdb_batch_create chooses by an estimate of both; this call chooses the
- * persistent kernel with the given shape.
+ * pimdb_batch_create chooses by an estimate of both.
+ * pimdb_batch_form tells the current form, and the waves that share a slice in
+ * the two-kernel one (1, 2 or 4); pimdb_batch_set_form changes it, PIMDB_E_ARG
+ * for two_kernel != 0 with a replica that does not take it.
+ * pimdb_batch_configure sets the shape of the persistent kernel and, unless
+ * both values are 0, chooses it.
  * Workgroup size of the persistent kernel (256, 512 or 1024; 0 keeps the
  * current one) and number of workgroups (0 keeps the current one; default
  * one of 1024 threads per compute unit, or two of 512 where there are more
@@ -271,6 +275,8 @@ int pimdb_batch_step(pimdb_batch* batch, int nsteps);
  * LDS, and every replica's phases are planned for that share (an exchange
  * workspace that does not fit goes to device memory, allocated here);
  * PIMDB_E_ARG (the previous shape kept) when some replica does not fit it. */
+int pimdb_batch_form(const pimdb_batch* batch, int* two_kernel, int* slice_waves);
+int pimdb_batch_set_form(pimdb_batch* batch, int two_kernel);
 int pimdb_batch_configure(pimdb_batch* batch, int threads, int resident);
 /* Times trial_steps steps for each launch shape (256, 512 or 1024 threads,
  * 1, 2 or 4 workgroups per compute unit, at most 1024 threads per CU) whose

@@ -844,7 +844,7 @@ int pimdb_batch_configure(pimdb_batch* b, int threads, int resident) {
     if (threads) b->threads = threads;
     if (resident) b->resident = resident;
     const bool split = b->split;
-    b->split = false;   // an explicit shape is the persistent kernel's
+    if (threads || resident) b->split = false;   // an explicit shape is the persistent kernel's
     const int rc = upload_schedule(b);
     if (rc == PIMDB_E_ARG) {   // this shape's LDS plan does not fit: keep the previous one
         const std::string why = b->err;
@@ -856,6 +856,24 @@ int pimdb_batch_configure(pimdb_batch* b, int threads, int resident) {
         return b->fail(PIMDB_E_ARG, why);
     }
     return rc;
+}
+
+int pimdb_batch_form(const pimdb_batch* b, int* two_kernel, int* slice_waves) {
+    if (!b) return PIMDB_E_ARG;
+    if (two_kernel) *two_kernel = b->split ? 1 : 0;
+    if (slice_waves) *slice_waves = b->split ? b->sp.share : 1;
+    return PIMDB_OK;
+}
+
+int pimdb_batch_set_form(pimdb_batch* b, int two_kernel) {
+    if (!b) return PIMDB_E_ARG;
+    if (two_kernel) {
+        if (!split_able(b)) return b->fail(PIMDB_E_ARG, "a replica does not take the two-kernel form");
+        const int rc = build_split(b);
+        if (rc) return rc;
+    }
+    b->split = two_kernel != 0;
+    return PIMDB_OK;
 }
 
 int pimdb_batch_time_step(pimdb_batch* b, int reps, double* ms_step) {

@@ -115,6 +115,8 @@ def lib():
         "pimdb_batch_get_state": (i, [vp, i, _DP, _DP, _DP]),
         "pimdb_batch_forces": (i, [vp]),
         "pimdb_batch_step": (i, [vp, i]),
+        "pimdb_batch_form": (i, [vp, C.POINTER(i), C.POINTER(i)]),
+        "pimdb_batch_set_form": (i, [vp, i]),
         "pimdb_batch_configure": (i, [vp, i, i]),
         "pimdb_batch_autotune": (i, [vp, i, C.POINTER(i), C.POINTER(i)]),
         "pimdb_batch_time_step": (i, [vp, i, _DP]),
@@ -274,6 +276,15 @@ class Batch:
 
     def step(self, nsteps=1):
         self._chk(lib().pimdb_batch_step(self.h, int(nsteps)))
+
+    def form(self):
+        """Whether steps take the two-kernel form, and the waves that share a slice there."""
+        t, w = C.c_int(), C.c_int()
+        self._chk(lib().pimdb_batch_form(self.h, C.byref(t), C.byref(w)))
+        return bool(t.value), w.value
+
+    def set_form(self, two_kernel):
+        self._chk(lib().pimdb_batch_set_form(self.h, int(two_kernel)))
 
     def configure(self, threads=0, resident=0):
         self._chk(lib().pimdb_batch_configure(self.h, int(threads), int(resident)))
