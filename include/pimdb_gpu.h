@@ -281,8 +281,9 @@ int pimdb_batch_configure(pimdb_batch* batch, int threads, int resident);
 /* Times trial_steps steps for each launch shape (256, 512 or 1024 threads,
  * 1, 2 or 4 workgroups per compute unit, at most 1024 threads per CU) whose
  * LDS plan fits, and the two-kernel form where it applies, keeps the fastest
- * and restores the state it started from.  The two-kernel form is reported as
- * 256 threads and the number of workgroups of its forces kernel. */
+ * and restores the state it started from.  The outputs are the persistent
+ * kernel's fastest shape, also where the two-kernel form is faster
+ * (pimdb_batch_form). */
 int pimdb_batch_autotune(pimdb_batch* batch, int trial_steps, int* threads_out, int* resident_out);
 /* nsteps MD steps of every replica, as pimdb_batch_step, with the device
  * time between events recorded on the batch's stream just before the first

@@ -1026,8 +1026,8 @@ int pimdb_batch_autotune(pimdb_batch* b, int trial_steps, int* threads_out, int*
     if (sfx) (void)hipFree(sfx);
     b->maybe_pending = pending;   // as the restored momenta are
     b->unsettled = true;
-    if (threads_out) *threads_out = b->split ? SPLIT_THREADS : b->threads;
-    if (resident_out) *resident_out = b->split ? b->sp.nforces : b->resident;
+    if (threads_out) *threads_out = b->threads;
+    if (resident_out) *resident_out = b->resident;
     return rc;
 }
 

@@ -1,6 +1,6 @@
 """Which form a batch steps in (the persistent kernel or two kernels a step):
 the default of batches far on either side of the choice, the waves per slice,
-what configure leaves, and both forms asked for by name, which
+what configure and the autotuner leave, and both forms asked for by name, which
 agree to rounding as in test_gpu_steps.  And single systems with a handful of
 particles that the one-workgroup form does not take, in their two kernels.
 """
@@ -45,7 +45,7 @@ def test_refused():
     b.close()
 
 
-def test_configure():
+def test_configure_and_autotune():
     systems = few()
     b = make(systems)
     assert b.form()[0]
@@ -54,7 +54,9 @@ def test_configure():
     with pytest.raises(G.PimdbError):
         b.configure(100, 0)
     assert b.form()[0]
-    b.configure(512, 0)
+    threads, resident = b.autotune(2)
+    assert threads in (256, 512, 1024) and 0 < resident <= 4 * G.device_cus()
+    b.configure(threads, resident)
     assert not b.form()[0]
     b.configure()
     assert not b.form()[0]
