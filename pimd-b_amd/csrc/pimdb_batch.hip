@@ -70,34 +70,40 @@ struct pimdb_batch {
         if (e_ != hipSuccess) return b->fail(PIMDB_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// Microseconds of one compute unit that a replica's step takes, fitted to both
-// forms at N = 8 .. 256, P = 8 .. 64, free, dipole and helium pairs, with and
-// without normal-mode coupling (split within about 15%, persistent 25%).
-// Pairs: 64-particle tiles, ns per pair; persistent: a fixed 55 us of barriers
-// and phase starts; split: the recursions' blocks, each a workgroup with waits
-// of its own, instead.
-static double pair_us(const pimdb_params& p) {
-    static const double ns[4] = {0.0, 0.2, 0.3, 0.55};   // free, harmonic, dipole, Aziz
-    const double T = (p.natoms + PTILE - 1) / PTILE;
-    return p.nbeads * (T * PTILE) * (T * PTILE) * 0.5e-3 * ns[p.int_kind & 3];
-}
-static double rep_cost(const pimdb_params& p) {
-    const double N = p.natoms, nd = N * p.nbeads * p.ndim;
-    return 55.0 + 0.004 * nd + (p.bosonic && p.nbeads > 1 ? 10.0 + 9e-4 * N * N : 0.0) + pair_us(p);
-}
-// Steps of the pair walk (two rows per lane) over one slice, and the
-// microseconds that a step costs one compute unit when the card is full.
+// Cost estimates in microseconds, fitted to 800 random batches (N = 3 .. 300, P = 2 .. 64, 2 .. 2000 replicas, every pair kind and
+// dimension; rings mostly without exchange, which costs the two-kernel form up to
+// a third more): 0.7 - 1.3 of the measured times in nine of ten.
+//
+// Steps of the pair walk (two rows per lane) over one slice; a step's cost in
+// units of `us`, per axis where the pair's arithmetic is short.
 static double walk_steps(const pimdb_params& p) {
     const int T = (p.natoms + PTILE - 1) / PTILE;
     return 17.0 * T + PTILE / 4 * T * (T - 1);
 }
-static double walk_step_us(const pimdb_params& p) {
-    return p.int_kind == PIMDB_POT_FREE ? 0.0 : p.int_kind == PIMDB_POT_AZIZ ? 0.06 : 0.018;
+static double walk_us(const pimdb_params& p, double harmonic, double dipole, double aziz) {
+    const double us = p.int_kind == PIMDB_POT_HARMONIC ? harmonic * p.ndim : p.int_kind == PIMDB_POT_DIPOLE ? dipole * p.ndim :
+                      p.int_kind == PIMDB_POT_AZIZ ? aziz : 0.0;
+    return us * walk_steps(p);
 }
+// A replica's step on a compute unit in the persistent kernel, with 16 waves a
+// workgroup or less (two workgroups of 8 waves a unit).  The beads take the waves
+// in whole rounds.
+static double rep_cost(const pimdb_params& p, int waves) {
+    const double N = p.natoms, P = p.nbeads, T = (p.natoms + PTILE - 1) / PTILE;
+    const double rounds = (double)((p.nbeads + waves - 1) / waves) * waves;
+    const bool ring = p.bosonic && p.nbeads > 1;
+    if (waves >= 16)
+        return 26.0 + 0.0057 * N * P * p.ndim + (p.nmthermostat ? 0.0013 * P * p.ndim * PTILE * T : 0.0) +
+               (ring ? 11.0 + 8.0 * T + 1e-4 * N * N : 0.0) + rounds * walk_us(p, 0.0062, 0.0093, 0.052);
+    return 14.0 + 0.0075 * N * P * p.ndim + (ring ? 6.0 + 5.3 * T + 2.4e-4 * N * N : 0.0) +
+           rounds * walk_us(p, 0.0055, 0.0089, 0.059);
+}
+// The same in the two-kernel form.  N^2: the exterior forces.
 static double rep_cost_split(const pimdb_params& p) {
-    const double T = (p.natoms + PTILE - 1) / PTILE, nd = (double)p.natoms * p.nbeads * p.ndim;
-    return 0.0079 * nd + (p.nmthermostat ? 0.0013 * p.nbeads * p.ndim * PTILE * T : 0.0) +
-           (p.bosonic && p.nbeads > 1 ? 14.0 * T : 0.0) + p.nbeads * walk_steps(p) * walk_step_us(p);
+    const double N = p.natoms, P = p.nbeads, T = (p.natoms + PTILE - 1) / PTILE;
+    return 0.008 * N * P * p.ndim + (p.nmthermostat ? 0.0012 * P * p.ndim * PTILE * T : 0.0) +
+           (p.bosonic && p.nbeads > 1 ? 7.5 * T + 2.8e-3 * N * N : 0.0) + 0.08 * P * T + 1.7 * p.ndim * T +
+           P * walk_us(p, 0.006, 0.0098, 0.077);
 }
 
 // Longest-processing-time-first assignment of replicas to `grid` workgroups.
@@ -105,7 +111,7 @@ static void build_schedule(pimdb_batch* b, std::vector<int>& sched, std::vector<
     std::vector<int> order(b->R);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int c) { return rep_cost(b->prm[a]) > rep_cost(b->prm[c]); });
+                     [&](int a, int c) { return rep_cost(b->prm[a], b->threads / WAVE) > rep_cost(b->prm[c], b->threads / WAVE); });
     using Item = std::pair<double, int>;
     std::priority_queue<Item, std::vector<Item>, std::greater<Item>> heap;
     for (int g = 0; g < b->grid; ++g) heap.push({0.0, g});
@@ -114,7 +120,7 @@ static void build_schedule(pimdb_batch* b, std::vector<int>& sched, std::vector<
         Item it = heap.top();
         heap.pop();
         lists[it.second].push_back(r);
-        heap.push({it.first + rep_cost(b->prm[r]), it.second});
+        heap.push({it.first + rep_cost(b->prm[r], b->threads / WAVE), it.second});
     }
     sched.clear();
     off.assign(1, 0);
@@ -181,13 +187,15 @@ static size_t plan_lds(pimdb_batch* b, int threads, int per_cu, std::vector<RepD
     return sizeof(double) * (16 + need);
 }
 
-// The largest load of a workgroup (us) in a schedule of `grid` workgroups.
-static double makespan(const pimdb_batch* b, int grid) {
+// The largest load of a compute unit (us) in a schedule of the persistent
+// kernel over the card, and the longest replica's.
+static double makespan(const pimdb_batch* b, int waves, double* longest = nullptr) {
     std::vector<double> c;
-    for (const pimdb_params& p : b->prm) c.push_back(rep_cost(p));
+    for (const pimdb_params& p : b->prm) c.push_back(rep_cost(p, waves));
     std::sort(c.rbegin(), c.rend());
+    if (longest) *longest = c[0];
     std::priority_queue<double, std::vector<double>, std::greater<double>> heap;
-    for (int g = 0; g < grid; ++g) heap.push(0.0);
+    for (int g = 0; g < std::min(b->R, b->cus); ++g) heap.push(0.0);
     double most = 0.0;
     for (double x : c) {
         const double t = heap.top() + x;
@@ -322,7 +330,8 @@ static void free_split(pimdb_batch* b) {
 // About how long a slice and a noise workgroup of the two-kernel form take (a
 // walk step of one of twelve waves on a compute unit, two draws per four beads).
 static double slice_wg_us(const pimdb_params& p, int share) {
-    return 3.0 + 12.0 * walk_step_us(p) * walk_steps(p) / share;
+    const double us = p.int_kind == PIMDB_POT_FREE ? 0.0 : p.int_kind == PIMDB_POT_AZIZ ? 0.06 : 0.018;
+    return 3.0 + 12.0 * us * walk_steps(p) / share;
 }
 static double noise_wg_us(const pimdb_params& p) { return 2.0 + 0.2 * p.nbeads; }
 
@@ -510,19 +519,22 @@ static int check_batch_status(pimdb_batch* b) {
     return PIMDB_OK;
 }
 
-// Launch shape and form of a new batch.  More replicas than compute units: two
-// workgroups of 512 threads per CU overlap each other's latencies (512
-// replicas: 8 - 33% faster than one of 1024 at every size tried), where their
-// LDS plan keeps every exchange workspace and force array in LDS.  The
-// two-kernel form where its load over the whole card is below the persistent
-// kernel's longest workgroup: fewer replicas than compute units (16 helium
-// replicas of N=256, P=64: 122 against 1240 us a step, 128 of them 716 against
-// 1278, but 256 of them 1486 against 1335), uneven ones, and small ones (512
-// uneven dipole replicas 210 against 277 us, 256 helium replicas of N=30, P=32
-// 104 against 133).
+// Launch shape and form of a new batch, from the estimates above.
+// More replicas than compute units: two workgroups of 512 threads per CU overlap
+// each other's latencies (8 - 33% faster than one of 1024), where their LDS plan
+// keeps every exchange workspace and force array in LDS and the longest replica,
+// which 512 threads take longer for, does not bound the whole (312 uneven
+// harmonic replicas of N <= 158, P <= 16: 185 us a step against 159).
+// The two-kernel form where it is not estimated more than a twentieth longer
+// than that.  Few replicas are many times faster in it (16 of helium, N=256,
+// P=64: 122 against 1240 us a step; 256 of them 1486 against 1335), uneven ones
+// faster (512 uneven dipole replicas 210 against 277), but hundreds of rings of
+// more than 64 particles with few beads slower, since each block of a ring is a
+// workgroup that waits (482 free ones of N=180, P=8: 233 against 100).  Of 600
+// other random batches 18 were more than 8% slower than in the better form.
 static int choose_form(pimdb_batch* b) {
-    double shape_gain = 1.0;
-    if (b->R > b->cus) {
+    double longest = 0.0, persistent = makespan(b, 1024 / WAVE, &longest);
+    if (b->R > b->cus && persistent > 1.3 * longest) {
         std::vector<RepDesc> one = b->desc, two = b->desc;
         std::vector<size_t> xdev(b->R, 0);
         std::string why;
@@ -532,15 +544,19 @@ static int choose_form(pimdb_batch* b) {
             if (same) {
                 b->threads = 512;
                 b->resident = 2 * b->cus;
-                shape_gain = 0.85;
+                persistent = makespan(b, 512 / WAVE);
             }
         }
     }
     const int rc = upload_schedule(b);
     if (rc || !split_able(b)) return rc;
-    double load = 0.0;
-    for (const pimdb_params& p : b->prm) load += rep_cost_split(p);
-    b->split = 22.0 + load / b->cus < 0.95 * shape_gain * makespan(b, std::min(b->R, b->cus));
+    double split = 0.0;
+    int blocks = 0;   // of the longest ring: its chain
+    for (int r = 0; r < b->R; ++r) {
+        split += rep_cost_split(b->prm[r]);
+        if (b->desc[r].bosonic) blocks = std::max(blocks, rec_blocks(b->prm[r].natoms));
+    }
+    b->split = 13.0 + 3.2 * blocks + split / b->cus < 1.05 * persistent;
     if (b->split && build_split(b) != PIMDB_OK) b->split = false;   // (no memory for its workspace)
     return PIMDB_OK;
 }

@@ -36,6 +36,24 @@ def test_default_and_waves(systems, waves):
     b.close()
 
 
+# (test_gpu_steps compares these with the persistent kernel)
+@pytest.mark.parametrize("mix", sorted(MIXES))
+@pytest.mark.parametrize("D", [2, 3])
+def test_default_of_the_mixes(mix, D):
+    b = make([system(N, P, D, 11 * r + N, **dict(kw, seed=50 + r)) for r, (N, P, kw) in enumerate(MIXES[mix])])
+    assert b.form()[0]
+    b.close()
+
+
+# hundreds of rings of several blocks with few beads
+@pytest.mark.parametrize("N,P,D,R", [(180, 8, 1, 400), (195, 8, 2, 500), (154, 2, 3, 500)])
+def test_default_of_many_rings(N, P, D, R):
+    kw, x, p = system(N, P, D, N, **TRAP)
+    b = G.Batch([G.make_params(**kw)] * R)
+    assert b.form() == (False, 1)
+    b.close()
+
+
 def test_refused():
     b = make(few(thermostat="nose_hoover_np"))
     assert b.form() == (False, 1)
