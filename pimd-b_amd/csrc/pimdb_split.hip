@@ -157,7 +157,7 @@ static __global__ void __launch_bounds__(SPLIT_THREADS, 4) k_split_forces(SplitP
     if (id < nx) {
         step_recursions<D, SPLIT_THREADS>(s, id, smem);
     } else if (id < nx + nn) {
-        step_noise<D, SPLIT_THREADS>(s, mode, id - nx, smem);
+        if (mode != STEP_FORCES) step_noise<D, SPLIT_THREADS>(s, mode, id - nx, smem);
     } else {
         split_slice<D, KIND>(sp.bp.reps[ri], sp.bp, smem, id - nx - nn, sp.share, split_slice_lds(N, D) <= sp.lds, s.fpart);
     }
