@@ -148,8 +148,8 @@ int pimdb_exchange_estimators(pimdb_ctx* ctx, double* prim, double* prob_distinc
  * counterpart (the reference has no graph capture). */
 int pimdb_graph_capture(pimdb_ctx* ctx);
 
-/* Average device time (ms) of `reps` launches of the physical-force kernel
- * of one force evaluation (ms_forces), of the exchange forward pass and
+/* Average device time (ms) of `reps` launches of the pair, external and spring
+ * forces as one force evaluation computes them (ms_forces), of the exchange forward pass and
  * exterior forces (ms_exchange) and of one MD step with device noise
  * (ms_step), measured with HIP events on the context stream; any output may
  * be NULL.  Side effects: the forces are recomputed from the current

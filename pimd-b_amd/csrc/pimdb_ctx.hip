@@ -249,9 +249,9 @@ static size_t tile_lds_bytes(int N, int D) {
 }
 
 template <int D>
-static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
+static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mode, bool ring) {
     const StepArgs a = step_args(ctx);
-    const int nx = forces && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = !forces ? 0 : a.pg.G ? a.pg.groups_of(ctx->P) : a.frows;
+    const int nx = forces && ring && ctx->dv.bosonic ? xw_grid(ctx->N) : 0, nf = !forces ? 0 : a.pg.G ? a.pg.groups_of(ctx->P) : a.frows;
     const int nn = noise ? step_noise_groups(a, D) : 0;
     if (nx + nf + nn == 0) return;
     size_t lds = 0;
@@ -269,12 +269,13 @@ static void launch_step_forces_d(pimdb_ctx* ctx, bool forces, bool noise, int mo
 }
 
 // The recursions and bead forces (forces: all but the exterior forces of beads
-// 1 and P) and the noise of the integration of this mode (noise).
-static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode) {
+// 1 and P) and the noise of the integration of this mode (noise).  ring false:
+// without the recursions.
+static void launch_step_forces(pimdb_ctx* ctx, bool forces, bool noise, int mode, bool ring = true) {
     switch (ctx->D) {
-    case 1: launch_step_forces_d<1>(ctx, forces, noise, mode); break;
-    case 2: launch_step_forces_d<2>(ctx, forces, noise, mode); break;
-    default: launch_step_forces_d<3>(ctx, forces, noise, mode); break;
+    case 1: launch_step_forces_d<1>(ctx, forces, noise, mode, ring); break;
+    case 2: launch_step_forces_d<2>(ctx, forces, noise, mode, ring); break;
+    default: launch_step_forces_d<3>(ctx, forces, noise, mode, ring); break;
     }
 }
 
@@ -1086,7 +1087,16 @@ int pimdb_time_kernels(pimdb_ctx* ctx, int reps, double* ms_forces, double* ms_e
     if (!ctx || reps < 1) return PIMDB_E_ARG;
     int rc = PIMDB_OK;
     if (ms_forces) {
-        rc = time_captured(ctx, reps, [&]() { launch_bead_forces(ctx, ctx->s0); return PIMDB_OK; }, ms_forces);
+        // what a force evaluation launches, without the exchange
+        rc = time_captured(ctx, reps, [&]() {
+            if (ctx->merged) {
+                launch_step_forces(ctx, true, false, STEP_CLOSE, false);
+                launch_pair_sum(ctx);
+            } else {
+                launch_bead_forces(ctx, ctx->s0);
+            }
+            return PIMDB_OK;
+        }, ms_forces);
         if (rc) return rc;
     }
     if (ms_exchange) {
@@ -1111,8 +1121,8 @@ int pimdb_time_kernels(pimdb_ctx* ctx, int reps, double* ms_forces, double* ms_e
         if (rc) return rc;
     }
     if (ms_step) {
-        // whole steps (device noise), as the benchmark replays them; this
-        // advances the state by 2 * reps steps
+        // whole steps (device noise), as pimdb_step launches them; this advances
+        // the state by 2 * reps steps
         hipGraphExec_t held = ctx->gexec;   // (a graph is not launched into a capture)
         ctx->gexec = nullptr;
         rc = time_captured(ctx, 1, [&]() { return enqueue_steps(ctx, reps); }, ms_step);
