@@ -160,10 +160,12 @@ k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f
 
 // Pair energy V and g with gradV = g d (harmonic.cpp:9-23, dipole.cpp:5-45,
 // aziz.cpp:18-106) from r^2, sharing the root, the exponentials and the
-// reciprocal powers; each elementary function within an ulp or so.
+// reciprocal powers; each elementary function within an ulp or so.  A distance
+// of 0, or one whose square overflows, gives what 1/r = inf or 0 does.
 template <int KIND>
 __device__ __forceinline__ void pair_energy_grad(double r2, double kpair, double strength, double& e, double& g) {
-    const double inv = rsqrt_refined(r2), norm = r2 * inv;
+    // (the refinement of an estimate of inf or 0 is NaN)
+    const double inv = r2 > 0.0 && r2 < INFINITY ? rsqrt_refined(r2) : __builtin_amdgcn_rsq(r2), norm = r2 * inv;
     if constexpr (KIND == POT_HARMONIC) {
         e = 0.5 * kpair * r2;
         g = kpair;
