@@ -207,6 +207,7 @@ class StagePool {
 
 public:
     static constexpr size_t CAP = (size_t)1 << 20;
+    StagePool() { idle.reserve(KEEP + 1); }   // (give allocates nothing)
     // a buffer of at least min(n, CAP) doubles and its size, or null
     std::pair<double*, size_t> take(size_t n) {
         size_t cap = LEAST;
