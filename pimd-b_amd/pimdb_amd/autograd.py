@@ -14,8 +14,7 @@ from . import XPlan
 def _in_memory(t):
     """t with its values in its memory: a lazily negated view (the imaginary part of a conjugate) holds the opposite
     ones there, and zeros that autograd makes may have no memory at all."""
-    t = t.resolve_neg()
-    return t.clone() if t._is_zerotensor() else t
+    return t.resolve_neg().clone() if t.is_neg() or t._is_zerotensor() else t
 
 
 class ExchangeVB(torch.autograd.Function):
