@@ -24,8 +24,6 @@ struct SplitPtrs {
     const int2* full_map;        // of k_split_integrate after forces
     const int2* open_map;        // and of an opening half
     int nforces, nnoise, nfull, nopen;
-    int nwait;                   // the first of forces_map: recursions of rings of several blocks
-    unsigned long long* places;  // their counter (xw_place)
     size_t lds;                  // dynamic LDS of k_split_forces
     int share;                   // waves per slice: 1, 2 or 4
 };

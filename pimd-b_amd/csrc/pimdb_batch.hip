@@ -346,7 +346,6 @@ static int build_split_buffers(pimdb_batch* b) {
         nd += 4 * D * N + (N + 1) + 2 * N + P * D * N + P * SPLIT_WAVES * D + D * (size_t)step_noise_tiles(p.natoms);
         if (b->desc[r].bosonic) nw += xw_pub_words(p.natoms);
     }
-    if (nw) nw += 1;   // the counter of their places, last
     BCK(hipMalloc((void**)&b->d_split, nd * sizeof(double)));
     b->npub = nw;
     if (nw) {
@@ -365,7 +364,6 @@ static int build_split_buffers(pimdb_batch* b) {
     while (fit && share < SPLIT_WAVES && beads * share < 8 * (size_t)b->cus) share *= 2;
     using Work = std::pair<double, int2>;
     std::vector<Work> rest;      // slices and noise, the longest first
-    std::vector<int2> alone;     // recursions of rings of one block
     std::vector<int2> maps[4];   // forces, noise, full, open
     size_t lds = 0, w = 0;
     b->hsteps.clear();
@@ -401,7 +399,7 @@ static int build_split_buffers(pimdb_batch* b) {
         a.seed = p.seed;
         b->hsteps.push_back(a);
         const int nx = d.bosonic ? xw_grid(p.natoms) : 0, ns = split_slices(p.nbeads, share), nn = step_noise_groups(a, D);
-        for (int i = 0; i < nx; ++i) (nx > 2 ? maps[0] : alone).push_back(int2{r, i});
+        for (int i = 0; i < nx; ++i) maps[0].push_back(int2{r, i});
         for (int i = nx; i < nx + nn; ++i) rest.push_back({noise_wg_us(p), int2{r, i}});
         for (int i = 0; i < ns; ++i) rest.push_back({slice_wg_us(p, share), int2{r, nx + nn + i}});
         for (int i = 0; i < nn; ++i) maps[1].push_back(int2{r, i});
@@ -412,9 +410,6 @@ static int build_split_buffers(pimdb_batch* b) {
         if (sl <= device_lds_limit()) lds = std::max(lds, sl);
         lds = std::max(lds, sizeof(double) * step_noise_lds_doubles<SPLIT_THREADS>(p.nbeads, a.thermostat && a.nm));
     }
-    b->sp.nwait = (int)maps[0].size();
-    b->sp.places = nw ? b->d_pub + nw - 1 : nullptr;
-    for (const int2& v : alone) maps[0].push_back(v);
     std::stable_sort(rest.begin(), rest.end(), [](const Work& a, const Work& c) { return a.first > c.first; });
     for (const Work& v : rest) maps[0].push_back(v.second);
     size_t nm = 0;

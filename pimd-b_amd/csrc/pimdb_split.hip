@@ -10,9 +10,8 @@
 // exchange term (the recursions and the exterior forces do not share them,
 // about 80 us of one CU per replica against 1090 for its pairs).
 //
-// The recursions of all replicas come first, those of several blocks in the
-// order of their start (xw_place), so that one waits only for running workgroups
-// of its own replica, then slices and noise tiles, the
+// The recursions of all replicas come first, a ring's blocks in the order of
+// their start (xw_place), then slices and noise tiles, the
 // longest first, so that the last round over the card is a short one.  Three
 // workgroups share a compute unit (44 KB of LDS, the ring of N=256), since the
 // noise no longer stages C^T (66 KB).  With these two and one particle a wave in
@@ -147,15 +146,13 @@ template <int D, int KIND>
 static __global__ void __launch_bounds__(SPLIT_THREADS, 4) k_split_forces(SplitPtrs sp, const int2* __restrict__ map,
                                                                         int only_noise, int mode) {
     extern __shared__ __align__(16) double smem[];
-    int at = blockIdx.x;
-    if (!only_noise && at < sp.nwait) at = xw_place(sp.places, sp.nwait, smem);
-    const int2 m = map[at];
+    const int2 m = map[blockIdx.x];
     const int ri = uni(m.x), id = uni(m.y);
     const StepArgs s = sp.steps[ri];   // (a copy: stores through it would make every use a load)
     const int N = s.fa.N, P = s.fa.P;
     const int nx = only_noise || !s.fa.bosonic ? 0 : xw_grid(N), nn = step_noise_groups(s, D);
     if (id < nx) {
-        step_recursions<D, SPLIT_THREADS>(s, id, smem);
+        step_recursions<D, SPLIT_THREADS>(s, xw_ring_place(s.pub, N, id, smem), smem);
     } else if (id < nx + nn) {
         if (mode != STEP_FORCES) step_noise<D, SPLIT_THREADS>(s, mode, id - nx, smem);
     } else {

@@ -6,11 +6,12 @@ whose kernels and inputs are the same: equal bits.
 import numpy as np
 import pytest
 
-import pimdb_amd as G
-from test_gpu_exchanging_rings import ring
+torch = pytest.importorskip("torch")   # (before the library, so that both share a HIP runtime)
+
+import pimdb_amd as G  # noqa: E402
+from test_gpu_exchanging_rings import ring  # noqa: E402
 
 pytestmark = pytest.mark.gpu
-
 
 LOST = 3   # PIMDB_E_HIP
 
@@ -61,7 +62,6 @@ def test_batch():
 
 
 def test_plan():
-    torch = pytest.importorskip("torch")
     from pimdb_amd.autograd import exchange_potential
     from test_gpu_autograd_saved import plan_for, ring as beads
     x1, xP = beads(300, 3, 1)
