@@ -9,7 +9,8 @@ rejection (raw uniform He at liquid density overlaps cores), replicated over
 beads; momenta Maxwell-Boltzmann at beta/P.  Device (Philox) noise.
 
 Forms measured:
-  plain    one system, one kernel per stage, captured as a hipGraph
+  plain    one system, two kernels per step (forces with the exchange
+           recursions and the noise; integration), launched directly
   batched  R independent replicas of the same workload in one persistent
            kernel per MD step (every replica starts from the same x and p and
            draws its own noise stream)
@@ -175,12 +176,12 @@ def bench_plain(kw, x, p, steps, warmup):
 
 
 def bench_batched(kw, x, p, replicas, steps, warmup, threads=0, resident=0, phases=True, run_length=0):
-    """R copies of the workload (distinct noise seeds) in the persistent
-    kernel.  Returns wall ms per batched step over the timed region, device ms
-    per launch from stream events around the same region, the launch shape,
-    finiteness, (optionally) per-phase device times and (optionally) the
-    device ms per launch of `steps` steps timed after `run_length` more steps
-    of evolution."""
+    """R copies of the workload (distinct noise seeds), in the form and launch
+    shape asked for or found by the autotuner.  Returns wall ms per batched step
+    over the timed region, device ms per step from stream events around the
+    same region, the persistent kernel's launch shape, finiteness, (optionally)
+    per-phase device times, (optionally) the device ms per step of `steps`
+    steps timed after `run_length` more steps of evolution, and the form."""
     params = []
     for r in range(replicas):
         k = dict(kw)
@@ -208,8 +209,9 @@ def bench_batched(kw, x, p, replicas, steps, warmup, threads=0, resident=0, phas
         later = b.step_timed(steps) / steps
     xs, _, fs = b.state(0)
     ok = bool(np.all(np.isfinite(xs)) and np.all(np.isfinite(fs)))
+    form = "two kernels a step" if b.form()[0] else "batched persistent kernel + hipGraph"
     b.close()
-    return (t1 - t0) / steps * 1e3, dev_ms / steps, tuned[0], tuned[1], ok, ph, later
+    return (t1 - t0) / steps * 1e3, dev_ms / steps, tuned[0], tuned[1], ok, ph, later, form
 
 
 def bench_uneven(steps, warmup):
@@ -223,10 +225,11 @@ def bench_uneven(steps, warmup):
     b.step(warmup)
     dev_ms = b.step_timed(steps) / steps
     finite = all(np.all(np.isfinite(b.state(r)[0])) for r in (0, len(reps) - 1))
+    form = "two kernels a step" if b.form()[0] else "batched persistent kernel + hipGraph"
     b.close()
     work = dict(replicas=len(reps), natoms_sum=int(sum(kw["natoms"] for kw, _, _ in reps)),
                 bead_particles=int(sum(kw["natoms"] * kw["nbeads"] for kw, _, _ in reps)))
-    return dict(value=len(reps) * 1e3 / dev_ms, unit="replica-steps/s", ms_per_step=dev_ms, steps=steps,
+    return dict(value=len(reps) * 1e3 / dev_ms, unit="replica-steps/s", ms_per_step=dev_ms, steps=steps, form=form,
                 batch_threads=threads, batch_grid=min(len(reps), resident), batch_resident=resident,
                 finite_state=bool(finite), workload="512 uneven replicas: N in {8..128}, P in {16,32,64}, "
                 "T in U[1,4] K, D=2, He-4, trap 3 meV + dipole pairs (strength U[0.5,2] a.u.), all pairs, "
@@ -318,7 +321,7 @@ def main():
 
     ms_plain, ms_forces, ms_exch, ms_step_graph = bench_plain(kw, x, p, args.plain_steps, 50)
     R = args.replicas
-    ms_batch, ms_launch, threads, resident, finite, phases, ms_later = bench_batched(
+    ms_batch, ms_launch, threads, resident, finite, phases, ms_later, form = bench_batched(
         kw, x, p, R, args.steps, args.warmup, args.threads, args.resident, not args.no_phases, args.run_length)
     value = R * 1e3 / ms_batch
     grid = min(R, resident)
@@ -370,7 +373,7 @@ def main():
                              "seeded uniform with a 2.2 A minimum-distance rejection, replicated over the "
                              "beads; every replica starts from the same x and p (Maxwell-Boltzmann) and "
                              "draws its own noise; timed from the start (warmup steps after it)",
-                    form="batched persistent kernel + hipGraph, %d replicas (value = replica-steps/s)" % R,
+                    form="%s, %d replicas (value = replica-steps/s)" % (form, R),
                     replicas=R, natoms=256, nbeads=64, pairs_per_step=n_pairs, pairs_in_cutoff=n_in,
                     batch_threads=threads, batch_grid=grid, batch_resident=resident),
         roofline=roofline,
@@ -380,7 +383,7 @@ def main():
             replica_steps_per_s=R * 1e3 / ms_later,
             note="the same batch timed again after the workload's run length (beads spread)"),
         plain=dict(steps_per_s=1e3 / ms_plain, ms_per_step=ms_plain, steps=args.plain_steps,
-                   form="one system, per-kernel launches replayed from a hipGraph",
+                   form="one system, two kernels a step, launched directly",
                    forces_kernel_ms=ms_forces, forces_kernel_tflops=achieved_f,
                    forces_kernel_frac=achieved_f / PEAK_FP64_TFLOPS, exchange_chain_ms=ms_exch,
                    step_graph_ms=ms_step_graph),

@@ -204,7 +204,9 @@ void pimdb_xplan_destroy(pimdb_xplan* plan);
 int pimdb_xplan_forward(pimdb_xplan* plan, const double* x1, const double* xP, double* VB, double* V,
                         double* Vb, void* stream);
 int pimdb_xplan_vb_grad(pimdb_xplan* plan, const double* x1, const double* xP, double* grad, void* stream);
-/* The pair for reverse-mode differentiation.  forward_saved reads particle i,
+/* A plan is used by one host thread at a time, as a context; its calls wait for
+ * their stream, but for backward_saved, which uses only its arguments.
+ * The pair for reverse-mode differentiation.  forward_saved reads particle i,
  * axis a of bead 1 at x1[i s1n + a s1d] (strides in doubles; xP alike), writes
  * V_B to VB and what the backward pass needs (V, Vb, the ring's prefix sums and
  * its own copy of the beads) to saved, pimdb_xplan_saved_doubles() doubles, and

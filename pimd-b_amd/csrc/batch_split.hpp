@@ -15,7 +15,7 @@ constexpr int SPLIT_THREADS = 256;
 constexpr int SPLIT_WAVES = SPLIT_THREADS / WAVE;
 
 // A workgroup's part of a forces launch: its replica and its index among the
-// replica's workgroups (recursions first, then slices, then noise).
+// replica's workgroups (recursions first, then noise, then slices).
 struct SplitPtrs {
     BatchPtrs bp;
     const StepArgs* steps;       // per replica

@@ -352,8 +352,8 @@ static int build_split_buffers(pimdb_batch* b) {
         BCK(hipMalloc((void**)&b->d_pub, nw * 8));
         BCK(hipMemset(b->d_pub, 0xFF, nw * 8));
     }
-    // waves per slice: enough of them for four per SIMD, where the slices alone
-    // are fewer and their force arrays fit the LDS
+    // waves per slice: enough of them for two per SIMD (8 per compute unit), where
+    // the slices alone are fewer and their force arrays fit the LDS
     size_t beads = 0;
     bool fit = true;
     for (const pimdb_params& p : b->prm) {

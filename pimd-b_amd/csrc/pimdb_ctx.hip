@@ -354,7 +354,6 @@ static size_t momenta_lds(pimdb_ctx* ctx) {
     return sizeof(double) * (2 * (size_t)ctx->P * ctx->tc + 256 / WAVE);
 }
 
-// One OBABO step; noise0/noise1: device noise of the two O-steps or null.
 // One Nose-Hoover O-step: the pending zeroMomentum (com_in), the half kick
 // (kick_f), the chains, the partial sums of the result (com_out).  Under
 // normal-mode coupling the chains act on the modes: transform (k_momenta
@@ -461,7 +460,8 @@ static void enqueue_close(pimdb_ctx* ctx, const double* noise1) {
     }
 }
 
-// One OBABO step; noise0/noise1: device noise of the two O-steps or null.
+// One OBABO step; noise0/noise1: host noise of the two O-steps, on the device, or
+// null for device noise.
 static int enqueue_step(pimdb_ctx* ctx, const double* noise0, const double* noise1) {
     enqueue_open(ctx, noise0);
     if (ctx->nh_close) {
@@ -589,7 +589,9 @@ static void launch_estimators(pimdb_ctx* ctx) {
     }
 }
 
-// Natoms that the reference-order estimator's workgroup held.
+// The exchange estimators' limit on natoms (about 20,000): what the workgroup of
+// their first form held.  The present kernels have none; larger rings stay
+// refused.
 static bool estimator_fits(int N) { return sizeof(double) * ((size_t)N + 1 + 16) <= device_lds_limit(); }
 
 template <int D>
@@ -979,7 +981,7 @@ int pimdb_observables(pimdb_ctx* ctx, double* out) {
     const size_t tail = obs_tail(N, P), all = obs_doubles(N, P);
     double* est = ctx->obs + tail;
     const bool ring = ctx->dv.bosonic && !factorial(ctx);
-    if (ring && !estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
+    if (ring && !estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the exchange estimators");
     if (ctx->merged) {
         switch (D) {
         case 1: launch_observe_d<1>(ctx); break;
@@ -1024,7 +1026,7 @@ int pimdb_exchange_estimators(pimdb_ctx* ctx, double* prim, double* prob_distinc
     if (factorial(ctx)) {
         launch_factorial(ctx, ctx->s0, nullptr, nullptr, nullptr, ctx->obs + tail);
     } else {
-        if (!estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the estimator workgroup");
+        if (!estimator_fits(N)) return ctx->fail(PIMDB_E_ARG, "natoms too large for the exchange estimators");
         launch_exchange_forward(ctx, ctx->s0);
         launch_estimators(ctx);
     }

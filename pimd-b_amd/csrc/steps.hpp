@@ -27,8 +27,9 @@
 //   only the integration needs them: it evaluates them itself.
 //
 // Forces kernel: workgroups take one of three parts, in this order: the
-// recursions (exchange_wide.hpp), the bead forces (forces.hpp or, batched,
-// batch.hpp), and tiles of H with the partial sums for the shift.  The
+// recursions (exchange_wide.hpp), tiles of H with the partial sums for the
+// shift, and the bead forces (forces.hpp, slice_groups.hpp or, batched,
+// pimdb_split.hip, where slices and tiles come longest first).  The
 // recursions' latency covers the rest of a single system up to about N = 500.
 // Integration kernel: the exterior forces and update of beads 1 and P, one
 // wave per particle and bead, and the update of the others, elementwise.
