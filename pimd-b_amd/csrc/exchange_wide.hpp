@@ -69,9 +69,9 @@
 // still lower ones: launches of other streams or processes that hold compute
 // units can delay a ring, but no set of waiting workgroups can keep each other's
 // predecessors out, as they could where the dies start a grid's workgroups
-// independently of each other.  The place costs an atomic per workgroup, 1 - 2 us
-// where the chain is the longest part (the differentiable exchange of N=500 140.7
-// -> 143.5 us a call, the observables of N=256 50.1 -> 50.9) and nothing where
+// independently of each other.  The place costs an atomic per workgroup, 0.6 us
+// where the chain is the longest part (V_B of N=65 20.4 -> 21.0 us a call, of
+// N=500 36.7 -> 37.3, the observables of N=256 50.1 -> 50.9) and nothing where
 // other work covers it (a helium step of N=256 or N=1000).
 #pragma once
 
