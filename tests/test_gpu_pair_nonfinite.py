@@ -31,6 +31,6 @@ def test_others_unaffected(N, kw):
         got = forces(kw, y)
         keep = np.arange(N) != j
         want = forces(dict(kw, natoms=N - 1), x[:, keep])
-        e = np.abs(got[:, keep] - want).max(axis=(1, 2)) / np.abs(want).max(axis=(1, 2))
-        assert np.all(e <= 1e-11), (j, value, e)
+        e = np.abs(got[1, keep] - want[1]).max() / np.abs(want[1]).max()   # (in the other beads it takes part)
+        assert e <= 1e-11, (j, value, e)
         assert not np.isfinite(got[1, j, 1])
