@@ -165,7 +165,11 @@ k_bead_forces(ForceArgs fa, const double* __restrict__ x, double* __restrict__ f
 template <int KIND>
 __device__ __forceinline__ void pair_energy_grad(double r2, double kpair, double strength, double& e, double& g) {
     // (the refinement of an estimate of inf or 0 is NaN)
-    const double inv = r2 > 0.0 && r2 < INFINITY ? rsqrt_refined(r2) : __builtin_amdgcn_rsq(r2), norm = r2 * inv;
+    double inv = rsqrt_refined(r2), norm = r2 * inv;
+    if (!__builtin_amdgcn_class(r2, 0x180)) {   // (positive, normal or not)
+        inv = __builtin_amdgcn_rsq(r2);
+        norm = r2;
+    }
     if constexpr (KIND == POT_HARMONIC) {
         e = 0.5 * kpair * r2;
         g = kpair;
@@ -243,12 +247,11 @@ __device__ __forceinline__ void bead_energies_tile(const ForceArgs& fa, int b, i
                     for (int a = 0; a < D; ++a) d[a] = disp_fast(sx[a * N + j], xi[a], pbc, fa.L, invL);
                     const double r2 = norm2<D>(d);
                     if (j > i && (all || r2 < fa.cut2)) {
-                        double e, g, xd = 0.0;
+                        double e, g;
                         pair_energy_grad<KIND>(r2, fa.int_k, fa.strength, e, g);
                         ipot += e;
 #pragma unroll
-                        for (int a = 0; a < D; ++a) xd = fma(xi[a], d[a], xd);
-                        vir = fma(g, xd, vir);
+                        for (int a = 0; a < D; ++a) vir = fma(xi[a], g * d[a], vir);
                     }
                 }
             }
