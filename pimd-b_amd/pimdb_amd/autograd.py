@@ -11,12 +11,6 @@ import torch
 from . import XPlan
 
 
-def _in_memory(t):
-    """t with its values in its memory: a lazily negated view (the imaginary part of a conjugate) holds the opposite
-    ones there, and zeros that autograd makes may have no memory at all."""
-    return t.resolve_neg().clone() if t.is_neg() or t._is_zerotensor() else t
-
-
 class ExchangeVB(torch.autograd.Function):
     """V_B(x1, xP) with its gradient from the adjoint kernel."""
 
@@ -26,7 +20,10 @@ class ExchangeVB(torch.autograd.Function):
             raise TypeError("ExchangeVB takes float64 CUDA tensors")
         if x1.shape != xP.shape or x1.dim() != 2 or x1.shape != (plan.natoms, plan.ndim):
             raise ValueError("x1 and xP must both have shape (%d, %d)" % (plan.natoms, plan.ndim))
-        x1, xP = _in_memory(x1), _in_memory(xP)
+        # the values in memory: a lazily negated view (the imaginary part of a conjugate) holds the opposite ones
+        # there, and zeros that autograd makes have no memory at all
+        if x1.is_neg() or xP.is_neg() or not (x1.data_ptr() and xP.data_ptr()):
+            x1, xP = x1.resolve_neg().clone(), xP.resolve_neg().clone()
         vb = torch.empty((), dtype=torch.float64, device=x1.device)
         saved = torch.empty(plan.saved_doubles, dtype=torch.float64, device=x1.device)
         stream = torch.cuda.current_stream(x1.device).cuda_stream
@@ -41,13 +38,13 @@ class ExchangeVB(torch.autograd.Function):
         plan = ctx.plan
         d1, dP = (torch.empty((plan.natoms, plan.ndim), dtype=torch.float64, device=saved.device) for _ in range(2))
         stream = torch.cuda.current_stream(saved.device).cuda_stream
-        # the product with g stays a torch operation where it is to be differentiated itself, and where g is many
-        # gradients at once (is_grads_batched), which have no memory to read
+        # the product with g stays a torch operation where it is to be differentiated itself, and where g's values are
+        # not in memory as they are: lazily negated, zeros without memory, or many gradients at once
+        # (is_grads_batched)
         scale = None
-        if not torch.is_grad_enabled():
-            g = _in_memory(g)
+        if not (torch.is_grad_enabled() or g.is_neg()):
             try:
-                scale = g.data_ptr()
+                scale = g.data_ptr() or None
             except RuntimeError:
                 pass
         plan.backward_saved(saved.data_ptr(), scale, d1.data_ptr(), dP.data_ptr(), stream)
