@@ -184,11 +184,9 @@ int pimdb_device_info(int* compute_units, long long* lds_bytes);
 int pimdb_math_probe(int fn, const double* x, double* y, long long n);
 /* For tests of the recovery from a wait between workgroups that ran out (the
  * exchange recursions' blocks wait for each other, a few seconds at most):
- * leave the object as such a kernel would and return what its call would,
+ * leaves the context as such a kernel would and returns what its call would,
  * PIMDB_E_HIP. */
 int pimdb_test_lost_wait(pimdb_ctx* ctx);
-int pimdb_xplan_test_lost_wait(struct pimdb_xplan* plan);
-int pimdb_batch_test_lost_wait(struct pimdb_batch* batch);
 
 /* ---------------------------------------------------------------------- */
 /* Exchange on caller-provided device arrays (the autograd harness).       */
@@ -218,6 +216,7 @@ int pimdb_xplan_forward_saved(pimdb_xplan* plan, const double* x1, long long s1n
                               long long sPn, long long sPd, double* VB, double* saved, void* stream);
 int pimdb_xplan_backward_saved(pimdb_xplan* plan, const double* saved, const double* scale, double* d1, double* dP,
                                void* stream);
+int pimdb_xplan_test_lost_wait(pimdb_xplan* plan);   /* as pimdb_test_lost_wait */
 
 /* pimdb_xplan_create + pimdb_xplan_forward (VB only) + pimdb_xplan_vb_grad in
  * one call that allocates nothing: the same kernels, with their workspace
@@ -300,6 +299,7 @@ int pimdb_batch_time_step(pimdb_batch* batch, int reps, double* ms_step);
  * forces) or 3 (O-steps, kicks and drift) for every replica; the state is
  * saved before and restored after. */
 int pimdb_batch_time_phase(pimdb_batch* batch, int phase, int reps, double* ms);
+int pimdb_batch_test_lost_wait(pimdb_batch* batch);   /* as pimdb_test_lost_wait */
 
 #ifdef __cplusplus
 }
